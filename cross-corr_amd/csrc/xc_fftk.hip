@@ -230,29 +230,68 @@ __device__ __forceinline__ void regs_sync() {
         wave_sync();
 }
 
-// Pass roots of fft_regs<LOGP> at lane position i: w[j] = exp(-2 pi i k / (8p)), k = i mod p,
-// for the j-th twiddled pass (p = 2^(LOGR0 + 3j)).  Kernels load them once, before their
-// first transform: a table read inside a pass would wait on memory after every LDS exchange.
+// Passes of fft_regs: radix 8 (no twiddles), twiddled radix-8 passes, and for log2 P mod 3 = 1
+// or 2 a last twiddled pass of radix 2 or 4.  The short radix stands last and not first because
+// a twiddled radix-2 or 4 pass multiplies 4 or 6 of a thread's 8 values where a radix-8 pass
+// multiplies 7 and forms 6 powers: per 8 points 92 FP64 instructions against 124 at 16 points,
+// 196 against 232 at 128, 312 against 340 at 1024 (234 against 248 at 256).
 template <int LOGP>
 struct regs_roots {
     static constexpr int REM = LOGP % 3;
-    static constexpr int LOGR0 = REM == 0 ? 3 : REM;  // log2 of the first (untwiddled) radix
-    static constexpr int N = (LOGP - LOGR0) / 3;     // twiddled radix-8 passes
+    static constexpr int N8 = LOGP / 3 - 1;  // twiddled radix-8 passes
+    static constexpr int N = N8 + (REM ? 1 : 0);
     double2 w[N];
 };
+// Pass roots at lane position i: w[j] = exp(-2 pi i k / (8p)), k = i mod p, p = 8^(j+1) for the
+// twiddled radix-8 passes, exp(-2 pi i i / P) for a last radix-2 or 4 pass.  Kernels load them
+// once, before their first transform: a table read inside a pass would wait on memory after
+// every LDS exchange.
 template <int LOGP>
 __device__ __forceinline__ regs_roots<LOGP> load_roots(int i, const double2* __restrict__ tw) {
+    using RR = regs_roots<LOGP>;
     regs_roots<LOGP> rr;
 #pragma unroll
-    for (int j = 0; j < regs_roots<LOGP>::N; ++j) {
-        const int logpp = regs_roots<LOGP>::LOGR0 + 3 * j;
+    for (int j = 0; j < RR::N8; ++j) {
+        const int logpp = 3 + 3 * j;
         rr.w[j] = tw[(i & ((1 << logpp) - 1)) << (kLogMaxP - logpp - 3)];
     }
+    if constexpr (RR::REM != 0) rr.w[RR::N8] = tw[i << (kLogMaxP - LOGP)];
     return rr;
 }
 
-// Radix-8 passes of fft_regs from p = 2^LOGPP on: middle passes through LDS, the last one
-// (p = P/8, k = i) leaves its outputs i + (P/8) r in registers.
+__device__ __forceinline__ double2 csqr(double2 a) {
+    return make_double2(a.x * a.x - a.y * a.y, (a.x + a.x) * a.y);
+}
+// a * exp(-2 pi i m / 8), m = 1, 2, 3
+template <int M>
+__device__ __forceinline__ double2 rot8(double2 a) {
+    constexpr double c = 0.70710678118654752440;  // sqrt(1/2)
+    if constexpr (M == 0) return a;
+    else if constexpr (M == 1) return make_double2(c * (a.x + a.y), c * (a.y - a.x));
+    else if constexpr (M == 2) return mul_mi(a);
+    else return make_double2(c * (a.y - a.x), -c * (a.x + a.y));
+}
+
+// The first pass's DFT of 8 values whose upper four are zero (a zero-padded input): 40 FP64
+// instructions against 56.
+__device__ __forceinline__ void dft8_half(double2 (&u)[8]) {
+    const double2 a0 = u[0], a1 = u[2], b0 = u[1], b1 = u[3];
+    const double2 ja = mul_mi(a1), jb = mul_mi(b1);
+    const double2 e0 = cadd(a0, a1), e1 = cadd(a0, ja), e2 = csub(a0, a1), e3 = csub(a0, ja);
+    const double2 o0 = cadd(b0, b1), o1 = rot8<1>(cadd(b0, jb)), o2 = mul_mi(csub(b0, b1)),
+                  o3 = rot8<3>(csub(b0, jb));
+    u[0] = cadd(e0, o0);
+    u[4] = csub(e0, o0);
+    u[1] = cadd(e1, o1);
+    u[5] = csub(e1, o1);
+    u[2] = cadd(e2, o2);
+    u[6] = csub(e2, o2);
+    u[3] = cadd(e3, o3);
+    u[7] = csub(e3, o3);
+}
+
+// Twiddled passes of fft_regs from p = 2^LOGPP on: middle passes through LDS, the last one
+// leaves its outputs i + (P/8) r in registers.
 template <int LOGP, int LOGPP>
 __device__ __forceinline__ void fft_regs_passes(double2 (&u)[8], double2* wb, int tl, int i,
                                                 const regs_roots<LOGP>& rr) {
@@ -268,59 +307,79 @@ __device__ __forceinline__ void fft_regs_passes(double2 (&u)[8], double2* wb, in
 #pragma unroll
         for (int r = 0; r < 8; ++r) u[r] = wb[at<LOGP>(tl, i + Q * r)];
     }
-    const int k = i & ((1 << LOGPP) - 1);
     // The root passes through an empty asm so that its powers are formed here, in this pass:
     // otherwise the compiler hoists the power chains of every pass (and keeps them for a second
     // transform with the same roots), which costs tens of VGPRs.
-    double2 w1 = rr.w[(LOGPP - regs_roots<LOGP>::LOGR0) / 3];
+    double2 w1 = rr.w[LOGPP / 3 - 1];
     asm volatile("" : "+v"(w1.x), "+v"(w1.y));
-    double2 w = w1;
+    if constexpr (LOGP - LOGPP == 1) {  // radix 2: butterfly i + Q m takes u[m], u[m + 4]
+        u[4] = cmul(u[4], w1);
+        u[5] = cmul(u[5], rot8<1>(w1));
+        u[6] = cmul(u[6], mul_mi(w1));
+        u[7] = cmul(u[7], rot8<3>(w1));
 #pragma unroll
-    for (int r = 1; r < 8; ++r) {
-        u[r] = cmul(u[r], w);
-        if (r + 1 < 8) w = cmul(w, w1);
-    }
-    dft<8>(u);
-    regs_sync<regs_of<LOGP>::BLOCK>();
-    if constexpr (LOGPP + 3 < LOGP) {
-#pragma unroll
-        for (int r = 0; r < 8; ++r) wb[at<LOGP>(tl, ((i - k) << 3) + k + (r << LOGPP))] = u[r];
+        for (int m = 0; m < 4; ++m) dft2(u[m], u[m + 4]);
         regs_sync<regs_of<LOGP>::BLOCK>();
-        fft_regs_passes<LOGP, LOGPP + 3>(u, wb, tl, i, rr);
+    } else if constexpr (LOGP - LOGPP == 2) {  // radix 4: butterfly i + Q m takes u[m + 2 r]
+#pragma unroll
+        for (int m = 0; m < 2; ++m) {
+            const double2 wm = m ? rot8<1>(w1) : w1;
+            const double2 w2 = csqr(wm);
+            u[m + 2] = cmul(u[m + 2], wm);
+            u[m + 4] = cmul(u[m + 4], w2);
+            u[m + 6] = cmul(u[m + 6], cmul(w2, wm));
+            dft4(u[m], u[m + 2], u[m + 4], u[m + 6]);
+        }
+        regs_sync<regs_of<LOGP>::BLOCK>();
+    } else {
+        // the powers as a tree: squares take 3 instructions and the chain is 3 long, not 6
+        u[1] = cmul(u[1], w1);
+        const double2 w2 = csqr(w1);
+        u[2] = cmul(u[2], w2);
+        const double2 w3 = cmul(w2, w1);
+        u[3] = cmul(u[3], w3);
+        const double2 w4 = csqr(w2);
+        u[4] = cmul(u[4], w4);
+        u[5] = cmul(u[5], cmul(w4, w1));
+        u[6] = cmul(u[6], csqr(w3));
+        u[7] = cmul(u[7], cmul(w4, w3));
+        dft<8>(u);
+        regs_sync<regs_of<LOGP>::BLOCK>();
+        if constexpr (LOGPP + 3 < LOGP) {
+            const int k = i & ((1 << LOGPP) - 1);
+#pragma unroll
+            for (int r = 0; r < 8; ++r) wb[at<LOGP>(tl, ((i - k) << 3) + k + (r << LOGPP))] = u[r];
+            regs_sync<regs_of<LOGP>::BLOCK>();
+            fft_regs_passes<LOGP, LOGPP + 3>(u, wb, tl, i, rr);
+        }
     }
 }
 
 // FFTs entered and left in registers, for P = 2^LOGP of 16..2048 points (regs_of).  Thread
 // (tl, i) of the owning wave (up to 512 points) or block (1024, 2048) -- tl = id / Q,
 // i = id mod Q, Q = P/8 -- holds elements i + Q s (s = 0..7) of its transform tl on entry, and
-// the transform's outputs at the same positions on return.  The first pass (radix R0 = 8, 2
-// or 4 as log2 P mod 3 is 0, 1, 2; 8/R0 butterflies per thread, no twiddles) reads registers
-// only and the last radix-8 pass writes registers only, so a kernel that moves those positions
-// to and from HBM needs LDS only for the exchanges between passes (one up to 64 points, two up
-// to 512, three for 1024 and 2048).  wb is the owner's first transform slot; transform tl lives
-// at wb + at<LOGP>(tl, .).  rr holds the pass roots of this thread (load_roots<LOGP>(i, table)).
-// A block-owned transform synchronises the block: every thread of it must call.  (tl, i) are
-// passed in (regs_pos) so that a kernel calling twice can keep the compiler from holding the
-// first call's LDS addresses in registers for the second.
-template <int LOGP>
+// the transform's outputs at the same positions on return.  The first pass (radix 8, butterfly
+// i, no twiddles) reads registers only and the last pass writes registers only, so a kernel
+// that moves those positions to and from HBM needs LDS only for the exchanges between passes
+// (one up to 64 points, two up to 512, three for 1024 and 2048).  HALF: the upper half of the
+// input is zero (u[4..7] are not read), as in every zero-padded forward transform.  wb is the
+// owner's first transform slot; transform tl lives at wb + at<LOGP>(tl, .).  rr holds the pass
+// roots of this thread (load_roots<LOGP>(i, table)).  A block-owned transform synchronises the
+// block: every thread of it must call.  (tl, i) are passed in (regs_pos) so that a kernel
+// calling twice can keep the compiler from holding the first call's LDS addresses in registers
+// for the second.
+template <int LOGP, bool HALF = false>
 __device__ __forceinline__ void fft_regs(double2 (&u)[8], double2* wb, const regs_roots<LOGP>& rr, int tl,
                                          int i) {
     static_assert(LOGP >= 4 && regs_of<LOGP>::ON, "register FFTs take 16..2048 points");
-    constexpr int Q = 1 << (LOGP - 3);
-    constexpr int LOGR0 = regs_roots<LOGP>::LOGR0;
-    constexpr int R0 = 1 << LOGR0;
-    // first pass (p = 1): butterfly b = i + Q m takes elements b + (P/R0) r = u[m + (8/R0) r]
+    if constexpr (HALF)
+        dft8_half(u);
+    else
+        dft<8>(u);
 #pragma unroll
-    for (int m = 0; m < 8 / R0; ++m) {
-        double2 v[R0];
-#pragma unroll
-        for (int r = 0; r < R0; ++r) v[r] = u[m + (8 / R0) * r];
-        dft<R0>(v);
-#pragma unroll
-        for (int r = 0; r < R0; ++r) wb[at<LOGP>(tl, (i + Q * m) * R0 + r)] = v[r];
-    }
+    for (int r = 0; r < 8; ++r) wb[at<LOGP>(tl, i * 8 + r)] = u[r];
     regs_sync<regs_of<LOGP>::BLOCK>();
-    fft_regs_passes<LOGP, LOGR0>(u, wb, tl, i, rr);
+    fft_regs_passes<LOGP, 3>(u, wb, tl, i, rr);
 }
 
 // Position of this thread in the register FFTs of its block: transform t, the first transform
@@ -436,9 +495,9 @@ __global__ __launch_bounds__(NT) void rows_fwd_regs_kernel(const Tin* __restrict
     };
     // Branch-free loads from clamped (in-bounds) addresses; out-of-range positions are zeroed
     // when the values are used.
-    auto fetch = [&](const where& w, Tin (&va)[8], Tin (&vb)[8]) {
+    auto fetch = [&](const where& w, Tin (&va)[4], Tin (&vb)[4]) {
 #pragma unroll
-        for (int r = 0; r < 8; ++r) {
+        for (int r = 0; r < 4; ++r) {  // W <= Pc / 2: the upper half of a row is padding
             const uint32_t c = i + Q * r, cc = c < w.Wm ? c : w.Wm - 1;
             va[r] = w.xa[cc];
             vb[r] = w.xb[cc];
@@ -447,14 +506,14 @@ __global__ __launch_bounds__(NT) void rows_fwd_regs_kernel(const Tin* __restrict
     uint32_t it = x * per + kb;
     if (it >= end) return;
     where cur = locate(it);
-    Tin va[8], vb[8];
+    Tin va[4], vb[4];
     fetch(cur, va, vb);
     while (true) {
         const uint32_t nxt = it + bpx;
         const bool more = nxt < end;
         double2 u[8];
 #pragma unroll
-        for (int r = 0; r < 8; ++r) {
+        for (int r = 0; r < 4; ++r) {
             const bool in = i + Q * r < (int)cur.Wm;
             u[r] = make_double2(cur.oka && in ? (double)va[r] : 0.0, cur.okb && in ? (double)vb[r] : 0.0);
         }
@@ -464,7 +523,7 @@ __global__ __launch_bounds__(NT) void rows_fwd_regs_kernel(const Tin* __restrict
             fetch(nw, va, vb);
         }
         if (cur.r0 < cur.Hm) {  // block-uniform: a row group beyond a smaller matrix is skipped
-            fft_regs<LOGPC>(u, buf + at<LOGPC>(t0, 0), rr, t - t0, i);
+            fft_regs<LOGPC, true>(u, buf + at<LOGPC>(t0, 0), rr, t - t0, i);
 #pragma unroll
             for (int r = 0; r < 8; ++r) buf[at<LOGPC>(t, i + Q * r)] = u[r];
             __syncthreads();
@@ -610,7 +669,7 @@ __global__ __launch_bounds__(cols_threads(LOGPR)) void cols_kernel(const double2
         const regs_roots<LOGPR> rr = load_roots<LOGPR>(i, tw);
         double2 u[8], lh[8];
 #pragma unroll
-        for (int r = 0; r < 8; ++r) {
+        for (int r = 0; r < 4; ++r) {  // Hq <= Pr / 2: the upper half of a column is padding
             const uint32_t rho = i + Q * r;
             u[r] = make_double2(0.0, 0.0);
             if (ok && rho < Hq) u[r] = Sm[(size_t)k * H + rho];
@@ -623,7 +682,7 @@ __global__ __launch_bounds__(cols_threads(LOGPR)) void cols_kernel(const double2
             lh[r] = make_double2(0.0, 0.0);
             if (MODE == 1 && ok) lh[r] = lk[i + Q * r];
         }
-        fft_regs<LOGPR>(u, wb, rr, ps.t - t0, i);
+        fft_regs<LOGPR, true>(u, wb, rr, ps.t - t0, i);
         if constexpr (MODE == 0) {
             if (ok) {
 #pragma unroll
@@ -954,9 +1013,9 @@ __global__ __launch_bounds__(rows3<LOGN>::NT) void rows_fwd3_kernel(
         return w;
     };
     // element n = i + Q r of sub-sequence m is column 3n + m; loads from clamped addresses
-    auto fetch = [&](const where& w, Tin (&va)[8], Tin (&vb)[8]) {
+    auto fetch = [&](const where& w, Tin (&va)[4], Tin (&vb)[4]) {
 #pragma unroll
-        for (int r = 0; r < 8; ++r) {
+        for (int r = 0; r < 4; ++r) {  // W <= P / 2: the upper half of a sub-sequence is padding
             const uint32_t c = 3u * (uint32_t)(i + Q * r) + (uint32_t)m, cc = c < w.Wm ? c : w.Wm - 1;
             va[r] = w.xa[cc];
             vb[r] = w.xb[cc];
@@ -965,14 +1024,14 @@ __global__ __launch_bounds__(rows3<LOGN>::NT) void rows_fwd3_kernel(
     uint32_t it = x * per + kb;
     if (it >= end) return;
     where cur = locate(it);
-    Tin va[8], vb[8];
+    Tin va[4], vb[4];
     fetch(cur, va, vb);
     while (true) {
         const uint32_t nxt = it + bpx;
         const bool more = nxt < end;
         double2 u[8];
 #pragma unroll
-        for (int r = 0; r < 8; ++r) {
+        for (int r = 0; r < 4; ++r) {
             const bool in = 3u * (uint32_t)(i + Q * r) + (uint32_t)m < cur.Wm;
             u[r] = make_double2(cur.oka && in ? (double)va[r] : 0.0, cur.okb && in ? (double)vb[r] : 0.0);
         }
@@ -982,7 +1041,7 @@ __global__ __launch_bounds__(rows3<LOGN>::NT) void rows_fwd3_kernel(
             fetch(nw, va, vb);
         }
         if (cur.r0 < cur.Hm) {  // block-uniform: a row group beyond a smaller matrix is skipped
-            fft_regs<LOGN>(u, buf + at<LOGN>(ps.t0, 0), rr, sub - ps.t0, i);
+            fft_regs<LOGN, true>(u, buf + at<LOGN>(ps.t0, 0), rr, sub - ps.t0, i);
 #pragma unroll
             for (int r = 0; r < 8; ++r) buf[at<LOGN>(sub, i + Q * r)] = u[r];
             __syncthreads();
