@@ -35,24 +35,13 @@
 #include <type_traits>
 #include <vector>
 
+#include "xc_fftk_core.hpp"
 #include "xc_methods.hpp"
 
 namespace xc {
 namespace {
 
-constexpr int kFT = 256;              // threads per block: slab kernels, block-owned column FFTs
-constexpr int kLogMaxP = 12;          // longest transform: 4096 (the twiddle table's length)
-constexpr int kSlab = 1 << kLogMaxP;  // twiddle table entries
-
-// LDS slot of element j of transform t (length P = 2^LOGP): one pad slot per 8 values, and a
-// transform stride of 9P/8 + 1 slots, so that lanes touching the same j of consecutive
-// transforms, or j = 8i, hit different banks.  With P a compile-time constant the pad and
-// stride arithmetic folds into immediate LDS offsets.
-template <int LOGP>
-__device__ __forceinline__ int at(int t, int j) {
-    constexpr int S = (1 << LOGP) + (1 << LOGP) / 8 + 1;
-    return t * S + j + (j >> 3);
-}
+constexpr int kFT = 256;  // threads per block: slab kernels, block-owned column FFTs
 
 // Slab (values per block) of a transform length: 2^11 values, or one transform of 4096.
 // Lengths of up to 2048 points are transformed in registers (fft_regs), 4096 in a slab.
@@ -60,62 +49,6 @@ template <int LOGP>
 struct slab_of {
     static constexpr int LOGS = LOGP <= 11 ? 11 : LOGP;
 };
-__device__ __forceinline__ double2 cmul(double2 a, double2 b) {
-    return make_double2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
-}
-__device__ __forceinline__ double2 cconj(double2 a) { return make_double2(a.x, -a.y); }
-__device__ __forceinline__ double2 cadd(double2 a, double2 b) { return make_double2(a.x + b.x, a.y + b.y); }
-__device__ __forceinline__ double2 csub(double2 a, double2 b) { return make_double2(a.x - b.x, a.y - b.y); }
-__device__ __forceinline__ double2 mul_mi(double2 a) { return make_double2(a.y, -a.x); }  // (-i) * a
-
-// In-register forward DFT of R points: X[k] = sum_j u[j] exp(-2 pi i jk / R).
-__device__ __forceinline__ void dft2(double2& a, double2& b) {
-    const double2 t = a;
-    a = cadd(t, b);
-    b = csub(t, b);
-}
-__device__ __forceinline__ void dft4(double2& u0, double2& u1, double2& u2, double2& u3) {
-    const double2 t0 = cadd(u0, u2), t1 = csub(u0, u2), t2 = cadd(u1, u3), t3 = mul_mi(csub(u1, u3));
-    u0 = cadd(t0, t2);
-    u2 = csub(t0, t2);
-    u1 = cadd(t1, t3);
-    u3 = csub(t1, t3);
-}
-template <int R>
-__device__ __forceinline__ void dft(double2 (&u)[R]) {
-    if constexpr (R == 2) {
-        dft2(u[0], u[1]);
-    } else if constexpr (R == 4) {
-        dft4(u[0], u[1], u[2], u[3]);
-    } else {
-        static_assert(R == 8, "radix");
-        constexpr double c = 0.70710678118654752440;  // sqrt(1/2)
-        double2 e0 = u[0], e1 = u[2], e2 = u[4], e3 = u[6];
-        double2 o0 = u[1], o1 = u[3], o2 = u[5], o3 = u[7];
-        dft4(e0, e1, e2, e3);
-        dft4(o0, o1, o2, o3);
-        // o_k *= exp(-2 pi i k / 8)
-        o1 = make_double2(c * (o1.x + o1.y), c * (o1.y - o1.x));
-        o2 = mul_mi(o2);
-        o3 = make_double2(c * (o3.y - o3.x), -c * (o3.x + o3.y));
-        u[0] = cadd(e0, o0);
-        u[4] = csub(e0, o0);
-        u[1] = cadd(e1, o1);
-        u[5] = csub(e1, o1);
-        u[2] = cadd(e2, o2);
-        u[6] = csub(e2, o2);
-        u[3] = cadd(e3, o3);
-        u[7] = csub(e3, o3);
-    }
-}
-
-// Barrier between the LDS phases of a wave-owned transform: every value a lane reads was
-// written by its own wave, so ordering the wave's LDS accesses is enough.
-__device__ __forceinline__ void wave_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-}
 
 // First radix of a length-2^LOGP transform (8, 2 or 4 as LOGP mod 3 is 0, 1, 2; it takes no
 // twiddles) and the number of twiddled radix-8 passes after it.
@@ -214,192 +147,6 @@ __device__ __forceinline__ void fft_slab(double2* buf, int T, const slab_roots<L
     radix8_passes<LOGP, LOGR0>(buf, T, sr);
 }
 
-// Transforms of up to 2048 points run in registers: P/8 threads hold one transform, 8 values
-// each.  Up to 512 points a transform lives in one wave (BLOCK false: the wave holds 512/P of
-// them); 1024 and 2048 points span two and four waves of the block.
-template <int LOGP>
-struct regs_of {
-    static constexpr bool ON = LOGP <= 11;
-    static constexpr bool BLOCK = LOGP > 9;
-};
-template <bool BLOCK>
-__device__ __forceinline__ void regs_sync() {
-    if constexpr (BLOCK)
-        __syncthreads();
-    else
-        wave_sync();
-}
-
-// Passes of fft_regs: radix 8 (no twiddles), twiddled radix-8 passes, and for log2 P mod 3 = 1
-// or 2 a last twiddled pass of radix 2 or 4.  The short radix stands last and not first because
-// a twiddled radix-2 or 4 pass multiplies 4 or 6 of a thread's 8 values where a radix-8 pass
-// multiplies 7 and forms 6 powers: per 8 points 92 FP64 instructions against 124 at 16 points,
-// 196 against 232 at 128, 312 against 340 at 1024 (234 against 248 at 256).
-template <int LOGP>
-struct regs_roots {
-    static constexpr int REM = LOGP % 3;
-    static constexpr int N8 = LOGP / 3 - 1;  // twiddled radix-8 passes
-    static constexpr int N = N8 + (REM ? 1 : 0);
-    double2 w[N];
-};
-// Pass roots at lane position i: w[j] = exp(-2 pi i k / (8p)), k = i mod p, p = 8^(j+1) for the
-// twiddled radix-8 passes, exp(-2 pi i i / P) for a last radix-2 or 4 pass.  Kernels load them
-// once, before their first transform: a table read inside a pass would wait on memory after
-// every LDS exchange.
-template <int LOGP>
-__device__ __forceinline__ regs_roots<LOGP> load_roots(int i, const double2* __restrict__ tw) {
-    using RR = regs_roots<LOGP>;
-    regs_roots<LOGP> rr;
-#pragma unroll
-    for (int j = 0; j < RR::N8; ++j) {
-        const int logpp = 3 + 3 * j;
-        rr.w[j] = tw[(i & ((1 << logpp) - 1)) << (kLogMaxP - logpp - 3)];
-    }
-    if constexpr (RR::REM != 0) rr.w[RR::N8] = tw[i << (kLogMaxP - LOGP)];
-    return rr;
-}
-
-__device__ __forceinline__ double2 csqr(double2 a) {
-    return make_double2(a.x * a.x - a.y * a.y, (a.x + a.x) * a.y);
-}
-// a * exp(-2 pi i m / 8), m = 1, 2, 3
-template <int M>
-__device__ __forceinline__ double2 rot8(double2 a) {
-    constexpr double c = 0.70710678118654752440;  // sqrt(1/2)
-    if constexpr (M == 0) return a;
-    else if constexpr (M == 1) return make_double2(c * (a.x + a.y), c * (a.y - a.x));
-    else if constexpr (M == 2) return mul_mi(a);
-    else return make_double2(c * (a.y - a.x), -c * (a.x + a.y));
-}
-
-// The first pass's DFT of 8 values whose upper four are zero (a zero-padded input): 40 FP64
-// instructions against 56.
-__device__ __forceinline__ void dft8_half(double2 (&u)[8]) {
-    const double2 a0 = u[0], a1 = u[2], b0 = u[1], b1 = u[3];
-    const double2 ja = mul_mi(a1), jb = mul_mi(b1);
-    const double2 e0 = cadd(a0, a1), e1 = cadd(a0, ja), e2 = csub(a0, a1), e3 = csub(a0, ja);
-    const double2 o0 = cadd(b0, b1), o1 = rot8<1>(cadd(b0, jb)), o2 = mul_mi(csub(b0, b1)),
-                  o3 = rot8<3>(csub(b0, jb));
-    u[0] = cadd(e0, o0);
-    u[4] = csub(e0, o0);
-    u[1] = cadd(e1, o1);
-    u[5] = csub(e1, o1);
-    u[2] = cadd(e2, o2);
-    u[6] = csub(e2, o2);
-    u[3] = cadd(e3, o3);
-    u[7] = csub(e3, o3);
-}
-
-// Twiddled passes of fft_regs from p = 2^LOGPP on: middle passes through LDS, the last one
-// leaves its outputs i + (P/8) r in registers.
-template <int LOGP, int LOGPP>
-__device__ __forceinline__ void fft_regs_passes(double2 (&u)[8], double2* wb, int tl, int i,
-                                                const regs_roots<LOGP>& rr) {
-    constexpr int Q = 1 << (LOGP - 3);
-    if constexpr (Q >= 8) {
-        // at(tl, i + Q r) = at(tl, i) + r (Q + Q/8) when 8 divides Q: one address register and
-        // constant offsets (the compiler does not split the shift of the sum by itself, and
-        // keeps eight addresses live through both transforms otherwise).
-        const int a = at<LOGP>(tl, i);
-#pragma unroll
-        for (int r = 0; r < 8; ++r) u[r] = wb[a + r * (Q + (Q >> 3))];
-    } else {
-#pragma unroll
-        for (int r = 0; r < 8; ++r) u[r] = wb[at<LOGP>(tl, i + Q * r)];
-    }
-    // The root passes through an empty asm so that its powers are formed here, in this pass:
-    // otherwise the compiler hoists the power chains of every pass (and keeps them for a second
-    // transform with the same roots), which costs tens of VGPRs.
-    double2 w1 = rr.w[LOGPP / 3 - 1];
-    asm volatile("" : "+v"(w1.x), "+v"(w1.y));
-    if constexpr (LOGP - LOGPP == 1) {  // radix 2: butterfly i + Q m takes u[m], u[m + 4]
-        u[4] = cmul(u[4], w1);
-        u[5] = cmul(u[5], rot8<1>(w1));
-        u[6] = cmul(u[6], mul_mi(w1));
-        u[7] = cmul(u[7], rot8<3>(w1));
-#pragma unroll
-        for (int m = 0; m < 4; ++m) dft2(u[m], u[m + 4]);
-        regs_sync<regs_of<LOGP>::BLOCK>();
-    } else if constexpr (LOGP - LOGPP == 2) {  // radix 4: butterfly i + Q m takes u[m + 2 r]
-#pragma unroll
-        for (int m = 0; m < 2; ++m) {
-            const double2 wm = m ? rot8<1>(w1) : w1;
-            const double2 w2 = csqr(wm);
-            u[m + 2] = cmul(u[m + 2], wm);
-            u[m + 4] = cmul(u[m + 4], w2);
-            u[m + 6] = cmul(u[m + 6], cmul(w2, wm));
-            dft4(u[m], u[m + 2], u[m + 4], u[m + 6]);
-        }
-        regs_sync<regs_of<LOGP>::BLOCK>();
-    } else {
-        // the powers as a tree: squares take 3 instructions and the chain is 3 long, not 6
-        u[1] = cmul(u[1], w1);
-        const double2 w2 = csqr(w1);
-        u[2] = cmul(u[2], w2);
-        const double2 w3 = cmul(w2, w1);
-        u[3] = cmul(u[3], w3);
-        const double2 w4 = csqr(w2);
-        u[4] = cmul(u[4], w4);
-        u[5] = cmul(u[5], cmul(w4, w1));
-        u[6] = cmul(u[6], csqr(w3));
-        u[7] = cmul(u[7], cmul(w4, w3));
-        dft<8>(u);
-        regs_sync<regs_of<LOGP>::BLOCK>();
-        if constexpr (LOGPP + 3 < LOGP) {
-            const int k = i & ((1 << LOGPP) - 1);
-#pragma unroll
-            for (int r = 0; r < 8; ++r) wb[at<LOGP>(tl, ((i - k) << 3) + k + (r << LOGPP))] = u[r];
-            regs_sync<regs_of<LOGP>::BLOCK>();
-            fft_regs_passes<LOGP, LOGPP + 3>(u, wb, tl, i, rr);
-        }
-    }
-}
-
-// FFTs entered and left in registers, for P = 2^LOGP of 16..2048 points (regs_of).  Thread
-// (tl, i) of the owning wave (up to 512 points) or block (1024, 2048) -- tl = id / Q,
-// i = id mod Q, Q = P/8 -- holds elements i + Q s (s = 0..7) of its transform tl on entry, and
-// the transform's outputs at the same positions on return.  The first pass (radix 8, butterfly
-// i, no twiddles) reads registers only and the last pass writes registers only, so a kernel
-// that moves those positions to and from HBM needs LDS only for the exchanges between passes
-// (one up to 64 points, two up to 512, three for 1024 and 2048).  HALF: the upper half of the
-// input is zero (u[4..7] are not read), as in every zero-padded forward transform.  wb is the
-// owner's first transform slot; transform tl lives at wb + at<LOGP>(tl, .).  rr holds the pass
-// roots of this thread (load_roots<LOGP>(i, table)).  A block-owned transform synchronises the
-// block: every thread of it must call.  (tl, i) are passed in (regs_pos) so that a kernel
-// calling twice can keep the compiler from holding the first call's LDS addresses in registers
-// for the second.
-template <int LOGP, bool HALF = false>
-__device__ __forceinline__ void fft_regs(double2 (&u)[8], double2* wb, const regs_roots<LOGP>& rr, int tl,
-                                         int i) {
-    static_assert(LOGP >= 4 && regs_of<LOGP>::ON, "register FFTs take 16..2048 points");
-    if constexpr (HALF)
-        dft8_half(u);
-    else
-        dft<8>(u);
-#pragma unroll
-    for (int r = 0; r < 8; ++r) wb[at<LOGP>(tl, i * 8 + r)] = u[r];
-    regs_sync<regs_of<LOGP>::BLOCK>();
-    fft_regs_passes<LOGP, 3>(u, wb, tl, i, rr);
-}
-
-// Position of this thread in the register FFTs of its block: transform t, the first transform
-// t0 of the owning wave (0 for block-owned transforms), and i within the transform.
-template <int LOGP>
-struct regs_pos {
-    int t0, t, i;
-    __device__ __forceinline__ regs_pos() {
-        constexpr int Q = 1 << (LOGP - 3);
-        if constexpr (regs_of<LOGP>::BLOCK) {
-            t0 = 0;
-            t = (int)threadIdx.x >> (LOGP - 3);
-        } else {
-            t0 = (int)(threadIdx.x >> 6) << (9 - LOGP);
-            t = t0 + ((int)(threadIdx.x & 63) >> (LOGP - 3));
-        }
-        i = (int)threadIdx.x & (Q - 1);
-    }
-};
-
 // Threads per block of the row kernels (INV: rows_inv): 256, or more for register transforms
 // of 1024 and 2048 points so that a block holds four transforms (8 rows: a column's piece of
 // S or Z is a whole 128-byte line) -- except rows_inv at 2048 points, where two transforms per
@@ -457,7 +204,7 @@ __global__ __launch_bounds__(NT) void rows_fwd_regs_kernel(const Tin* __restrict
     static_assert(regs_of<LOGPC>::ON, "register transforms only");
     constexpr int Q = 1 << (LOGPC - 3);
     extern __shared__ double2 buf[];
-    const regs_pos<LOGPC> ps;
+    const regs_pos<LOGPC> ps((int)threadIdx.x);
     const int t0 = ps.t0, t = ps.t, i = ps.i;
     const regs_roots<LOGPC> rr = load_roots<LOGPC>(i, tw);
     // this block's items: x * per + k + j * bpx, j = 0, 1, ... below min((x + 1) * per, items)
@@ -661,7 +408,7 @@ __global__ __launch_bounds__(cols_threads(LOGPR)) void cols_kernel(const double2
         // C = 8 * threads / Pr: the columns go from HBM to HBM through fft_regs; the product with
         // conj(Lhat) happens in registers between the two FFTs.
         constexpr int Q = 1 << (LOGPR - 3);
-        const regs_pos<LOGPR> ps;
+        const regs_pos<LOGPR> ps((int)threadIdx.x);
         const int t0 = ps.t0, i = ps.i;
         const uint32_t k = k0 + ps.t;
         const bool ok = k < Kc;
@@ -807,7 +554,7 @@ __global__ __launch_bounds__(NT) void rows_inv_kernel(const double2* __restrict_
     regs_roots<LOGPC> rr{};
     slab_roots<LOGPC> sr{};
     if constexpr (regs_of<LOGPC>::ON)
-        rr = load_roots<LOGPC>((int)threadIdx.x & ((1 << (LOGPC - 3)) - 1), tw);
+        rr = load_roots<LOGPC>(regs_pos<LOGPC>((int)threadIdx.x).i, tw);
     else
         sr = load_slab_roots<LOGPC>(tw);
     // One thread per (column kk, transform t) loads the two rows' values A[kk], B[kk] (32
@@ -846,7 +593,7 @@ __global__ __launch_bounds__(NT) void rows_inv_kernel(const double2* __restrict_
         // T = 8 NT / Pc: the transforms (row pairs) go through fft_regs and are written from
         // registers: thread (t, i) holds circular columns c = i + Q r of rows rho0 + 2t, +1.
         constexpr int Q = 1 << (LOGPC - 3);
-        const regs_pos<LOGPC> ps;
+        const regs_pos<LOGPC> ps((int)threadIdx.x);
         const int t0 = ps.t0, t = ps.t, i = ps.i;
         double2 u[8];
 #pragma unroll
@@ -977,7 +724,7 @@ __global__ __launch_bounds__(rows3<LOGN>::NT) void rows_fwd3_kernel(
     constexpr int N = G::N, P = G::P, Q = G::Q, T = G::T;
     constexpr uint32_t Kc = P / 2 + 1;
     extern __shared__ double2 buf[];
-    const regs_pos<LOGN> ps;
+    const regs_pos<LOGN> ps((int)threadIdx.x);
     const int sub = ps.t, tt = sub / 3, m = sub - 3 * tt, i = ps.i;
     const regs_roots<LOGN> rr = load_roots<LOGN>(i, tw);
     const r3_roots<LOGN> w3 = load_r3_roots<LOGN>(tw3);
@@ -1106,7 +853,7 @@ __global__ __launch_bounds__(rows3<LOGN>::NT) void rows_inv3_kernel(
     const uint32_t z0 = g * (2 * T);
     if (z0 >= 2 * H) return;
     const double2* Zq = Z + (size_t)item * Kc * Ys;
-    const regs_pos<LOGN> ps;
+    const regs_pos<LOGN> ps((int)threadIdx.x);
     const int sub = ps.t, tt = sub / 3, m = sub - 3 * tt, i = ps.i;
     const regs_roots<LOGN> rr = load_roots<LOGN>(i, tw);
     const r3_roots<LOGN> w3 = load_r3_roots<LOGN>(tw3);
@@ -1296,8 +1043,12 @@ struct fftk_geom {
     uint32_t Pr, Pc, Kc;
     slab_shape v1, vc, v3;
     uint32_t g1, cg, g3;
+    // A pair's half spectrum fits one block (xc_fftk_small.hip): lengths 2^logPrs x 2^logPcs; the
+    // right spectra take S's place (column spectra of Pr values), Z and the left S are not used.
+    bool small;
+    int logPrs, logPcs;
     uint32_t Ys;  // column stride of Z: 2H (the 2H-1 circular rows of the result, z_row)
-    size_t s_bytes, col_bytes, z_bytes;
+    size_t s_bytes, sl_bytes, col_bytes, z_bytes;  // S per right and per left, Lhat per left, Z per pair
 };
 
 fftk_geom geom_of(uint32_t H, uint32_t W, bool pow2_rows = false) {
@@ -1330,6 +1081,15 @@ fftk_geom geom_of(uint32_t H, uint32_t W, bool pow2_rows = false) {
     g.s_bytes = sizeof(double2) * (size_t)g.Kc * H;
     g.col_bytes = sizeof(double2) * (size_t)g.Kc * g.Pr;
     g.z_bytes = sizeof(double2) * (size_t)g.Kc * g.Ys;
+    g.sl_bytes = g.s_bytes;
+    g.logPrs = std::max(5, g.logPr);
+    g.logPcs = std::max(5, ilog2_ceil(2 * W - 1));
+    g.small = fftk_small_fits(g.logPrs, g.logPcs);
+    if (g.small) {
+        g.col_bytes = sizeof(double2) * (size_t)((1u << g.logPcs) / 2 + 1) << g.logPrs;
+        g.s_bytes = g.col_bytes;
+        g.sl_bytes = g.z_bytes = 0;
+    }
     return g;
 }
 
@@ -1360,24 +1120,18 @@ uint32_t resident_grid(const void* kernel, int threads, uint32_t lds, uint32_t i
     return std::max<uint32_t>(g, 1);
 }
 
-// Launch, with the kernel's own start and end recorded under `name` while kernel timing is on.
-template <typename K, typename... Args>
-void launch_timed(const char* name, bool timing, K kernel, dim3 grid, dim3 block, uint32_t lds, hipStream_t s,
-                  Args... args) {
-    if (timing && timing_enabled()) {
-        hipEvent_t a = nullptr, b = nullptr;
-        timing_launch_events(name, &a, &b);
-        hipExtLaunchKernelGGL(kernel, grid, block, lds, s, a, b, 0, args...);
-    } else {
-        hipLaunchKernelGGL(kernel, grid, block, lds, s, args...);
-    }
-}
-
 template <typename Tio>
 void launch_job(const fftk_job& j, const Tio* L, const Tio* R, Tio* O, const fftk_ws& ws, hipStream_t s,
                 bool timing) {
     const uint32_t H = j.H, W = j.W;
     const fftk_geom g = geom_of(H, W, j.pow2_rows);
+    if (g.small) {
+        if constexpr (std::is_same<Tio, float>::value)
+            fftk_small_f32(j, g.logPrs, g.logPcs, L, R, O, ws, s, timing);
+        else
+            fftk_small_f64(j, g.logPrs, g.logPcs, L, R, O, ws, s, timing);
+        return;
+    }
     const double2* tw = twiddles();
     double2* SR = static_cast<double2*>(ws.sr);
     double2* SL = static_cast<double2*>(ws.sl);
@@ -1526,7 +1280,7 @@ struct noalloc_part {
 
 // Scratch bytes of a part with nl left and nr right spectra and `chunk` pairs of Z.
 size_t part_bytes(const fftk_geom& g, uint32_t nl, uint32_t nr, uint32_t chunk) {
-    return align256(g.s_bytes * nr) + align256(g.s_bytes * nl) + align256(g.col_bytes * nl) +
+    return align256(g.s_bytes * nr) + align256(g.sl_bytes * nl) + align256(g.col_bytes * nl) +
            align256(g.z_bytes * chunk);
 }
 
@@ -1586,7 +1340,7 @@ std::vector<noalloc_part> plan_noalloc(const family_args& a, const fftk_geom& g)
                 const uint32_t c = std::min(gl, a.n - l0);
                 // as many pairs per launch as the rest of the array holds (at least m: gl fits them)
                 const size_t rest = B - part_bytes(g, c, a.m, 0);
-                uint32_t chunk = (uint32_t)std::min<size_t>((size_t)c * a.m, rest / g.z_bytes);
+                uint32_t chunk = (uint32_t)std::min<size_t>((size_t)c * a.m, g.z_bytes ? rest / g.z_bytes : SIZE_MAX);
                 while (chunk > a.m && part_bytes(g, c, a.m, chunk) > B) --chunk;
                 parts.push_back({XC_N_TO_M, c, a.m, c * a.m, l0 * hw, 0, (size_t)l0 * a.m * out_elems, chunk});
             }
@@ -1624,7 +1378,7 @@ void run_fftk_noalloc_f32(const family_args& a, const float* L, const float* R, 
         ws.sr = q;
         q += align256(g.s_bytes * j.nr);
         ws.sl = q;
-        q += align256(g.s_bytes * j.nl);
+        q += align256(g.sl_bytes * j.nl);
         ws.lh = q;
         q += align256(g.col_bytes * j.nl);
         ws.z = q;
@@ -1634,6 +1388,8 @@ void run_fftk_noalloc_f32(const family_args& a, const float* L, const float* R, 
         launch_job<float>(j, L + p.loff, R + p.roff, O + p.ooff, ws, s, false);
     }
 }
+
+const double2* fftk_twiddles() { return twiddles(); }
 
 uint32_t fftk_col_len(uint32_t rows) {
     uint32_t p = 16;
@@ -1648,16 +1404,22 @@ uint32_t fftk_row_len(uint32_t cols) {
     return p;
 }
 
+std::pair<uint32_t, uint32_t> fftk_class(uint32_t rows, uint32_t cols) {
+    const fftk_geom g = geom_of(rows, cols);
+    if (g.small) return {1u << g.logPrs, 1u << g.logPcs};
+    return {g.Pr, g.Pc};
+}
+
 fftk_ws_sizes fftk_sizes(const fftk_job& j) {
     const fftk_geom g = geom_of(j.H, j.W, j.pow2_rows);
     fftk_ws_sizes z{};
     // Z is processed in chunks of pairs of at most ~2 GiB.
-    z.chunk = (uint32_t)std::max<size_t>(1, std::min<size_t>(j.pairs, (size_t(2) << 30) / g.z_bytes));
+    z.chunk = (uint32_t)std::max<size_t>(1, std::min<size_t>(j.pairs, (size_t(2) << 30) / std::max<size_t>(g.z_bytes, 1)));
     if (j.max_chunk) z.chunk = std::min(z.chunk, j.max_chunk);
     z.sr = std::max<size_t>(g.s_bytes * j.nr, 16);
-    z.sl = std::max<size_t>(g.s_bytes * j.nl, 16);
+    z.sl = std::max<size_t>(g.sl_bytes * j.nl, 16);
     z.lh = std::max<size_t>(g.col_bytes * j.nl, 16);
-    z.z = g.z_bytes * z.chunk;
+    z.z = std::max<size_t>(g.z_bytes * z.chunk, 16);
     return z;
 }
 

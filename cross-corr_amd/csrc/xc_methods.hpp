@@ -1,6 +1,7 @@
 // Method-level entry points behind the C ABI (one per algorithm family of the library).
 #pragma once
 
+#include <utility>
 #include <vector>
 
 #include "xc_internal.hpp"
@@ -98,8 +99,20 @@ fftk_ws_sizes fftk_sizes(const fftk_job& j);
 // 16); rows that, or 3 * 2^n (n = 4..9) when that is shorter.  Matrices of one job share them.
 uint32_t fftk_col_len(uint32_t rows);
 uint32_t fftk_row_len(uint32_t cols);
+// Matrices of equal fftk_class may share a job: the lengths above, or those of the one-block
+// kernels where they take the size (fftk_small_fits).
+std::pair<uint32_t, uint32_t> fftk_class(uint32_t rows, uint32_t cols);
 void fftk_prepare();  // device tables the kernels read (call before stream capture)
 void fftk_launch_f32(const fftk_job& j, const float* L, const float* R, float* O, const fftk_ws& ws, hipStream_t s);
+
+// One-block variant of a job (xc_fftk_small.hip): padded lengths 2^lr x 2^lc of at most 2^14
+// values.  ws.lh holds the left and ws.sr the right spectra, (2^lc / 2 + 1) 2^lr values each.
+constexpr int kSmallLog = 14;
+bool fftk_small_fits(int lr, int lc);
+void fftk_small_f32(const fftk_job& j, int lr, int lc, const float* L, const float* R, float* O, const fftk_ws& ws,
+                    hipStream_t s, bool timing);
+void fftk_small_f64(const fftk_job& j, int lr, int lc, const double* L, const double* R, double* O, const fftk_ws& ws,
+                    hipStream_t s, bool timing);
 
 // FFT method on the library's own FP64 FFT kernels (xc_fftk.hip): rows, cols <= 2048.
 // The own FFT without any allocation: scratch memory is a fixed array of the code object
