@@ -161,11 +161,11 @@ struct rows_block {
 };
 
 // The block's T transformed row pairs (spectra in natural order in LDS) -> the half spectra
-// of rows r0 .. r0 + 2T - 1 (those below Hm), written column-major into Sm (column stride H):
+// of rows r0 .. r0 + 2T - 1 (those below Hm), written column-major into Sm (column stride Hs):
 // with z = FFT(a + i b), A[k] = (z[k] + conj(z[P-k]))/2 and B[k] = (z[k] - conj(z[P-k]))/(2i).
 template <int LOGPC, int NT>
 __device__ __forceinline__ void split_rows(const double2* buf, double2* __restrict__ Sm, uint32_t r0, uint32_t Hm,
-                                           uint32_t H, int logT) {
+                                           uint32_t Hs, int logT) {
     constexpr int Pc = 1 << LOGPC;
     constexpr uint32_t Kc = Pc / 2 + 1;
     const int rows2 = 2 << logT;
@@ -183,7 +183,7 @@ __device__ __forceinline__ void split_rows(const double2* buf, double2* __restri
             const double2 d = mul_mi(csub(zk, zn));
             v = make_double2(0.5 * d.x, 0.5 * d.y);
         }
-        Sm[(size_t)k * H + r] = v;
+        Sm[(size_t)k * Hs + r] = v;
     }
 }
 
@@ -198,7 +198,7 @@ template <typename Tin, int LOGPC, int NT = rows_block<LOGPC, false>::NT>
 __global__ __launch_bounds__(NT) void rows_fwd_regs_kernel(const Tin* __restrict__ XL, const Tin* __restrict__ XR,
                                                            const uint64_t* __restrict__ moff,
                                                            const uint2* __restrict__ mdims, uint32_t nl, uint32_t H,
-                                                           uint32_t W, int logT, uint32_t groups, uint32_t items,
+                                                           uint32_t Hs, uint32_t W, int logT, uint32_t groups, uint32_t items,
                                                            double2* __restrict__ SL, double2* __restrict__ SR,
                                                            const double2* __restrict__ tw) {
     static_assert(regs_of<LOGPC>::ON, "register transforms only");
@@ -274,8 +274,8 @@ __global__ __launch_bounds__(NT) void rows_fwd_regs_kernel(const Tin* __restrict
 #pragma unroll
             for (int r = 0; r < 8; ++r) buf[at<LOGPC>(t, i + Q * r)] = u[r];
             __syncthreads();
-            split_rows<LOGPC, NT>(buf, (cur.left ? SL : SR) + (size_t)cur.mat * ((1 << LOGPC) / 2 + 1) * H, cur.r0,
-                                  cur.Hm, H, logT);
+            split_rows<LOGPC, NT>(buf, (cur.left ? SL : SR) + (size_t)cur.mat * ((1 << LOGPC) / 2 + 1) * Hs, cur.r0,
+                                  cur.Hm, Hs, logT);
             __syncthreads();  // the next item's transform reuses the slab
         }
         if (!more) break;
@@ -288,12 +288,12 @@ __global__ __launch_bounds__(NT) void rows_fwd_regs_kernel(const Tin* __restrict
 // matrices 0..nl-1 are the left ones (into SL), the rest the right ones (into SR).  Matrix i
 // starts at element moff[i] of its input when the offset table is given (uneven batches),
 // else at i * H * W.  With mdims (uneven batches), matrix i is mdims[i].x x mdims[i].y, at
-// most H x W (the padded lengths are those of H x W); S keeps a column stride of H.
+// most H x W (the padded lengths are those of H x W); S keeps a column stride of Hs.
 template <typename Tin, int LOGPC, int NT = rows_block<LOGPC, false>::NT>
 __global__ __launch_bounds__(NT) void rows_fwd_slab_kernel(const Tin* __restrict__ XL, const Tin* __restrict__ XR,
                                                            const uint64_t* __restrict__ moff,
                                                            const uint2* __restrict__ mdims, uint32_t nl, uint32_t H,
-                                                           uint32_t W, int logT, uint32_t groups,
+                                                           uint32_t Hs, uint32_t W, int logT, uint32_t groups,
                                                            double2* __restrict__ SL, double2* __restrict__ SR,
                                                            const double2* __restrict__ tw) {
     static_assert(!regs_of<LOGPC>::ON && NT == kFT, "slab transforms");
@@ -342,25 +342,33 @@ __global__ __launch_bounds__(NT) void rows_fwd_slab_kernel(const Tin* __restrict
     }
     __syncthreads();
     fft_slab<LOGPC>(buf, T, sr);
-    split_rows<LOGPC, NT>(buf, S + (size_t)mat * (Pc / 2 + 1) * H, r0, Hm, H, logT);
+    split_rows<LOGPC, NT>(buf, S + (size_t)mat * (Pc / 2 + 1) * Hs, r0, Hm, Hs, logT);
 }
 
+// S and Z are column-major with column strides Hs and Ys = 2 Hs, Hs = the job's row count H
+// rounded up to 8: every column starts on a 128-byte line, and so does each group of 8 rows that
+// the row kernels move (off the lines, at 299 rows, fftk_rows_inv took 131 us where 304 rows took
+// 115: 64 pairs of 512 columns).
+//
 // Row of Z that keeps circular row rho of a pair with H rows: the result's shifts dy = rho
-// (rho < H) stay in place, dy = rho - Pr (rho > Pr - H) move down by Pr - 2H to rows
-// H + 1 .. 2H - 1, so that both halves start on the same alignment as in the transform (and
-// for Pr = 2H nothing moves); -1 for the rows in between and for rho >= Pr.  Row H of Z is
-// never written.
-__device__ __forceinline__ int z_row(uint32_t rho, uint32_t H, uint32_t Pr) {
+// (rho < H) stay in place, dy = rho - Pr (rho > Pr - H) move down by Pr - Ys to the rows below
+// Ys, so that both halves keep the transform's alignment (and for Pr = Ys nothing moves); -1 for
+// the rows in between.
+__device__ __forceinline__ int z_row(uint32_t rho, uint32_t H, uint32_t Ys, uint32_t Pr) {
     if (rho < H) return (int)rho;
-    if (rho > Pr - H && rho < Pr) return (int)(rho - (Pr - 2 * H));
+    if (rho > Pr - H && rho < Pr) return (int)(rho - (Pr - Ys));
     return -1;
 }
 
-// Output row (dy + H - 1) of row z of Z (z_row's inverse): -1 for row H and rows >= 2H.
-__device__ __forceinline__ int out_row_of_z(uint32_t z, uint32_t H) {
+// Output row (dy + H - 1) of row z of Z (z_row's inverse), -1 for the rows in between.
+__device__ __forceinline__ int out_row_of_z(uint32_t z, uint32_t H, uint32_t Ys) {
     if (z < H) return (int)(z + H - 1);
-    if (z > H && z < 2 * H) return (int)(z - H - 1);
+    if (z > Ys - H && z < Ys) return (int)(z + H - 1 - Ys);
     return -1;
+}
+// Whether none of the `rows` rows from z0 on is a row of a result.
+__device__ __forceinline__ bool z_gap(uint32_t z0, uint32_t rows, uint32_t H, uint32_t Ys) {
+    return z0 >= Ys || (z0 >= H && z0 + rows <= Ys - H + 1);
 }
 
 // Threads per block of the column kernel: one wave for wave-owned register transforms (up to
@@ -371,19 +379,19 @@ constexpr int cols_threads(int logP) { return logP <= 9 ? 64 : kFT; }
 // cols: block (item, group of C columns k).  mode 0: item = left matrix l, writes its full
 // column spectra Lhat[l][k][rho] (the FFT along rho of SL[l][k][0..H), zero padded).  With
 // mdims (uneven batches) a matrix has mdims[i].x rows of its own (i = l, or nl + r for the
-// right of a pair); S keeps a column stride of H.
+// right of a pair); S keeps a column stride of Hs.
 // mode 1: item = pair q0 + item (left l, right r from the family's order, or from the pair
 // table of an uneven batch): X = the same FFT of SR[r][k], then a second FFT of
 // conj(Lhat) * X, conjugated: Pr * IFFT_rho(Lhat * conj(X)), whose circular row rho goes to
-// Z[item][k][z_row(rho)] (column stride Ys = 2H; the rows between the result's two halves
-// are dropped).
+// Z[item][k][z_row(rho)] (column stride Ys; the rows between the result's two halves are
+// dropped).
 // Blocks are ordered column-group major through the XCD remap, so the pairs that read the
 // same Lhat columns run on one XCD and find them in its L2.
 template <int LOGPR, int MODE>
 __global__ __launch_bounds__(cols_threads(LOGPR)) void cols_kernel(const double2* __restrict__ S, double2* __restrict__ Lhat,
                                                    double2* __restrict__ Z, const uint2* __restrict__ ptab,
                                                    const uint2* __restrict__ mdims, uint32_t nl, int family,
-                                                   uint32_t n, uint32_t m, uint32_t q0, uint32_t items, uint32_t H,
+                                                   uint32_t n, uint32_t m, uint32_t q0, uint32_t items, uint32_t H, uint32_t Hs,
                                                    uint32_t Kc, uint32_t Ys, int logC,
                                                    const double2* __restrict__ tw) {
     constexpr int logPr = LOGPR;
@@ -402,7 +410,7 @@ __global__ __launch_bounds__(cols_threads(LOGPR)) void cols_kernel(const double2
         }
     }
     const uint32_t Hq = mdims ? mdims[MODE == 1 ? nl + r : l].x : H;  // rows of this item's matrices
-    const double2* Sm = S + (size_t)r * Kc * H;
+    const double2* Sm = S + (size_t)r * Kc * Hs;
     double2* Ll = Lhat + (size_t)l * Kc * Pr;
     if constexpr (regs_of<LOGPR>::ON) {
         // C = 8 * threads / Pr: the columns go from HBM to HBM through fft_regs; the product with
@@ -419,7 +427,7 @@ __global__ __launch_bounds__(cols_threads(LOGPR)) void cols_kernel(const double2
         for (int r = 0; r < 4; ++r) {  // Hq <= Pr / 2: the upper half of a column is padding
             const uint32_t rho = i + Q * r;
             u[r] = make_double2(0.0, 0.0);
-            if (ok && rho < Hq) u[r] = Sm[(size_t)k * H + rho];
+            if (ok && rho < Hq) u[r] = Sm[(size_t)k * Hs + rho];
         }
         double2* lk = Ll + (size_t)k * Pr;
         // The left spectrum is loaded together with the column (its latency overlaps the
@@ -448,14 +456,14 @@ __global__ __launch_bounds__(cols_threads(LOGPR)) void cols_kernel(const double2
             // rows from the opaque i2, so that the row indices of the loads are not kept live
             // through both transforms for these stores
             // z_row with constant offsets from two bases: rows below Hq in place, rows from
-            // Pr - Hq on down by Pr - 2Hq (for Pr = 2Hq one base and every row, row Hq
+            // Pr - Hq on down by Pr - Ys (for Pr = 2Hq one base and every row, row Hq
             // included, which the row kernel reads as zero)
             double2* zlo = Z + (size_t)item * Kc * Ys + (size_t)k * Ys + i2;
             if (Pr == 2 * (int)Hq) {
 #pragma unroll
                 for (int r = 0; r < 8; ++r) zlo[Q * r] = cconj(u[r]);
             } else {
-                double2* zhi = zlo - (Pr - 2 * (int)Hq);
+                double2* zhi = zlo - (Pr - (int)Ys);
 #pragma unroll
                 for (int r = 0; r < 8; ++r) {
                     const uint32_t rho = (uint32_t)(i2 + Q * r);
@@ -479,7 +487,7 @@ __global__ __launch_bounds__(cols_threads(LOGPR)) void cols_kernel(const double2
         const int idx = threadIdx.x + kFT * q;
         const uint32_t k = k0 + (idx >> logPr), rho = idx & (Pr - 1);
         const uint32_t kk = k < Kc ? k : Kc - 1;
-        xs[q] = Sm[(size_t)kk * H + (rho < Hq ? rho : Hq - 1)];
+        xs[q] = Sm[(size_t)kk * Hs + (rho < Hq ? rho : Hq - 1)];
         lh[q] = MODE == 1 ? Ll[(size_t)kk * Pr + rho] : make_double2(0.0, 0.0);
     }
 #pragma unroll
@@ -513,7 +521,7 @@ __global__ __launch_bounds__(cols_threads(LOGPR)) void cols_kernel(const double2
     for (int q = 0; q < NI; ++q) {
         const int idx = threadIdx.x + kFT * q;
         const uint32_t k = k0 + (idx >> logPr);
-        const int y = z_row((uint32_t)(idx & (Pr - 1)), Hq, (uint32_t)Pr);
+        const int y = z_row((uint32_t)(idx & (Pr - 1)), Hq, Ys, (uint32_t)Pr);
         if (k < Kc && y >= 0) Zq[(size_t)k * Ys + y] = cconj(buf[at<LOGPR>(idx >> logPr, idx & (Pr - 1))]);
     }
     }
@@ -549,7 +557,7 @@ __global__ __launch_bounds__(NT) void rows_inv_kernel(const double2* __restrict_
     const uint32_t SX = 2 * W - 1;
     const uint32_t z0 = g << (logT + 1);
     const int rows2 = 2 << logT;
-    if (z0 >= 2 * H) return;  // a smaller pair of an uneven batch
+    if (z_gap(z0, (uint32_t)rows2, H, Ys)) return;  // between the two halves of the result
     const double2* Zq = Z + (size_t)item * Kc * Ys;
     regs_roots<LOGPC> rr{};
     slab_roots<LOGPC> sr{};
@@ -575,8 +583,8 @@ __global__ __launch_bounds__(NT) void rows_inv_kernel(const double2* __restrict_
             const double2* zc = Zq + (size_t)kk * Ys + za;
             A[q] = make_double2(0.0, 0.0);
             B[q] = make_double2(0.0, 0.0);
-            if (idx < items && out_row_of_z(za, H) >= 0) A[q] = zc[0];
-            if (idx < items && out_row_of_z(za + 1, H) >= 0) B[q] = zc[1];
+            if (idx < items && out_row_of_z(za, H, Ys) >= 0) A[q] = zc[0];
+            if (idx < items && out_row_of_z(za + 1, H, Ys) >= 0) B[q] = zc[1];
         }
 #pragma unroll
         for (int q = 0; q < NQ; ++q) {
@@ -601,7 +609,7 @@ __global__ __launch_bounds__(NT) void rows_inv_kernel(const double2* __restrict_
         // a block-owned transform's first pass overwrites slots other waves still read
         if constexpr (regs_of<LOGPC>::BLOCK) __syncthreads();
         fft_regs<LOGPC>(u, buf + at<LOGPC>(t0, 0), rr, t - t0, i);
-        const int oa = out_row_of_z(z0 + 2 * t, H), ob = out_row_of_z(z0 + 2 * t + 1, H);
+        const int oa = out_row_of_z(z0 + 2 * t, H, Ys), ob = out_row_of_z(z0 + 2 * t + 1, H, Ys);
 #pragma unroll
         for (int r = 0; r < 8; ++r) {
             const int c = i + Q * r;
@@ -615,7 +623,7 @@ __global__ __launch_bounds__(NT) void rows_inv_kernel(const double2* __restrict_
     fft_slab<LOGPC>(buf, T, sr);
     // IFFT(Y) = conj(FFT(conj(Y))) / Pc: row A is the real part, row B minus the imaginary.
     for (int rr = threadIdx.x >> 6; rr < rows2; rr += NT / 64) {
-        const int oy = out_row_of_z(z0 + rr, H);
+        const int oy = out_row_of_z(z0 + rr, H, Ys);
         if (oy < 0) continue;
         Tout* orow = Oq + (size_t)oy * SX;
         const int t = rr >> 1;
@@ -717,8 +725,8 @@ __device__ __forceinline__ void radix3_pass(const double2* buf, const r3_roots<L
 template <typename Tin, int LOGN>
 __global__ __launch_bounds__(rows3<LOGN>::NT) void rows_fwd3_kernel(
     const Tin* __restrict__ XL, const Tin* __restrict__ XR, const uint64_t* __restrict__ moff,
-    const uint2* __restrict__ mdims, uint32_t nl, uint32_t H, uint32_t W, uint32_t groups, uint32_t items,
-    double2* __restrict__ SL, double2* __restrict__ SR, const double2* __restrict__ tw,
+    const uint2* __restrict__ mdims, uint32_t nl, uint32_t H, uint32_t Hs, uint32_t W, uint32_t groups,
+    uint32_t items, double2* __restrict__ SL, double2* __restrict__ SR, const double2* __restrict__ tw,
     const double2* __restrict__ tw3) {
     using G = rows3<LOGN>;
     constexpr int N = G::N, P = G::P, Q = G::Q, T = G::T;
@@ -806,7 +814,7 @@ __global__ __launch_bounds__(rows3<LOGN>::NT) void rows_fwd3_kernel(
             }
             __syncthreads();
             // split into the two rows' half spectra (as split_rows), column-major into S
-            double2* Sm = (cur.left ? SL : SR) + (size_t)cur.mat * Kc * H;
+            double2* Sm = (cur.left ? SL : SR) + (size_t)cur.mat * Kc * Hs;
             for (int idx = threadIdx.x; idx < (int)Kc * 2 * T; idx += G::NT) {
                 const int k = idx >> (G::LOGT + 1), rw = idx & (2 * T - 1);
                 const uint32_t r = cur.r0 + rw;
@@ -821,7 +829,7 @@ __global__ __launch_bounds__(rows3<LOGN>::NT) void rows_fwd3_kernel(
                     const double2 d = mul_mi(csub(zk, zn));
                     v = make_double2(0.5 * d.x, 0.5 * d.y);
                 }
-                Sm[(size_t)k * H + r] = v;
+                Sm[(size_t)k * Hs + r] = v;
             }
             __syncthreads();  // the next item's transform reuses the slab
         }
@@ -851,7 +859,7 @@ __global__ __launch_bounds__(rows3<LOGN>::NT) void rows_inv3_kernel(
     }
     const uint32_t SX = 2 * W - 1;
     const uint32_t z0 = g * (2 * T);
-    if (z0 >= 2 * H) return;
+    if (z_gap(z0, 2 * T, H, Ys)) return;
     const double2* Zq = Z + (size_t)item * Kc * Ys;
     const regs_pos<LOGN> ps((int)threadIdx.x);
     const int sub = ps.t, tt = sub / 3, m = sub - 3 * tt, i = ps.i;
@@ -869,8 +877,8 @@ __global__ __launch_bounds__(rows3<LOGN>::NT) void rows_inv3_kernel(
             const double2* zc = Zq + (size_t)(idx < (int)Kc * T ? kk : 0) * Ys + za;
             A[q] = make_double2(0.0, 0.0);
             B[q] = make_double2(0.0, 0.0);
-            if (idx < (int)Kc * T && out_row_of_z(za, H) >= 0) A[q] = zc[0];
-            if (idx < (int)Kc * T && out_row_of_z(za + 1, H) >= 0) B[q] = zc[1];
+            if (idx < (int)Kc * T && out_row_of_z(za, H, Ys) >= 0) A[q] = zc[0];
+            if (idx < (int)Kc * T && out_row_of_z(za + 1, H, Ys) >= 0) B[q] = zc[1];
         }
 #pragma unroll
         for (int q = 0; q < NQ; ++q) {
@@ -899,7 +907,7 @@ __global__ __launch_bounds__(rows3<LOGN>::NT) void rows_inv3_kernel(
         const int idx = (int)threadIdx.x + G::NT * q;
         if (idx >= T * N) continue;
         const int t2 = idx >> LOGN, k = idx & (N - 1);
-        const int oa = out_row_of_z(z0 + 2 * t2, H), ob = out_row_of_z(z0 + 2 * t2 + 1, H);
+        const int oa = out_row_of_z(z0 + 2 * t2, H, Ys), ob = out_row_of_z(z0 + 2 * t2 + 1, H, Ys);
 #pragma unroll
         for (int j = 0; j < 3; ++j) {
             const int c = k + N * j;
@@ -1047,11 +1055,13 @@ struct fftk_geom {
     // right spectra take S's place (column spectra of Pr values), Z and the left S are not used.
     bool small;
     int logPrs, logPcs;
-    uint32_t Ys;  // column stride of Z: 2H (the 2H-1 circular rows of the result, z_row)
+    uint32_t Hs, Ys;  // column strides of S and Z (z_row)
     size_t s_bytes, sl_bytes, col_bytes, z_bytes;  // S per right and per left, Lhat per left, Z per pair
 };
 
-fftk_geom geom_of(uint32_t H, uint32_t W, bool pow2_rows = false) {
+// plain: the layout that takes the least memory per matrix (no one-block kernels, no rounding of
+// the column strides).
+fftk_geom geom_of(uint32_t H, uint32_t W, bool pow2_rows = false, bool plain = false) {
     if (H == 0 || W == 0 || 2 * H - 1 > (uint32_t)kSlab || 2 * W - 1 > (uint32_t)kSlab)
         fail(XC_ERR_UNSUPPORTED, "own-FFT method: rows and cols must be 1..2048");
     fftk_geom g{};
@@ -1076,15 +1086,16 @@ fftk_geom geom_of(uint32_t H, uint32_t W, bool pow2_rows = false) {
     }
     g.g1 = (H + (2u << g.v1.logT) - 1) >> (g.v1.logT + 1);
     g.cg = (g.Kc + (1u << g.vc.logT) - 1) >> g.vc.logT;
-    g.g3 = (2 * H + (2u << g.v3.logT) - 1) >> (g.v3.logT + 1);  // a block may be taller
-    g.Ys = 2 * H;
-    g.s_bytes = sizeof(double2) * (size_t)g.Kc * H;
+    g.Hs = plain ? H : (H + 7) & ~7u;
+    g.Ys = 2 * g.Hs;
+    g.g3 = (g.Ys + (2u << g.v3.logT) - 1) >> (g.v3.logT + 1);  // a block may be taller
+    g.s_bytes = sizeof(double2) * (size_t)g.Kc * g.Hs;
     g.col_bytes = sizeof(double2) * (size_t)g.Kc * g.Pr;
     g.z_bytes = sizeof(double2) * (size_t)g.Kc * g.Ys;
     g.sl_bytes = g.s_bytes;
     g.logPrs = std::max(5, g.logPr);
     g.logPcs = std::max(5, ilog2_ceil(2 * W - 1));
-    g.small = fftk_small_fits(g.logPrs, g.logPcs);
+    g.small = !plain && fftk_small_fits(g.logPrs, g.logPcs);
     if (g.small) {
         g.col_bytes = sizeof(double2) * (size_t)((1u << g.logPcs) / 2 + 1) << g.logPrs;
         g.s_bytes = g.col_bytes;
@@ -1124,7 +1135,7 @@ template <typename Tio>
 void launch_job(const fftk_job& j, const Tio* L, const Tio* R, Tio* O, const fftk_ws& ws, hipStream_t s,
                 bool timing) {
     const uint32_t H = j.H, W = j.W;
-    const fftk_geom g = geom_of(H, W, j.pow2_rows);
+    const fftk_geom g = geom_of(H, W, j.pow2_rows, j.plain);
     if (g.small) {
         if constexpr (std::is_same<Tio, float>::value)
             fftk_small_f32(j, g.logPrs, g.logPcs, L, R, O, ws, s, timing);
@@ -1153,7 +1164,7 @@ void launch_job(const fftk_job& j, const Tio* L, const Tio* R, Tio* O, const fft
                 const uint32_t items = (j.nl + j.nr) * g.g1;
                 const uint32_t grid = resident_grid(reinterpret_cast<const void*>(k), G3::NT, g.v1.lds, items);
                 launch_timed("fftk_rows_fwd", timing, k, dim3(grid), dim3(G3::NT), g.v1.lds, s, L, R, j.moff, mdims,
-                             j.nl, H, W, g.g1, items, SL, SR, tw, tw3);
+                             j.nl, H, g.Hs, W, g.g1, items, SL, SR, tw, tw3);
             }
         });
     } else
@@ -1166,12 +1177,12 @@ void launch_job(const fftk_job& j, const Tio* L, const Tio* R, Tio* O, const fft
             const uint32_t grid = resident_grid(reinterpret_cast<const void*>(k), rows_threads(LOGPC, false),
                                                 g.v1.lds, items);
             launch_timed("fftk_rows_fwd", timing, k, dim3(grid), dim3(rows_threads(LOGPC, false)), g.v1.lds, s, L, R,
-                         j.moff, mdims, j.nl, H, W, g.v1.logT, g.g1, items, SL, SR, tw);
+                         j.moff, mdims, j.nl, H, g.Hs, W, g.v1.logT, g.g1, items, SL, SR, tw);
         } else {
             auto k = rows_fwd_slab_kernel<Tio, LOGPC>;
             allow_lds(k, g.v1.lds);
             launch_timed("fftk_rows_fwd", timing, k, dim3(items), dim3(kFT), g.v1.lds, s, L, R, j.moff, mdims, j.nl, H,
-                         W, g.v1.logT, g.g1, SL, SR, tw);
+                         g.Hs, W, g.v1.logT, g.g1, SL, SR, tw);
         }
     });
     auto cols = [&](const char* name, const double2* S, double2* Zout, auto MODE, uint32_t items,
@@ -1180,7 +1191,7 @@ void launch_job(const fftk_job& j, const Tio* L, const Tio* R, Tio* O, const fft
             auto k = cols_kernel<decltype(LP)::value, decltype(MODE)::value>;
             allow_lds(k, g.vc.lds);
             launch_timed(name, timing, k, dim3(items * g.cg), dim3(cols_threads(g.logPr)), g.vc.lds, s, S, LH, Zout,
-                         ptab, mdims, j.nl, j.family, j.n, j.m, q0, items, H, g.Kc, g.Ys, g.vc.logT, tw);
+                         ptab, mdims, j.nl, j.family, j.n, j.m, q0, items, H, g.Hs, g.Kc, g.Ys, g.vc.logT, tw);
         });
     };
     cols("fftk_cols_left", SL, nullptr, std::integral_constant<int, 0>{}, j.nl, 0);
@@ -1340,7 +1351,7 @@ std::vector<noalloc_part> plan_noalloc(const family_args& a, const fftk_geom& g)
                 const uint32_t c = std::min(gl, a.n - l0);
                 // as many pairs per launch as the rest of the array holds (at least m: gl fits them)
                 const size_t rest = B - part_bytes(g, c, a.m, 0);
-                uint32_t chunk = (uint32_t)std::min<size_t>((size_t)c * a.m, g.z_bytes ? rest / g.z_bytes : SIZE_MAX);
+                uint32_t chunk = (uint32_t)std::min<size_t>((size_t)c * a.m, rest / g.z_bytes);
                 while (chunk > a.m && part_bytes(g, c, a.m, chunk) > B) --chunk;
                 parts.push_back({XC_N_TO_M, c, a.m, c * a.m, l0 * hw, 0, (size_t)l0 * a.m * out_elems, chunk});
             }
@@ -1361,9 +1372,19 @@ std::vector<noalloc_part> plan_noalloc(const family_args& a, const fftk_geom& g)
 
 void run_fftk_noalloc_f32(const family_args& a, const float* L, const float* R, float* O, hipStream_t s) {
     char* base = scratch_of_device();
-    const fftk_geom g = geom_of(a.rows, a.cols);
     (void)tables_of_device();
-    for (const noalloc_part& p : plan_noalloc(a, g)) {
+    // The plain layout decides what fits and how a call is split; a call that fits whole in the
+    // faster layout of the allocating calls takes that one.
+    fftk_geom g = geom_of(a.rows, a.cols, false, true);
+    std::vector<noalloc_part> parts = plan_noalloc(a, g);
+    const bool one = a.family == XC_ONE_TO_ONE || a.family == XC_ONE_TO_MANY;
+    const fftk_geom fast = geom_of(a.rows, a.cols);
+    const bool whole = part_bytes(fast, one ? 1 : a.n, a.family == XC_ONE_TO_ONE ? 1 : a.m, a.pairs) <= kScratchBytes;
+    if (whole) {
+        g = fast;
+        parts = {{a.family, one ? 1 : a.n, a.family == XC_ONE_TO_ONE ? 1 : a.m, a.pairs, 0, 0, 0, a.pairs}};
+    }
+    for (const noalloc_part& p : parts) {
         fftk_job j{};
         j.H = a.rows;
         j.W = a.cols;
@@ -1373,6 +1394,7 @@ void run_fftk_noalloc_f32(const family_args& a, const float* L, const float* R, 
         j.nl = p.family == XC_ONE_TO_ONE || p.family == XC_ONE_TO_MANY ? 1 : p.n;
         j.nr = p.m;
         j.pairs = p.pairs;
+        j.plain = !whole;
         fftk_ws ws{};
         char* q = base;
         ws.sr = q;
@@ -1411,7 +1433,7 @@ std::pair<uint32_t, uint32_t> fftk_class(uint32_t rows, uint32_t cols) {
 }
 
 fftk_ws_sizes fftk_sizes(const fftk_job& j) {
-    const fftk_geom g = geom_of(j.H, j.W, j.pow2_rows);
+    const fftk_geom g = geom_of(j.H, j.W, j.pow2_rows, j.plain);
     fftk_ws_sizes z{};
     // Z is processed in chunks of pairs of at most ~2 GiB.
     z.chunk = (uint32_t)std::max<size_t>(1, std::min<size_t>(j.pairs, (size_t(2) << 30) / std::max<size_t>(g.z_bytes, 1)));

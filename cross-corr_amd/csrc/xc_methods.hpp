@@ -85,6 +85,8 @@ struct fftk_job {
     uint32_t max_chunk = 0;
     // Row transforms of the power of two >= 2W-1 even where 3 * 2^n is shorter.
     bool pow2_rows = false;
+    // The layout of the least memory per matrix (the allocation-free entry point's split calls).
+    bool plain = false;
 };
 struct fftk_ws_sizes {
     size_t sr, sl, lh, z;
