@@ -227,7 +227,9 @@ xc_status xc_normalize_fft_f64(const double* res, double* norm, uint32_t rows, u
  * src/one_to_many.hpp:679-745, src/n_to_m.hpp:700-736).  If `normalize` is 0 the
  * results are the unnormalised (2*rows) x (2*cols) circular correlations the
  * reference stores without -n; otherwise (2*rows-1) x (2*cols-1) as every other
- * method.  Plans are cached per (device, stream, shape, batch, precision). */
+ * method.  Plans are cached per (device, stream, shape, batch, precision).  Normalised
+ * float results of up to 2048 x 2048 are computed by the own FFT kernels in FP64 whatever
+ * fp64_transform says (it picks the precision of the rocFFT transforms of the rest). */
 xc_status xc_fft_cross_corr_f32(xc_family family, const float* left, const float* right, float* out,
                                 uint32_t rows, uint32_t cols, uint32_t n, uint32_t m, int normalize,
                                 int fp64_transform, xc_stream_t stream);
