@@ -336,24 +336,31 @@ uint32_t rights_per_left(const family_args& a) {
     }
 }
 
-// Whether the lanes-over-pairs kernel serves this batch by default: at least 48 rights per
-// left (a wave's lanes at least 3/4 busy below 64), and its copy of the rights (the register-
-// tile kernel needs none) at most 16 GiB.
-bool pairs_kernel_applies(const family_args& a) {
+// Waves of the lanes-over-pairs kernel.
+uint64_t pairs_kernel_waves(const family_args& a) {
+    const uint32_t nl = a.family == XC_ONE_TO_MANY ? 1 : a.n;
+    return (uint64_t)nl * ((rights_per_left(a) + 63) / 64) * ((2 * a.rows - 1 + kPairsTY - 1) / kPairsTY) *
+           ((2 * a.cols - 1 + 3) / 4);
+}
+
+// Whether the lanes-over-pairs kernel serves this batch by default: at least 48 rights per left
+// (a wave's lanes at least 3/4 busy below 64), its copy of the rights (the other kernels need
+// none) at most 16 GiB, and enough waves.  Double data, and float data with every lane busy: 2048
+// waves (against the register tiles 0.45-0.9x at 128-1024 waves, 1.14x at 2048, 1.6-2.2x from
+// 4096).  Float data with idle lanes competes with the 16 x 16 shifts kernel: a wave's time does
+// not shrink with its pairs, so the line lies at waves * (busy lanes)^3 = 4500, at least 7 lanes
+// in 10 busy.  Measured us, pairs / shifts: 48 of 128^2 869 / 635, 100 of 128^2 1563 / 1287, 4 x 50
+// of 100^2 950 / 1283, 56 of 200^2 3805 / 4499, 80 of 256^2 16620 / 15070, 100 of 256^2 17350 / 18830.
+bool pairs_kernel_applies(const family_args& a, bool float_data) {
     const uint32_t mpl = rights_per_left(a);
     if (mpl < 48) return false;
     const uint64_t lefts = a.family == XC_ONE_TO_MANY ? 1 : a.n;
     const uint64_t slots = (a.family == XC_N_TO_MN ? lefts : 1) * ((mpl + 63) / 64 * 64);
     const uint64_t copy = slots * a.rows * (a.cols + 24) * sizeof(float);
-    return copy <= (16ull << 30);
-}
-
-// Waves of the lanes-over-pairs kernel.  Measured against the register-tile kernel (one_to_many
-// and n_to_m, 16^2 to 256^2): 0.45-0.9x at 128-1024 waves, 1.14x at 2048, 1.6-2.2x from 4096.
-uint64_t pairs_kernel_waves(const family_args& a) {
-    const uint32_t nl = a.family == XC_ONE_TO_MANY ? 1 : a.n;
-    return (uint64_t)nl * ((rights_per_left(a) + 63) / 64) * ((2 * a.rows - 1 + kPairsTY - 1) / kPairsTY) *
-           ((2 * a.cols - 1 + 3) / 4);
+    if (copy > (16ull << 30)) return false;
+    const double busy = (double)mpl / (double)((mpl + 63) / 64 * 64), waves = (double)pairs_kernel_waves(a);
+    if (!float_data || busy == 1.0) return waves >= 2048;
+    return busy >= 0.7 && waves * busy * busy * busy >= 4500;
 }
 
 template <typename T>
@@ -404,11 +411,242 @@ void launch_direct_pairs(const family_args& a, const T* L, const T* R, T* O, hip
     XC_HIP(hipGetLastError());
 }
 
+// ---------------------------------------------------------------- lanes over shifts and rows
+// Definition-based FP32 kernel for batches with few rights per left.  A block takes one pair and
+// a tile of 16 dy x 16 dx; its NW waves have four groups of 16 lanes each, and each of the 4 NW
+// groups sums its share of the tile's right rows.  A lane holds 4 x 4 outputs (lane gx + 4 gy of
+// a group: dx0 + 4 gx .., dy0 + 4 gy ..).  The inputs go through the wave's own LDS in panels of
+// 8 right rows x 16 columns (zeros outside the matrices), the next panel's values loaded into
+// registers meanwhile; per right row and 4 columns a lane does 64 FMAs from three 16-byte LDS
+// reads (two quads of the right row: the 7 values of its window; one quad of the left row that
+// enters, the other three rows stay in registers):
+//   out(dy0+y, dx0+x) += L[j+dy0+y][c0+t] * R[j][c0+t-dx0-x].
+// No barriers until the groups' FP64 totals are added through LDS at the end, in a fixed order.
+//
+// Bound: FP32 FMAs (LDS a fifth of the FMAs' time): 22.8 T products/s at 40 pairs of 256^2, where
+// the register tiles run 17.8; n_to_m 2 x 6 of 100x120 349 -> 137 us, 1 pair of 512^2 9.5 -> 3.4 ms.  All lanes of a tile share one column range
+// and one row range, the unions over 16 shifts: (W/2 + 8)(H/2 + 8) products issued per W/2 * H/2,
+// where the register tiles' 64-dx waves issue W/2 + 32 columns and take 32 4-byte LDS reads per
+// 128 FMAs.  Panels that hold a NaN or an infinity are summed product by product, so that a
+// shift's sum never meets a value outside its overlap (0 * inf).
+struct ds_args {
+    int family, H, W;
+    uint32_t n, m, pairs, tiles_x, tiles_y;
+};
+
+template <int NW>
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(3))) void direct_shifts_kernel(const float* __restrict__ L,
+                                                                const float* __restrict__ R, float* __restrict__ O,
+                                                                ds_args a) {
+    constexpr int JP = 8, CP = 16;           // panel: right rows x columns
+    constexpr int NLR = JP + 15;             // left rows of a panel
+    constexpr int RQ = 68, LQ = 129, LS = 5;  // quads: right part, left part of a group, left row stride (bank spread)
+    constexpr int WQ = 4 * (RQ + LQ);        // quads of a wave
+    __shared__ float4 smem[NW * WQ];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int g = lane >> 4, l16 = lane & 15, gx = lane & 3, gy = (lane >> 2) & 3;
+    // tiles nearest the centre (the longest sums) first, all pairs of a tile together
+    uint32_t bid = xcd_remap(blockIdx.x, gridDim.x);
+    const uint32_t pair = bid % a.pairs;
+    bid /= a.pairs;
+    const int tx = center_first((int)(bid % a.tiles_x), (int)a.tiles_x);
+    const int ty = center_first((int)(bid / a.tiles_x), (int)a.tiles_y);
+    const int H = a.H, W = a.W, dx0 = -(W - 1) + 16 * tx, dy0 = -(H - 1) + 16 * ty;
+    uint32_t li, ri;
+    pair_of(a.family, a.n, a.m, pair, li, ri);
+    const float* __restrict__ Lp = L + (size_t)li * H * W;
+    const float* __restrict__ Rp = R + (size_t)ri * H * W;
+    const int jlo = max(0, -(dy0 + 15)), cnt = min(H, H - dy0) - jlo;
+    const int clo = max(0, dx0), chi = min(W, W + dx0 + 15);
+    const int split = wave * 4 + g;
+    const int js = jlo + cnt * split / (4 * NW), je = jlo + cnt * (split + 1) / (4 * NW);
+    const int jpanels = (cnt + 4 * NW * JP - 1) / (4 * NW * JP), cpanels = (chi - clo + CP - 1) / CP;
+
+    float4* const rq = smem + wave * WQ + g * RQ;
+    float4* const lq = smem + wave * WQ + 4 * RQ + g * LQ;
+    float* const rw = reinterpret_cast<float*>(rq) + l16;
+    float* const lw = reinterpret_cast<float*>(lq) + l16;
+    float pr[2 * JP], pl[NLR];
+    // This lane's share of the panel at right row j0, column c0: right columns c0 - dx0 - 16 + l16
+    // and the 16 after, left column c0 + l16.  Bounds-checked buffer loads: rows outside a matrix
+    // fall outside its bytes, columns outside it get an offset that does (kOut; the launcher keeps
+    // matrices below 2^31 bytes), and both read zero without a select after the load, which
+    // would have to wait for it.
+    constexpr uint32_t kOut = 0x80000000u;
+    const uint32_t bytes = (uint32_t)H * (uint32_t)W * 4u, pitch = (uint32_t)W * 4u;
+    const __amdgpu_buffer_rsrc_t rl = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(Lp), 0, bytes, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rr = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(Rp), 0, bytes, 0x00020000);
+    auto load = [](const __amdgpu_buffer_rsrc_t rsrc, uint32_t offset) {
+        return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrc, (int)offset, 0, 0));
+    };
+    auto fetch = [&](int j0, int c0) {
+        const int q0 = c0 - dx0 - 16 + l16, q1 = q0 + 16, c = c0 + l16;
+        const uint32_t row = (uint32_t)j0 * pitch;
+        const uint32_t o0 = q0 >= 0 && q0 < W ? row + (uint32_t)q0 * 4u : kOut;
+        const uint32_t o1 = q1 >= 0 && q1 < W ? row + (uint32_t)q1 * 4u : kOut;
+        const uint32_t ol = c < W ? (uint32_t)(j0 + dy0) * pitch + (uint32_t)c * 4u : kOut;
+#pragma unroll
+        for (int k = 0; k < JP; ++k) {
+            const bool in = j0 + k < je;  // the group's share of the rows ends here
+            pr[2 * k] = load(rr, in ? o0 + k * pitch : kOut);
+            pr[2 * k + 1] = load(rr, in ? o1 + k * pitch : kOut);
+        }
+#pragma unroll
+        for (int k = 0; k < NLR; ++k) pl[k] = load(rl, ol + k * pitch);
+    };
+    float acc[4][4];
+    double tot[4][4];
+#pragma unroll
+    for (int y = 0; y < 4; ++y)
+#pragma unroll
+        for (int x = 0; x < 4; ++x) acc[y][x] = 0.f, tot[y][x] = 0.0;
+    auto flush = [&] {
+#pragma unroll
+        for (int y = 0; y < 4; ++y)
+#pragma unroll
+            for (int x = 0; x < 4; ++x) {
+                tot[y][x] += (double)acc[y][x];
+                acc[y][x] = 0.f;
+            }
+    };
+    auto lds_sync = [] {  // the wave's own LDS: ordering its accesses is enough
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+    };
+
+    // The products of the first JN right rows of the panel in LDS.
+    auto sum_panel = [&](auto JN) {
+#pragma unroll 1
+        for (int q = 0; q < CP / 4; ++q) {
+            const float4* rrow = rq + (q - gx + 3);
+            const float4* lrow = lq + 4 * gy * LS + q;
+            float4 lv[4];
+#pragma unroll
+            for (int y = 0; y < 3; ++y) lv[y + 1] = lrow[y * LS];
+#pragma unroll
+            for (int j = 0; j < decltype(JN)::value; ++j) {
+#pragma unroll
+                for (int y = 0; y < 3; ++y) lv[y] = lv[y + 1];
+                lv[3] = lrow[(j + 3) * LS];
+                float4 w0 = rrow[j * 8];
+                const float4 w1 = rrow[j * 8 + 1];
+                asm volatile("" : "+v"(w0.x));  // not used: keeps the quad one 16-byte read
+                const float w[8] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w};
+#pragma unroll
+                for (int y = 0; y < 4; ++y) {
+                    const float l[4] = {lv[y].x, lv[y].y, lv[y].z, lv[y].w};
+#pragma unroll
+                    for (int t = 0; t < 4; ++t)
+#pragma unroll
+                        for (int x = 0; x < 4; ++x) acc[y][x] = fmaf(l[t], w[t - x + 4], acc[y][x]);
+                }
+            }
+            if (q & 1) flush();  // at most 64 products per FP32 sum
+        }
+    };
+
+    const int panels = jpanels * cpanels, share = (cnt + 4 * NW - 1) / (4 * NW);
+    fetch(js, clo);
+    int jp = 0, cp = 0;
+    for (int p = 0; p < panels; ++p) {
+#pragma unroll
+        for (int k = 0; k < 2 * JP; ++k) rw[k * 16] = pr[k];
+#pragma unroll
+        for (int k = 0; k < NLR; ++k) lw[k * 4 * LS] = pl[k];
+        const int rows_left = share - jp * JP;  // of the longest group
+        if (++cp == cpanels) cp = 0, ++jp;
+        if (p + 1 < panels) fetch(js + jp * JP, clo + cp * CP);
+        lds_sync();
+        if (rows_left > JP / 2)
+            sum_panel(std::integral_constant<int, JP>{});
+        else
+            sum_panel(std::integral_constant<int, JP / 2>{});
+        lds_sync();  // the next panel overwrites this one
+    }
+    // A value that is not finite makes a total of every lane that met it so, overlap or not (0 *
+    // inf): such a wave sums its shifts again, each over its own overlap only.
+    bool finite = true;
+#pragma unroll
+    for (int y = 0; y < 4; ++y)
+#pragma unroll
+        for (int x = 0; x < 4; ++x) finite = finite & __builtin_isfinite(tot[y][x]);
+    if (!__all(finite)) {
+#pragma unroll 1
+        for (int o = 0; o < 16; ++o) {
+            const int dy = dy0 + 4 * gy + (o >> 2), dx = dx0 + 4 * gx + (o & 3);
+            double v = 0.0;
+            for (int j = max(js, -dy); j < min(je, H - dy); ++j) {
+                float part = 0.f;
+                for (int c = max(0, dx); c < min(W, W + dx); ++c)
+                    part = fmaf(Lp[(size_t)(j + dy) * W + c], Rp[(size_t)j * W + c - dx], part);
+                v += (double)part;
+            }
+#pragma unroll
+            for (int i = 0; i < 16; ++i)
+                if (i == o) tot[i >> 2][i & 3] = v;
+        }
+    }
+    // The groups' totals, added in order.
+    double* const td = reinterpret_cast<double*>(smem + wave * WQ) + g * 256;
+#pragma unroll
+    for (int y = 0; y < 4; ++y)
+#pragma unroll
+        for (int x = 0; x < 4; ++x) td[(4 * gy + y) * 16 + 4 * gx + x] = tot[y][x];
+    __syncthreads();
+    const int SX = 2 * W - 1, SY = 2 * H - 1;
+    float* __restrict__ Op = O + (size_t)pair * SX * SY;
+    for (int o = threadIdx.x; o < 256; o += 64 * NW) {
+        double v = 0.0;
+        for (int w = 0; w < NW; ++w)
+#pragma unroll
+            for (int k = 0; k < 4; ++k) v += reinterpret_cast<const double*>(smem + w * WQ)[k * 256 + o];
+        const int oy = 16 * ty + (o >> 4), ox = 16 * tx + (o & 15);
+        if (oy < SY && ox < SX) Op[(size_t)oy * SX + ox] = (float)v;
+    }
+}
+
+// Waves per block, each with four of the tile's 4 NW shares of right rows: more waves while the
+// shares keep about 4 rows and the tiles are too few to balance the 256 CUs (the longer the sums,
+// the more of them it takes).  Measured us with 1 / 2 / 4 waves: 1 pair of 64^2 43 / 24 / 18, 8 of
+// 128^2 194 / 150 / 114, 64 of 64^2 72 / 70 / 90, 40 of 32^2 14 / 13 / 18, 40 of 256^2 7630 / 7880 /
+// 8110, 64 of 50x80 87 / 92 / 107.
+int direct_shifts_waves(uint64_t tiles, uint32_t rows) {
+    int nw = 1;
+    while (nw < 4 && rows >= 20u * nw && tiles * nw < 72ull * rows) nw *= 2;
+    return nw;
+}
+
+void launch_direct_shifts(const family_args& a, const float* L, const float* R, float* O, hipStream_t s) {
+    ds_args k{};
+    k.family = a.family;
+    k.H = (int)a.rows;
+    k.W = (int)a.cols;
+    k.n = a.family == XC_ONE_TO_ONE || a.family == XC_ONE_TO_MANY ? 1 : a.n;
+    k.m = a.m;
+    k.pairs = a.pairs;
+    k.tiles_x = (2 * a.cols - 1 + 15) / 16;
+    k.tiles_y = (2 * a.rows - 1 + 15) / 16;
+    const uint64_t tiles = (uint64_t)a.pairs * k.tiles_x * k.tiles_y;
+    if (tiles > 0x7fffffffULL) fail(XC_ERR_INVALID_ARGUMENT, "problem too large for one launch");
+    const int nw = direct_shifts_waves(tiles, a.rows);
+    const dim3 grid((uint32_t)tiles), block(64 * nw);
+    record_launch("direct_kernel<f32> 16x16 shifts, rows over lanes", grid, block, 0, a.rows, a.cols, a.pairs, 1);
+    timed td("direct_kernel", s);
+    if (nw == 1)
+        hipLaunchKernelGGL(direct_shifts_kernel<1>, grid, block, 0, s, L, R, O, k);
+    else if (nw == 2)
+        hipLaunchKernelGGL(direct_shifts_kernel<2>, grid, block, 0, s, L, R, O, k);
+    else
+        hipLaunchKernelGGL(direct_shifts_kernel<4>, grid, block, 0, s, L, R, O, k);
+    XC_HIP(hipGetLastError());
+}
+
 template <typename T>
 void launch_direct(const family_args& a, const T* L, const T* R, T* O, const xc_options& opt, hipStream_t s) {
     if (a.cols > (uint32_t)kMaxCols) fail(XC_ERR_UNSUPPORTED, "direct kernel: cols above 32768");
-    // tile 0: the lanes-over-pairs kernel where it applies, the batch gives 2048 waves or more
-    // and no register tile or work distribution is requested; 1: the register-tile kernel;
+    // tile 0, with no register tile or work distribution requested: the lanes-over-pairs kernel
+    // where it applies, else (float data) the 16 x 16 shifts kernel; 1: the register-tile kernel;
     // 2: the lanes-over-pairs kernel (float and double data alike)
     if (opt.tile > 2)
         fail(XC_ERR_INVALID_ARGUMENT, "direct-method tile must be 0 (default), 1 (register tiles) or 2 (lanes over pairs)");
@@ -416,9 +654,20 @@ void launch_direct(const family_args& a, const T* L, const T* R, T* O, const xc_
                       opt.rows_per_step || opt.waves_per_block || opt.split || opt.rows_per_block;
     if (opt.tile == 2 && rights_per_left(a) == 0)
         fail(XC_ERR_UNSUPPORTED, "direct-method tile 2 (lanes over pairs) does not serve one_to_one");
-    if (opt.tile == 2 || (opt.tile == 0 && !keys && pairs_kernel_applies(a) && pairs_kernel_waves(a) >= 2048)) {
+    if (opt.tile == 2 || (opt.tile == 0 && !keys && pairs_kernel_applies(a, sizeof(T) == 4))) {
         launch_direct_pairs<T>(a, L, R, O, s);
         return;
+    }
+    if constexpr (std::is_same<T, float>::value) {
+        // Few rights per left: 16 x 16 shifts per wave or block, unless the matrices are so flat
+        // that a tile's 16 dy are mostly padding (16 rows < cols).  Measured, 16 pairs, us, against
+        // the register tiles: 20x100 29 / 41, 20x300 110 / 109, 20x1000 833 / 676, 40x1000 1970 /
+        // 1850, 64x1000 2950 / 4960, 1000x20 640 / 1150; its buffer offsets need matrices below
+        // 2^31 bytes.
+        if (opt.tile == 0 && !keys && 16ull * a.rows >= a.cols && (uint64_t)a.rows * a.cols < (1u << 29)) {
+            launch_direct_shifts(a, L, R, O, s);
+            return;
+        }
     }
     direct_plan d = plan_direct<T>(a, opt);
     if (d.lds > 160 * 1024) {
