@@ -1109,24 +1109,24 @@ fftk_geom geom_of(uint32_t H, uint32_t W, bool pow2_rows = false, bool plain = f
 // there are at least 8.  The occupancy is queried once per kernel and size.
 uint32_t resident_grid(const void* kernel, int threads, uint32_t lds, uint32_t items) {
     static std::mutex mu;
-    static std::vector<std::tuple<const void*, int, uint32_t, int, int>> known;  // kernel, threads, lds, dev, blocks
+    static std::vector<std::tuple<const void*, int, uint32_t, int, uint32_t>> known;  // kernel, threads, lds, dev, blocks
     int dev = 0;
     XC_HIP(hipGetDevice(&dev));
-    int per_cu = 0;
+    uint32_t resident = 0;
     {
         std::lock_guard<std::mutex> lock(mu);
         for (const auto& e : known)
             if (std::get<0>(e) == kernel && std::get<1>(e) == threads && std::get<2>(e) == lds && std::get<3>(e) == dev)
-                per_cu = std::get<4>(e);
-        if (per_cu == 0) {
+                resident = std::get<4>(e);
+        if (resident == 0) {
+            int per_cu = 0, cus = 0;
             XC_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, threads, lds));
-            per_cu = std::max(per_cu, 1);
-            known.emplace_back(kernel, threads, lds, dev, per_cu);
+            XC_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+            resident = (uint32_t)cus * (uint32_t)std::max(per_cu, 1);
+            known.emplace_back(kernel, threads, lds, dev, resident);
         }
     }
-    int cus = 0;
-    XC_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-    uint32_t g = std::min<uint32_t>(items, (uint32_t)cus * (uint32_t)per_cu);
+    uint32_t g = std::min<uint32_t>(items, resident);
     if (g >= 8) g -= g % 8;
     return std::max<uint32_t>(g, 1);
 }

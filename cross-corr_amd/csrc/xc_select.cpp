@@ -309,28 +309,34 @@ void cost_model_predict(const xc_workload& w, float* ms) {
 }
 
 int select_method(const xc_workload& w, xc_options& chosen) {
-    float f[kFeatures];
-    workload_features(w, f, kFeatures);
+    // The tables first: their keys are workloads that passed the checks below, and the features
+    // (some twenty logarithms) cost more than both lookups.
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) {
         (void)hipGetLastError();
         dev = -1;
     }
-    std::lock_guard<std::mutex> lock(g_mu);
-    auto it = g_tuned.find(std::make_tuple(w.family, w.rows, w.cols, w.n, w.m, dev));
-    if (it != g_tuned.end()) {
-        chosen = candidate(it->second);
-        return XC_SELECT_TUNED;
+    const auto wkey = std::make_tuple(w.family, w.rows, w.cols, w.n, w.m);
+    const bool tune = auto_mode() == "autotune";
+    {
+        std::lock_guard<std::mutex> lock(g_mu);
+        auto it = g_tuned.find(std::make_tuple(w.family, w.rows, w.cols, w.n, w.m, dev));
+        if (it != g_tuned.end()) {
+            chosen = candidate(it->second);
+            return XC_SELECT_TUNED;
+        }
+        auto pit = g_predicted.find(wkey);
+        if (!tune && pit != g_predicted.end()) {
+            chosen = candidate(pit->second);
+            return XC_SELECT_MODEL;
+        }
     }
-    if (auto_mode() == "autotune") return XC_SELECT_NONE;
+    float f[kFeatures];
+    workload_features(w, f, kFeatures);
+    if (tune) return XC_SELECT_NONE;
+    std::lock_guard<std::mutex> lock(g_mu);
     ensure_model_locked();
     if (!g_model.loaded || !in_domain(g_model, f)) return XC_SELECT_NONE;
-    const auto wkey = std::make_tuple(w.family, w.rows, w.cols, w.n, w.m);
-    auto pit = g_predicted.find(wkey);
-    if (pit != g_predicted.end()) {
-        chosen = candidate(pit->second);
-        return XC_SELECT_MODEL;
-    }
     std::vector<float> ms(g_model.cands.size());
     predict(g_model, f, ms.data());
     // A candidate is considered only up to twice the largest work it was timed on.
