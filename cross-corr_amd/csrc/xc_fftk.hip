@@ -11,7 +11,7 @@
 //              split into the two half spectra, written transposed as S[mat][k][r]
 //              (k = 0..Pc/2, only the H nonzero rows r);
 //   cols     : per (pair, column k): X = FFT of length Pr of S[right][k][0..H-1] (zero
-//              padded), then a second FFT of conj(Lhat) * X, conjugated:
+//              padded), then a second FFT of conj(Lhat) * X: the conjugate of
 //              Pr * IFFT(Lhat * conj(X)) (Lhat = the left's 2D spectrum, made by the same
 //              kernel in "left" mode), of which only the 2H-1 circular rows of the result
 //              are kept: Z[pair][k][z_row(rho)];
@@ -187,7 +187,8 @@ __device__ __forceinline__ void split_rows(const double2* buf, double2* __restri
     }
 }
 
-// rows_fwd for register transforms (up to 2048 points): a persistent grid of the blocks that
+// rows_fwd for register transforms (up to 2048 points; 65 matrices of 256^2 in 17.9 us, 4.8 TB/s;
+// 20.2 with index arithmetic per split value): a persistent grid of the blocks that
 // fit at once, each taking row groups (items: matrix, group of 2T rows) in turn and loading
 // the next item's rows into registers while it transforms and stores the current one, so
 // that HBM latency is paid once per block rather than once per item.  Items are dealt so
@@ -198,11 +199,13 @@ template <typename Tin, int LOGPC, int NT = rows_block<LOGPC, false>::NT>
 __global__ __launch_bounds__(NT) void rows_fwd_regs_kernel(const Tin* __restrict__ XL, const Tin* __restrict__ XR,
                                                            const uint64_t* __restrict__ moff,
                                                            const uint2* __restrict__ mdims, uint32_t nl, uint32_t H,
-                                                           uint32_t Hs, uint32_t W, int logT, uint32_t groups, uint32_t items,
+                                                           uint32_t Hs, uint32_t W, uint32_t groups, uint32_t items,
                                                            double2* __restrict__ SL, double2* __restrict__ SR,
                                                            const double2* __restrict__ tw) {
     static_assert(regs_of<LOGPC>::ON, "register transforms only");
-    constexpr int Q = 1 << (LOGPC - 3);
+    constexpr int Pc = 1 << LOGPC, Q = Pc / 8, T = 8 * NT / Pc, LOGT = rows_block<LOGPC, false>::LOGS - LOGPC;
+    constexpr uint32_t Kc = Pc / 2 + 1;
+    static_assert(T == 1 << LOGT, "transforms per block");
     extern __shared__ double2 buf[];
     const regs_pos<LOGPC> ps((int)threadIdx.x);
     const int t0 = ps.t0, t = ps.t, i = ps.i;
@@ -212,42 +215,35 @@ __global__ __launch_bounds__(NT) void rows_fwd_regs_kernel(const Tin* __restrict
     const uint32_t x = blockIdx.x % nx, kb = blockIdx.x / nx, bpx = gridDim.x / nx;
     const uint32_t per = (items + nx - 1) / nx;
     const uint32_t end = min((x + 1) * per, items);
-    // where item `it` lives: input rows a, b of this thread, sizes, output
+    // the matrix of item `it`, its size and the first row of its group
     struct where {
-        const Tin* xa;
-        const Tin* xb;
-        uint32_t Hm, Wm, r0, mat;
-        bool left, oka, okb;
+        uint32_t matg, r0, Hm, Wm;
     };
     auto locate = [&](uint32_t it) {
         where w;
-        const uint32_t matg = it / groups, g = it - matg * groups;
-        w.left = matg < nl;
-        w.mat = w.left ? matg : matg - nl;
-        w.r0 = g << (logT + 1);
+        w.matg = it / groups;
+        w.r0 = (it - w.matg * groups) << (LOGT + 1);
         w.Hm = H;
         w.Wm = W;
         if (mdims) {
-            const uint2 d = mdims[matg];
+            const uint2 d = mdims[w.matg];
             w.Hm = d.x;
             w.Wm = d.y;
         }
-        const Tin* Xm = (w.left ? XL : XR) + (moff ? moff[matg] : (size_t)w.mat * H * W);
-        const uint32_t a = w.r0 + 2 * t, b = a + 1;
-        w.oka = a < w.Hm;
-        w.okb = b < w.Hm;
-        w.xa = Xm + (w.oka ? (size_t)a * w.Wm : 0);
-        w.xb = Xm + (w.okb ? (size_t)b * w.Wm : 0);
         return w;
     };
-    // Branch-free loads from clamped (in-bounds) addresses; out-of-range positions are zeroed
-    // when the values are used.
+    // Rows r0 + 2t and the next; rows and columns outside the matrix read zero (W <= Pc / 2: the
+    // upper half of a row is padding).
     auto fetch = [&](const where& w, Tin (&va)[4], Tin (&vb)[4]) {
+        const uint32_t mat = w.matg < nl ? w.matg : w.matg - nl;
+        const Tin* Xm = (w.matg < nl ? XL : XR) + (moff ? moff[w.matg] : (size_t)mat * H * W);
+        const __amdgpu_buffer_rsrc_t rx = buf_of(Xm, w.Hm * w.Wm * (uint32_t)sizeof(Tin));
+        const uint32_t row = ((w.r0 + 2 * (uint32_t)t) * w.Wm + (uint32_t)i) * (uint32_t)sizeof(Tin);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {  // W <= Pc / 2: the upper half of a row is padding
-            const uint32_t c = i + Q * r, cc = c < w.Wm ? c : w.Wm - 1;
-            va[r] = w.xa[cc];
-            vb[r] = w.xb[cc];
+        for (int r = 0; r < 4; ++r) {
+            const uint32_t off = (uint32_t)(i + Q * r) < w.Wm ? row + (uint32_t)(Q * r * sizeof(Tin)) : kOut;
+            va[r] = buf_load_real<Tin>(rx, off, 0);
+            vb[r] = buf_load_real<Tin>(rx, off, w.Wm * (uint32_t)sizeof(Tin));
         }
     };
     uint32_t it = x * per + kb;
@@ -260,10 +256,7 @@ __global__ __launch_bounds__(NT) void rows_fwd_regs_kernel(const Tin* __restrict
         const bool more = nxt < end;
         double2 u[8];
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const bool in = i + Q * r < (int)cur.Wm;
-            u[r] = make_double2(cur.oka && in ? (double)va[r] : 0.0, cur.okb && in ? (double)vb[r] : 0.0);
-        }
+        for (int r = 0; r < 4; ++r) u[r] = make_double2((double)va[r], (double)vb[r]);
         where nw{};
         if (more) {  // the next item's rows are in flight during this item's transform and stores
             nw = locate(nxt);
@@ -272,10 +265,35 @@ __global__ __launch_bounds__(NT) void rows_fwd_regs_kernel(const Tin* __restrict
         if (cur.r0 < cur.Hm) {  // block-uniform: a row group beyond a smaller matrix is skipped
             fft_regs<LOGPC, true>(u, buf + at<LOGPC>(t0, 0), rr, t - t0, i);
 #pragma unroll
-            for (int r = 0; r < 8; ++r) buf[at<LOGPC>(t, i + Q * r)] = u[r];
+            for (int r = 0; r < 8; ++r)
+                buf[Q % 8 == 0 ? at<LOGPC>(t, i) + r * (Q + Q / 8) : at<LOGPC>(t, i + Q * r)] = u[r];
             __syncthreads();
-            split_rows<LOGPC, NT>(buf, (cur.left ? SL : SR) + (size_t)cur.mat * ((1 << LOGPC) / 2 + 1) * Hs, cur.r0,
-                                  cur.Hm, Hs, logT);
+            // Split into the rows' half spectra, column-major into S: with z = FFT(a + i b), A[k] =
+            // (z[k] + conj(z[P-k]))/2 and B[k] = (z[k] - conj(z[P-k]))/(2i).  A thread takes row rw
+            // of the group (an A or a B) at columns k0 + (Q/2) q; the component of z that the sum
+            // takes is the real one for A and the imaginary one for B, the other goes into the
+            // difference, so both read as 8-byte values at a lane's own offset.
+            const int rw = (int)threadIdx.x & (2 * T - 1), tq = rw >> 1, odd = rw & 1;
+            const int k0 = (int)threadIdx.x >> (LOGT + 1);
+            constexpr int KS = Q / 2;
+            const double hs = odd ? -0.5 : 0.5;
+            const double* zs = reinterpret_cast<const double*>(buf) + odd;      // the sum's component
+            const double* zd = reinterpret_cast<const double*>(buf) + 1 - odd;  // the difference's
+            const bool left = cur.matg < nl;
+            const size_t mat = left ? cur.matg : cur.matg - nl;
+            const __amdgpu_buffer_rsrc_t rs = buf_of((left ? SL : SR) + mat * Kc * Hs, Kc * Hs * 16u);
+            const uint32_t row = cur.r0 + (uint32_t)rw, step = KS * Hs * 16u;
+            const uint32_t off = row < cur.Hm ? ((uint32_t)k0 * Hs + row) * 16u : kOut;
+#pragma unroll
+            for (int q = 0; q < 8; ++q) {
+                const int a = KS % 8 == 0 ? at<LOGPC>(tq, k0) + q * (KS + KS / 8) : at<LOGPC>(tq, k0 + KS * q);
+                const int b = q == 0        ? at<LOGPC>(tq, (Pc - k0) & (Pc - 1))
+                              : KS % 8 == 0 ? at<LOGPC>(tq, Pc - k0) - q * (KS + KS / 8)
+                                            : at<LOGPC>(tq, Pc - k0 - KS * q);
+                buf_store(make_double2(0.5 * (zs[2 * a] + zs[2 * b]), hs * (zd[2 * a] - zd[2 * b])), rs, off, q * step);
+            }
+            if (k0 == 0)  // column Pc / 2
+                buf_store(make_double2(zs[2 * at<LOGPC>(tq, Pc / 2)], 0.0), rs, off, 8 * step);
             __syncthreads();  // the next item's transform reuses the slab
         }
         if (!more) break;
@@ -382,7 +400,7 @@ constexpr int cols_threads(int logP) { return logP <= 9 ? 64 : kFT; }
 // right of a pair); S keeps a column stride of Hs.
 // mode 1: item = pair q0 + item (left l, right r from the family's order, or from the pair
 // table of an uneven batch): X = the same FFT of SR[r][k], then a second FFT of
-// conj(Lhat) * X, conjugated: Pr * IFFT_rho(Lhat * conj(X)), whose circular row rho goes to
+// conj(Lhat) * X: the conjugate of Pr * IFFT_rho(Lhat * conj(X)), whose circular row rho goes to
 // Z[item][k][z_row(rho)] (column stride Ys; the rows between the result's two halves are
 // dropped).
 // Blocks are ordered column-group major through the XCD remap, so the pairs that read the
@@ -415,34 +433,30 @@ __global__ __launch_bounds__(cols_threads(LOGPR)) void cols_kernel(const double2
     if constexpr (regs_of<LOGPR>::ON) {
         // C = 8 * threads / Pr: the columns go from HBM to HBM through fft_regs; the product with
         // conj(Lhat) happens in registers between the two FFTs.
-        constexpr int Q = 1 << (LOGPR - 3);
+        constexpr int Q = 1 << (LOGPR - 3), P = 1 << LOGPR;
         const regs_pos<LOGPR> ps((int)threadIdx.x);
         const int t0 = ps.t0, i = ps.i;
         const uint32_t k = k0 + ps.t;
         const bool ok = k < Kc;
         double2* wb = buf + at<LOGPR>(t0, 0);
         const regs_roots<LOGPR> rr = load_roots<LOGPR>(i, tw);
+        const __amdgpu_buffer_rsrc_t rs = buf_of(Sm, Kc * Hs * 16u), rl = buf_of(Ll, Kc * (uint32_t)P * 16u);
+        const uint32_t so = (k * Hs + (uint32_t)i) * 16u, lo = ok ? (k * (uint32_t)P + (uint32_t)i) * 16u : kOut;
+        const uint32_t rows = ok ? Hq : 0;
         double2 u[8], lh[8];
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {  // Hq <= Pr / 2: the upper half of a column is padding
-            const uint32_t rho = i + Q * r;
-            u[r] = make_double2(0.0, 0.0);
-            if (ok && rho < Hq) u[r] = Sm[(size_t)k * Hs + rho];
-        }
-        double2* lk = Ll + (size_t)k * Pr;
+        for (int r = 0; r < 4; ++r)  // Hq <= Pr / 2: the upper half of a column is padding
+            u[r] = buf_load(rs, (uint32_t)(i + Q * r) < rows ? so + 16u * Q * r : kOut, 0);
         // The left spectrum is loaded together with the column (its latency overlaps the
         // first transform's).
+        if constexpr (MODE == 1) {
 #pragma unroll
-        for (int r = 0; r < 8; ++r) {
-            lh[r] = make_double2(0.0, 0.0);
-            if (MODE == 1 && ok) lh[r] = lk[i + Q * r];
+            for (int r = 0; r < 8; ++r) lh[r] = buf_load(rl, lo, 16u * Q * r);
         }
         fft_regs<LOGPR, true>(u, wb, rr, ps.t - t0, i);
         if constexpr (MODE == 0) {
-            if (ok) {
 #pragma unroll
-                for (int r = 0; r < 8; ++r) lk[i + Q * r] = u[r];
-            }
+            for (int r = 0; r < 8; ++r) buf_store(u[r], rl, lo, 16u * Q * r);
             return;
         }
 #pragma unroll
@@ -452,27 +466,15 @@ __global__ __launch_bounds__(cols_threads(LOGPR)) void cols_kernel(const double2
         int tl2 = ps.t - t0, i2 = i;
         asm volatile("" : "+v"(tl2), "+v"(i2));
         fft_regs<LOGPR>(u, wb, rr, tl2, i2);
-        if (ok) {
-            // rows from the opaque i2, so that the row indices of the loads are not kept live
-            // through both transforms for these stores
-            // z_row with constant offsets from two bases: rows below Hq in place, rows from
-            // Pr - Hq on down by Pr - Ys (for Pr = 2Hq one base and every row, row Hq
-            // included, which the row kernel reads as zero)
-            double2* zlo = Z + (size_t)item * Kc * Ys + (size_t)k * Ys + i2;
-            if (Pr == 2 * (int)Hq) {
+        // z_row: rows below Hq (r < 4: Hq <= Pr / 2) in place, rows above Pr - Hq (r >= 4) down by
+        // Pr - Ys; indices from the opaque i2, so that those of the loads are not kept live.
+        const __amdgpu_buffer_rsrc_t rz = buf_of(Z + (size_t)item * Kc * Ys, Kc * Ys * 16u);
+        const uint32_t zlo = (k * Ys + (uint32_t)i2) * 16u, zhi = zlo - ((uint32_t)P - Ys) * 16u;
 #pragma unroll
-                for (int r = 0; r < 8; ++r) zlo[Q * r] = cconj(u[r]);
-            } else {
-                double2* zhi = zlo - (Pr - (int)Ys);
-#pragma unroll
-                for (int r = 0; r < 8; ++r) {
-                    const uint32_t rho = (uint32_t)(i2 + Q * r);
-                    if (rho < Hq)
-                        zlo[Q * r] = cconj(u[r]);
-                    else if (rho >= (uint32_t)Pr - Hq)
-                        zhi[Q * r] = cconj(u[r]);
-                }
-            }
+        for (int r = 0; r < 8; ++r) {
+            const uint32_t rho = (uint32_t)(i2 + Q * r);
+            const bool in = r < 4 ? rho < rows : rho + rows > (uint32_t)P;
+            buf_store(u[r], rz, in ? (r < 4 ? zlo : zhi) + 16u * Q * r : kOut, 0);
         }
         return;
     } else {
@@ -522,7 +524,7 @@ __global__ __launch_bounds__(cols_threads(LOGPR)) void cols_kernel(const double2
         const int idx = threadIdx.x + kFT * q;
         const uint32_t k = k0 + (idx >> logPr);
         const int y = z_row((uint32_t)(idx & (Pr - 1)), Hq, Ys, (uint32_t)Pr);
-        if (k < Kc && y >= 0) Zq[(size_t)k * Ys + y] = cconj(buf[at<LOGPR>(idx >> logPr, idx & (Pr - 1))]);
+        if (k < Kc && y >= 0) Zq[(size_t)k * Ys + y] = buf[at<LOGPR>(idx >> logPr, idx & (Pr - 1))];
     }
     }
 }
@@ -534,7 +536,7 @@ __global__ __launch_bounds__(cols_threads(LOGPR)) void cols_kernel(const double2
 // is read as zero); output column ox = dx + W - 1 takes circular column dx mod Pc.  Pair q's
 // result starts at ooff[q] when the table is given, else at q times the result size.
 template <typename Tout, int LOGPC, int NT = rows_block<LOGPC, true>::NT>
-__global__ __launch_bounds__(NT) void rows_inv_kernel(const double2* __restrict__ Z, Tout* __restrict__ O,
+__global__ __launch_bounds__(NT) void rows_inv_slab_kernel(const double2* __restrict__ Z, Tout* __restrict__ O,
                                                        const uint64_t* __restrict__ ooff,
                                                        const uint2* __restrict__ ptab, const uint2* __restrict__ mdims,
                                                        uint32_t nl, uint32_t q0, uint32_t H, uint32_t W, uint32_t Ys,
@@ -559,15 +561,11 @@ __global__ __launch_bounds__(NT) void rows_inv_kernel(const double2* __restrict_
     const int rows2 = 2 << logT;
     if (z_gap(z0, (uint32_t)rows2, H, Ys)) return;  // between the two halves of the result
     const double2* Zq = Z + (size_t)item * Kc * Ys;
-    regs_roots<LOGPC> rr{};
-    slab_roots<LOGPC> sr{};
-    if constexpr (regs_of<LOGPC>::ON)
-        rr = load_roots<LOGPC>(regs_pos<LOGPC>((int)threadIdx.x).i, tw);
-    else
-        sr = load_slab_roots<LOGPC>(tw);
+    static_assert(!regs_of<LOGPC>::ON && NT == kFT, "slab transforms");
+    const slab_roots<LOGPC> sr = load_slab_roots<LOGPC>(tw);
     // One thread per (column kk, transform t) loads the two rows' values A[kk], B[kk] (32
-    // adjacent bytes) and writes both slots kk and Pc-kk of conj(Y), Y[k] = A[k] + i B[k]
-    // extended by A[Pc-k] = conj(A[k]), B[Pc-k] = conj(B[k]).
+    // adjacent bytes, conjugated) and writes both slots kk and Pc-kk of conj(Y), Y[k] = A[k] +
+    // i B[k] extended by A[Pc-k] = conj(A[k]), B[Pc-k] = conj(B[k]).
     {
         // At most TMAX = 2^LOGS / Pc transforms, so (Kc << logT) <= (Pc/2 + 1) * TMAX items: all
         // loads first, then the writes.
@@ -591,35 +589,12 @@ __global__ __launch_bounds__(NT) void rows_inv_kernel(const double2* __restrict_
             const int idx = threadIdx.x + NT * q;
             if (idx >= items) continue;
             const int kk = idx >> logT, t = idx & (T - 1);
-            buf[at<LOGPC>(t, kk)] = cadd(cconj(A[q]), mul_mi(cconj(B[q])));
-            if (kk > 0 && kk < half) buf[at<LOGPC>(t, Pc - kk)] = cadd(A[q], mul_mi(B[q]));
+            buf[at<LOGPC>(t, kk)] = cadd(A[q], mul_mi(B[q]));
+            if (kk > 0 && kk < half) buf[at<LOGPC>(t, Pc - kk)] = cadd(cconj(A[q]), mul_mi(cconj(B[q])));
         }
     }
     __syncthreads();
     Tout* Oq = O + (ooff ? ooff[q0 + item] : (size_t)(q0 + item) * (2 * H - 1) * SX);
-    if constexpr (regs_of<LOGPC>::ON) {
-        // T = 8 NT / Pc: the transforms (row pairs) go through fft_regs and are written from
-        // registers: thread (t, i) holds circular columns c = i + Q r of rows rho0 + 2t, +1.
-        constexpr int Q = 1 << (LOGPC - 3);
-        const regs_pos<LOGPC> ps((int)threadIdx.x);
-        const int t0 = ps.t0, t = ps.t, i = ps.i;
-        double2 u[8];
-#pragma unroll
-        for (int r = 0; r < 8; ++r) u[r] = buf[at<LOGPC>(t, i + Q * r)];
-        // a block-owned transform's first pass overwrites slots other waves still read
-        if constexpr (regs_of<LOGPC>::BLOCK) __syncthreads();
-        fft_regs<LOGPC>(u, buf + at<LOGPC>(t0, 0), rr, t - t0, i);
-        const int oa = out_row_of_z(z0 + 2 * t, H, Ys), ob = out_row_of_z(z0 + 2 * t + 1, H, Ys);
-#pragma unroll
-        for (int r = 0; r < 8; ++r) {
-            const int c = i + Q * r;
-            const int ox = c <= (int)W - 1 ? c + (int)W - 1 : (c >= Pc - (int)W + 1 ? c - (Pc - (int)W + 1) : -1);
-            if (ox < 0) continue;
-            if (oa >= 0) Oq[(size_t)oa * SX + ox] = (Tout)(u[r].x * scale);
-            if (ob >= 0) Oq[(size_t)ob * SX + ox] = (Tout)(-u[r].y * scale);
-        }
-        return;
-    } else {
     fft_slab<LOGPC>(buf, T, sr);
     // IFFT(Y) = conj(FFT(conj(Y))) / Pc: row A is the real part, row B minus the imaginary.
     for (int rr = threadIdx.x >> 6; rr < rows2; rr += NT / 64) {
@@ -633,6 +608,92 @@ __global__ __launch_bounds__(NT) void rows_inv_kernel(const double2* __restrict_
             orow[ox] = (Tout)(((rr & 1) ? -f.y : f.x) * scale);
         }
     }
+}
+
+// rows_inv for register transforms (up to 2048 points), T row pairs per block.  A thread's columns
+// kk0 + Q q and its LDS slots are a constant apart (Q = Pc / 8 threads per row pair), and rows and
+// columns outside the result are dropped by their buffer offsets, so that little but the FP64 work
+// is left: 422 VALU instructions at 512 points for 294 of FP64, where branches and index
+// arithmetic had made them 700 for 316 (64 pairs of 256^2 35.8 -> 33.1 us, 32 of 1024^2 430 -> 368).
+template <typename Tout, int LOGPC, int NT = rows_block<LOGPC, true>::NT>
+__global__ __launch_bounds__(NT) void rows_inv_regs_kernel(const double2* __restrict__ Z, Tout* __restrict__ O,
+                                                           const uint64_t* __restrict__ ooff,
+                                                           const uint2* __restrict__ ptab,
+                                                           const uint2* __restrict__ mdims, uint32_t nl, uint32_t q0,
+                                                           uint32_t H, uint32_t W, uint32_t Ys, uint32_t groups,
+                                                           double scale, const double2* __restrict__ tw) {
+    static_assert(regs_of<LOGPC>::ON, "register transforms only");
+    constexpr int Pc = 1 << LOGPC, half = Pc / 2, Q = Pc / 8;
+    constexpr uint32_t Kc = half + 1;
+    constexpr int T = 8 * NT / Pc, LOGT = rows_block<LOGPC, true>::LOGS - LOGPC;
+    static_assert(T == 1 << LOGT, "transforms per block");
+    extern __shared__ double2 buf[];
+    // XCD-aware order: the row groups of one pair run on one XCD, so the lines of Z that
+    // neighbouring groups read in pieces (2T rows of a column) are fetched into its L2 once.
+    const uint32_t bid = xcd_remap(blockIdx.x, gridDim.x);
+    const uint32_t item = bid / groups, g = bid - item * groups;
+    if (mdims) {  // uneven batch: this pair's own size (at most H x W)
+        const uint2 d = mdims[nl + ptab[q0 + item].y];
+        H = d.x;
+        W = d.y;
+    }
+    const uint32_t z0 = g << (LOGT + 1);
+    if (z_gap(z0, 2 * T, H, Ys)) return;  // between the two halves of the result
+    const regs_pos<LOGPC> ps((int)threadIdx.x);
+    const regs_roots<LOGPC> rr = load_roots<LOGPC>(ps.i, tw);
+    // Columns kk0 + Q q of row pair tq: A, B (conjugated) -> slots kk and Pc - kk of conj(Y), Y[k] =
+    // A[k] + i B[k] extended by A[Pc-k] = conj(A[k]), B[Pc-k] = conj(B[k]).
+    {
+        const int tq = (int)threadIdx.x & (T - 1), kk0 = (int)threadIdx.x >> LOGT;
+        const uint32_t za = z0 + 2 * tq;
+        const bool oka = out_row_of_z(za, H, Ys) >= 0, okb = out_row_of_z(za + 1, H, Ys) >= 0;
+        const __amdgpu_buffer_rsrc_t rz = buf_of(Z + (size_t)item * Kc * Ys, Kc * Ys * 16u);
+        const uint32_t voff = ((uint32_t)kk0 * Ys + za) * 16u, va = oka ? voff : kOut, vb = okb ? voff + 16u : kOut;
+        const uint32_t step = Q * Ys * 16u;
+        double2 A[4], B[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            A[q] = buf_load(rz, va, q * step);
+            B[q] = buf_load(rz, vb, q * step);
+        }
+        if (kk0 == 0) {  // column Pc / 2
+            const double2 a = buf_load(rz, va, 4 * step), b = buf_load(rz, vb, 4 * step);
+            buf[at<LOGPC>(tq, half)] = cadd(a, mul_mi(b));
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const double2 a = A[q], b = B[q];
+            // at(t, kk0 + Q q) = at(t, kk0) + q (Q + Q/8) when 8 divides Q, at(t, Pc - kk) likewise;
+            // slot Pc, for column 0, is the pad slot behind transform t
+            const int s0 = Q % 8 == 0 ? at<LOGPC>(tq, kk0) + q * (Q + Q / 8) : at<LOGPC>(tq, kk0 + Q * q);
+            const int s1 = Q % 8 == 0 ? at<LOGPC>(tq, Pc - kk0) - q * (Q + Q / 8) : at<LOGPC>(tq, Pc - kk0 - Q * q);
+            buf[s0] = make_double2(a.x + b.y, a.y - b.x);
+            buf[s1] = make_double2(a.x - b.y, -a.y - b.x);
+        }
+    }
+    __syncthreads();
+    const int t = ps.t, i = ps.i;
+    double2 u[8];
+#pragma unroll
+    for (int r = 0; r < 8; ++r)
+        u[r] = buf[Q % 8 == 0 ? at<LOGPC>(t, i) + r * (Q + Q / 8) : at<LOGPC>(t, i + Q * r)];
+    // a block-owned transform's first pass overwrites slots other waves still read
+    if constexpr (regs_of<LOGPC>::BLOCK) __syncthreads();
+    fft_regs<LOGPC>(u, buf + at<LOGPC>(ps.t0, 0), rr, t - ps.t0, i);
+    // IFFT(Y) = conj(FFT(conj(Y))) / Pc: row A is the real part, row B minus the imaginary; circular
+    // column c = i + Q r is shift c for r < 4 and c - Pc above (W <= Pc / 2).
+    const int SX = 2 * (int)W - 1;
+    Tout* Oq = O + (ooff ? ooff[q0 + item] : (size_t)(q0 + item) * (2 * H - 1) * SX);
+    const __amdgpu_buffer_rsrc_t ro = buf_of(Oq, (2 * H - 1) * (uint32_t)SX * (uint32_t)sizeof(Tout));
+    const int oa = out_row_of_z(z0 + 2 * t, H, Ys), ob = out_row_of_z(z0 + 2 * t + 1, H, Ys);
+    const uint32_t va = oa >= 0 ? (uint32_t)(oa * SX + i) * (uint32_t)sizeof(Tout) : kOut;
+    const uint32_t vb = ob >= 0 ? (uint32_t)(ob * SX + i) * (uint32_t)sizeof(Tout) : kOut;
+#pragma unroll
+    for (int r = 0; r < 8; ++r) {
+        const bool in = r < 4 ? i + Q * r < (int)W : i + Q * r > Pc - (int)W;
+        const uint32_t off = (uint32_t)(Q * r + (r < 4 ? (int)W - 1 : (int)W - 1 - Pc)) * (uint32_t)sizeof(Tout);
+        buf_store((Tout)(u[r].x * scale), ro, in && oa >= 0 ? va + off : kOut, 0);
+        buf_store((Tout)(-u[r].y * scale), ro, in && ob >= 0 ? vb + off : kOut, 0);
     }
 }
 
@@ -865,7 +926,7 @@ __global__ __launch_bounds__(rows3<LOGN>::NT) void rows_inv3_kernel(
     const int sub = ps.t, tt = sub / 3, m = sub - 3 * tt, i = ps.i;
     const regs_roots<LOGN> rr = load_roots<LOGN>(i, tw);
     const r3_roots<LOGN> w3 = load_r3_roots<LOGN>(tw3);
-    // Hermitian extension of the two rows of each transform (conjugated, as rows_inv_kernel)
+    // Hermitian extension of the two rows of each transform (conjugated, as rows_inv_regs_kernel)
     {
         constexpr int NQ = ((int)Kc * T + G::NT - 1) / G::NT;
         double2 A[NQ], B[NQ];
@@ -885,8 +946,8 @@ __global__ __launch_bounds__(rows3<LOGN>::NT) void rows_inv3_kernel(
             const int idx = threadIdx.x + G::NT * q;
             if (idx >= (int)Kc * T) continue;
             const int kk = idx >> G::LOGT, t = idx & (T - 1);
-            buf[xat<LOGN>(t, kk)] = cadd(cconj(A[q]), mul_mi(cconj(B[q])));
-            if (kk > 0 && kk < P / 2) buf[xat<LOGN>(t, P - kk)] = cadd(A[q], mul_mi(B[q]));
+            buf[xat<LOGN>(t, kk)] = cadd(A[q], mul_mi(B[q]));
+            if (kk > 0 && kk < P / 2) buf[xat<LOGN>(t, P - kk)] = cadd(cconj(A[q]), mul_mi(cconj(B[q])));
         }
     }
     __syncthreads();
@@ -1177,7 +1238,7 @@ void launch_job(const fftk_job& j, const Tio* L, const Tio* R, Tio* O, const fft
             const uint32_t grid = resident_grid(reinterpret_cast<const void*>(k), rows_threads(LOGPC, false),
                                                 g.v1.lds, items);
             launch_timed("fftk_rows_fwd", timing, k, dim3(grid), dim3(rows_threads(LOGPC, false)), g.v1.lds, s, L, R,
-                         j.moff, mdims, j.nl, H, g.Hs, W, g.v1.logT, g.g1, items, SL, SR, tw);
+                         j.moff, mdims, j.nl, H, g.Hs, W, g.g1, items, SL, SR, tw);
         } else {
             auto k = rows_fwd_slab_kernel<Tio, LOGPC>;
             allow_lds(k, g.v1.lds);
@@ -1214,11 +1275,19 @@ void launch_job(const fftk_job& j, const Tio* L, const Tio* R, Tio* O, const fft
             continue;
         }
         with_logp(g.logPc, [&](auto LP) {
-            auto k = rows_inv_kernel<Tio, decltype(LP)::value>;
-            allow_lds(k, g.v3.lds);
-            launch_timed("fftk_rows_inv", timing, k, dim3(nq * g.g3), dim3(rows_threads(g.logPc, true)), g.v3.lds, s,
-                         (const double2*)Zw, O, j.ooff, ptab, mdims, j.nl, q0, H, W, g.Ys,
-                         g.v3.logT, g.g3, scale, tw);
+            constexpr int LOGPC = decltype(LP)::value;
+            const dim3 grid(nq * g.g3), block(rows_threads(LOGPC, true));
+            if constexpr (regs_of<LOGPC>::ON) {
+                auto k = rows_inv_regs_kernel<Tio, LOGPC>;
+                allow_lds(k, g.v3.lds);
+                launch_timed("fftk_rows_inv", timing, k, grid, block, g.v3.lds, s, (const double2*)Zw, O, j.ooff, ptab,
+                             mdims, j.nl, q0, H, W, g.Ys, g.g3, scale, tw);
+            } else {
+                auto k = rows_inv_slab_kernel<Tio, LOGPC>;
+                allow_lds(k, g.v3.lds);
+                launch_timed("fftk_rows_inv", timing, k, grid, block, g.v3.lds, s, (const double2*)Zw, O, j.ooff, ptab,
+                             mdims, j.nl, q0, H, W, g.Ys, g.v3.logT, g.g3, scale, tw);
+            }
         });
     }
     XC_HIP(hipGetLastError());
@@ -1427,9 +1496,9 @@ uint32_t fftk_row_len(uint32_t cols) {
 }
 
 std::pair<uint32_t, uint32_t> fftk_class(uint32_t rows, uint32_t cols) {
-    const fftk_geom g = geom_of(rows, cols);
-    if (g.small) return {1u << g.logPrs, 1u << g.logPcs};
-    return {g.Pr, g.Pc};
+    const int lr = std::max(5, ilog2_ceil(2 * rows - 1)), lc = std::max(5, ilog2_ceil(2 * cols - 1));
+    if (fftk_small_fits(lr, lc)) return {1u << lr, 1u << lc};
+    return {fftk_col_len(rows), fftk_row_len(cols)};
 }
 
 fftk_ws_sizes fftk_sizes(const fftk_job& j) {

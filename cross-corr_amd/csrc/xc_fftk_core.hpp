@@ -35,6 +35,36 @@ __device__ __forceinline__ double2 cadd(double2 a, double2 b) { return make_doub
 __device__ __forceinline__ double2 csub(double2 a, double2 b) { return make_double2(a.x - b.x, a.y - b.y); }
 __device__ __forceinline__ double2 mul_mi(double2 a) { return make_double2(a.y, -a.x); }  // (-i) * a
 
+// Bounds-checked buffer accesses relative to a wave-uniform base: `voff` bytes per lane plus a
+// uniform `soff`; past `bytes` (below 2^31: kOut always is) loads give zero and stores do nothing,
+// so a condition costs one select of the offset instead of a branch and a cleared register.
+constexpr uint32_t kOut = 0x80000000u;
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t buf_of(const void* base, uint32_t bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, bytes, 0x00020000);
+}
+typedef int i32x4 __attribute__((ext_vector_type(4)));
+typedef int i32x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ double2 buf_load(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) {
+    const i32x4 v = __builtin_amdgcn_raw_buffer_load_b128(r, (int)voff, (int)soff, 0);
+    return __builtin_bit_cast(double2, v);
+}
+template <typename T>
+__device__ __forceinline__ T buf_load_real(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) {
+    if constexpr (sizeof(T) == 4)
+        return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b32(r, (int)voff, (int)soff, 0));
+    else
+        return __builtin_bit_cast(T, (i32x2)__builtin_amdgcn_raw_buffer_load_b64(r, (int)voff, (int)soff, 0));
+}
+__device__ __forceinline__ void buf_store(double2 v, __amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) {
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(i32x4, v), r, (int)voff, (int)soff, 0);
+}
+__device__ __forceinline__ void buf_store(float v, __amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) {
+    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, v), r, (int)voff, (int)soff, 0);
+}
+__device__ __forceinline__ void buf_store(double v, __amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) {
+    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(i32x2, v), r, (int)voff, (int)soff, 0);
+}
+
 // In-register forward DFT of R points: X[k] = sum_j u[j] exp(-2 pi i jk / R).
 __device__ __forceinline__ void dft2(double2& a, double2& b) {
     const double2 t = a;
@@ -48,6 +78,33 @@ __device__ __forceinline__ void dft4(double2& u0, double2& u1, double2& u2, doub
     u1 = cadd(t1, t3);
     u3 = csub(t1, t3);
 }
+// The last two levels of an 8-point DFT from its first: t0, t1 = x0 +- x4, t2, t3 = x2 +- x6,
+// s0, s1 = x1 +- x5, s2, s3 = x3 +- x7.  The rotations by odd eighths, c (p, q), go into the sums
+// as FMAs: 36 instructions where rotating first took 40.
+__device__ __forceinline__ void dft8_last(double2 t0, double2 t1, double2 t2, double2 t3, double2 s0, double2 s1,
+                                          double2 s2, double2 s3, double2 (&u)[8]) {
+    constexpr double c = 0.70710678118654752440;  // sqrt(1/2)
+    const double2 e0 = cadd(t0, t2), e2 = csub(t0, t2), o0 = cadd(s0, s2), o2 = csub(s0, s2);
+    const double2 e1 = make_double2(t1.x + t3.y, t1.y - t3.x), e3 = make_double2(t1.x - t3.y, t1.y + t3.x);
+    const double2 o1 = make_double2(s1.x + s3.y, s1.y - s3.x), o3 = make_double2(s1.x - s3.y, s1.y + s3.x);
+    u[0] = cadd(e0, o0);
+    u[4] = csub(e0, o0);
+    u[2] = make_double2(e2.x + o2.y, e2.y - o2.x);
+    u[6] = make_double2(e2.x - o2.y, e2.y + o2.x);
+    const double p1 = o1.x + o1.y, q1 = o1.y - o1.x, p3 = o3.y - o3.x, q3 = o3.x + o3.y;
+    u[1] = make_double2(fma(c, p1, e1.x), fma(c, q1, e1.y));
+    u[5] = make_double2(fma(-c, p1, e1.x), fma(-c, q1, e1.y));
+    u[3] = make_double2(fma(c, p3, e3.x), fma(-c, q3, e3.y));
+    u[7] = make_double2(fma(-c, p3, e3.x), fma(c, q3, e3.y));
+}
+// s = a + w b, d = a - w b = 2 a - s: 6 FMAs where product, sum and difference took 8
+// instructions.
+__device__ __forceinline__ void bfly(double2 a, double2 w, double2 b, double2& s, double2& d) {
+    s.x = fma(w.x, b.x, fma(-w.y, b.y, a.x));
+    s.y = fma(w.x, b.y, fma(w.y, b.x, a.y));
+    d.x = fma(2.0, a.x, -s.x);
+    d.y = fma(2.0, a.y, -s.y);
+}
 template <int R>
 __device__ __forceinline__ void dft(double2 (&u)[R]) {
     if constexpr (R == 2) {
@@ -56,23 +113,9 @@ __device__ __forceinline__ void dft(double2 (&u)[R]) {
         dft4(u[0], u[1], u[2], u[3]);
     } else {
         static_assert(R == 8, "radix");
-        constexpr double c = 0.70710678118654752440;  // sqrt(1/2)
-        double2 e0 = u[0], e1 = u[2], e2 = u[4], e3 = u[6];
-        double2 o0 = u[1], o1 = u[3], o2 = u[5], o3 = u[7];
-        dft4(e0, e1, e2, e3);
-        dft4(o0, o1, o2, o3);
-        // o_k *= exp(-2 pi i k / 8)
-        o1 = make_double2(c * (o1.x + o1.y), c * (o1.y - o1.x));
-        o2 = mul_mi(o2);
-        o3 = make_double2(c * (o3.y - o3.x), -c * (o3.x + o3.y));
-        u[0] = cadd(e0, o0);
-        u[4] = csub(e0, o0);
-        u[1] = cadd(e1, o1);
-        u[5] = csub(e1, o1);
-        u[2] = cadd(e2, o2);
-        u[6] = csub(e2, o2);
-        u[3] = cadd(e3, o3);
-        u[7] = csub(e3, o3);
+        const double2 t0 = cadd(u[0], u[4]), t1 = csub(u[0], u[4]), t2 = cadd(u[2], u[6]), t3 = csub(u[2], u[6]);
+        const double2 s0 = cadd(u[1], u[5]), s1 = csub(u[1], u[5]), s2 = cadd(u[3], u[7]), s3 = csub(u[3], u[7]);
+        dft8_last(t0, t1, t2, t3, s0, s1, s2, s3, u);
     }
 }
 
@@ -142,22 +185,10 @@ __device__ __forceinline__ double2 rot8(double2 a) {
     else return make_double2(c * (a.y - a.x), -c * (a.x + a.y));
 }
 
-// The first pass's DFT of 8 values whose upper four are zero (a zero-padded input): 40 FP64
-// instructions against 56.
+// The first pass's DFT of 8 values whose upper four are zero (a zero-padded input): 36 FP64
+// instructions against 52.
 __device__ __forceinline__ void dft8_half(double2 (&u)[8]) {
-    const double2 a0 = u[0], a1 = u[2], b0 = u[1], b1 = u[3];
-    const double2 ja = mul_mi(a1), jb = mul_mi(b1);
-    const double2 e0 = cadd(a0, a1), e1 = cadd(a0, ja), e2 = csub(a0, a1), e3 = csub(a0, ja);
-    const double2 o0 = cadd(b0, b1), o1 = rot8<1>(cadd(b0, jb)), o2 = mul_mi(csub(b0, b1)),
-                  o3 = rot8<3>(csub(b0, jb));
-    u[0] = cadd(e0, o0);
-    u[4] = csub(e0, o0);
-    u[1] = cadd(e1, o1);
-    u[5] = csub(e1, o1);
-    u[2] = cadd(e2, o2);
-    u[6] = csub(e2, o2);
-    u[3] = cadd(e3, o3);
-    u[7] = csub(e3, o3);
+    dft8_last(u[0], u[0], u[2], u[2], u[1], u[1], u[3], u[3], u);
 }
 
 // Swap of one register index bit with bit 5 (4) of the lane: a holds index 0, b index 1.
@@ -233,35 +264,34 @@ __device__ __forceinline__ void fft_regs_passes(double2 (&u)[8], double2* wb, in
     double2 w1 = rr.w[LOGPP / 3 - 1];
     asm volatile("" : "+v"(w1.x), "+v"(w1.y));
     if constexpr (LOGP - LOGPP == 1) {  // radix 2: butterfly i + Q m takes u[m], u[m + 4]
-        u[4] = cmul(u[4], w1);
-        u[5] = cmul(u[5], rot8<1>(w1));
-        u[6] = cmul(u[6], mul_mi(w1));
-        u[7] = cmul(u[7], rot8<3>(w1));
-#pragma unroll
-        for (int m = 0; m < 4; ++m) dft2(u[m], u[m + 4]);
+        bfly(u[0], w1, u[4], u[0], u[4]);
+        bfly(u[1], rot8<1>(w1), u[5], u[1], u[5]);
+        bfly(u[2], mul_mi(w1), u[6], u[2], u[6]);
+        bfly(u[3], rot8<3>(w1), u[7], u[3], u[7]);
     } else if constexpr (LOGP - LOGPP == 2) {  // radix 4: butterfly i + Q m takes u[m + 2 r]
 #pragma unroll
         for (int m = 0; m < 2; ++m) {
             const double2 wm = m ? rot8<1>(w1) : w1;
             const double2 w2 = csqr(wm);
-            u[m + 2] = cmul(u[m + 2], wm);
-            u[m + 4] = cmul(u[m + 4], w2);
-            u[m + 6] = cmul(u[m + 6], cmul(w2, wm));
-            dft4(u[m], u[m + 2], u[m + 4], u[m + 6]);
+            double2 t0, t1, t2, t3;
+            bfly(u[m], w2, u[m + 4], t0, t1);
+            bfly(cmul(u[m + 2], wm), cmul(w2, wm), u[m + 6], t2, t3);
+            u[m] = cadd(t0, t2);
+            u[m + 4] = csub(t0, t2);
+            u[m + 2] = make_double2(t1.x + t3.y, t1.y - t3.x);
+            u[m + 6] = make_double2(t1.x - t3.y, t1.y + t3.x);
         }
     } else {
-        // the powers as a tree: squares take 3 instructions and the chain is 3 long, not 6
-        u[1] = cmul(u[1], w1);
-        const double2 w2 = csqr(w1);
-        u[2] = cmul(u[2], w2);
-        const double2 w3 = cmul(w2, w1);
-        u[3] = cmul(u[3], w3);
-        const double2 w4 = csqr(w2);
-        u[4] = cmul(u[4], w4);
-        u[5] = cmul(u[5], cmul(w4, w1));
-        u[6] = cmul(u[6], csqr(w3));
-        u[7] = cmul(u[7], cmul(w4, w3));
-        dft<8>(u);
+        // The powers as a tree (squares take 3 instructions and the chain is 3 long, not 6); the
+        // products of the upper four inputs go into the first level's sums (bfly): 93 FP64
+        // instructions against 105.
+        const double2 w2 = csqr(w1), w3 = cmul(w2, w1), w4 = csqr(w2);
+        double2 t0, t1, t2, t3, s0, s1, s2, s3;
+        bfly(u[0], w4, u[4], t0, t1);
+        bfly(cmul(u[1], w1), cmul(w4, w1), u[5], s0, s1);
+        bfly(cmul(u[2], w2), csqr(w3), u[6], t2, t3);
+        bfly(cmul(u[3], w3), cmul(w4, w3), u[7], s2, s3);
+        dft8_last(t0, t1, t2, t3, s0, s1, s2, s3, u);
         regs_sync<regs_of<LOGP>::BLOCK>();
         if constexpr (LOGPP + 3 < LOGP) fft_regs_next<LOGP, LOGPP + 3>(u, wb, tl, i, rr);
     }
