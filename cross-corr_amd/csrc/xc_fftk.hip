@@ -243,7 +243,7 @@ __global__ __launch_bounds__(NT) void rows_fwd_regs_kernel(const Tin* __restrict
         for (int r = 0; r < 4; ++r) {
             const uint32_t off = (uint32_t)(i + Q * r) < w.Wm ? row + (uint32_t)(Q * r * sizeof(Tin)) : kOut;
             va[r] = buf_load_real<Tin>(rx, off, 0);
-            vb[r] = buf_load_real<Tin>(rx, off, w.Wm * (uint32_t)sizeof(Tin));
+            vb[r] = buf_load_real<Tin>(rx, off + w.Wm * (uint32_t)sizeof(Tin), 0);
         }
     };
     uint32_t it = x * per + kb;

@@ -36,8 +36,9 @@ __device__ __forceinline__ double2 csub(double2 a, double2 b) { return make_doub
 __device__ __forceinline__ double2 mul_mi(double2 a) { return make_double2(a.y, -a.x); }  // (-i) * a
 
 // Bounds-checked buffer accesses relative to a wave-uniform base: `voff` bytes per lane plus a
-// uniform `soff`; past `bytes` (below 2^31: kOut always is) loads give zero and stores do nothing,
-// so a condition costs one select of the offset instead of a branch and a cleared register.
+// uniform `soff`; with `voff` past `bytes` (below 2^31: kOut always is) loads give zero and stores do
+// nothing, so a condition costs one select of the offset instead of a branch and a cleared
+// register.  Only `voff` may be what leaves the buffer: `soff` stays inside it by construction.
 constexpr uint32_t kOut = 0x80000000u;
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t buf_of(const void* base, uint32_t bytes) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, bytes, 0x00020000);
