@@ -698,11 +698,22 @@ __global__ __launch_bounds__(NT) void rows_inv_regs_kernel(const double2* __rest
 }
 
 // Row transforms of P = 3N points (N = 2^LOGN, 16..512), for widths where 3N >= 2W - 1 is
-// shorter than the power of two.  Each of a block's T transforms (row pairs) is split into
-// the three sub-sequences x[3n + m] (m = 0, 1, 2) of N points, which go through fft_regs<LOGN>
-// as 3T wave-owned transforms (sub-transform s = 3t + m); a radix-3 pass through LDS combines
-// them (decimation in time): with F_m the sub-spectra and w = exp(-2 pi i / P),
-//   X[k + N j] = F_0[k] + W_3^j w^k F_1[k] + W_3^2j w^2k F_2[k],  j = 0, 1, 2.
+// shorter than the power of two.  A transform (row pair) is three of N points through
+// fft_regs<LOGN> (3T wave-owned transforms per block, sub-transform 3t + m) and one radix-3 step,
+// with w = exp(-2 pi i / P) and W_3 = w^N:
+//   forward (decimation in time): F_m = FFT of x[3n + m]; the split into the two rows' spectra is
+//     done on the F_m, a_m[k] = (F_m[k] + conj(F_m[N-k])) / 2 and b_m[k] = (F_m[k] -
+//     conj(F_m[N-k])) / 2i, and row A's bins are A[k + N j] = sum_m w^(km) W_3^(jm) a_m[k] for
+//     k = 0..N/2 (bin k + 2N is the conjugate of bin N - k), so the spectrum of the pair never
+//     goes through LDS;
+//   inverse (decimation in frequency): from the conjugated bins k, N + k, N - k of rows A and B,
+//     ah_m = w^(km) sum_j W_3^(jm) conj(A[k + N j]) and bh_m, the sub-sequences of the extended
+//     row are y_m[k] = ah_m - i bh_m and y_m[N - k] = conj(ah_m) - i conj(bh_m); their transforms
+//     give X[3q + m], which go through LDS as real output values so that rows are stored whole.
+// HBM-bound.  Splitting the sub-transforms' spectra instead of the whole one saves a write and a
+// read of all values through LDS with a barrier in both directions, and bounds-checked loads and
+// stores a branch per element: at 65 matrices of 350^2 rows_fwd3 54 -> 43 us (3.9 TB/s), rows_inv3
+// 125 -> 111 us (3.6 TB/s); the whole call 291 -> 254 us, 640^2 1124 -> 977, 190^2 69.7 -> 63.8.
 // A block holds T transforms (3T N / 8 threads, a multiple of 64): 2 at 1536 points (two
 // blocks per CU measured faster than one), 4 from 384 to 768, more below (192 threads).
 constexpr int rows3_t(int logN) { return logN >= 9 ? 2 : (logN >= 7 ? 4 : 512 >> logN); }
@@ -712,71 +723,27 @@ struct rows3 {
     static constexpr int T = rows3_t(LOGN);                 // transforms (row pairs) per block
     static constexpr int NT = 3 * T * N / 8;
     static constexpr int LOGT = T == 2 ? 1 : (T == 4 ? 2 : (T == 8 ? 3 : (T == 16 ? 4 : 5)));
-    static constexpr int XS = P + P / 8 + 1;                // LDS stride of a whole transform
-    static constexpr int SLOTS = 3 * T * (N + N / 8 + 1) > T * XS ? 3 * T * (N + N / 8 + 1) : T * XS;
-    static constexpr int NI = (T * N + NT - 1) / NT;        // radix-3 butterflies per thread
+    static constexpr int SLOTS = 3 * T * (N + N / 8 + 1);
+    static constexpr int FS = NT / (2 * T), IS = NT / T;    // k steps of the split and of the extension
+    static constexpr int FQ = 3, IQ = 2;                    // and their number: k = 0..N/2
     static_assert(NT % 64 == 0 && NT <= 1024 && (1 << LOGT) == T && 8 * NT == T * P, "rows3 geometry");
+    static_assert(FS * FQ > N / 2 && IS * IQ > N / 2, "rows3 steps");
 };
-template <int LOGN>
-__device__ __forceinline__ int xat(int t, int p) {
-    return t * rows3<LOGN>::XS + p + (p >> 3);
-}
 
 // tw3[j] = exp(-2 pi i j / 12288): the P-th roots for P = 3 * 2^n <= 12288, one table per
 // device, kept for the process.
 constexpr int kTw3 = 3 * kSlab;
 const double2* twiddles3();
 
-// Radix-3 butterfly of the combine pass: (a, b, c) = (F_0, w^k F_1, w^2k F_2) -> X[k + N j].
+// 3-point DFT: x0 = a + b + c, x1 and x2 its other bins.
 __device__ __forceinline__ void dft3(const double2 a, const double2 b, const double2 c, double2& x0, double2& x1,
                                      double2& x2) {
     constexpr double h = 0.86602540378443864676;  // sqrt(3) / 2
     const double2 sm = cadd(b, c), df = csub(b, c);
     const double2 t1 = make_double2(a.x - 0.5 * sm.x, a.y - 0.5 * sm.y);
-    const double2 t2 = make_double2(h * df.y, -h * df.x);  // -i sqrt(3)/2 (b - c)
     x0 = cadd(a, sm);
-    x1 = cadd(t1, t2);
-    x2 = csub(t1, t2);
-}
-
-// Twiddles w^k, w^2k of this thread's radix-3 butterflies (idx = threadIdx + NT q, k = idx mod
-// N), read at kernel start like the pass roots (a table read between two LDS phases would
-// wait on memory).
-template <int LOGN>
-struct r3_roots {
-    double2 w1[rows3<LOGN>::NI], w2[rows3<LOGN>::NI];
-};
-template <int LOGN>
-__device__ __forceinline__ r3_roots<LOGN> load_r3_roots(const double2* __restrict__ tw3) {
-    using G = rows3<LOGN>;
-    r3_roots<LOGN> w;
-#pragma unroll
-    for (int q = 0; q < G::NI; ++q) {
-        const int k = ((int)threadIdx.x + G::NT * q) & (G::N - 1);
-        w.w1[q] = tw3[k * (kTw3 / G::P)];
-        w.w2[q] = tw3[2 * k * (kTw3 / G::P)];
-    }
-    return w;
-}
-
-// The radix-3 pass of the block's T transforms: sub-spectra F_m[k] at at<LOGN>(3t + m, k) in
-// buf -> X[t][k + N j] in registers (this thread's butterflies idx = threadIdx + NT q,
-// t = idx / N, k = idx mod N).
-template <int LOGN>
-__device__ __forceinline__ void radix3_pass(const double2* buf, const r3_roots<LOGN>& w,
-                                            double2 (&X)[rows3<LOGN>::NI][3]) {
-    using G = rows3<LOGN>;
-#pragma unroll
-    for (int q = 0; q < G::NI; ++q) {
-        const int idx = (int)threadIdx.x + G::NT * q;
-        const int tt = idx >> LOGN, k = idx & (G::N - 1);
-        if (idx < G::T * G::N) {
-            const double2 f0 = buf[at<LOGN>(3 * tt, k)];
-            const double2 f1 = cmul(w.w1[q], buf[at<LOGN>(3 * tt + 1, k)]);
-            const double2 f2 = cmul(w.w2[q], buf[at<LOGN>(3 * tt + 2, k)]);
-            dft3(f0, f1, f2, X[q][0], X[q][1], X[q][2]);
-        }
-    }
+    x1 = make_double2(fma(h, df.y, t1.x), fma(-h, df.x, t1.y));
+    x2 = make_double2(fma(-h, df.y, t1.x), fma(h, df.x, t1.y));
 }
 
 // rows_fwd for P = 3N: a persistent grid as rows_fwd_regs_kernel (items: matrix, group of 2T
@@ -790,51 +757,51 @@ __global__ __launch_bounds__(rows3<LOGN>::NT) void rows_fwd3_kernel(
     uint32_t items, double2* __restrict__ SL, double2* __restrict__ SR, const double2* __restrict__ tw,
     const double2* __restrict__ tw3) {
     using G = rows3<LOGN>;
-    constexpr int N = G::N, P = G::P, Q = G::Q, T = G::T;
+    constexpr int N = G::N, P = G::P, Q = G::Q, T = G::T, FS = G::FS;
     constexpr uint32_t Kc = P / 2 + 1;
     extern __shared__ double2 buf[];
     const regs_pos<LOGN> ps((int)threadIdx.x);
     const int sub = ps.t, tt = sub / 3, m = sub - 3 * tt, i = ps.i;
     const regs_roots<LOGN> rr = load_roots<LOGN>(i, tw);
-    const r3_roots<LOGN> w3 = load_r3_roots<LOGN>(tw3);
+    // the split: row rw of the group (an A or a B of row pair tq) at k = k0 + FS q
+    const int rw = (int)threadIdx.x & (2 * T - 1), tq = rw >> 1, odd = rw & 1;
+    const int k0 = (int)threadIdx.x >> (G::LOGT + 1);
+    double2 w1[G::FQ];
+#pragma unroll
+    for (int q = 0; q < G::FQ; ++q) w1[q] = tw3[(k0 + FS * q) * (kTw3 / P)];
     const uint32_t nx = gridDim.x >= 8 ? 8 : 1;
     const uint32_t x = blockIdx.x % nx, kb = blockIdx.x / nx, bpx = gridDim.x / nx;
     const uint32_t per = (items + nx - 1) / nx;
     const uint32_t end = min((x + 1) * per, items);
     struct where {
-        const Tin* xa;
-        const Tin* xb;
-        uint32_t Hm, Wm, r0, mat;
-        bool left, oka, okb;
+        uint32_t matg, r0, Hm, Wm;
     };
     auto locate = [&](uint32_t it) {
         where w;
-        const uint32_t matg = it / groups, g = it - matg * groups;
-        w.left = matg < nl;
-        w.mat = w.left ? matg : matg - nl;
-        w.r0 = g * (2 * T);
+        w.matg = it / groups;
+        w.r0 = (it - w.matg * groups) * (2 * T);
         w.Hm = H;
         w.Wm = W;
         if (mdims) {
-            const uint2 d = mdims[matg];
+            const uint2 d = mdims[w.matg];
             w.Hm = d.x;
             w.Wm = d.y;
         }
-        const Tin* Xm = (w.left ? XL : XR) + (moff ? moff[matg] : (size_t)w.mat * H * W);
-        const uint32_t a = w.r0 + 2 * tt, b = a + 1;
-        w.oka = a < w.Hm;
-        w.okb = b < w.Hm;
-        w.xa = Xm + (w.oka ? (size_t)a * w.Wm : 0);
-        w.xb = Xm + (w.okb ? (size_t)b * w.Wm : 0);
         return w;
     };
-    // element n = i + Q r of sub-sequence m is column 3n + m; loads from clamped addresses
+    // element n = i + Q r of sub-sequence m is column 3n + m; rows and columns outside the matrix
+    // read zero (W <= P / 2: the upper half of a sub-sequence is padding)
     auto fetch = [&](const where& w, Tin (&va)[4], Tin (&vb)[4]) {
+        const uint32_t mat = w.matg < nl ? w.matg : w.matg - nl;
+        const Tin* Xm = (w.matg < nl ? XL : XR) + (moff ? moff[w.matg] : (size_t)mat * H * W);
+        const __amdgpu_buffer_rsrc_t rx = buf_of(Xm, w.Hm * w.Wm * (uint32_t)sizeof(Tin));
+        const uint32_t c0 = 3u * (uint32_t)i + (uint32_t)m;
+        const uint32_t row = ((w.r0 + 2 * (uint32_t)tt) * w.Wm + c0) * (uint32_t)sizeof(Tin);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {  // W <= P / 2: the upper half of a sub-sequence is padding
-            const uint32_t c = 3u * (uint32_t)(i + Q * r) + (uint32_t)m, cc = c < w.Wm ? c : w.Wm - 1;
-            va[r] = w.xa[cc];
-            vb[r] = w.xb[cc];
+        for (int r = 0; r < 4; ++r) {
+            const uint32_t off = c0 + 3u * Q * r < w.Wm ? row + (uint32_t)(3 * Q * r * sizeof(Tin)) : kOut;
+            va[r] = buf_load_real<Tin>(rx, off, 0);
+            vb[r] = buf_load_real<Tin>(rx, off + w.Wm * (uint32_t)sizeof(Tin), 0);
         }
     };
     uint32_t it = x * per + kb;
@@ -847,10 +814,7 @@ __global__ __launch_bounds__(rows3<LOGN>::NT) void rows_fwd3_kernel(
         const bool more = nxt < end;
         double2 u[8];
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const bool in = 3u * (uint32_t)(i + Q * r) + (uint32_t)m < cur.Wm;
-            u[r] = make_double2(cur.oka && in ? (double)va[r] : 0.0, cur.okb && in ? (double)vb[r] : 0.0);
-        }
+        for (int r = 0; r < 4; ++r) u[r] = make_double2((double)va[r], (double)vb[r]);
         where nw{};
         if (more) {
             nw = locate(nxt);
@@ -859,38 +823,35 @@ __global__ __launch_bounds__(rows3<LOGN>::NT) void rows_fwd3_kernel(
         if (cur.r0 < cur.Hm) {  // block-uniform: a row group beyond a smaller matrix is skipped
             fft_regs<LOGN, true>(u, buf + at<LOGN>(ps.t0, 0), rr, sub - ps.t0, i);
 #pragma unroll
-            for (int r = 0; r < 8; ++r) buf[at<LOGN>(sub, i + Q * r)] = u[r];
+            for (int r = 0; r < 8; ++r)
+                buf[Q % 8 == 0 ? at<LOGN>(sub, i) + r * (Q + Q / 8) : at<LOGN>(sub, i + Q * r)] = u[r];
             __syncthreads();
-            double2 X[G::NI][3];
-            radix3_pass<LOGN>(buf, w3, X);
-            __syncthreads();  // X overwrites the sub-spectra
+            // the components of F_m that row rw takes, as in rows_fwd_regs_kernel
+            const double hs = odd ? -0.5 : 0.5;
+            const double* zs = reinterpret_cast<const double*>(buf) + odd;
+            const double* zd = reinterpret_cast<const double*>(buf) + 1 - odd;
+            const bool left = cur.matg < nl;
+            const size_t mat = left ? cur.matg : cur.matg - nl;
+            const __amdgpu_buffer_rsrc_t rs = buf_of((left ? SL : SR) + mat * Kc * Hs, Kc * Hs * 16u);
+            const uint32_t row = cur.r0 + (uint32_t)rw;
 #pragma unroll
-            for (int q = 0; q < G::NI; ++q) {
-                const int idx = (int)threadIdx.x + G::NT * q;
-                if (idx < T * N) {
-                    const int t2 = idx >> LOGN, k = idx & (N - 1);
+            for (int q = 0; q < G::FQ; ++q) {
+                const int k = k0 + FS * q;
+                if (k > N / 2) continue;
+                double2 f[3];
 #pragma unroll
-                    for (int j = 0; j < 3; ++j) buf[xat<LOGN>(t2, k + N * j)] = X[q][j];
+                for (int mm = 0; mm < 3; ++mm) {
+                    const int a = at<LOGN>(3 * tq + mm, k), b = at<LOGN>(3 * tq + mm, (N - k) & (N - 1));
+                    f[mm] = make_double2(0.5 * (zs[2 * a] + zs[2 * b]), hs * (zd[2 * a] - zd[2 * b]));
                 }
-            }
-            __syncthreads();
-            // split into the two rows' half spectra (as split_rows), column-major into S
-            double2* Sm = (cur.left ? SL : SR) + (size_t)cur.mat * Kc * Hs;
-            for (int idx = threadIdx.x; idx < (int)Kc * 2 * T; idx += G::NT) {
-                const int k = idx >> (G::LOGT + 1), rw = idx & (2 * T - 1);
-                const uint32_t r = cur.r0 + rw;
-                if (r >= cur.Hm) continue;
-                const int t2 = rw >> 1;
-                const double2 zk = buf[xat<LOGN>(t2, k)];
-                const double2 zn = cconj(buf[xat<LOGN>(t2, k == 0 ? 0 : P - k)]);
-                double2 v;
-                if ((rw & 1) == 0) {
-                    v = make_double2(0.5 * (zk.x + zn.x), 0.5 * (zk.y + zn.y));
-                } else {
-                    const double2 d = mul_mi(csub(zk, zn));
-                    v = make_double2(0.5 * d.x, 0.5 * d.y);
-                }
-                Sm[(size_t)k * Hs + r] = v;
+                double2 x0, x1, x2;
+                dft3(f[0], cmul(w1[q], f[1]), cmul(csqr(w1[q]), f[2]), x0, x1, x2);
+                const uint32_t off = row < cur.Hm ? ((uint32_t)k * Hs + row) * 16u : kOut;
+                buf_store(x0, rs, off, 0);
+                buf_store(x1, rs, off, N * Hs * 16u);
+                // bin N - k; k = 0 and N/2 have it already
+                const bool third = k != 0 && k != N / 2 && row < cur.Hm;
+                buf_store(cconj(x2), rs, third ? ((uint32_t)(N - k) * Hs + row) * 16u : kOut, 0);
             }
             __syncthreads();  // the next item's transform reuses the slab
         }
@@ -901,14 +862,14 @@ __global__ __launch_bounds__(rows3<LOGN>::NT) void rows_fwd3_kernel(
 }
 
 // rows_inv for P = 3N: block (pair item, group of 2T rows z0 = 2T g ... of Z), otherwise as
-// rows_inv_kernel (Z rows by z_row, output rows out_row_of_z, crop and quadrant swap by index).
+// rows_inv_regs_kernel (Z rows by z_row, output rows out_row_of_z, crop and quadrant swap by index).
 template <typename Tout, int LOGN>
 __global__ __launch_bounds__(rows3<LOGN>::NT) void rows_inv3_kernel(
     const double2* __restrict__ Z, Tout* __restrict__ O, const uint64_t* __restrict__ ooff,
     const uint2* __restrict__ ptab, const uint2* __restrict__ mdims, uint32_t nl, uint32_t q0, uint32_t H, uint32_t W,
     uint32_t Ys, uint32_t groups, double scale, const double2* __restrict__ tw, const double2* __restrict__ tw3) {
     using G = rows3<LOGN>;
-    constexpr int N = G::N, P = G::P, Q = G::Q, T = G::T;
+    constexpr int N = G::N, P = G::P, Q = G::Q, T = G::T, IS = G::IS;
     constexpr uint32_t Kc = P / 2 + 1;
     extern __shared__ double2 buf[];
     const uint32_t bid = xcd_remap(blockIdx.x, gridDim.x);
@@ -918,64 +879,78 @@ __global__ __launch_bounds__(rows3<LOGN>::NT) void rows_inv3_kernel(
         H = d.x;
         W = d.y;
     }
-    const uint32_t SX = 2 * W - 1;
     const uint32_t z0 = g * (2 * T);
     if (z_gap(z0, 2 * T, H, Ys)) return;
-    const double2* Zq = Z + (size_t)item * Kc * Ys;
     const regs_pos<LOGN> ps((int)threadIdx.x);
     const int sub = ps.t, tt = sub / 3, m = sub - 3 * tt, i = ps.i;
     const regs_roots<LOGN> rr = load_roots<LOGN>(i, tw);
-    const r3_roots<LOGN> w3 = load_r3_roots<LOGN>(tw3);
-    // Hermitian extension of the two rows of each transform (conjugated, as rows_inv_regs_kernel)
+    // The extension: row pair tq at k = k0 + IS q, the bins k, N + k and N - k of both rows (Z holds
+    // them conjugated).
     {
-        constexpr int NQ = ((int)Kc * T + G::NT - 1) / G::NT;
-        double2 A[NQ], B[NQ];
+        const int tq = (int)threadIdx.x & (T - 1), k0 = (int)threadIdx.x >> G::LOGT;
+        const uint32_t za = z0 + 2 * tq;
+        const bool oka = out_row_of_z(za, H, Ys) >= 0, okb = out_row_of_z(za + 1, H, Ys) >= 0;
+        const __amdgpu_buffer_rsrc_t rz = buf_of(Z + (size_t)item * Kc * Ys, Kc * Ys * 16u);
+        double2 A[G::IQ][3], B[G::IQ][3], w1[G::IQ];
 #pragma unroll
-        for (int q = 0; q < NQ; ++q) {
-            const int idx = threadIdx.x + G::NT * q;
-            const int kk = idx >> G::LOGT, t = idx & (T - 1);
-            const uint32_t za = z0 + 2 * t;
-            const double2* zc = Zq + (size_t)(idx < (int)Kc * T ? kk : 0) * Ys + za;
-            A[q] = make_double2(0.0, 0.0);
-            B[q] = make_double2(0.0, 0.0);
-            if (idx < (int)Kc * T && out_row_of_z(za, H, Ys) >= 0) A[q] = zc[0];
-            if (idx < (int)Kc * T && out_row_of_z(za + 1, H, Ys) >= 0) B[q] = zc[1];
+        for (int q = 0; q < G::IQ; ++q) {
+            const int k = k0 + IS * q;
+            const uint32_t lo = ((uint32_t)k * Ys + za) * 16u, hi = ((uint32_t)(N - k) * Ys + za) * 16u;
+            const bool ka = oka && k <= N / 2, kb = okb && k <= N / 2;
+            w1[q] = tw3[(k <= N / 2 ? k : 0) * (kTw3 / P)];
+            A[q][0] = buf_load(rz, ka ? lo : kOut, 0);
+            B[q][0] = buf_load(rz, kb ? lo + 16u : kOut, 0);
+            A[q][1] = buf_load(rz, ka ? lo : kOut, N * Ys * 16u);
+            B[q][1] = buf_load(rz, kb ? lo + 16u : kOut, N * Ys * 16u);
+            A[q][2] = buf_load(rz, ka ? hi : kOut, 0);
+            B[q][2] = buf_load(rz, kb ? hi + 16u : kOut, 0);
         }
 #pragma unroll
-        for (int q = 0; q < NQ; ++q) {
-            const int idx = threadIdx.x + G::NT * q;
-            if (idx >= (int)Kc * T) continue;
-            const int kk = idx >> G::LOGT, t = idx & (T - 1);
-            buf[xat<LOGN>(t, kk)] = cadd(A[q], mul_mi(B[q]));
-            if (kk > 0 && kk < P / 2) buf[xat<LOGN>(t, P - kk)] = cadd(cconj(A[q]), mul_mi(cconj(B[q])));
+        for (int q = 0; q < G::IQ; ++q) {
+            const int k = k0 + IS * q;
+            if (k > N / 2) continue;
+            const double2 w2 = csqr(w1[q]);
+            double2 a[3], b[3];
+            dft3(A[q][0], A[q][1], cconj(A[q][2]), a[0], a[1], a[2]);
+            dft3(B[q][0], B[q][1], cconj(B[q][2]), b[0], b[1], b[2]);
+            a[1] = cmul(w1[q], a[1]);
+            b[1] = cmul(w1[q], b[1]);
+            a[2] = cmul(w2, a[2]);
+            b[2] = cmul(w2, b[2]);
+#pragma unroll
+            for (int mm = 0; mm < 3; ++mm) {  // slot N, for k = 0, is the pad slot behind the sub-transform
+                buf[at<LOGN>(3 * tq + mm, k)] = make_double2(a[mm].x + b[mm].y, a[mm].y - b[mm].x);
+                buf[at<LOGN>(3 * tq + mm, N - k)] = make_double2(a[mm].x - b[mm].y, -a[mm].y - b[mm].x);
+            }
         }
     }
     __syncthreads();
     double2 u[8];
 #pragma unroll
-    for (int r = 0; r < 8; ++r) u[r] = buf[xat<LOGN>(tt, 3 * (i + Q * r) + m)];
-    __syncthreads();  // the sub-transforms' slots overlap the extended rows
+    for (int r = 0; r < 8; ++r)
+        u[r] = buf[Q % 8 == 0 ? at<LOGN>(sub, i) + r * (Q + Q / 8) : at<LOGN>(sub, i + Q * r)];
+    wave_sync();
     fft_regs<LOGN>(u, buf + at<LOGN>(ps.t0, 0), rr, sub - ps.t0, i);
+    __syncthreads();  // the output rows overlap the sub-transforms' slots
+    // IFFT(Y) = conj(FFT(conj(Y))) / P: row A is the real part, row B minus the imaginary; element
+    // q = i + Q r of sub-transform m is circular column 3q + m
+    Tout* rows = reinterpret_cast<Tout*>(buf);
 #pragma unroll
-    for (int r = 0; r < 8; ++r) buf[at<LOGN>(sub, i + Q * r)] = u[r];
+    for (int r = 0; r < 8; ++r) {
+        const int c = 3 * (i + Q * r) + m;
+        rows[(2 * tt) * P + c] = (Tout)(u[r].x * scale);
+        rows[(2 * tt + 1) * P + c] = (Tout)(-u[r].y * scale);
+    }
     __syncthreads();
-    double2 X[G::NI][3];
-    radix3_pass<LOGN>(buf, w3, X);
-    // IFFT(Y) = conj(FFT(conj(Y))) / P: row A is the real part, row B minus the imaginary
+    const int SX = 2 * (int)W - 1;
     Tout* Oq = O + (ooff ? ooff[q0 + item] : (size_t)(q0 + item) * (2 * H - 1) * SX);
 #pragma unroll
-    for (int q = 0; q < G::NI; ++q) {
-        const int idx = (int)threadIdx.x + G::NT * q;
-        if (idx >= T * N) continue;
-        const int t2 = idx >> LOGN, k = idx & (N - 1);
-        const int oa = out_row_of_z(z0 + 2 * t2, H, Ys), ob = out_row_of_z(z0 + 2 * t2 + 1, H, Ys);
-#pragma unroll
-        for (int j = 0; j < 3; ++j) {
-            const int c = k + N * j;
-            const int ox = c <= (int)W - 1 ? c + (int)W - 1 : (c >= P - (int)W + 1 ? c - (P - (int)W + 1) : -1);
-            if (ox < 0) continue;
-            if (oa >= 0) Oq[(size_t)oa * SX + ox] = (Tout)(X[q][j].x * scale);
-            if (ob >= 0) Oq[(size_t)ob * SX + ox] = (Tout)(-X[q][j].y * scale);
+    for (int z = 0; z < 2 * T; ++z) {
+        const int oy = out_row_of_z(z0 + z, H, Ys);
+        if (oy < 0) continue;
+        for (int ox = (int)threadIdx.x; ox < SX; ox += G::NT) {
+            const int c = ox - ((int)W - 1);
+            Oq[(size_t)oy * SX + ox] = rows[z * P + (c < 0 ? c + P : c)];
         }
     }
 }
@@ -1137,8 +1112,7 @@ fftk_geom geom_of(uint32_t H, uint32_t W, bool pow2_rows = false, bool plain = f
     // rows_inv 2T output rows.
     g.vc = shape_for(g.logPr, g.Kc, cols_threads(g.logPr));
     if (g.f3) {  // rows3<logN>: T = 8 NT / P transforms per block of NT threads
-        const uint32_t n = g.Pc / 3, t = (uint32_t)rows3_t(g.logN);
-        const uint32_t slots = std::max(3 * t * (n + n / 8 + 1), t * (g.Pc + g.Pc / 8 + 1));
+        const uint32_t n = g.Pc / 3, t = (uint32_t)rows3_t(g.logN), slots = 3 * t * (n + n / 8 + 1);
         g.v1 = slab_shape{0, true, ilog2_ceil(t), slots * (uint32_t)sizeof(double2)};
         g.v3 = g.v1;
     } else {
