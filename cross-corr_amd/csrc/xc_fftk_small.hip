@@ -17,10 +17,18 @@
 // are rho and rho + Pr/2: a column thread holds both after its FFT (elements i + Q r and
 // i + Q (r + 4)), so the Hermitian extension needs no exchange between lanes.
 //
-// Bound: FP64 VALU and LDS inside the block (one 1024-thread block per CU at 128 x 128 points;
-// four of 256 at 64 x 64), then the spectra from L2.  Against the three passes (one call, float):
-// n_to_m 16 x 64 of 64^2 77.9 -> 52.7 us, of 32^2 36 -> 17, 1 x 64 of 10^2 20.3 -> 13.9, 1 x 256
-// of 40^2 38.4 -> 32.0 (there with 96-point rows); double, 16 x 64 of 64^2 85.1 -> 64.2.
+// Bound: FP64 VALU and LDS inside the block, then the spectra from L2.  Against the three passes
+// (one call, float): n_to_m 16 x 64 of 64^2 77.9 -> 42.5 us, of 32^2 36 -> 16, 1 x 64 of 10^2 20.3 ->
+// 13.9, 1 x 256 of 40^2 38.4 -> 32.0 (there with 96-point rows).
+//
+// small_pairs with one column per thread loads, transforms and stores in turn: at 128 x 128 points
+// its 1024-thread block fills the CU's LDS, and nothing runs while it waits for the spectra.  With
+// two columns per thread (the second column's transform after the first, in the same scratch) and
+// the rows in two passes through half the slots, a pair takes half the threads and LDS, and the
+// blocks that share a CU overlap each other's phases.  It is taken for more pairs than the chip
+// holds at once in the other form: 16 x 64 of 64^2 53.8 -> 42.5 us, 32 x 128 201 -> 136; of 60 x 30
+// 28.8 -> 26.3 and 78 -> 65.5; of 30^2 17.4 -> 16.4 and 39.8 -> 34.3.  Fewer pairs, where a pair's
+// own latency counts, are 0.5 us faster to 2 us slower that way (one pair of 60 x 30 12.1 -> 14.0).
 #include <hip/hip_ext.h>
 #include <hip/hip_runtime.h>
 
@@ -42,6 +50,14 @@ struct small_geom {
     static constexpr int SLOTS = NC * SR > NR * SC ? NC * SR : NR * SC;
     static constexpr uint32_t LDS = (uint32_t)(SLOTS * (int)sizeof(double2));
     static_assert(NT >= 64 && NT <= 1024 && LR >= 5 && LC >= 5 && LR <= 9 && LC <= 9, "one block per pair");
+};
+
+// small_pairs with PS columns per thread and PS passes of rows: threads and LDS of a block.
+template <int LR, int LC, int PS>
+struct pairs_geom : small_geom<LR, LC> {
+    using G = small_geom<LR, LC>;
+    static constexpr int NT = G::NT / PS;
+    static constexpr uint32_t LDS = G::LDS / PS;
 };
 
 // Matrices 0..nl-1 are the left ones (XL into FL), the rest the right ones (XR into FR); moff and
@@ -121,13 +137,13 @@ __global__ __launch_bounds__((small_geom<LR, LC>::NT)) void small_spec_kernel(
 
 // Pair order: the pairs of one right are consecutive for n_to_m (an XCD's share of the pairs
 // then reads few rights with all lefts, which its L2 holds), else the family's own order.
-template <typename Tout, int LR, int LC>
-__global__ __launch_bounds__((small_geom<LR, LC>::NT)) void small_pairs_kernel(
+template <typename Tout, int LR, int LC, int PS>
+__global__ __launch_bounds__((pairs_geom<LR, LC, PS>::NT), 4) void small_pairs_kernel(
     const double2* __restrict__ FL, const double2* __restrict__ FR, Tout* __restrict__ O,
     const uint64_t* __restrict__ ooff, const uint2* __restrict__ ptab, const uint2* __restrict__ mdims, uint32_t nl,
     int family, uint32_t n, uint32_t m, uint32_t H, uint32_t W, double scale,
     const double2* __restrict__ tw) {
-    using G = small_geom<LR, LC>;
+    using G = pairs_geom<LR, LC, PS>;
     extern __shared__ double2 buf[];
     const int tp = (int)threadIdx.x;
     uint32_t q = xcd_remap(blockIdx.x, gridDim.x), l, r;
@@ -146,80 +162,95 @@ __global__ __launch_bounds__((small_geom<LR, LC>::NT)) void small_pairs_kernel(
         H = d.x;
         W = d.y;
     }
+    // Columns pc.t + h NC/PS: the products' transforms, combined to the row transforms' inputs.
+    const regs_pos<LR> pc(tp);
+    const int i = pc.i;
+    const bool wave0 = tp < 64;  // holds column 0 (selects in every wave cost 60 instructions)
+    double2 u[PS][8];
     {
-        const regs_pos<LR> pc(tp);
-        const regs_roots<LR> rr = load_roots<LR>(pc.i, tw);
-        const int k = pc.t, i = pc.i;
-        const size_t col = (size_t)k * G::Pr + i, nyq = (size_t)G::NC * G::Pr;
-        const double2* Lf = FL + (size_t)l * (G::NC + 1) * G::Pr + col;
-        const double2* Rf = FR + (size_t)r * (G::NC + 1) * G::Pr + col;
-        double2 u[8], v[8];
+        const regs_roots<LR> rr = load_roots<LR>(i, tw);
+        const size_t nyq = (size_t)G::NC * G::Pr;
 #pragma unroll
-        for (int s = 0; s < 8; ++s) {
-            u[s] = Rf[G::Qr * s];
-            v[s] = Lf[G::Qr * s];
-        }
-#pragma unroll
-        for (int s = 0; s < 8; ++s) u[s] = cmul(cconj(v[s]), u[s]);
-        // the wave of column 0 (alone: selects in every wave cost 60 instructions)
-        const bool wave0 = tp < 64;
-        if (wave0 && k == 0) {
+        for (int h = 0; h < PS; ++h) {
+            const int k = pc.t + h * (G::NC / PS);
+            const size_t col = (size_t)k * G::Pr + i;
+            const double2* Lf = FL + (size_t)l * (G::NC + 1) * G::Pr + col;
+            const double2* Rf = FR + (size_t)r * (G::NC + 1) * G::Pr + col;
+            double2 v[8];
 #pragma unroll
             for (int s = 0; s < 8; ++s) {
-                const double2 g = cmul(cconj(Lf[nyq + G::Qr * s]), Rf[nyq + G::Qr * s]);
-                u[s] = make_double2(u[s].x - g.y, u[s].y + g.x);
+                u[h][s] = Rf[G::Qr * s];
+                v[s] = Lf[G::Qr * s];
             }
-        }
-        fft_regs<LR>(u, buf + at<LR>(pc.t0, 0), rr, pc.t - pc.t0, i);
-        __syncthreads();  // the rows' slots overlap other columns' scratch
-        // conj(Y) of row transform rho: with a, b the conjugated column results at rho and
-        // rho + Pr/2, a - i b at k and conj(a) - i conj(b) at Pc - k; column 0 carries the two
-        // real columns 0 and Pc/2.
-        double2* y0 = buf + at<LC>(i, k);
-        double2* y1 = buf + at<LC>(i, wave0 && k == 0 ? G::Pc / 2 : G::Pc - k);
-        if (wave0 && k == 0) {
 #pragma unroll
-            for (int s = 0; s < 4; ++s) {
-                const double2 a = u[s], b = u[s + 4];
-                u[s] = make_double2(a.x, -b.x);
-                u[s + 4] = make_double2(a.y, -b.y);
+            for (int s = 0; s < 8; ++s) u[h][s] = cmul(cconj(v[s]), u[h][s]);
+            if (h == 0 && wave0 && k == 0) {
+#pragma unroll
+                for (int s = 0; s < 8; ++s) {
+                    const double2 g = cmul(cconj(Lf[nyq + G::Qr * s]), Rf[nyq + G::Qr * s]);
+                    u[h][s] = make_double2(u[h][s].x - g.y, u[h][s].y + g.x);
+                }
             }
-        } else {
+            fft_regs<LR>(u[h], buf + at<LR>(pc.t0, 0), rr, pc.t - pc.t0, i);
+            // conj(Y) of row transform rho: with a, b the conjugated column results at rho and
+            // rho + Pr/2, a - i b at k and conj(a) - i conj(b) at Pc - k; column 0 carries the two
+            // real columns 0 and Pc/2.
+            if (h == 0 && wave0 && pc.t == 0) {
 #pragma unroll
-            for (int s = 0; s < 4; ++s) {
-                const double2 a = u[s], b = u[s + 4];
-                u[s] = make_double2(a.x + b.y, a.y - b.x);
-                u[s + 4] = make_double2(a.x - b.y, -a.y - b.x);
+                for (int s = 0; s < 4; ++s) {
+                    const double2 a = u[h][s], b = u[h][s + 4];
+                    u[h][s] = make_double2(a.x, -b.x);
+                    u[h][s + 4] = make_double2(a.y, -b.y);
+                }
+            } else {
+#pragma unroll
+                for (int s = 0; s < 4; ++s) {
+                    const double2 a = u[h][s], b = u[h][s + 4];
+                    u[h][s] = make_double2(a.x + b.y, a.y - b.x);
+                    u[h][s + 4] = make_double2(a.x - b.y, -a.y - b.x);
+                }
             }
-        }
-#pragma unroll
-        for (int s = 0; s < 4; ++s) {
-            y0[s * G::Qr * G::SC] = u[s];
-            y1[s * G::Qr * G::SC] = u[s + 4];
         }
     }
-    __syncthreads();
     const regs_pos<LC> pr(tp);
     const regs_roots<LC> rr = load_roots<LC>(pr.i, tw);
-    double2 u[8];
-#pragma unroll
-    for (int s = 0; s < 8; ++s) u[s] = buf[at<LC>(pr.t, pr.i + G::Qc * s)];
-    wave_sync();
-    fft_regs<LC>(u, buf + at<LC>(pr.t0, 0), rr, pr.t - pr.t0, pr.i);
-    // Circular row rho = t (shifts 0..H-1) and t + Pr/2 (shifts -(H-1)..-1 are rho > Pr - H);
-    // circular columns i + Qc s likewise, s < 4 and s >= 4 (H <= Pr/2, W <= Pc/2).
     const int SX = 2 * (int)W - 1;
     Tout* Oq = O + (ooff ? ooff[q] : (size_t)q * (2 * H - 1) * SX);
-    const bool oka = pr.t < (int)H, okb = pr.t + G::Pr / 2 > G::Pr - (int)H;
-    Tout* oa = Oq + (pr.t + (int)H - 1) * SX + pr.i;
-    Tout* ob = Oq + (pr.t - (G::Pr / 2 - (int)H + 1)) * SX + pr.i;
     const int wlo = (int)W - 1, whi = -(G::Pc - (int)W + 1);
+    // Row transforms rho = pass NR/PS + pr.t.
 #pragma unroll
-    for (int s = 0; s < 8; ++s) {
-        const int c = pr.i + G::Qc * s, off = G::Qc * s + (s < 4 ? wlo : whi);
-        const bool in = s < 4 ? c < (int)W : c > G::Pc - (int)W;
-        if (in && oka) oa[off] = (Tout)(u[s].x * scale);
-        if (in && okb) ob[off] = (Tout)(-u[s].y * scale);
+    for (int pass = 0; pass < PS; ++pass) {
+        __syncthreads();  // the rows' slots overlap the columns' scratch, or the last pass's rows
+#pragma unroll
+        for (int h = 0; h < PS; ++h) {
+            const int k = pc.t + h * (G::NC / PS);
+            double2* y0 = buf + at<LC>(i, k);
+            double2* y1 = buf + at<LC>(i, h == 0 && wave0 && k == 0 ? G::Pc / 2 : G::Pc - k);
+#pragma unroll
+            for (int s = 0; s < 4 / PS; ++s) {
+                y0[s * G::Qr * G::SC] = u[h][pass * (4 / PS) + s];
+                y1[s * G::Qr * G::SC] = u[h][pass * (4 / PS) + s + 4];
+            }
+        }
+        __syncthreads();
+        double2 w[8];
+#pragma unroll
+        for (int s = 0; s < 8; ++s) w[s] = buf[at<LC>(pr.t, pr.i + G::Qc * s)];
+        wave_sync();
+        fft_regs<LC>(w, buf + at<LC>(pr.t0, 0), rr, pr.t - pr.t0, pr.i);
+        // Circular row rho (shifts 0..H-1) and rho + Pr/2 (shifts -(H-1)..-1 are rows > Pr - H);
+        // circular columns i + Qc s likewise, s < 4 and s >= 4 (H <= Pr/2, W <= Pc/2).
+        const int rho = pr.t + pass * (G::NR / PS);
+        const bool oka = rho < (int)H, okb = rho + G::Pr / 2 > G::Pr - (int)H;
+        Tout* oa = Oq + (rho + (int)H - 1) * SX + pr.i;
+        Tout* ob = Oq + (rho - (G::Pr / 2 - (int)H + 1)) * SX + pr.i;
+#pragma unroll
+        for (int s = 0; s < 8; ++s) {
+            const int c = pr.i + G::Qc * s, off = G::Qc * s + (s < 4 ? wlo : whi);
+            const bool in = s < 4 ? c < (int)W : c > G::Pc - (int)W;
+            if (in && oka) oa[off] = (Tout)(w[s].x * scale);
+            if (in && okb) ob[off] = (Tout)(-w[s].y * scale);
+        }
     }
 }
 
@@ -264,17 +295,29 @@ void launch_small(const fftk_job& j, int lr, int lc, const Tio* L, const Tio* R,
     with_small(lr, lc, [&](auto LR, auto LC) {
         using G = small_geom<decltype(LR)::value, decltype(LC)::value>;
         auto ks = small_spec_kernel<Tio, decltype(LR)::value, decltype(LC)::value>;
-        auto kp = small_pairs_kernel<Tio, decltype(LR)::value, decltype(LC)::value>;
         allow_lds(ks, G::LDS);
-        allow_lds(kp, G::LDS);
         launch_timed("fftk_small_spec", timing, ks, dim3(j.nl + j.nr), dim3(G::NT), G::LDS, s, L, R, j.moff, mdims,
                      j.nl, j.H, j.W, FL, FR, tw);
-        const dim3 grid(j.pairs);
-        launch_timed("fftk_small_pairs", timing, kp, grid, dim3(G::NT), G::LDS, s, (const double2*)FL,
-                     (const double2*)FR, O, j.ooff, ptab, mdims, j.nl, j.family, j.n, j.m, j.H, j.W,
-                     1.0 / ((double)G::Pr * (double)G::Pc), tw);
+        auto pairs = [&](auto PS) {
+            using P = pairs_geom<decltype(LR)::value, decltype(LC)::value, decltype(PS)::value>;
+            auto kp = small_pairs_kernel<Tio, decltype(LR)::value, decltype(LC)::value, decltype(PS)::value>;
+            allow_lds(kp, P::LDS);
+            const dim3 grid(j.pairs);
+            launch_timed("fftk_small_pairs", timing, kp, grid, dim3(P::NT), P::LDS, s, (const double2*)FL,
+                         (const double2*)FR, O, j.ooff, ptab, mdims, j.nl, j.family, j.n, j.m, j.H, j.W,
+                         1.0 / ((double)G::Pr * (double)G::Pc), tw);
+            record_launch("fftk_small_pairs", grid, dim3(P::NT), P::LDS, j.H, j.W, j.pairs, 1);
+        };
+        if constexpr (G::NT >= 128) {
+            // More pairs than the 256 CUs hold at once with one column per thread (1024 threads each).
+            if (j.pairs > 256 * 1024 / G::NT)
+                pairs(std::integral_constant<int, 2>{});
+            else
+                pairs(std::integral_constant<int, 1>{});
+        } else {
+            pairs(std::integral_constant<int, 1>{});
+        }
         XC_HIP(hipGetLastError());
-        record_launch("fftk_small_pairs", grid, dim3(G::NT), G::LDS, j.H, j.W, j.pairs, 1);
     });
 }
 

@@ -67,3 +67,35 @@ def test_uneven_batch_of_small_matrices():
             err, _ = norm_error(res, oracle_family(0, lm, rm), oracle_family(0, lm, rm, absval=True))
             assert err <= 1e-6, (r, c, err)
     plan.close()
+
+
+# rows, cols, lefts, rights: more pairs than the chip holds with one column per thread
+MANY = [(64, 64, 5, 52), (16, 200, 5, 52), (200, 16, 5, 52), (30, 100, 5, 52), (100, 30, 5, 52), (60, 30, 9, 58),
+        (30, 60, 9, 58), (120, 16, 9, 58), (16, 120, 9, 58), (30, 30, 19, 54), (16, 60, 19, 54), (60, 16, 19, 54),
+        (16, 30, 33, 63), (30, 16, 33, 63)]
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("rows,cols,n,m", MANY)
+def test_many_pairs(rows, cols, n, m, dtype):
+    """Two columns per thread: the first and last matrices against the oracle, every pair against the
+    one-left calls (one column per thread).  Those differ by the transforms' rounding, below 1e-14
+    of the norms' product, and one rounding of the output."""
+    x = xcorr()
+    left = seeded((n, rows, cols), "normal", 95, dtype)
+    right = seeded((m, rows, cols), "u11", 96, dtype)
+    dl, dr = torch.from_numpy(left).cuda(), torch.from_numpy(right).cuda()
+    out = x.cross_corr("n_to_m", dl, dr, precision="fft64", tile=1)
+    threads = x.last_launch()["block"]
+    got = out.cpu().numpy().reshape(n, m, 2 * rows - 1, 2 * cols - 1)
+    parts = [x.cross_corr("one_to_many", dl[k:k + 1], dr, precision="fft64", tile=1) for k in range(n)]
+    assert x.last_launch()["block"] != threads
+    one = torch.stack(parts).cpu().numpy().reshape(got.shape).astype(np.float64)
+    norm = np.sqrt((left.astype(np.float64) ** 2).sum((1, 2))[:, None] * (right.astype(np.float64) ** 2).sum((1, 2)))
+    bound = 1e-14 * norm[:, :, None, None] + np.finfo(dtype).eps * np.abs(one)
+    assert (np.abs(got - one) <= bound).all()
+    l64, r64 = left[[0, -1]].astype(np.float64), right[[0, -1]].astype(np.float64)
+    ref = oracle_family("n_to_m", l64, r64)
+    err, _ = norm_error(got[np.ix_([0, n - 1], [0, m - 1])].reshape(ref.shape), ref,
+                        oracle_family("n_to_m", l64, r64, absval=True))
+    assert err <= (1e-6 if dtype is np.float32 else 1e-9), (rows, cols, err)
