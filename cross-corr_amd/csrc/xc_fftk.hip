@@ -13,8 +13,9 @@
 //   cols     : per (pair, column k): X = FFT of length Pr of S[right][k][0..H-1] (zero
 //              padded), then a second FFT of conj(Lhat) * X: the conjugate of
 //              Pr * IFFT(Lhat * conj(X)) (Lhat = the left's 2D spectrum, made by the same
-//              kernel in "left" mode), of which only the 2H-1 circular rows of the result
-//              are kept: Z[pair][k][z_row(rho)];
+//              kernel in "left" mode, or inside the block where few pairs share a left:
+//              cols_group), of which only the 2H-1 circular rows of the result are kept:
+//              Z[pair][k][z_row(rho)];
 //   rows_inv : per pair, two output rows per complex FFT of length Pc: the Hermitian half
 //              rows of Z are extended, inverse transformed, scaled by 1/(Pr*Pc) and written
 //              straight into the cropped (2H-1) x (2W-1) result (quadrant swap by index).
@@ -405,6 +406,84 @@ constexpr int cols_threads(int logP) { return logP <= 9 ? 64 : kFT; }
 // dropped).
 // Blocks are ordered column-group major through the XCD remap, so the pairs that read the
 // same Lhat columns run on one XCD and find them in its L2.
+// cols_group: block (group of C columns k, G consecutive pairs from q0 + item G): the columns of
+// the pairs' left matrix are transformed here and kept in registers while the left stays the
+// same, so the left spectra are neither written to Lhat nor read back, and one launch is saved;
+// the rest as cols mode 1 below.  Against that path a left's columns are transformed once per
+// block instead of once per call, and the registers of the left stay occupied during the second
+// transform of a pair (118 instead of 96 at 512 points: 4 waves per SIMD for 5).  So it is taken for
+// at most 4 pairs per left (64 pairs of n_to_mn at 256^2: one per left 189 -> 131 us, two 151 ->
+// 108, four 110 -> 101; eight 100 -> 100, sixteen 94 -> 95; the uneven batch of 128 x 4 pairs 796 ->
+// 720) and where the pairs' columns are at most 6144 waves, so that the launch counts (one pair of
+// 128^2 15.9 -> 13.6 us, of 512^2 32.2 -> 28.6, 1 x 16 of 256^2 40.0 -> 37.4; 1 x 24 46.6 -> 46.0, 1 x
+// 32 55.2 -> 56.1).  G = 2 above 4608 waves (the batch 772 -> 740 in one run), G = 1 below (1 x 4 of
+// 256^2 20.7 against 22.1, 64 x 64 of 128^2 37.7 against 39.7).
+template <int LOGPR>
+__global__ __launch_bounds__(cols_threads(LOGPR)) void cols_group_kernel(
+    const double2* __restrict__ SL, const double2* __restrict__ SR, double2* __restrict__ Z,
+    const uint2* __restrict__ ptab, const uint2* __restrict__ mdims, uint32_t nl, int family, uint32_t n, uint32_t m,
+    uint32_t q0, uint32_t pairs, uint32_t G, uint32_t items, uint32_t H, uint32_t Hs, uint32_t Kc, uint32_t Ys,
+    const double2* __restrict__ tw) {
+    extern __shared__ double2 buf[];
+    constexpr int Q = 1 << (LOGPR - 3), P = 1 << LOGPR;
+    constexpr uint32_t C = 8 * cols_threads(LOGPR) / P;
+    const uint32_t bid = xcd_remap(blockIdx.x, gridDim.x);
+    const uint32_t cg = bid / items, first = (bid - cg * items) * G, last = min(first + G, pairs);
+    const regs_pos<LOGPR> ps((int)threadIdx.x);
+    const uint32_t k = cg * C + ps.t;
+    const bool ok = k < Kc;
+    double2* wb = buf + at<LOGPR>(ps.t0, 0);
+    const regs_roots<LOGPR> rr = load_roots<LOGPR>(ps.i, tw);
+    auto column = [&](const double2* S, uint32_t mat, uint32_t rows, int i, double2 (&u)[8]) {
+        const __amdgpu_buffer_rsrc_t rs = buf_of(S + (size_t)mat * Kc * Hs, Kc * Hs * 16u);
+        const uint32_t so = (k * Hs + (uint32_t)i) * 16u;
+#pragma unroll
+        for (int r = 0; r < 4; ++r)  // rows <= Pr / 2: the upper half of a column is padding
+            u[r] = buf_load(rs, (uint32_t)(i + Q * r) < rows ? so + 16u * Q * r : kOut, 0);
+    };
+    double2 lh[8];
+    uint32_t have = ~0u;
+    for (uint32_t p = first; p < last; ++p) {
+        uint32_t l, r;
+        if (ptab) {
+            l = ptab[q0 + p].x;
+            r = ptab[q0 + p].y;
+        } else {
+            pair_of(family, n, m, q0 + p, l, r);
+        }
+        const uint32_t Hq = mdims ? mdims[nl + r].x : H, rows = ok ? Hq : 0;
+        // opaque copies of the position: no transform keeps another one's LDS addresses live
+        int tl = ps.t - ps.t0, i = ps.i;
+        double2 u[8];
+        if (l != have) {  // block-uniform
+            asm volatile("" : "+v"(tl), "+v"(i));
+            column(SL, l, rows, i, lh);
+            column(SR, r, rows, i, u);
+            fft_regs<LOGPR, true>(lh, wb, rr, tl, i);
+            have = l;
+        } else {
+            asm volatile("" : "+v"(tl), "+v"(i));
+            column(SR, r, rows, i, u);
+        }
+        asm volatile("" : "+v"(tl), "+v"(i));
+        fft_regs<LOGPR, true>(u, wb, rr, tl, i);
+#pragma unroll
+        for (int s = 0; s < 8; ++s) u[s] = cmul(cconj(lh[s]), u[s]);
+        asm volatile("" : "+v"(tl), "+v"(i));
+        fft_regs<LOGPR>(u, wb, rr, tl, i);
+        // z_row: rows below Hq (s < 4: Hq <= Pr / 2) in place, rows above Pr - Hq (s >= 4) down by
+        // Pr - Ys
+        const __amdgpu_buffer_rsrc_t rz = buf_of(Z + (size_t)p * Kc * Ys, Kc * Ys * 16u);
+        const uint32_t zlo = (k * Ys + (uint32_t)i) * 16u, zhi = zlo - ((uint32_t)P - Ys) * 16u;
+#pragma unroll
+        for (int s = 0; s < 8; ++s) {
+            const uint32_t rho = (uint32_t)(i + Q * s);
+            const bool in = s < 4 ? rho < rows : rho + rows > (uint32_t)P;
+            buf_store(u[s], rz, in ? (s < 4 ? zlo : zhi) + 16u * Q * s : kOut, 0);
+        }
+    }
+}
+
 template <int LOGPR, int MODE>
 __global__ __launch_bounds__(cols_threads(LOGPR)) void cols_kernel(const double2* __restrict__ S, double2* __restrict__ Lhat,
                                                    double2* __restrict__ Z, const uint2* __restrict__ ptab,
@@ -1229,11 +1308,31 @@ void launch_job(const fftk_job& j, const Tio* L, const Tio* R, Tio* O, const fft
                          ptab, mdims, j.nl, j.family, j.n, j.m, q0, items, H, g.Hs, g.Kc, g.Ys, g.vc.logT, tw);
         });
     };
-    cols("fftk_cols_left", SL, nullptr, std::integral_constant<int, 0>{}, j.nl, 0);
+    // Column kernel of a chunk: grouped (cols_group_kernel has the reasons for both lines) or from Lhat.
+    const uint32_t waves = std::min(chunk, j.pairs) * g.cg * (uint32_t)cols_threads(g.logPr) / 64;
+    const bool grouped = g.logPr <= 11 && (j.pairs <= 4 * j.nl || waves <= 6144);
+    const uint32_t G = waves > 4608 && j.pairs > j.nl ? 2 : 1;
+    auto cols_group = [&](uint32_t nq, uint32_t q0) {
+        with_logp(g.logPr, [&](auto LP) {
+            constexpr int LOGPR = decltype(LP)::value;
+            if constexpr (regs_of<LOGPR>::ON) {
+                auto k = cols_group_kernel<LOGPR>;
+                allow_lds(k, g.vc.lds);
+                const uint32_t items = (nq + G - 1) / G;
+                launch_timed("fftk_cols", timing, k, dim3(items * g.cg), dim3(cols_threads(g.logPr)), g.vc.lds, s,
+                             (const double2*)SL, (const double2*)SR, Zw, ptab, mdims, j.nl, j.family, j.n, j.m, q0, nq,
+                             G, items, H, g.Hs, g.Kc, g.Ys, tw);
+            }
+        });
+    };
+    if (!grouped) cols("fftk_cols_left", SL, nullptr, std::integral_constant<int, 0>{}, j.nl, 0);
     const double scale = 1.0 / ((double)g.Pr * (double)g.Pc);
     for (uint32_t q0 = 0; q0 < j.pairs; q0 += chunk) {
         const uint32_t nq = std::min(chunk, j.pairs - q0);
-        cols("fftk_cols", SR, Zw, std::integral_constant<int, 1>{}, nq, q0);
+        if (grouped)
+            cols_group(nq, q0);
+        else
+            cols("fftk_cols", SR, Zw, std::integral_constant<int, 1>{}, nq, q0);
         if (g.f3) {
             with_logp(g.logN, [&](auto LN) {
                 constexpr int LOGN = decltype(LN)::value;
