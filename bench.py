@@ -46,11 +46,12 @@ ROWS = COLS = 256
 NUM_RIGHT = 64
 ERR_BAR = 2e-6
 HBM_GBPS = 8000.0
-# Peaks of the arithmetic each definition-based kernel issues: non-packed FP32 FMA (the
-# direct kernel does not use packed FP32 instructions: half the published 157.3 TFLOP/s),
-# FP64 VALU, dense BF16/FP16 MFMA.
+# Peaks of the arithmetic each definition-based kernel issues: non-packed FP32 FMA (the VALU
+# direct kernels do not use packed FP32 instructions: half the published 157.3 TFLOP/s; the FP32
+# matrix instructions reach all of it), FP64 VALU, dense BF16/FP16 MFMA.
+FP32_MATRIX_TFLOPS = 157.3
 TFLOPS = {"direct_kernel": 78.6, "direct_kernel_f64": 78.6, "mfma_kernel": 2500.0, "batch_kernel": 2500.0}
-# fp32: the library's FP32 default (the lanes-over-pairs kernel where it applies); fp32tiles: the
+# fp32: the library's FP32 default (the FP32 matrix instructions at this size); fp32tiles: the
 # register-tile kernel (FP32 tile 1), for comparison runs only.
 METHODS = {"fp32": dict(precision="fp32"), "fp32tiles": dict(precision="fp32", tile=1),
            "bf16x3": dict(precision="bf16x3"), "fp16x3": dict(precision="fp16x3"),
@@ -274,10 +275,12 @@ def main():
     if "ms_per_step" in results.get("fp32", {}):
         t32 = kernels_of(lambda: step("fp32"), 2)
         fp32_roof = roofline(t32, lambda k: None, lambda k: 2.0 * NUM_RIGHT * macs)
-        # "direct_kernel" is the direct method's timer, shared by its two kernels: name the
+        # "direct_kernel" is the direct method's timer, shared by its kernels: name the
         # kernel that ran.
         fp32_roof["timer"] = fp32_roof["kernel"]
         fp32_roof["kernel"] = results["fp32"].get("last_kernel", fp32_roof["kernel"])
+        if "matrix" in fp32_roof["kernel"]:
+            fp32_roof.update(bound="mfma", peak=FP32_MATRIX_TFLOPS, frac=fp32_roof["achieved"] / FP32_MATRIX_TFLOPS)
 
     # CPU baseline: the oracle's FP32 restatement of cpu_cross_corr_one_to_many
     # (src/validate.hpp:231-247), single thread, on a bounded sample of the same workload.

@@ -2,6 +2,7 @@
 // plan of a launch (tile, block shape, work distribution) and the launchers; the float
 // instances of the kernel.
 #include <algorithm>
+#include <cmath>
 #include <cstdio>
 #include <vector>
 
@@ -160,6 +161,8 @@ struct dp_args {
     uint32_t r_count;                 // matrices in the right copy
     int Q4, PL, Hl, Wl;               // right copy: quads per row, column offset; left copy: rows, row length
     int by_unit;                      // block order (see the kernel)
+    uint32_t mp;                      // slots of the right copy per left (n_to_mn) or in all: mpl rounded up
+    uint32_t gpl;                     // direct_matrix_kernel: groups of 16 rights per left
 };
 
 // Four consecutive elements of a row: 16 bytes (float) or 32 bytes (double).
@@ -184,9 +187,11 @@ struct quad_of<double> {
 
 template <typename T, int TY>
 __global__ __launch_bounds__(256) void direct_pairs_kernel(const T* __restrict__ Lc, const T* __restrict__ Rq,
-                                                           T* __restrict__ O, dp_args a) {
+                                                           T* __restrict__ O, dp_args a,
+                                                           const uint32_t* __restrict__ only_if) {
     using Q = typename quad_of<T>::type;
     constexpr int TX = 4, FLUSHC = 16;  // FLUSHC chunks of 4 columns per partial sum
+    if (only_if && *only_if == 0) return;  // direct_matrix_kernel has done the batch
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
     // Blocks go round-robin to the 8 XCDs; tiles run nearest the centre (largest overlap)
@@ -208,7 +213,7 @@ __global__ __launch_bounds__(256) void direct_pairs_kernel(const T* __restrict__
     // last right read a zero slot and store nothing)
     const uint32_t li = g / a.wpl, t = (g % a.wpl) * 64 + (uint32_t)lane;
     const bool valid = t < a.mpl;
-    const uint32_t slot = (a.family == XC_N_TO_MN ? li * a.wpl * 64 : 0) + t;
+    const uint32_t slot = (a.family == XC_N_TO_MN ? li * a.mp : 0) + min(t, a.mp - 1);
     const uint32_t pk = a.family == XC_N_TO_M ? li * a.m + t : (a.family == XC_N_TO_MN ? li + a.n * t : t);
     // right rows: those that meet a dy of the tile; columns: the union over the tile's dx,
     // from a multiple of 4
@@ -281,30 +286,40 @@ __global__ __launch_bounds__(256) void direct_pairs_kernel(const T* __restrict__
     }
 }
 
-// Left copy: count matrices of H x W into rows of Wl (zero past W) with pad zero rows above
-// and below: element (r, c) of matrix i at (i * Hl + r + pad) * Wl + c.
+// Left copy: count matrices of H x W into rows of Wl (zero outside the matrix) with pad zero rows
+// above and below: element (r, c) of matrix i at (i * Hl + r + pad) * Wl + c + padc.  Clears
+// *flag when one is given.
 template <typename T>
 __global__ __launch_bounds__(256) void pairs_copy_left_kernel(const T* __restrict__ X, T* __restrict__ Xc,
-                                                              uint32_t count, int H, int W, int Hl, int Wl, int pad) {
+                                                              uint32_t count, int H, int W, int Hl, int Wl, int pad,
+                                                              int padc, uint32_t* __restrict__ flag) {
+    if (flag && blockIdx.x == 0 && threadIdx.x == 0) *flag = 0;
     const uint64_t total = (uint64_t)count * Hl * Wl;
     for (uint64_t e = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; e < total; e += (uint64_t)gridDim.x * blockDim.x) {
-        const int c = (int)(e % (uint64_t)Wl);
+        const int c = (int)(e % (uint64_t)Wl) - padc;
         const uint64_t rest = e / (uint64_t)Wl;
         const int r = (int)(rest % (uint64_t)Hl) - pad;
         const uint64_t i = rest / (uint64_t)Hl;
-        Xc[e] = (r >= 0 && r < H && c < W) ? X[(i * H + r) * W + c] : T(0);
+        Xc[e] = (r >= 0 && r < H && c >= 0 && c < W) ? X[(i * H + r) * W + c] : T(0);
     }
 }
 
 // Right copy: quad position p of row j of slot i at ((j * Q4 + p) * count + i) * 4, holding
 // columns 4p - PL .. 4p - PL + 3 (zero outside [0, W)) of the slot's matrix: with ln = 0 slot
 // i is matrix i (zero for i >= nmat); with ln lefts (n_to_mn), slot l*MP + t is matrix
-// l + ln*t (zero for t >= mpl).  Thread e writes quad e.
+// l + ln*t (zero for t >= mpl).  Thread e writes quad e.  With a flag given, *flag is set if a
+// value here, or one of the lsize values of the left copy Lc, is an infinity or a NaN.
 template <typename T>
 __global__ __launch_bounds__(256) void pairs_copy_right_kernel(const T* __restrict__ X, T* __restrict__ Xq,
                                                                uint32_t count, uint32_t nmat, uint32_t ln,
-                                                               uint32_t mp, uint32_t mpl, int H, int W, int Q4, int PL) {
+                                                               uint32_t mp, uint32_t mpl, int H, int W, int Q4, int PL,
+                                                               const T* __restrict__ Lc, uint64_t lsize,
+                                                               uint32_t* __restrict__ flag) {
     const uint64_t total = (uint64_t)count * H * Q4;
+    bool bad = false;
+    if (flag)
+        for (uint64_t e = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; e < lsize; e += (uint64_t)gridDim.x * blockDim.x)
+            bad |= !isfinite(Lc[e]);
     for (uint64_t e = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; e < total; e += (uint64_t)gridDim.x * blockDim.x) {
         const uint64_t i = e % count, rest = e / count;
         const int p = (int)(rest % (uint64_t)Q4), j = (int)(rest / (uint64_t)Q4);
@@ -319,7 +334,124 @@ __global__ __launch_bounds__(256) void pairs_copy_right_kernel(const T* __restri
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
             const int q = 4 * p + t - PL;
-            Xq[e * 4 + t] = (ok && q >= 0 && q < W) ? row[q] : T(0);
+            const T v = (ok && q >= 0 && q < W) ? row[q] : T(0);
+            bad |= !isfinite(v);
+            Xq[e * 4 + t] = v;
+        }
+    }
+    if (flag && bad) *flag = 1;  // every writer stores the same value
+}
+
+// The same sums on the FP32 matrix instructions (v_mfma_f32_16x16x4_f32: FP32 products and FP32
+// sums at 256 FLOPs per CU and clock, twice the rate of FP32 FMAs that are not packed).  For one
+// left, rights x shifts is a matrix product over the pixels: A = 16 rights x 4 pixels, B = 4 pixels
+// of the left x 16 consecutive dx.  A block takes 16 rights of one left and a tile of 4 dy x 16 dx; its four waves split the tile's (right row, 16 columns) steps evenly, each wave with its own
+// FP32 partial sums of 32 products and FP64 totals, which are added through LDS in a fixed
+// order.  The order of the 16 pixels of a step is free as long as A and B agree: lane group k = lane /
+// 16 takes columns q + 4k .. q + 4k + 3, so that a lane's four A values are one quad of the
+// lanes-over-pairs kernel's right copy, and its four B values four neighbours in the left copy.  Five
+// 16-byte loads, one step ahead, feed 16 instructions of 32 cycles: no LDS, no barriers.  Bound: the
+// matrix instructions, 4.0 ms at 2.4 GHz of the 4.57 that 64 of 256^2 take (lanes over pairs 9.12; 120
+// TFLOP/s of the definition); partial sums of 64 took 4.36, of 32 bring the error of signed
+// data from 1.43e-7 to 1.04e-7 (lanes over pairs 1.45e-7); two groups of rights per wave took 4.57 too,
+// with 149 registers, and twice as long where the second was idle.  16 x 64 of 64^2 700 -> 465 us.
+// Columns are the union over 16 dx, rounded up to 16 (about 16 more than a single dx has), rows
+// the union over 4 dy.  A zero of the copies' padding must not meet an infinity or a NaN: a batch
+// that holds one (*nonfinite) is left to direct_pairs_kernel, which reads the same copies.
+constexpr int kMatrixPadC = 20;  // zero columns of the left copy before column 0
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void direct_matrix_kernel(
+    const float* __restrict__ Lc, const float* __restrict__ Rq, float* __restrict__ O, dp_args a,
+    const uint32_t* __restrict__ nonfinite) {
+    typedef float f32x4 __attribute__((ext_vector_type(4)));
+    constexpr int TY = 4;
+    __shared__ double part[4][2 * 4 * 64];  // a wave's totals of two of the tile's dy
+    if (*nonfinite) return;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lane = threadIdx.x & 63, l16 = lane & 15, kg = lane >> 4;
+    const uint32_t groups = a.n * a.gpl;
+    uint32_t u, band;
+    if (!block_order(blockIdx.x, groups * a.tiles_x, a.tiles_y, a.by_unit, u, band)) return;
+    const uint32_t g = u % groups, li = g / a.gpl, t0 = (g % a.gpl) * 16;
+    const int H = a.H, W = a.W;
+    const int dy0 = -(H - 1) + TY * center_first((int)band, (int)a.tiles_y);
+    const int dx0 = -(W - 1) + 16 * center_first((int)(u / groups), (int)a.tiles_x);
+    // right rows and columns that meet the tile, the first column on a quad of the right copy
+    const int jlo = max(0, -(dy0 + TY - 1)), jhi = min(H, H - dy0);
+    const int qmin = max(0, -(dx0 + 15)), qlo = qmin - ((qmin + a.PL) & 3);
+    const int nch = (min(W, W - dx0) - qlo + 15) >> 4;
+    const int steps = (jhi - jlo) * nch;
+    const int s0 = (int)((int64_t)steps * wave >> 2), s1 = (int)((int64_t)steps * (wave + 1) >> 2);
+    const int64_t rq = (int64_t)a.r_count * 4;  // elements between quad positions of one row
+    const uint32_t slot = (a.family == XC_N_TO_MN ? li * a.mp : 0) + t0 + (uint32_t)l16;
+    const uint32_t a_off = (uint32_t)kg * (uint32_t)(rq * 4) + slot * 16u;
+    const uint32_t b_off = (uint32_t)(4 * kg + l16) * 4u;
+    const float* __restrict__ at = Rq + (int64_t)((qlo + a.PL) >> 2) * rq;
+    const float* __restrict__ bt = Lc + ((int64_t)li * a.Hl + dy0 + TY - 1) * a.Wl + kMatrixPadC + qlo + dx0;
+    f32x4 acc[TY];
+    double tot[TY][4];
+#pragma unroll
+    for (int y = 0; y < TY; ++y)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) tot[y][r] = 0.0;
+    auto load = [&](int j, int ch, float4& av, float4 (&bv)[TY]) {
+        const float* bp = bt + (int64_t)j * a.Wl + 16 * ch;
+        av = buffer_quad(at + ((int64_t)j * a.Q4 + 4 * ch) * rq, a_off, 0);
+#pragma unroll
+        for (int y = 0; y < TY; ++y) bv[y] = buffer_quad(bp + (int64_t)y * a.Wl, b_off, 0);
+    };
+    if (s0 < s1) {
+        int j = jlo + s0 / nch, ch = s0 % nch;
+        float4 a0, b0[TY], a1, b1[TY];
+        auto next = [&](int s, float4& av, float4 (&bv)[TY]) {
+            if (s + 1 < s1 && ++ch == nch) {  // the last step loads itself again
+                ch = 0;
+                ++j;
+            }
+            load(j, ch, av, bv);
+            __builtin_amdgcn_sched_barrier(0);  // in flight before this step's products, not behind them
+        };
+        auto products = [&](const float4& av, const float4 (&bv)[TY], auto first) {
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+#pragma unroll
+                for (int y = 0; y < TY; ++y) {
+                    const f32x4 c = decltype(first)::value && t == 0 ? f32x4{0, 0, 0, 0} : acc[y];
+                    acc[y] = __builtin_amdgcn_mfma_f32_16x16x4f32((&av.x)[t], (&bv[y].x)[t], c, 0, 0, 0);
+                }
+        };
+        load(j, ch, a0, b0);
+        for (int s = s0; s < s1; s += 2) {
+            next(s, a1, b1);
+            products(a0, b0, std::true_type{});
+            if (s + 1 < s1) {
+                next(s + 1, a0, b0);
+                products(a1, b1, std::false_type{});
+            }
+#pragma unroll
+            for (int y = 0; y < TY; ++y)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) tot[y][r] += (double)acc[y][r];
+        }
+    }
+    // the waves' totals, two dy at a time; lane `el` of a tile holds dx el % 16 of rights 4 (el / 16) + r
+    const int SX = 2 * W - 1, SY = 2 * H - 1;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        if (h) __syncthreads();
+#pragma unroll
+        for (int y = 0; y < 2; ++y)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) part[wave][(4 * y + r) * 64 + lane] = tot[2 * h + y][r];
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            const int e = (int)threadIdx.x + 256 * q;
+            const double v = ((part[0][e] + part[1][e]) + part[2][e]) + part[3][e];
+            const int el = e & 63, r = (e >> 6) & 3, y = e >> 8;
+            const int oy = dy0 + 2 * h + y + H - 1, ox = dx0 + (el & 15) + W - 1;
+            const uint32_t t = t0 + (uint32_t)(4 * (el >> 4) + r);
+            const uint32_t pk = a.family == XC_N_TO_M ? li * a.m + t : (a.family == XC_N_TO_MN ? li + a.n * t : t);
+            if (t < a.mpl && oy < SY && ox < SX) O[((size_t)pk * SY + oy) * SX + ox] = (float)v;
         }
     }
 }
@@ -363,8 +495,36 @@ bool pairs_kernel_applies(const family_args& a, bool float_data) {
     return busy >= 0.7 && waves * busy * busy * busy >= 4500;
 }
 
+// Whether direct_matrix_kernel serves this float batch by default: its copy of the rights at most 16
+// GiB, and a shorter estimated time than the 16 x 16 shifts kernel's.  Both estimates are products
+// issued (the padding of tiles and of groups of 16 rights among them) over a rate, plus the launches;
+// the matrix kernel's also six steps per wave for its start and end, and 0.6 of its longest wave,
+// which small grids wait for.  Measured us, matrix / shifts: 8 of 128^2 127 / 115, 10 of 128^2 127 / 143,
+// 48 of 128^2 298 / 590, 64 of 128^2 380 / 800 (lanes over pairs 898), 16 of 64^2 34 / 27, 32 of 64^2 37 / 47,
+// 20 x 10 of 64^2 149 / 190, 64 of 32^2 18 / 14, 256 of 32^2 28 / 33, 8 of 256^2 1228 / 1552.  Below 16 columns most of
+// its 16 dx and 16 columns are padding: the lanes-over-pairs kernel keeps the batches it serves (200 x 64 of
+// 10^2 59 / 86 us).
+bool matrix_kernel_applies(const family_args& a) {
+    const uint32_t mpl = rights_per_left(a);
+    if (mpl == 0) return false;
+    const double lefts = a.family == XC_ONE_TO_MANY ? 1 : a.n, groups = lefts * ((mpl + 15) / 16);
+    const double slots = (a.family == XC_N_TO_MN ? lefts : 1) * ((mpl + 15) / 16 * 16);
+    const double H = a.rows, W = a.cols;
+    if (slots * H * (W + 27) * sizeof(float) > (double)(16ull << 30) || slots * 64 >= (double)(1u << 31)) return false;
+    if (a.cols < 16 && pairs_kernel_applies(a, true)) return false;
+    const double SX = (2 * a.cols - 1 + 15) / 16 * 16, SY = (2 * a.rows - 1 + 3) / 4 * 4;
+    const double SYs = (2 * a.rows - 1 + 15) / 16 * 16;
+    const double step = 512 / 2.4e3, waves = groups * (SX / 16) * (SY / 4) * 4;  // us of a step; waves
+    const double matrix = 12 + groups * 16 * SX * SY * (H / 2 + 2) * (W / 2 + 16.5) / 68e6 +
+                          waves * 6 * step / 1024 + 0.6 * step * (H / 4) * std::ceil((W + 15) / 16);
+    const double shifts = 10 + lefts * mpl * SX * SYs * (H / 2 + 8) * (W / 2 + 8) / 25e6;
+    return matrix < shifts;
+}
+
+// matrix: by direct_matrix_kernel, with direct_pairs_kernel behind it for data that is not finite;
+// false (nothing launched) if there is no memory for its copies.
 template <typename T>
-void launch_direct_pairs(const family_args& a, const T* L, const T* R, T* O, hipStream_t s) {
+bool launch_direct_pairs(const family_args& a, const T* L, const T* R, T* O, hipStream_t s, bool matrix) {
     constexpr int TY = kPairsTY;
     const int H = (int)a.rows, W = (int)a.cols;
     const uint32_t nl = a.family == XC_ONE_TO_MANY ? 1 : a.n;
@@ -378,37 +538,64 @@ void launch_direct_pairs(const family_args& a, const T* L, const T* R, T* O, hip
     k.mpl = rights_per_left(a);
     k.wpl = (k.mpl + 63) / 64;
     k.groups = nl * k.wpl;
-    // right slots: the rights in order, padded to a multiple of 64; n_to_mn: per left, its
-    // rights, padded to a multiple of 64 each
-    const uint32_t nr = a.family == XC_N_TO_MN ? nl * k.wpl * 64 : k.wpl * 64;
+    // right slots: the rights in order, padded to a multiple of 64 (16 for the matrix kernel);
+    // n_to_mn: per left, its rights, padded to such a multiple each
+    k.mp = matrix ? (k.mpl + 15) / 16 * 16 : k.wpl * 64;
+    const uint32_t nr = a.family == XC_N_TO_MN ? nl * k.mp : k.mp;
     k.tiles_y = (uint32_t)(2 * H - 1 + TY - 1) / TY;
     k.tiles_x = (uint32_t)(2 * W - 1 + 3) / 4;
     k.nbx = (k.tiles_x + 3) / 4;
     k.r_count = nr;
     k.PL = 8 + (4 - W % 4) % 4;
-    k.Q4 = (k.PL + W + 12 + 3) / 4;  // a quad past the last window
+    k.Q4 = (k.PL + W + (matrix ? 16 : 12) + 3) / 4;  // a quad past the last window; a step of 16 columns
     k.Hl = H + 2 * (TY - 1);
-    k.Wl = (W + 3) / 4 * 4 + 4;       // a chunk past the last one (prefetch)
+    // a chunk past the last one (prefetch); 16 columns and 16 dx past the last column
+    const int padc = matrix ? kMatrixPadC : 0;
+    k.Wl = matrix ? (padc + W + 32 + 3) / 4 * 4 : (W + 3) / 4 * 4 + 4;
     if ((uint64_t)nr * 4 * sizeof(T) + 16 >= (1ull << 31)) fail(XC_ERR_UNSUPPORTED, "direct kernel: too many right matrices");
     const uint64_t lsize = (uint64_t)nl * k.Hl * k.Wl, rsize = (uint64_t)nr * H * k.Q4 * 4;
-    T* Lc = static_cast<T*>(workspace(WS_DIRECT, sizeof(T) * (lsize + rsize), s));
+    const size_t bytes = sizeof(T) * (lsize + rsize) + sizeof(uint32_t);
+    T* Lc = static_cast<T*>(matrix ? workspace_if_free(WS_DIRECT, bytes, s) : workspace(WS_DIRECT, bytes, s));
+    if (!Lc) return false;
     T* Rq = Lc + lsize;
+    uint32_t* flag = matrix ? reinterpret_cast<uint32_t*>(Rq + rsize) : nullptr;
     auto blocks_for = [](uint64_t n) { return (uint32_t)std::min<uint64_t>((n + 255) / 256, 16384); };
     hipLaunchKernelGGL(pairs_copy_left_kernel<T>, dim3(blocks_for(lsize)), dim3(256), 0, s, L, Lc, nl, H, W, k.Hl,
-                       k.Wl, TY - 1);
+                       k.Wl, TY - 1, padc, flag);
     XC_HIP(hipGetLastError());
     hipLaunchKernelGGL(pairs_copy_right_kernel<T>, dim3(blocks_for(rsize / 4)), dim3(256), 0, s, R, Rq, nr, a.m,
-                       a.family == XC_N_TO_MN ? nl : 0u, k.wpl * 64, k.mpl, H, W, k.Q4, k.PL);
+                       a.family == XC_N_TO_MN ? nl : 0u, k.mp, k.mpl, H, W, k.Q4, k.PL, Lc, lsize, flag);
     XC_HIP(hipGetLastError());
     k.by_unit = rsize * sizeof(T) > (4u << 20);  // larger than one XCD's L2
+    if constexpr (std::is_same<T, float>::value) {
+        if (matrix) {
+            dp_args mk = k;
+            mk.gpl = k.mp / 16;
+            mk.tiles_x = (uint32_t)(2 * W - 1 + 15) / 16;
+            const uint32_t units = nl * mk.gpl * mk.tiles_x;
+            // a unit's bands on one XCD (16 of 128^2 127 us; bands dealt to the XCDs in turn 179: each CU's
+            // blocks are then the same units of several bands), unless that leaves XCDs idle
+            mk.by_unit = (units + 7) / 8 * 8 * 10 <= units * 11;
+            const uint64_t mblocks = blocks_for_order(units, mk.tiles_y, mk.by_unit);
+            if (mblocks > 0x7fffffffULL) fail(XC_ERR_INVALID_ARGUMENT, "problem too large for one launch");
+            const dim3 grid((uint32_t)mblocks), block(256);
+            record_launch("direct_pairs_kernel<f32> matrix instructions", grid, block, 0, a.rows, a.cols, a.pairs, 1);
+            timed td("direct_kernel", s);
+            hipLaunchKernelGGL(direct_matrix_kernel, grid, block, 0, s, Lc, Rq, O, mk, flag);
+            XC_HIP(hipGetLastError());
+        }
+    }
     const uint64_t nblocks = blocks_for_order(k.groups * k.nbx, k.tiles_y, k.by_unit);
     if (nblocks > 0x7fffffffULL) fail(XC_ERR_INVALID_ARGUMENT, "problem too large for one launch");
     dim3 grid((uint32_t)nblocks), block(256);
-    record_launch(sizeof(T) == 4 ? "direct_pairs_kernel<f32> ty4 tx4" : "direct_pairs_kernel<f64> ty4 tx4", grid, block,
-                  0, a.rows, a.cols, a.pairs, 1);
-    timed td("direct_kernel", s);
-    hipLaunchKernelGGL((direct_pairs_kernel<T, TY>), grid, block, 0, s, Lc, Rq, O, k);
+    if (!matrix)
+        record_launch(sizeof(T) == 4 ? "direct_pairs_kernel<f32> ty4 tx4" : "direct_pairs_kernel<f64> ty4 tx4", grid,
+                      block, 0, a.rows, a.cols, a.pairs, 1);
+    timed td("direct_kernel", s, !matrix);
+    hipLaunchKernelGGL((direct_pairs_kernel<T, TY>), grid, block, 0, s, Lc + padc, Rq, O, k,
+                       static_cast<const uint32_t*>(flag));
     XC_HIP(hipGetLastError());
+    return true;
 }
 
 // ---------------------------------------------------------------- lanes over shifts and rows
@@ -645,8 +832,9 @@ void launch_direct_shifts(const family_args& a, const float* L, const float* R, 
 template <typename T>
 void launch_direct(const family_args& a, const T* L, const T* R, T* O, const xc_options& opt, hipStream_t s) {
     if (a.cols > (uint32_t)kMaxCols) fail(XC_ERR_UNSUPPORTED, "direct kernel: cols above 32768");
-    // tile 0, with no register tile or work distribution requested: the lanes-over-pairs kernel
-    // where it applies, else (float data) the 16 x 16 shifts kernel; 1: the register-tile kernel;
+    // tile 0, with no register tile or work distribution requested: float data by the matrix kernel
+    // where it applies, then the lanes-over-pairs kernel where it applies, else (float data) the 16 x
+    // 16 shifts kernel; 1: the register-tile kernel;
     // 2: the lanes-over-pairs kernel (float and double data alike)
     if (opt.tile > 2)
         fail(XC_ERR_INVALID_ARGUMENT, "direct-method tile must be 0 (default), 1 (register tiles) or 2 (lanes over pairs)");
@@ -654,8 +842,12 @@ void launch_direct(const family_args& a, const T* L, const T* R, T* O, const xc_
                       opt.rows_per_step || opt.waves_per_block || opt.split || opt.rows_per_block;
     if (opt.tile == 2 && rights_per_left(a) == 0)
         fail(XC_ERR_UNSUPPORTED, "direct-method tile 2 (lanes over pairs) does not serve one_to_one");
-    if (opt.tile == 2 || (opt.tile == 0 && !keys && pairs_kernel_applies(a, sizeof(T) == 4))) {
-        launch_direct_pairs<T>(a, L, R, O, s);
+    const bool free_choice = opt.tile == 0 && !keys;
+    if (std::is_same<T, float>::value && free_choice && matrix_kernel_applies(a) &&
+        launch_direct_pairs<T>(a, L, R, O, s, true))
+        return;
+    if (opt.tile == 2 || (free_choice && pairs_kernel_applies(a, sizeof(T) == 4))) {
+        launch_direct_pairs<T>(a, L, R, O, s, false);
         return;
     }
     if constexpr (std::is_same<T, float>::value) {
@@ -664,7 +856,7 @@ void launch_direct(const family_args& a, const T* L, const T* R, T* O, const xc_
         // the register tiles: 20x100 29 / 41, 20x300 110 / 109, 20x1000 833 / 676, 40x1000 1970 /
         // 1850, 64x1000 2950 / 4960, 1000x20 640 / 1150; its buffer offsets need matrices below
         // 2^31 bytes.
-        if (opt.tile == 0 && !keys && 16ull * a.rows >= a.cols && (uint64_t)a.rows * a.cols < (1u << 29)) {
+        if (free_choice && 16ull * a.rows >= a.cols && (uint64_t)a.rows * a.cols < (1u << 29)) {
             launch_direct_shifts(a, L, R, O, s);
             return;
         }

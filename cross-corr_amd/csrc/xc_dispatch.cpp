@@ -32,9 +32,18 @@ std::map<std::pair<int, hipStream_t>, std::vector<ws_slot>> g_ws;
 // slot, so what is retired stays below the slot's final size.
 std::vector<void*> g_ws_retired;
 
-}  // namespace
+bool capturing(hipStream_t s) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &st) != hipSuccess) {  // the null stream while another one captures
+        (void)hipGetLastError();
+        return true;
+    }
+    return st != hipStreamCaptureStatusNone;
+}
 
-void* workspace(int slot, size_t bytes, hipStream_t s) {
+// The slot's buffer of at least `bytes`; nullptr if there is no memory for it or, with `optional`,
+// if it is too small while `s` captures.
+void* workspace_buffer(int slot, size_t bytes, hipStream_t s, bool optional) {
     std::lock_guard<std::mutex> lock(g_ws_mutex);
     int dev = 0;
     XC_HIP(hipGetDevice(&dev));
@@ -42,6 +51,7 @@ void* workspace(int slot, size_t bytes, hipStream_t s) {
     if ((int)v.size() <= slot) v.resize(slot + 1);
     ws_slot& w = v[slot];
     if (w.bytes < bytes) {
+        if (optional && capturing(s)) return nullptr;
         size_t size = w.ptr ? std::max(bytes, 2 * w.bytes) : bytes;
         void* p = nullptr;
         if (hipMalloc(&p, size) != hipSuccess) {
@@ -49,7 +59,7 @@ void* workspace(int slot, size_t bytes, hipStream_t s) {
             size = bytes;
             if (hipMalloc(&p, size) != hipSuccess) {
                 (void)hipGetLastError();
-                fail(XC_ERR_NO_MEMORY, "workspace allocation of " + std::to_string(bytes) + " bytes failed");
+                return nullptr;
             }
         }
         if (w.ptr) g_ws_retired.push_back(w.ptr);
@@ -58,6 +68,16 @@ void* workspace(int slot, size_t bytes, hipStream_t s) {
     }
     return w.ptr;
 }
+
+}  // namespace
+
+void* workspace(int slot, size_t bytes, hipStream_t s) {
+    void* p = workspace_buffer(slot, bytes, s, false);
+    if (!p && bytes) fail(XC_ERR_NO_MEMORY, "workspace allocation of " + std::to_string(bytes) + " bytes failed");
+    return p;
+}
+
+void* workspace_if_free(int slot, size_t bytes, hipStream_t s) { return workspace_buffer(slot, bytes, s, true); }
 
 void allow_dynamic_lds(const void* kernel, uint32_t bytes) {
     static std::mutex mu;

@@ -10,6 +10,8 @@ namespace xc {
 
 // Grow-only device workspace, one per purpose; released at process exit.
 void* workspace(int slot, size_t bytes, hipStream_t s);
+// The same, or nullptr where it would have to allocate and cannot: no memory, or `s` captures a graph.
+void* workspace_if_free(int slot, size_t bytes, hipStream_t s);
 
 // On-device error checks in FP64 (xc_check.hip); they synchronise `s` to return the values.
 void validate_result_f32(const float* r, const float* v, uint64_t n, double* out5, hipStream_t s);

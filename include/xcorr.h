@@ -58,7 +58,8 @@ typedef enum xc_family {
 
 /* Arithmetic used for float inputs.  Every method accumulates in FP32 with a
  * two-level (per row-pair, then total) sum.
- *  XC_PREC_FP32     exact FP32 products on the VALU (wave64 direct kernel)
+ *  XC_PREC_FP32     FP32 products and partial sums, on the VALU (wave64 direct kernels) or, with
+ *                   many rights per left, on the FP32 matrix instructions
  *  XC_PREC_BF16X3   MFMA implicit GEMM, each operand split into bf16 hi + lo,
  *                   hi*hi + hi*lo + lo*hi; outputs whose overlap is smaller than
  *                   the border threshold are recomputed exactly in FP32
