@@ -491,8 +491,10 @@ template <int KIND, int WX, int WY, int KC, int FLUSH, bool KAHAN, int OCC, int 
 __global__ __launch_bounds__(256, OCC) void mfma_kernel(const float* __restrict__ L, const float* __restrict__ R,
                                                       float* __restrict__ O, int family, uint32_t rows,
                                                       uint32_t cols, uint32_t n, uint32_t m, uint32_t tiles_x,
-                                                      uint32_t tiles_y, uint32_t skip_area) {
+                                                      uint32_t tiles_y, uint32_t skip_area,
+                                                      const uint32_t* __restrict__ only_if) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
+    if (only_if && *only_if == 0) return;  // mfma_rights_kernel has done the batch
     const int H = (int)rows, W = (int)cols;
     uint32_t bid = xcd_remap(blockIdx.x, gridDim.x);
     const uint32_t tx = bid % tiles_x;
@@ -812,8 +814,10 @@ template <int KIND, int NS, int KC, int FLUSH, int OCC, bool PIPE_ROWS>
 __global__ __launch_bounds__(256, OCC) void mfma_rows_kernel(const float* __restrict__ L, const float* __restrict__ R,
                                                            float* __restrict__ O, int family, uint32_t rows,
                                                            uint32_t cols, uint32_t n, uint32_t m, uint32_t tiles_x,
-                                                           uint32_t tiles_y, uint32_t skip_area) {
+                                                           uint32_t tiles_y, uint32_t skip_area,
+                                                           const uint32_t* __restrict__ only_if) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
+    if (only_if && *only_if == 0) return;  // mfma_rights_kernel has done the batch
     const int H = (int)rows, W = (int)cols;
     uint32_t bid = xcd_remap(blockIdx.x, gridDim.x);
     const uint32_t tx = bid % tiles_x;
@@ -1086,7 +1090,8 @@ __global__ __launch_bounds__(256) void frame_kernel(const float* __restrict__ Ln
 }
 
 template <int KIND, int WX, int WY, int KC, int FLUSH, bool KAHAN, int OCC, int JR = 1>
-void launch(const family_args& a, const float* L, const float* R, float* O, uint32_t skip_area, hipStream_t s) {
+void launch(const family_args& a, const float* L, const float* R, float* O, uint32_t skip_area, hipStream_t s,
+            const uint32_t* only_if) {
     using G = geom<WX, WY, split_traits<KIND>::planes, KC, JR>;
     const uint32_t SX = 2 * a.cols - 1, SY = 2 * a.rows - 1;
     const uint32_t tiles_x = (SX + G::BX - 1) / G::BX;
@@ -1095,19 +1100,21 @@ void launch(const family_args& a, const float* L, const float* R, float* O, uint
     if (nblocks > 0x7fffffffULL) fail(XC_ERR_INVALID_ARGUMENT, "problem too large for one launch");
     allow_dynamic_lds(reinterpret_cast<const void*>(&mfma_kernel<KIND, WX, WY, KC, FLUSH, KAHAN, OCC, JR>), G::BYTES);
     dim3 grid((uint32_t)nblocks), block(256);
-    record_launch(KIND == XC_PREC_BF16X3   ? "mfma_kernel<bf16x3>"
+    if (!only_if)
+        record_launch(KIND == XC_PREC_BF16X3   ? "mfma_kernel<bf16x3>"
                   : KIND == XC_PREC_FP16X3 ? "mfma_kernel<fp16x3>"
                   : KIND == XC_PREC_BF16   ? "mfma_kernel<bf16>"
                                            : "mfma_kernel<fp16>",
                   grid, block, G::BYTES, a.rows, a.cols, a.pairs, 1);
-    timed tm("mfma_kernel", s);
+    timed tm("mfma_kernel", s, !only_if);
     hipLaunchKernelGGL((mfma_kernel<KIND, WX, WY, KC, FLUSH, KAHAN, OCC, JR>), grid, block, G::BYTES, s, L, R, O, a.family, a.rows, a.cols, a.n,
-                       a.m, tiles_x, tiles_y, skip_area);
+                       a.m, tiles_x, tiles_y, skip_area, only_if);
     XC_HIP(hipGetLastError());
 }
 
 template <int KIND, int NS, int KC, int FLUSH, int OCC, bool PIPE_ROWS = (OCC == 1)>
-void launch_rows(const family_args& a, const float* L, const float* R, float* O, uint32_t skip_area, hipStream_t s) {
+void launch_rows(const family_args& a, const float* L, const float* R, float* O, uint32_t skip_area, hipStream_t s,
+            const uint32_t* only_if) {
     using G = rgeom<NS, split_traits<KIND>::planes, KC>;
     const uint32_t SX = 2 * a.cols - 1, SY = 2 * a.rows - 1;
     const uint32_t tiles_x = (SX + G::BX - 1) / G::BX;
@@ -1116,15 +1123,304 @@ void launch_rows(const family_args& a, const float* L, const float* R, float* O,
     if (nblocks > 0x7fffffffULL) fail(XC_ERR_INVALID_ARGUMENT, "problem too large for one launch");
     allow_dynamic_lds(reinterpret_cast<const void*>(&mfma_rows_kernel<KIND, NS, KC, FLUSH, OCC, PIPE_ROWS>), G::BYTES);
     dim3 grid((uint32_t)nblocks), block(256);
-    record_launch(KIND == XC_PREC_BF16X3   ? "mfma_rows_kernel<bf16x3>"
+    if (!only_if)
+        record_launch(KIND == XC_PREC_BF16X3   ? "mfma_rows_kernel<bf16x3>"
                   : KIND == XC_PREC_FP16X3 ? "mfma_rows_kernel<fp16x3>"
                   : KIND == XC_PREC_BF16   ? "mfma_rows_kernel<bf16>"
                                            : "mfma_rows_kernel<fp16>",
                   grid, block, G::BYTES, a.rows, a.cols, a.pairs, 1);
-    timed tm("mfma_kernel", s);
+    timed tm("mfma_kernel", s, !only_if);
     hipLaunchKernelGGL((mfma_rows_kernel<KIND, NS, KC, FLUSH, OCC, PIPE_ROWS>), grid, block, G::BYTES, s, L, R, O, a.family, a.rows,
-                       a.cols, a.n, a.m, tiles_x, tiles_y, skip_area);
+                       a.cols, a.n, a.m, tiles_x, tiles_y, skip_area, only_if);
     XC_HIP(hipGetLastError());
+}
+
+// ---------------------------------------------------------------- lanes over rights
+// The three-product sums for batches with many rights per left: for one left, rights x shifts is a
+// matrix product over the pixels, A = 32 rights x 16 pixels, B = 16 pixels of the left x 32
+// consecutive dx (v_mfma_f32_32x32x16).  A block takes 64 rights of one left and a tile of 4 dy x 32
+// dx; its waves split the tile's steps (16 columns of one right row), column chunks outermost, so
+// that along the right rows a wave's left rows slide: a step loads 64 rights (hi and lo, 4
+// loads) and one new left row (2 loads) for 24 instructions of 32 cycles.  Operands come from split
+// copies: the rights as octets of 8 columns interleaved over slots, the lefts row-major, twice, the
+// second a column ahead, so that every 8 columns a lane wants start on 4 bytes of one of them.  No
+// LDS and no barriers before the waves' totals are added at the end, where the tiles above read every
+// B value from LDS for 64 rows of one pair only.
+// Bound: the load latency of one wave per SIMD (its 256 sums and totals leave no room for a second);
+// with the loads one step ahead the matrix cores were busy 55% of the time, with two rows per
+// iteration (two steps ahead) 64 of 256^2 took 1530 us instead of 1605.  Against the tiles, with the
+// frame, us: bf16x3 64 of 256^2 2029 -> 1530, of 128^2 305 -> 234, 16 x 64 of 64^2 421 -> 347, 64 of 200x20 277 ->
+// 118; fp16x3 64 of 256^2 2040 -> 1529, 16 x 64 of 64^2 306 -> 225.
+// FP32 partial sums of `flush` steps, FP32 totals: the rounding of both grows with their length, so
+// that their product, a wave's steps, is shared evenly between them (error at 256^2, u01: 8 steps 7.8e-8,
+// 16 6.4e-8, 32 5.8e-8, the tiles 6.9e-8; at 32^2 8 steps 4.9e-8, 16 7.2e-8, the tiles 6.0e-8, fp16x3).
+// Batches with a value that is not finite after the split are left to the tiles (*nonfinite).
+struct mr_args {
+    int family, H, W;
+    uint32_t n, m, mpl, mp;        // mpl: rights per left; mp: its slots (a multiple of 64)
+    uint32_t gpl, nr;              // groups of 64 rights per left; slots in all
+    uint32_t tiles_x, tiles_y;
+    int Q8, Hl, Wl, by_unit;       // right copy: octets per row; left copy: rows, row length
+    uint32_t skip_area;
+    int flush;                     // steps of 16 pixels per FP32 partial sum (even)
+};
+constexpr int kRightsPadC = 40;    // zero columns of the left copy before column 0
+constexpr int kRightsTY = 4;
+
+template <int KIND>
+__device__ __forceinline__ bool split_finite(float x, uint16_t& hi, uint16_t& lo) {
+    split_traits<KIND>::split(x, hi, lo);
+    const uint16_t e = KIND == XC_PREC_FP16X3 ? 0x7C00 : 0x7F80;
+    return (hi & e) != e;
+}
+
+// Left copy: element (r, c) of plane p (hi, lo) and copy k at ((i * Hl + r + 3) * 4 + 2 p + k) * Wl +
+// c + kRightsPadC - k; zero outside the matrix.  Clears *flag.
+template <int KIND>
+__global__ __launch_bounds__(256) void rights_copy_left_kernel(const float* __restrict__ X, uint16_t* __restrict__ Xc,
+                                                               uint32_t count, int H, int W, int Hl, int Wl,
+                                                               uint32_t* __restrict__ flag) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) *flag = 0;
+    const uint64_t total = (uint64_t)count * Hl * 2 * Wl;
+    for (uint64_t e = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; e < total; e += (uint64_t)gridDim.x * blockDim.x) {
+        const int x = (int)(e % (uint64_t)Wl);
+        const uint64_t rest = e / (uint64_t)Wl, row = rest / 2;
+        const int k = (int)(rest & 1), c = x - kRightsPadC + k, r = (int)(row % (uint64_t)Hl) - (kRightsTY - 1);
+        uint16_t hi = 0, lo = 0;
+        if (r >= 0 && r < H && c >= 0 && c < W) split_traits<KIND>::split(X[(row / Hl * H + r) * W + c], hi, lo);
+        Xc[(row * 4 + k) * Wl + x] = hi;
+        Xc[(row * 4 + 2 + k) * Wl + x] = lo;
+    }
+}
+
+// Right copy: octet p of row j, plane q, slot i at ((j * Q8 + p) * 2 + q) * nr + i, holding columns 8p
+// .. 8p + 7 (zero past W and in slots without a matrix).  n_to_mn (ln lefts): slot l * mp + t is
+// right l + ln t.  Sets *flag if a value here or in the lefts L does not stay finite.
+template <int KIND>
+__global__ __launch_bounds__(256) void rights_copy_right_kernel(const float* __restrict__ X, uint4* __restrict__ Xq,
+                                                                uint32_t nr, uint32_t ln, uint32_t mp, uint32_t mpl,
+                                                                int H, int W, int Q8, const float* __restrict__ L,
+                                                                uint64_t lcount, uint32_t* __restrict__ flag) {
+    const uint64_t total = (uint64_t)nr * H * Q8, stride = (uint64_t)gridDim.x * blockDim.x;
+    const uint64_t first = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    bool ok = true;
+    for (uint64_t e = first; e < lcount; e += stride) {
+        uint16_t hi, lo;
+        ok &= split_finite<KIND>(L[e], hi, lo);
+    }
+    for (uint64_t e = first; e < total; e += stride) {
+        const uint64_t i = e % nr, rest = e / nr, l = i / mp, t = i % mp;
+        const int p = (int)(rest % (uint64_t)Q8), j = (int)(rest / (uint64_t)Q8);
+        const float* __restrict__ row = X + (((ln ? l + ln * t : t) * H) + j) * (uint64_t)W;
+        uint16_t h[8], o[8];
+#pragma unroll
+        for (int c = 0; c < 8; ++c) {
+            h[c] = o[c] = 0;
+            if (t < mpl && 8 * p + c < W) ok &= split_finite<KIND>(row[8 * p + c], h[c], o[c]);
+        }
+        auto pack = [](const uint16_t (&v)[8]) {
+            return make_uint4(v[0] | (uint32_t)v[1] << 16, v[2] | (uint32_t)v[3] << 16, v[4] | (uint32_t)v[5] << 16,
+                              v[6] | (uint32_t)v[7] << 16);
+        };
+        Xq[rest * 2 * nr + i] = pack(h);
+        Xq[(rest * 2 + 1) * nr + i] = pack(o);
+    }
+    if (!ok) *flag = 1;  // every writer stores the same value
+}
+
+template <int KIND>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void mfma_rights_kernel(
+    const uint16_t* __restrict__ Lc, const uint4* __restrict__ Rq, float* __restrict__ O, mr_args a,
+    const uint32_t* __restrict__ nonfinite) {
+    constexpr int TY = kRightsTY;
+    __shared__ float part[4][2][16][64];
+    if (*nonfinite) return;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lane = threadIdx.x & 63, l32 = lane & 31, kg = lane >> 5;
+    const uint32_t groups = a.n * a.gpl;
+    uint32_t u, band;
+    if (!block_order(blockIdx.x, groups * a.tiles_x, a.tiles_y, a.by_unit, u, band)) return;
+    const uint32_t g = u % groups, li = g / a.gpl, t0 = (g % a.gpl) * 64;
+    const int H = a.H, W = a.W;
+    const int dy0 = -(H - 1) + TY * center_first((int)band, (int)a.tiles_y);
+    const int dx0 = -(W - 1) + 32 * center_first((int)(u / groups), (int)a.tiles_x);
+    const int jlo = max(0, -(dy0 + TY - 1)), rows = min(H, H - dy0) - jlo;
+    const int qlo = max(0, -(dx0 + 31)) & ~7;
+    const int nch = (min(W, W - dx0) - qlo + 15) >> 4;
+    const int steps = rows * nch;
+    const int s0 = (int)((int64_t)steps * wave >> 2), s1 = (int)((int64_t)steps * (wave + 1) >> 2);
+    const uint32_t nr16 = a.nr * 16u;  // bytes between planes; twice that between octets
+    const uint32_t slot = (a.family == XC_N_TO_MN ? li * a.mp : 0) + t0 + (uint32_t)l32;
+    const uint32_t a_off = (uint32_t)kg * 2 * nr16 + slot * 16u;
+    const int e0 = kRightsPadC + qlo + dx0, par = (e0 + l32) & 1;  // the lane's copy of the left
+    const uint32_t b_off = (uint32_t)(par * a.Wl + (e0 & 1) + 8 * kg + l32 - par) * 2u;
+    const uint4* __restrict__ at = Rq + (int64_t)(qlo >> 3) * 2 * a.nr;
+    const uint16_t* __restrict__ bt = Lc + ((int64_t)li * a.Hl + dy0 + TY - 1) * 4 * a.Wl + (e0 & ~1);
+    auto quad = [](const void* base, uint32_t lane_bytes, uint32_t uniform) {
+        return __builtin_bit_cast(uint4, buffer_quad(static_cast<const float*>(base), lane_bytes, uniform));
+    };
+    struct rights { uint4 v[2][2]; };  // [32 rights][plane]
+    struct lrow { uint4 v[2]; };
+    auto load_a = [&](int j, int ch) {
+        const uint4* p = at + ((int64_t)j * a.Q8 + 2 * ch) * 2 * a.nr;
+        rights r;
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int q = 0; q < 2; ++q) r.v[i][q] = quad(p, a_off, (uint32_t)q * nr16 + 512u * i);
+        return r;
+    };
+    auto load_b = [&](int j, int ch) {  // left row j + dy0
+        const uint16_t* p = bt + (int64_t)j * 4 * a.Wl + 16 * ch;
+        lrow r;
+#pragma unroll
+        for (int q = 0; q < 2; ++q) r.v[q] = quad(p, b_off, (uint32_t)(4 * q * a.Wl));
+        return r;
+    };
+    f32x16 acc[TY][2], tot[TY][2];
+#pragma unroll
+    for (int y = 0; y < TY; ++y)
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[y][i][r] = tot[y][i][r] = 0.0f;
+    for (int s = s0; s < s1;) {
+        // one column chunk's right rows j .. je - 1, the left rows j + dy0 .. j + dy0 + 3 in w
+        const int ch = s / rows, js = s - ch * rows, je = jlo + min(rows, js + (s1 - s));
+        int j = jlo + js;
+        s += je - j;
+        rights cur[2] = {load_a(j, ch), load_a(min(j + 1, je - 1), ch)};
+        lrow w[TY + 1];
+#pragma unroll
+        for (int y = 0; y <= TY; ++y) w[y] = load_b(min(j + y, je + TY - 2), ch);
+        while (j < je) {
+            const int stop = min(je, j + a.flush);
+            do {  // two right rows; the last ones load their own again
+                const rights nxt[2] = {load_a(min(j + 2, je - 1), ch), load_a(min(j + 3, je - 1), ch)};
+                const lrow bn[2] = {load_b(min(j + TY + 1, je + TY - 2), ch), load_b(min(j + TY + 2, je + TY - 2), ch)};
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int k = 0; k < 2; ++k) {
+                    if (k && j + 1 == je) break;
+#pragma unroll
+                    for (int p = 0; p < 3; ++p)  // hi lo, lo hi, hi hi
+#pragma unroll
+                        for (int y = 0; y < TY; ++y)
+#pragma unroll
+                            for (int i = 0; i < 2; ++i)
+                                acc[y][i] = mma<KIND>(cur[k].v[i][p == 1], w[y + k].v[p == 0], acc[y][i]);
+                }
+                cur[0] = nxt[0], cur[1] = nxt[1];
+#pragma unroll
+                for (int y = 0; y < TY - 1; ++y) w[y] = w[y + 2];
+                w[TY - 1] = bn[0], w[TY] = bn[1];
+                j += 2;
+            } while (j < stop);
+#pragma unroll
+            for (int y = 0; y < TY; ++y)
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) tot[y][i][r] += acc[y][i][r], acc[y][i][r] = 0.0f;
+        }
+    }
+    const int SX = 2 * W - 1, SY = 2 * H - 1;
+#pragma unroll
+    for (int y = 0; y < TY; ++y) {
+        const int dy = dy0 + y, oy = dy + H - 1;
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) part[wave][i][r][lane] = tot[y][i][r];
+        __syncthreads();
+        const float* pd = &part[0][0][0][0];
+        if (oy < SY) {
+#pragma unroll
+            for (int q = 0; q < 8; ++q) {
+                const int e = (int)threadIdx.x + 256 * q;
+                const double v = (((double)pd[e] + pd[2048 + e]) + pd[4096 + e]) + pd[6144 + e];
+                const int el = e & 63, r = (e >> 6) & 15, i = e >> 10, dx = dx0 + (el & 31);
+                const uint32_t t = t0 + (uint32_t)(32 * i + 8 * (r >> 2) + 4 * (el >> 5) + (r & 3));
+                const uint32_t pk = a.family == XC_N_TO_M ? li * a.m + t : (a.family == XC_N_TO_MN ? li + a.n * t : t);
+                const uint32_t area = (uint32_t)(H - abs(dy)) * (uint32_t)(W - abs(dx));
+                if (t < a.mpl && dx < W && area >= a.skip_area) O[((size_t)pk * SY + oy) * SX + dx + W - 1] = (float)v;
+            }
+        }
+    }
+}
+
+template <int KIND>
+void launch_tile(const family_args& a, const float* L, const float* R, float* O, uint32_t tile, uint32_t skip_area,
+                 hipStream_t s, const uint32_t* only_if = nullptr);
+
+// Whether mfma_rights_kernel serves this batch by default.  Its time does not shrink with a group's
+// missing rights: 3/4 of the slots busy, or 17/20 up to 64 columns (48 of 256^2 1402 us against
+// the tiles' 1541, 80 of 128^2 288 / 341); up to 64 columns also half of them where the grid is small and the tiles'
+// blocks are few (32 of 32^2 64 / 84, 40 of 64^2 94 / 159).  Flat images spend much of a wave on the
+// start of its column chunks: above 64 columns at least 48 rows, all groups counted (64 of 32x200 125 /
+// 108, of 48x200 157 / 176, 256 of 20x200 128 / 180, 64 of 40x66 90 / 76).  10^2 takes as long either way.
+bool rights_kernel_applies(const family_args& a) {
+    if (a.family == XC_ONE_TO_ONE || (uint64_t)a.rows * a.cols < 256) return false;
+    const uint64_t lefts = a.family == XC_ONE_TO_MANY ? 1 : a.n, mpl = a.family == XC_N_TO_MN ? a.m / a.n : a.m;
+    const uint64_t mp = (mpl + 63) / 64 * 64, nr = (a.family == XC_N_TO_MN ? lefts : 1) * mp;
+    if (nr * a.rows * (a.cols + 22) * 4 > (16ull << 30) || nr * 80 + 4096 >= (1ull << 31)) return false;
+    const uint64_t group_rows = lefts * (mp / 64) * a.rows;
+    if (a.cols > 64) return 4 * mpl >= 3 * mp && group_rows >= 48;
+    return 20 * mpl >= 17 * mp || (2 * mpl >= mp && group_rows <= 128);
+}
+
+// The batch by mfma_rights_kernel, with the tiles behind it for data that does not stay finite in
+// the split; false (nothing launched) if it does not apply or there is no memory for its copies.
+template <int KIND>
+bool launch_rights(const family_args& a, const float* L, const float* R, float* O, uint32_t skip_area, hipStream_t s) {
+    if (!rights_kernel_applies(a)) return false;
+    mr_args k{};
+    k.family = a.family;
+    k.H = (int)a.rows;
+    k.W = (int)a.cols;
+    k.n = a.family == XC_ONE_TO_MANY ? 1 : a.n;
+    k.m = a.m;
+    k.mpl = a.family == XC_N_TO_MN ? a.m / a.n : a.m;
+    k.mp = (k.mpl + 63) / 64 * 64;
+    k.gpl = k.mp / 64;
+    k.nr = a.family == XC_N_TO_MN ? k.n * k.mp : k.mp;
+    k.tiles_x = (2 * a.cols - 1 + 31) / 32;
+    k.tiles_y = (2 * a.rows - 1 + kRightsTY - 1) / kRightsTY;
+    k.Q8 = (k.W + 15 + 7) / 8;                     // a step of 16 columns past the last column
+    k.Hl = k.H + 2 * (kRightsTY - 1);
+    k.Wl = (kRightsPadC + k.W + 48 + 1) / 2 * 2;   // 16 columns and 32 dx past it
+    k.skip_area = skip_area;
+    k.flush = 8;
+    while (k.flush < 64 && (uint64_t)a.rows * a.cols >= 256ull * k.flush * k.flush) k.flush *= 2;
+    const uint32_t units = k.n * k.gpl * k.tiles_x;
+    k.by_unit = (units + 7) / 8 * 8 * 10 <= units * 11;
+    const uint64_t blocks = blocks_for_order(units, k.tiles_y, k.by_unit);
+    if (blocks > 0x7fffffffULL) return false;
+    const uint64_t rbytes = 32ull * k.nr * k.H * k.Q8, lelem = 4ull * k.n * k.Hl * k.Wl;
+    char* ws = static_cast<char*>(workspace_if_free(WS_SPLIT, rbytes + 2 * lelem + 16, s));
+    if (!ws) return false;
+    uint4* Rq = reinterpret_cast<uint4*>(ws);
+    uint16_t* Lc = reinterpret_cast<uint16_t*>(ws + rbytes);
+    uint32_t* flag = reinterpret_cast<uint32_t*>(ws + rbytes + (2 * lelem + 15) / 16 * 16);
+    auto blocks_for = [](uint64_t n) { return dim3((uint32_t)std::min<uint64_t>((n + 255) / 256, 16384)); };
+    hipLaunchKernelGGL(rights_copy_left_kernel<KIND>, blocks_for(lelem / 2), dim3(256), 0, s, L, Lc, k.n, k.H, k.W, k.Hl,
+                       k.Wl, flag);
+    XC_HIP(hipGetLastError());
+    hipLaunchKernelGGL(rights_copy_right_kernel<KIND>, blocks_for(rbytes / 32), dim3(256), 0, s, R, Rq, k.nr,
+                       a.family == XC_N_TO_MN ? k.n : 0u, k.mp, k.mpl, k.H, k.W, k.Q8, L,
+                       (uint64_t)k.n * a.rows * a.cols, flag);
+    XC_HIP(hipGetLastError());
+    const dim3 grid((uint32_t)blocks), block(256);
+    record_launch(KIND == XC_PREC_BF16X3 ? "mfma_rights_kernel<bf16x3>" : "mfma_rights_kernel<fp16x3>", grid, block, 0,
+                  a.rows, a.cols, a.pairs, 1);
+    {
+        timed tm("mfma_kernel", s);
+        hipLaunchKernelGGL(mfma_rights_kernel<KIND>, grid, block, 0, s, Lc, Rq, O, k, flag);
+        XC_HIP(hipGetLastError());
+    }
+    launch_tile<KIND>(a, L, R, O, 0, skip_area, s, flag);
+    return true;
 }
 
 }  // namespace
@@ -1326,21 +1622,21 @@ namespace {
 
 template <int KIND>
 void launch_tile(const family_args& a, const float* L, const float* R, float* O, uint32_t tile, uint32_t skip_area,
-                 hipStream_t s) {
+                 hipStream_t s, const uint32_t* only_if) {
     if (tile == 0) tile = a.cols <= 64 ? 6 : 9;
     switch (tile) {
-    case 1: launch<KIND, 4, 1, 128, 4, false, 2>(a, L, R, O, skip_area, s); break;
-    case 2: launch<KIND, 4, 1, 256, 2, true, 1>(a, L, R, O, skip_area, s); break;
-    case 3: launch<KIND, 4, 1, 128, 2, true, 1>(a, L, R, O, skip_area, s); break;
-    case 4: launch<KIND, 4, 1, 128, 8, false, 2>(a, L, R, O, skip_area, s); break;
-    case 5: launch<KIND, 4, 1, 64, 8, false, 2>(a, L, R, O, skip_area, s); break;
-    case 6: launch<KIND, 2, 2, 64, 4, false, 2>(a, L, R, O, skip_area, s); break;
-    case 7: launch<KIND, 4, 1, 128, 8, false, 2, 2>(a, L, R, O, skip_area, s); break;
-    case 8: launch<KIND, 4, 1, 128, 8, false, 1, 2>(a, L, R, O, skip_area, s); break;
-    case 9: launch_rows<KIND, 2, 128, 8, 2>(a, L, R, O, skip_area, s); break;
-    case 10: launch_rows<KIND, 2, 64, 8, 2>(a, L, R, O, skip_area, s); break;
-    case 11: launch_rows<KIND, 2, 128, 4, 2>(a, L, R, O, skip_area, s); break;
-    case 12: launch_rows<KIND, 1, 64, 8, 3>(a, L, R, O, skip_area, s); break;
+    case 1: launch<KIND, 4, 1, 128, 4, false, 2>(a, L, R, O, skip_area, s, only_if); break;
+    case 2: launch<KIND, 4, 1, 256, 2, true, 1>(a, L, R, O, skip_area, s, only_if); break;
+    case 3: launch<KIND, 4, 1, 128, 2, true, 1>(a, L, R, O, skip_area, s, only_if); break;
+    case 4: launch<KIND, 4, 1, 128, 8, false, 2>(a, L, R, O, skip_area, s, only_if); break;
+    case 5: launch<KIND, 4, 1, 64, 8, false, 2>(a, L, R, O, skip_area, s, only_if); break;
+    case 6: launch<KIND, 2, 2, 64, 4, false, 2>(a, L, R, O, skip_area, s, only_if); break;
+    case 7: launch<KIND, 4, 1, 128, 8, false, 2, 2>(a, L, R, O, skip_area, s, only_if); break;
+    case 8: launch<KIND, 4, 1, 128, 8, false, 1, 2>(a, L, R, O, skip_area, s, only_if); break;
+    case 9: launch_rows<KIND, 2, 128, 8, 2>(a, L, R, O, skip_area, s, only_if); break;
+    case 10: launch_rows<KIND, 2, 64, 8, 2>(a, L, R, O, skip_area, s, only_if); break;
+    case 11: launch_rows<KIND, 2, 128, 4, 2>(a, L, R, O, skip_area, s, only_if); break;
+    case 12: launch_rows<KIND, 1, 64, 8, 3>(a, L, R, O, skip_area, s, only_if); break;
     default: fail(XC_ERR_INVALID_ARGUMENT, "tile code " + std::to_string(tile) + " is not in the MFMA tile catalog");
     }
 }
@@ -1354,13 +1650,15 @@ void launch_mfma_f32(const family_args& a, const float* L, const float* R, float
     switch (kind) {
     case XC_PREC_BF16X3: {
         const uint32_t thresh = border ? border : kDefaultBorder;
-        launch_tile<XC_PREC_BF16X3>(a, L, R, O, tile, thresh, s);
+        if (tile || !launch_rights<XC_PREC_BF16X3>(a, L, R, O, thresh, s))
+            launch_tile<XC_PREC_BF16X3>(a, L, R, O, tile, thresh, s);
         launch_frame_f32(a, L, R, O, thresh, s);
         break;
     }
     case XC_PREC_FP16X3: {
         const uint32_t thresh = border ? border : kDefaultBorderFp16x3;
-        launch_tile<XC_PREC_FP16X3>(a, L, R, O, tile, thresh, s);
+        if (tile || !launch_rights<XC_PREC_FP16X3>(a, L, R, O, thresh, s))
+            launch_tile<XC_PREC_FP16X3>(a, L, R, O, tile, thresh, s);
         launch_frame_f32(a, L, R, O, thresh, s);
         break;
     }
