@@ -1146,11 +1146,11 @@ void launch_rows(const family_args& a, const float* L, const float* R, float* O,
 // second a column ahead, so that every 8 columns a lane wants start on 4 bytes of one of them.  No
 // LDS and no barriers before the waves' totals are added at the end, where the tiles above read every
 // B value from LDS for 64 rows of one pair only.
-// Bound: the load latency of one wave per SIMD (its 256 sums and totals leave no room for a second);
-// with the loads one step ahead the matrix cores were busy 55% of the time, with two rows per
-// iteration (two steps ahead) 64 of 256^2 took 1530 us instead of 1605.  Against the tiles, with the
-// frame, us: bf16x3 64 of 256^2 2029 -> 1530, of 128^2 305 -> 234, 16 x 64 of 64^2 421 -> 347, 64 of 200x20 277 ->
-// 118; fp16x3 64 of 256^2 2040 -> 1529, 16 x 64 of 64^2 306 -> 225.
+// Bound: one wave per SIMD (its 256 sums and totals leave no room for a second), so that whatever
+// it issues between two rows' products idles the matrix cores, busy 0.66 of the time: 64 of 256^2 1605 us with
+// one row per iteration, 1530 with two (loads two steps ahead), 1320..1420 with running pointers instead of
+// clamped row numbers.  Against the tiles, with the frame, us: bf16x3 64 of 256^2 1985 -> 1322, of 128^2 305 ->
+// 223, 16 x 64 of 64^2 421 -> 333, 64 of 200x20 277 -> 112; fp16x3 64 of 256^2 2040 -> 1426, 16 x 64 of 64^2 306 -> 215.
 // FP32 partial sums of `flush` steps, FP32 totals: the rounding of both grows with their length, so
 // that their product, a wave's steps, is shared evenly between them (error at 256^2, u01: 8 steps 7.8e-8,
 // 16 6.4e-8, 32 5.8e-8, the tiles 6.9e-8; at 32^2 8 steps 4.9e-8, 16 7.2e-8, the tiles 6.0e-8, fp16x3).
@@ -1162,7 +1162,7 @@ struct mr_args {
     uint32_t tiles_x, tiles_y;
     int Q8, Hl, Wl, by_unit;       // right copy: octets per row; left copy: rows, row length
     uint32_t skip_area;
-    int flush;                     // steps of 16 pixels per FP32 partial sum (even)
+    int flush;                     // steps of 16 pixels per FP32 partial sum (a power of two >= 8)
 };
 constexpr int kRightsPadC = 40;    // zero columns of the left copy before column 0
 constexpr int kRightsTY = 4;
@@ -1261,22 +1261,22 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     };
     struct rights { uint4 v[2][2]; };  // [32 rights][plane]
     struct lrow { uint4 v[2]; };
-    auto load_a = [&](int j, int ch) {
-        const uint4* p = at + ((int64_t)j * a.Q8 + 2 * ch) * 2 * a.nr;
+    const int64_t a_row = (int64_t)a.Q8 * 2 * a.nr, b_row = 4 * (int64_t)a.Wl;  // a row of the copies
+    auto load_a = [&](const uint4* p, uint32_t below) {
         rights r;
 #pragma unroll
         for (int i = 0; i < 2; ++i)
 #pragma unroll
-            for (int q = 0; q < 2; ++q) r.v[i][q] = quad(p, a_off, (uint32_t)q * nr16 + 512u * i);
+            for (int q = 0; q < 2; ++q) r.v[i][q] = quad(p, a_off, below + (uint32_t)q * nr16 + 512u * i);
         return r;
     };
-    auto load_b = [&](int j, int ch) {  // left row j + dy0
-        const uint16_t* p = bt + (int64_t)j * 4 * a.Wl + 16 * ch;
+    auto load_b = [&](const uint16_t* p, uint32_t below) {
         lrow r;
 #pragma unroll
-        for (int q = 0; q < 2; ++q) r.v[q] = quad(p, b_off, (uint32_t)(4 * q * a.Wl));
+        for (int q = 0; q < 2; ++q) r.v[q] = quad(p, b_off, below + (uint32_t)(4 * q * a.Wl));
         return r;
     };
+    const uint32_t a_next = (uint32_t)(a_row * 16), b_next = (uint32_t)(b_row * 2);  // bytes to the row below
     f32x16 acc[TY][2], tot[TY][2];
 #pragma unroll
     for (int y = 0; y < TY; ++y)
@@ -1289,16 +1289,24 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
         const int ch = s / rows, js = s - ch * rows, je = jlo + min(rows, js + (s1 - s));
         int j = jlo + js;
         s += je - j;
-        rights cur[2] = {load_a(j, ch), load_a(min(j + 1, je - 1), ch)};
+        // running pointers to the next right rows and left rows; loads past the segment (and up to 6
+        // rows past the copies' last rows, which have that slack) are not used
+        const uint4* __restrict__ pa = at + (int64_t)j * a_row + 4 * (int64_t)ch * a.nr;
+        const uint16_t* __restrict__ pb = bt + (int64_t)j * b_row + 16 * ch;
+        rights cur[2] = {load_a(pa, 0), load_a(pa, a_next)};
         lrow w[TY + 1];
 #pragma unroll
-        for (int y = 0; y <= TY; ++y) w[y] = load_b(min(j + y, je + TY - 2), ch);
+        for (int y = 0; y <= TY; ++y) w[y] = load_b(pb + y * b_row, 0);
+        pa += 2 * a_row;
+        pb += (TY + 1) * b_row;
         while (j < je) {
             const int stop = min(je, j + a.flush);
-            do {  // two right rows; the last ones load their own again
-                const rights nxt[2] = {load_a(min(j + 2, je - 1), ch), load_a(min(j + 3, je - 1), ch)};
-                const lrow bn[2] = {load_b(min(j + TY + 1, je + TY - 2), ch), load_b(min(j + TY + 2, je + TY - 2), ch)};
-                __builtin_amdgcn_sched_barrier(0);
+            do {  // two right rows
+                const rights nxt[2] = {load_a(pa, 0), load_a(pa, a_next)};
+                const lrow bn[2] = {load_b(pb, 0), load_b(pb, b_next)};
+                pa += 2 * a_row;
+                pb += 2 * b_row;
+                __builtin_amdgcn_sched_barrier(0xF);  // loads stay here; arithmetic may pass (1348 -> 1331 us)
 #pragma unroll
                 for (int k = 0; k < 2; ++k) {
                     if (k && j + 1 == je) break;
@@ -1355,11 +1363,11 @@ void launch_tile(const family_args& a, const float* L, const float* R, float* O,
                  hipStream_t s, const uint32_t* only_if = nullptr);
 
 // Whether mfma_rights_kernel serves this batch by default.  Its time does not shrink with a group's
-// missing rights: 3/4 of the slots busy, or 17/20 up to 64 columns (48 of 256^2 1402 us against
-// the tiles' 1541, 80 of 128^2 288 / 341); up to 64 columns also half of them where the grid is small and the tiles'
-// blocks are few (32 of 32^2 64 / 84, 40 of 64^2 94 / 159).  Flat images spend much of a wave on the
+// missing rights: 3/4 of the slots busy, or 17/20 up to 64 columns (48 of 256^2 1341 us against
+// the tiles' 1541); up to 64 columns also half of them where the grid is small and the tiles'
+// blocks are few (32 of 32^2 64 / 84, 40 of 64^2 91 / 159).  Flat images spend much of a wave on the
 // start of its column chunks: above 64 columns at least 48 rows, all groups counted (64 of 32x200 125 /
-// 108, of 48x200 157 / 176, 256 of 20x200 128 / 180, 64 of 40x66 90 / 76).  10^2 takes as long either way.
+// 108, of 48x200 151 / 176, 256 of 20x200 122 / 180, 64 of 40x66 90 / 76).  10^2 takes as long either way.
 bool rights_kernel_applies(const family_args& a) {
     if (a.family == XC_ONE_TO_ONE || (uint64_t)a.rows * a.cols < 256) return false;
     const uint64_t lefts = a.family == XC_ONE_TO_MANY ? 1 : a.n, mpl = a.family == XC_N_TO_MN ? a.m / a.n : a.m;
@@ -1397,12 +1405,15 @@ bool launch_rights(const family_args& a, const float* L, const float* R, float* 
     k.by_unit = (units + 7) / 8 * 8 * 10 <= units * 11;
     const uint64_t blocks = blocks_for_order(units, k.tiles_y, k.by_unit);
     if (blocks > 0x7fffffffULL) return false;
-    const uint64_t rbytes = 32ull * k.nr * k.H * k.Q8, lelem = 4ull * k.n * k.Hl * k.Wl;
-    char* ws = static_cast<char*>(workspace_if_free(WS_SPLIT, rbytes + 2 * lelem + 16, s));
+    // the kernel's loads run up to 6 rows past the last row of each copy
+    const uint64_t rbytes = 32ull * k.nr * k.H * k.Q8, rslack = 32ull * k.nr * 6 * k.Q8;
+    const uint64_t lelem = 4ull * k.n * k.Hl * k.Wl, lslack = 4ull * 6 * k.Wl;
+    if (32ull * k.nr * k.Q8 >= (1ull << 30) || 8ull * k.Wl >= (1ull << 30)) return false;  // offsets of 31 bits
+    char* ws = static_cast<char*>(workspace_if_free(WS_SPLIT, rbytes + rslack + 2 * (lelem + lslack) + 16, s));
     if (!ws) return false;
     uint4* Rq = reinterpret_cast<uint4*>(ws);
-    uint16_t* Lc = reinterpret_cast<uint16_t*>(ws + rbytes);
-    uint32_t* flag = reinterpret_cast<uint32_t*>(ws + rbytes + (2 * lelem + 15) / 16 * 16);
+    uint16_t* Lc = reinterpret_cast<uint16_t*>(ws + rbytes + rslack);
+    uint32_t* flag = reinterpret_cast<uint32_t*>(ws + rbytes + rslack + 2 * (lelem + lslack));
     auto blocks_for = [](uint64_t n) { return dim3((uint32_t)std::min<uint64_t>((n + 255) / 256, 16384)); };
     hipLaunchKernelGGL(rights_copy_left_kernel<KIND>, blocks_for(lelem / 2), dim3(256), 0, s, L, Lc, k.n, k.H, k.W, k.Hl,
                        k.Wl, flag);
