@@ -549,8 +549,11 @@ void run_batch_f32(const xc_pair* pairs, uint32_t num_pairs, const float* L, con
             }
         }
     }
-    static std::mutex mu;
-    static std::list<std::pair<std::string, std::unique_ptr<xc_batch_plan>>> cache;
+    // Never destroyed: at process exit the plans' graphs, streams and events would be given back to a
+    // HIP runtime that may have freed them itself by then (exit handlers that it registers after the
+    // first plan run before this one would).
+    static std::mutex& mu = *new std::mutex;
+    static auto& cache = *new std::list<std::pair<std::string, std::unique_ptr<xc_batch_plan>>>;
     // per stream too: a plan's workspaces and work counter serve one execution at a time
     std::string key(reinterpret_cast<const char*>(&o), sizeof(o));
     key.append(pairs_key(pairs, num_pairs));
