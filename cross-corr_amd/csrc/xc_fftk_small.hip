@@ -32,6 +32,7 @@
 #include <hip/hip_ext.h>
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <type_traits>
 
 #include "xc_fftk_core.hpp"
@@ -135,18 +136,19 @@ __global__ __launch_bounds__((small_geom<LR, LC>::NT)) void small_spec_kernel(
     for (int r = 0; r < 8; ++r) F[G::Qr * r] = u[r];
 }
 
-// Pair order: the pairs of one right are consecutive for n_to_m (an XCD's share of the pairs
-// then reads few rights with all lefts, which its L2 holds), else the family's own order.
+// Pairs q0 .. q0 + gridDim.x - 1 of the job in this order: the pairs of one right are consecutive
+// for n_to_m (an XCD's share of the pairs then reads few rights with all lefts, which its L2
+// holds), else the family's own order.
 template <typename Tout, int LR, int LC, int PS>
 __global__ __launch_bounds__((pairs_geom<LR, LC, PS>::NT), 4) void small_pairs_kernel(
     const double2* __restrict__ FL, const double2* __restrict__ FR, Tout* __restrict__ O,
     const uint64_t* __restrict__ ooff, const uint2* __restrict__ ptab, const uint2* __restrict__ mdims, uint32_t nl,
-    int family, uint32_t n, uint32_t m, uint32_t H, uint32_t W, double scale,
+    int family, uint32_t n, uint32_t m, uint32_t q0, uint32_t H, uint32_t W, double scale,
     const double2* __restrict__ tw) {
     using G = pairs_geom<LR, LC, PS>;
     extern __shared__ double2 buf[];
     const int tp = (int)threadIdx.x;
-    uint32_t q = xcd_remap(blockIdx.x, gridDim.x), l, r;
+    uint32_t q = q0 + xcd_remap(blockIdx.x, gridDim.x), l, r;
     if (ptab) {
         l = ptab[q].x;
         r = ptab[q].y;
@@ -302,11 +304,14 @@ void launch_small(const fftk_job& j, int lr, int lc, const Tio* L, const Tio* R,
             using P = pairs_geom<decltype(LR)::value, decltype(LC)::value, decltype(PS)::value>;
             auto kp = small_pairs_kernel<Tio, decltype(LR)::value, decltype(LC)::value, decltype(PS)::value>;
             allow_lds(kp, P::LDS);
-            const dim3 grid(j.pairs);
-            launch_timed("fftk_small_pairs", timing, kp, grid, dim3(P::NT), P::LDS, s, (const double2*)FL,
-                         (const double2*)FR, O, j.ooff, ptab, mdims, j.nl, j.family, j.n, j.m, j.H, j.W,
-                         1.0 / ((double)G::Pr * (double)G::Pc), tw);
-            record_launch("fftk_small_pairs", grid, dim3(P::NT), P::LDS, j.H, j.W, j.pairs, 1);
+            // one launch holds fewer than 2^32 threads (67 M pairs of up to 16 x 16)
+            constexpr uint32_t kMost = 0xffffffffu / P::NT;
+            for (uint32_t q0 = 0; q0 < j.pairs; q0 += std::min(kMost, j.pairs - q0))
+                launch_timed("fftk_small_pairs", timing, kp, dim3(std::min(kMost, j.pairs - q0)), dim3(P::NT), P::LDS,
+                             s, (const double2*)FL, (const double2*)FR, O, j.ooff, ptab, mdims, j.nl, j.family, j.n,
+                             j.m, q0, j.H, j.W, 1.0 / ((double)G::Pr * (double)G::Pc), tw);
+            record_launch("fftk_small_pairs", dim3(std::min(kMost, j.pairs)), dim3(P::NT), P::LDS, j.H, j.W, j.pairs,
+                          1);
         };
         if constexpr (G::NT >= 128) {
             // More pairs than the 256 CUs hold at once with one column per thread (1024 threads each).
