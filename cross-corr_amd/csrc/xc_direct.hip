@@ -522,7 +522,8 @@ bool matrix_kernel_applies(const family_args& a) {
 }
 
 // matrix: by direct_matrix_kernel, with direct_pairs_kernel behind it for data that is not finite;
-// false (nothing launched) if there is no memory for its copies.
+// false (nothing launched) if there is no memory for its copies.  False too where a grid does not
+// fit one launch.
 template <typename T>
 bool launch_direct_pairs(const family_args& a, const T* L, const T* R, T* O, hipStream_t s, bool matrix) {
     constexpr int TY = kPairsTY;
@@ -555,6 +556,19 @@ bool launch_direct_pairs(const family_args& a, const T* L, const T* R, T* O, hip
     if ((uint64_t)nr * 4 * sizeof(T) + 16 >= (1ull << 31)) fail(XC_ERR_UNSUPPORTED, "direct kernel: too many right matrices");
     const uint64_t lsize = (uint64_t)nl * k.Hl * k.Wl, rsize = (uint64_t)nr * H * k.Q4 * 4;
     const size_t bytes = sizeof(T) * (lsize + rsize) + sizeof(uint32_t);
+    k.by_unit = rsize * sizeof(T) > (4u << 20);  // larger than one XCD's L2
+    const uint64_t punits = (uint64_t)k.groups * k.nbx;
+    const uint64_t nblocks = blocks_for_order((uint32_t)punits, k.tiles_y, k.by_unit);
+    dp_args mk = k;  // of the matrix kernel
+    mk.gpl = k.mp / 16;
+    mk.tiles_x = (uint32_t)(2 * W - 1 + 15) / 16;
+    const uint64_t units = (uint64_t)nl * mk.gpl * mk.tiles_x;
+    // a unit's bands on one XCD (16 of 128^2 127 us; bands dealt to the XCDs in turn 179: each CU's
+    // blocks are then the same units of several bands), unless that leaves XCDs idle
+    mk.by_unit = (units + 7) / 8 * 8 * 10 <= units * 11;
+    const uint64_t mblocks = blocks_for_order((uint32_t)units, k.tiles_y, mk.by_unit);
+    if (!fits_one_launch(std::max(punits, nblocks), 256) || (matrix && !fits_one_launch(std::max(units, mblocks), 256)))
+        return false;
     T* Lc = static_cast<T*>(matrix ? workspace_if_free(WS_DIRECT, bytes, s) : workspace(WS_DIRECT, bytes, s));
     if (!Lc) return false;
     T* Rq = Lc + lsize;
@@ -566,18 +580,8 @@ bool launch_direct_pairs(const family_args& a, const T* L, const T* R, T* O, hip
     hipLaunchKernelGGL(pairs_copy_right_kernel<T>, dim3(blocks_for(rsize / 4)), dim3(256), 0, s, R, Rq, nr, a.m,
                        a.family == XC_N_TO_MN ? nl : 0u, k.mp, k.mpl, H, W, k.Q4, k.PL, Lc, lsize, flag);
     XC_HIP(hipGetLastError());
-    k.by_unit = rsize * sizeof(T) > (4u << 20);  // larger than one XCD's L2
     if constexpr (std::is_same<T, float>::value) {
         if (matrix) {
-            dp_args mk = k;
-            mk.gpl = k.mp / 16;
-            mk.tiles_x = (uint32_t)(2 * W - 1 + 15) / 16;
-            const uint32_t units = nl * mk.gpl * mk.tiles_x;
-            // a unit's bands on one XCD (16 of 128^2 127 us; bands dealt to the XCDs in turn 179: each CU's
-            // blocks are then the same units of several bands), unless that leaves XCDs idle
-            mk.by_unit = (units + 7) / 8 * 8 * 10 <= units * 11;
-            const uint64_t mblocks = blocks_for_order(units, mk.tiles_y, mk.by_unit);
-            if (mblocks > 0x7fffffffULL) fail(XC_ERR_INVALID_ARGUMENT, "problem too large for one launch");
             const dim3 grid((uint32_t)mblocks), block(256);
             record_launch("direct_pairs_kernel<f32> matrix instructions", grid, block, 0, a.rows, a.cols, a.pairs, 1);
             timed td("direct_kernel", s);
@@ -585,8 +589,6 @@ bool launch_direct_pairs(const family_args& a, const T* L, const T* R, T* O, hip
             XC_HIP(hipGetLastError());
         }
     }
-    const uint64_t nblocks = blocks_for_order(k.groups * k.nbx, k.tiles_y, k.by_unit);
-    if (nblocks > 0x7fffffffULL) fail(XC_ERR_INVALID_ARGUMENT, "problem too large for one launch");
     dim3 grid((uint32_t)nblocks), block(256);
     if (!matrix)
         record_launch(sizeof(T) == 4 ? "direct_pairs_kernel<f32> ty4 tx4" : "direct_pairs_kernel<f64> ty4 tx4", grid,
@@ -804,7 +806,8 @@ int direct_shifts_waves(uint64_t tiles, uint32_t rows) {
     return nw;
 }
 
-void launch_direct_shifts(const family_args& a, const float* L, const float* R, float* O, hipStream_t s) {
+// False (nothing launched) where the grid does not fit one launch.
+bool launch_direct_shifts(const family_args& a, const float* L, const float* R, float* O, hipStream_t s) {
     ds_args k{};
     k.family = a.family;
     k.H = (int)a.rows;
@@ -815,8 +818,8 @@ void launch_direct_shifts(const family_args& a, const float* L, const float* R, 
     k.tiles_x = (2 * a.cols - 1 + 15) / 16;
     k.tiles_y = (2 * a.rows - 1 + 15) / 16;
     const uint64_t tiles = (uint64_t)a.pairs * k.tiles_x * k.tiles_y;
-    if (tiles > 0x7fffffffULL) fail(XC_ERR_INVALID_ARGUMENT, "problem too large for one launch");
     const int nw = direct_shifts_waves(tiles, a.rows);
+    if (!fits_one_launch(tiles, 64 * nw)) return false;
     const dim3 grid((uint32_t)tiles), block(64 * nw);
     record_launch("direct_kernel<f32> 16x16 shifts, rows over lanes", grid, block, 0, a.rows, a.cols, a.pairs, 1);
     timed td("direct_kernel", s);
@@ -827,6 +830,7 @@ void launch_direct_shifts(const family_args& a, const float* L, const float* R, 
     else
         hipLaunchKernelGGL(direct_shifts_kernel<4>, grid, block, 0, s, L, R, O, k);
     XC_HIP(hipGetLastError());
+    return true;
 }
 
 template <typename T>
@@ -846,20 +850,19 @@ void launch_direct(const family_args& a, const T* L, const T* R, T* O, const xc_
     if (std::is_same<T, float>::value && free_choice && matrix_kernel_applies(a) &&
         launch_direct_pairs<T>(a, L, R, O, s, true))
         return;
-    if (opt.tile == 2 || (free_choice && pairs_kernel_applies(a, sizeof(T) == 4))) {
-        launch_direct_pairs<T>(a, L, R, O, s, false);
+    if ((opt.tile == 2 || (free_choice && pairs_kernel_applies(a, sizeof(T) == 4))) &&
+        launch_direct_pairs<T>(a, L, R, O, s, false))
         return;
-    }
+    if (opt.tile == 2) fail(XC_ERR_INVALID_ARGUMENT, "problem too large for one launch");
     if constexpr (std::is_same<T, float>::value) {
         // Few rights per left: 16 x 16 shifts per wave or block, unless the matrices are so flat
         // that a tile's 16 dy are mostly padding (16 rows < cols).  Measured, 16 pairs, us, against
         // the register tiles: 20x100 29 / 41, 20x300 110 / 109, 20x1000 833 / 676, 40x1000 1970 /
         // 1850, 64x1000 2950 / 4960, 1000x20 640 / 1150; its buffer offsets need matrices below
         // 2^31 bytes.
-        if (free_choice && 16ull * a.rows >= a.cols && (uint64_t)a.rows * a.cols < (1u << 29)) {
-            launch_direct_shifts(a, L, R, O, s);
+        if (free_choice && 16ull * a.rows >= a.cols && (uint64_t)a.rows * a.cols < (1u << 29) &&
+            launch_direct_shifts(a, L, R, O, s))
             return;
-        }
     }
     direct_plan d = plan_direct<T>(a, opt);
     if (d.lds > 160 * 1024) {
@@ -872,7 +875,8 @@ void launch_direct(const family_args& a, const T* L, const T* R, T* O, const xc_
         if (d.lds > 160 * 1024) fail(XC_ERR_UNSUPPORTED, "matrix too wide for the direct kernel's LDS row buffer");
     }
     const uint64_t nblocks = (uint64_t)d.tiles_x * d.tiles_y * d.chunks * d.groups_r * d.groups_l;
-    if (nblocks == 0 || nblocks > 0x7fffffffULL) fail(XC_ERR_INVALID_ARGUMENT, "problem too large for one launch");
+    if (nblocks == 0 || !fits_one_launch(nblocks, 64 * d.nwx * d.nwy))
+        fail(XC_ERR_INVALID_ARGUMENT, "problem too large for one launch");
     dk_args k{};
     k.family = a.family;
     k.H = (int)a.rows;

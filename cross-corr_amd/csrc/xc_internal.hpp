@@ -55,6 +55,10 @@ struct timed {
     timed& operator=(const timed&) = delete;
 };
 
+// Whether one launch holds the grid: from 2^32 threads on the grid's size wraps, and most of its
+// blocks do not run, without an error.
+inline bool fits_one_launch(uint64_t blocks, uint32_t threads) { return blocks < (1ull << 32) / threads; }
+
 // Raises the dynamic-LDS limit of `kernel` to `bytes` on the current device, once per
 // (kernel, device, size); thread-safe.
 void allow_dynamic_lds(const void* kernel, uint32_t bytes);

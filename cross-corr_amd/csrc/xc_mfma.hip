@@ -1404,7 +1404,7 @@ bool launch_rights(const family_args& a, const float* L, const float* R, float* 
     const uint32_t units = k.n * k.gpl * k.tiles_x;
     k.by_unit = (units + 7) / 8 * 8 * 10 <= units * 11;
     const uint64_t blocks = blocks_for_order(units, k.tiles_y, k.by_unit);
-    if (blocks > 0x7fffffffULL) return false;
+    if (!fits_one_launch(blocks, 256)) return false;
     // the kernel's loads run up to 6 rows past the last row of each copy
     const uint64_t rbytes = 32ull * k.nr * k.H * k.Q8, rslack = 32ull * k.nr * 6 * k.Q8;
     const uint64_t lelem = 4ull * k.n * k.Hl * k.Wl, lslack = 4ull * 6 * k.Wl;
