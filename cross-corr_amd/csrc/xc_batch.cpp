@@ -103,40 +103,33 @@ void* plan_alloc(xc_batch_plan* plan, size_t bytes) {
     return p;
 }
 
-// Own-FFT plan: pairs grouped into classes of equal transform lengths (fftk_class), one job per
-// class whose matrices keep their own sizes (the
-// job's per-matrix size table); per class the distinct left and right matrices (by offset and
-// size) are transformed once and every pair of the class is one result of the job.  Classes
-// are dealt to `branches` (1..8) parallel graph branches.
-xc_batch_plan* fft_plan_create(const xc_pair* pairs, uint32_t num_pairs, uint32_t branches) {
-    auto plan = std::make_unique<xc_batch_plan>();
-    plan->fft = true;
-    plan->kind = XC_PREC_FFT64;
-    plan->n_items = num_pairs;
-    plan->pairs.assign(pairs, pairs + num_pairs);
-    XC_HIP(hipGetDevice(&plan->device));
-    fftk_prepare();
-    using mkey = std::tuple<uint64_t, uint32_t, uint32_t>;  // offset, rows, cols
-    struct cls {
-        std::vector<uint64_t> loffs, roffs, ooffs;
-        std::vector<uint32_t> ldims, rdims, ptab;
-        std::map<mkey, uint32_t> lidx, ridx;
-        uint32_t H = 0, W = 0;
-        double work = 0.0;
-    };
-    std::map<std::pair<uint32_t, uint32_t>, cls> classes;
+// Size classes of an own-FFT plan: pairs of equal transform lengths (fftk_class, or the three-pass
+// lengths for the plain layout), with the distinct left and right matrices (by offset and size) of
+// each.
+struct fft_class {
+    std::vector<uint64_t> loffs, roffs, ooffs;
+    std::vector<uint32_t> ldims, rdims, ptab;
+    std::map<std::tuple<uint64_t, uint32_t, uint32_t>, uint32_t> lidx, ridx;  // offset, rows, cols
+    uint32_t H = 0, W = 0;
+    double work = 0.0;
+};
+using fft_classes = std::map<std::pair<uint32_t, uint32_t>, fft_class>;
+
+fft_classes classes_of(const xc_pair* pairs, uint32_t num_pairs, bool plain) {
+    fft_classes classes;
     for (uint32_t i = 0; i < num_pairs; ++i) {
         const xc_pair& p = pairs[i];
         if (2 * p.rows - 1 > 4096 || 2 * p.cols - 1 > 4096)
             fail(XC_ERR_UNSUPPORTED, "pair " + std::to_string(i) + ": the FFT batch plan takes rows, cols <= 2048");
-        cls& c = classes[fftk_class(p.rows, p.cols)];
-        auto li = c.lidx.emplace(mkey{p.left_off, p.rows, p.cols}, (uint32_t)c.loffs.size());
+        fft_class& c = classes[plain ? std::make_pair(fftk_col_len(p.rows), fftk_row_len(p.cols))
+                                     : fftk_class(p.rows, p.cols)];
+        auto li = c.lidx.emplace(std::make_tuple(p.left_off, p.rows, p.cols), (uint32_t)c.loffs.size());
         if (li.second) {
             c.loffs.push_back(p.left_off);
             c.ldims.insert(c.ldims.end(), {p.rows, p.cols});
             c.work += (double)p.rows * p.cols;
         }
-        auto ri = c.ridx.emplace(mkey{p.right_off, p.rows, p.cols}, (uint32_t)c.roffs.size());
+        auto ri = c.ridx.emplace(std::make_tuple(p.right_off, p.rows, p.cols), (uint32_t)c.roffs.size());
         if (ri.second) {
             c.roffs.push_back(p.right_off);
             c.rdims.insert(c.rdims.end(), {p.rows, p.cols});
@@ -149,9 +142,71 @@ xc_batch_plan* fft_plan_create(const xc_pair* pairs, uint32_t num_pairs, uint32_
         c.W = std::max(c.W, p.cols);
         c.work += 2.0 * p.rows * p.cols;
     }
+    return classes;
+}
+
+// The classes' jobs (without their tables), dealt largest first to the least loaded of at most
+// `branches` branches, and the workspaces of each branch: the largest that one of its jobs needs.
+struct fft_layout {
+    std::vector<fftk_job> jobs;
+    std::vector<uint32_t> job_branch;
+    std::vector<fftk_ws_sizes> need;
+    size_t bytes = 0;
+};
+
+fft_layout layout_of(const fft_classes& classes, uint32_t branches, bool plain) {
+    fft_layout v;
+    std::vector<double> cost;  // work estimate: FFT points transformed (padded lengths are proportional)
+    for (const auto& kv : classes) {
+        const fft_class& c = kv.second;
+        fftk_job j{};
+        j.H = c.H;
+        j.W = c.W;
+        j.nl = (uint32_t)c.loffs.size();
+        j.nr = (uint32_t)c.roffs.size();
+        j.pairs = (uint32_t)c.ooffs.size();
+        j.plain = plain;
+        v.jobs.push_back(j);
+        cost.push_back(c.work);
+    }
+    const uint32_t nb = (uint32_t)std::max<size_t>(1, std::min<size_t>(branches, v.jobs.size()));
+    std::vector<size_t> order(v.jobs.size());
+    for (size_t c = 0; c < order.size(); ++c) order[c] = c;
+    std::stable_sort(order.begin(), order.end(), [&](size_t a, size_t b) { return cost[a] > cost[b]; });
+    std::vector<double> load(nb, 0.0);
+    v.job_branch.assign(v.jobs.size(), 0);
+    v.need.assign(nb, fftk_ws_sizes{16, 16, 16, 16, 1});
+    for (size_t c : order) {
+        const uint32_t b = (uint32_t)(std::min_element(load.begin(), load.end()) - load.begin());
+        v.job_branch[c] = b;
+        load[b] += cost[c];
+        const fftk_ws_sizes z = fftk_sizes(v.jobs[c]);
+        v.need[b].sr = std::max(v.need[b].sr, z.sr);
+        v.need[b].sl = std::max(v.need[b].sl, z.sl);
+        v.need[b].lh = std::max(v.need[b].lh, z.lh);
+        v.need[b].z = std::max(v.need[b].z, z.z);
+    }
+    for (const fftk_ws_sizes& z : v.need) v.bytes += z.sr + z.sl + z.lh + z.z;
+    return v;
+}
+
+// Own-FFT plan: one job per class whose matrices keep their own sizes (the job's per-matrix size
+// table); a class's distinct matrices are transformed once and every pair of the class is one
+// result of the job.  Classes are dealt to `branches` (1..8) parallel graph branches.
+xc_batch_plan* fft_plan_build(const xc_pair* pairs, uint32_t num_pairs, const fft_classes& classes,
+                              const fft_layout& layout) {
+    auto plan = std::make_unique<xc_batch_plan>();
+    plan->fft = true;
+    plan->kind = XC_PREC_FFT64;
+    plan->n_items = num_pairs;
+    plan->pairs.assign(pairs, pairs + num_pairs);
+    plan->jobs = layout.jobs;
+    plan->job_branch = layout.job_branch;
+    XC_HIP(hipGetDevice(&plan->device));
+    fftk_prepare();
     // One device buffer for every class's tables.
     size_t words64 = 0, words32 = 0;
-    for (auto& kv : classes) {
+    for (const auto& kv : classes) {
         words64 += kv.second.loffs.size() + kv.second.roffs.size() + kv.second.ooffs.size();
         words32 += kv.second.ptab.size() + kv.second.ldims.size() + kv.second.rdims.size();
     }
@@ -163,9 +218,8 @@ xc_batch_plan* fft_plan_create(const xc_pair* pairs, uint32_t num_pairs, uint32_
         size_t moff, ooff, ptab, dims;
     };
     std::vector<span> spans;
-    std::vector<double> cost;
-    for (auto& kv : classes) {
-        cls& c = kv.second;
+    for (const auto& kv : classes) {
+        const fft_class& c = kv.second;
         span sp{t64.size(), 0, t32.size(), 0};
         t64.insert(t64.end(), c.loffs.begin(), c.loffs.end());
         t64.insert(t64.end(), c.roffs.begin(), c.roffs.end());
@@ -176,15 +230,6 @@ xc_batch_plan* fft_plan_create(const xc_pair* pairs, uint32_t num_pairs, uint32_
         t32.insert(t32.end(), c.ldims.begin(), c.ldims.end());
         t32.insert(t32.end(), c.rdims.begin(), c.rdims.end());
         spans.push_back(sp);
-        fftk_job j{};
-        j.H = c.H;
-        j.W = c.W;
-        j.nl = (uint32_t)c.loffs.size();
-        j.nr = (uint32_t)c.roffs.size();
-        j.pairs = (uint32_t)c.ooffs.size();
-        plan->jobs.push_back(j);
-        // work estimate: FFT points transformed (padded lengths are proportional)
-        cost.push_back(c.work);
     }
     uint64_t* d64 = static_cast<uint64_t*>(plan_alloc(plan.get(), t64.size() * sizeof(uint64_t)));
     uint32_t* d32 = static_cast<uint32_t*>(plan_alloc(plan.get(), t32.size() * sizeof(uint32_t)));
@@ -196,30 +241,12 @@ xc_batch_plan* fft_plan_create(const xc_pair* pairs, uint32_t num_pairs, uint32_
         plan->jobs[c].ptab = d32 + spans[c].ptab;
         plan->jobs[c].mdims = d32 + spans[c].dims;
     }
-    // Classes, largest first, to the least loaded branch.
-    const uint32_t nb = (uint32_t)std::max<size_t>(1, std::min<size_t>(branches, plan->jobs.size()));
-    std::vector<size_t> order(plan->jobs.size());
-    for (size_t c = 0; c < order.size(); ++c) order[c] = c;
-    std::stable_sort(order.begin(), order.end(), [&](size_t a, size_t b) { return cost[a] > cost[b]; });
-    std::vector<double> load(nb, 0.0);
-    plan->job_branch.assign(plan->jobs.size(), 0);
-    std::vector<fftk_ws_sizes> need(nb, fftk_ws_sizes{16, 16, 16, 16, 1});
-    for (size_t c : order) {
-        const uint32_t b = (uint32_t)(std::min_element(load.begin(), load.end()) - load.begin());
-        plan->job_branch[c] = b;
-        load[b] += cost[c];
-        const fftk_ws_sizes z = fftk_sizes(plan->jobs[c]);
-        need[b].sr = std::max(need[b].sr, z.sr);
-        need[b].sl = std::max(need[b].sl, z.sl);
-        need[b].lh = std::max(need[b].lh, z.lh);
-        need[b].z = std::max(need[b].z, z.z);
-    }
-    for (uint32_t b = 0; b < nb; ++b) {
+    for (const fftk_ws_sizes& need : layout.need) {
         fftk_ws w{};
-        w.sr = plan_alloc(plan.get(), need[b].sr);
-        w.sl = plan_alloc(plan.get(), need[b].sl);
-        w.lh = plan_alloc(plan.get(), need[b].lh);
-        w.z = plan_alloc(plan.get(), need[b].z);
+        w.sr = plan_alloc(plan.get(), need.sr);
+        w.sl = plan_alloc(plan.get(), need.sl);
+        w.lh = plan_alloc(plan.get(), need.lh);
+        w.z = plan_alloc(plan.get(), need.z);
         w.zchunk = 0;  // per job below
         plan->branch_ws.push_back(w);
         hipStream_t st = nullptr;
@@ -232,6 +259,25 @@ xc_batch_plan* fft_plan_create(const xc_pair* pairs, uint32_t num_pairs, uint32_
     XC_HIP(hipEventCreateWithFlags(&plan->fork, hipEventDisableTiming));
     XC_HIP(hipStreamCreateWithFlags(&plan->capture_stream, hipStreamNonBlocking));
     return plan.release();
+}
+
+// The faster layout of the spectra, or the plain one where that saves more than kFftkExtra bytes in
+// all or where there is no memory for the faster one.
+xc_batch_plan* fft_plan_create(const xc_pair* pairs, uint32_t num_pairs, uint32_t branches) {
+    {
+        const fft_classes classes = classes_of(pairs, num_pairs, false);
+        const fft_layout fast = layout_of(classes, branches, false);
+        if (fast.bytes <= kFftkExtra ||
+            fast.bytes <= layout_of(classes_of(pairs, num_pairs, true), branches, true).bytes + kFftkExtra) {
+            try {
+                return fft_plan_build(pairs, num_pairs, classes, fast);
+            } catch (const error& e) {
+                if (e.status != XC_ERR_NO_MEMORY) throw;
+            }
+        }
+    }
+    const fft_classes classes = classes_of(pairs, num_pairs, true);
+    return fft_plan_build(pairs, num_pairs, classes, layout_of(classes, branches, true));
 }
 
 // Enqueues every class of an FFT plan: on `s` alone, or forked over the branch streams.

@@ -1369,6 +1369,8 @@ void launch_job(const fftk_job& j, const Tio* L, const Tio* R, Tio* O, const fft
                   g.v3.lds, H, W, j.pairs, 1);
 }
 
+size_t bytes_of(const fftk_ws_sizes& z) { return z.sr + z.sl + z.lh + z.z; }
+
 template <typename Tio>
 void run_fftk(const family_args& a, const Tio* L, const Tio* R, Tio* O, uint32_t max_chunk, bool pow2_rows,
               hipStream_t s) {
@@ -1383,13 +1385,27 @@ void run_fftk(const family_args& a, const Tio* L, const Tio* R, Tio* O, uint32_t
     j.family = a.family;
     j.n = a.n;
     j.m = a.m;
-    const fftk_ws_sizes z = fftk_sizes(j);
+    // The faster layout where kFftkExtra lets it and its memory is there, the right spectra (the
+    // bulk of it) last; else the plain one.
+    const fftk_ws_sizes fast = fftk_sizes(j);
+    j.plain = true;
+    const fftk_ws_sizes plain = fftk_sizes(j);
     fftk_ws ws{};
-    ws.sr = workspace(WS_FK_SR, z.sr, s);
-    ws.sl = workspace(WS_FK_SL, z.sl, s);
-    ws.lh = workspace(WS_FK_LHAT, z.lh, s);
-    ws.z = workspace(WS_FK_Z, z.z, s);
-    ws.zchunk = z.chunk;
+    if (bytes_of(fast) <= bytes_of(plain) + kFftkExtra) {
+        ws.z = workspace_if_free(WS_FK_Z, fast.z, s);
+        ws.lh = ws.z ? workspace_if_free(WS_FK_LHAT, fast.lh, s) : nullptr;
+        ws.sl = ws.lh ? workspace_if_free(WS_FK_SL, fast.sl, s) : nullptr;
+        ws.sr = ws.sl ? workspace_if_free(WS_FK_SR, fast.sr, s) : nullptr;
+        ws.zchunk = fast.chunk;
+        j.plain = !ws.sr;
+    }
+    if (j.plain) {
+        ws.sr = workspace(WS_FK_SR, plain.sr, s);
+        ws.sl = workspace(WS_FK_SL, plain.sl, s);
+        ws.lh = workspace(WS_FK_LHAT, plain.lh, s);
+        ws.z = workspace(WS_FK_Z, plain.z, s);
+        ws.zchunk = plain.chunk;
+    }
     launch_job<Tio>(j, L, R, O, ws, s, true);
 }
 

@@ -87,7 +87,8 @@ struct fftk_job {
     uint32_t max_chunk = 0;
     // Row transforms of the power of two >= 2W-1 even where 3 * 2^n is shorter.
     bool pow2_rows = false;
-    // The layout of the least memory per matrix (the allocation-free entry point's split calls).
+    // The layout of the least memory per matrix (the allocation-free entry point's split calls; jobs
+    // whose faster layout would take kFftkExtra bytes more).
     bool plain = false;
 };
 struct fftk_ws_sizes {
@@ -99,6 +100,11 @@ struct fftk_ws {
     uint32_t zchunk;
 };
 fftk_ws_sizes fftk_sizes(const fftk_job& j);
+// The faster layout (spectra of the one-block kernels, column strides on 128-byte lines) takes 8
+// times the plain one's memory for matrices of few rows and 32 times for flat small ones: 131 KB
+// for 4 KB per right of 1 x 256.  It is taken while that is at most 4 GiB more, twice what Z may take:
+// 65 000 rights of 64^2, where it takes twice as much.
+constexpr size_t kFftkExtra = size_t(4) << 30;
 // Transform lengths of the own-FFT method: columns the power of two >= 2 rows - 1 (at least
 // 16); rows that, or 3 * 2^n (n = 4..9) when that is shorter.  Matrices of one job share them.
 uint32_t fftk_col_len(uint32_t rows);
