@@ -495,7 +495,7 @@ bool pairs_kernel_applies(const family_args& a, bool float_data) {
     return busy >= 0.7 && waves * busy * busy * busy >= 4500;
 }
 
-// Whether direct_matrix_kernel serves this float batch by default: its copy of the rights at most 16
+// Whether direct_matrix_kernel serves this float batch by default: its copies of both sides at most 16
 // GiB, and a shorter estimated time than the 16 x 16 shifts kernel's.  Both estimates are products
 // issued (the padding of tiles and of groups of 16 rights among them) over a rate, plus the launches;
 // the matrix kernel's also six steps per wave for its start and end, and 0.6 of its longest wave,
@@ -510,7 +510,8 @@ bool matrix_kernel_applies(const family_args& a) {
     const double lefts = a.family == XC_ONE_TO_MANY ? 1 : a.n, groups = lefts * ((mpl + 15) / 16);
     const double slots = (a.family == XC_N_TO_MN ? lefts : 1) * ((mpl + 15) / 16 * 16);
     const double H = a.rows, W = a.cols;
-    if (slots * H * (W + 27) * sizeof(float) > (double)(16ull << 30) || slots * 64 >= (double)(1u << 31)) return false;
+    const double copies = slots * H * (W + 27) + lefts * (H + 6) * (W + 55);
+    if (copies * sizeof(float) > (double)(16ull << 30) || slots * 64 >= (double)(1u << 31)) return false;
     if (a.cols < 16 && pairs_kernel_applies(a, true)) return false;
     const double SX = (2 * a.cols - 1 + 15) / 16 * 16, SY = (2 * a.rows - 1 + 3) / 4 * 4;
     const double SYs = (2 * a.rows - 1 + 15) / 16 * 16;

@@ -1372,7 +1372,8 @@ bool rights_kernel_applies(const family_args& a) {
     if (a.family == XC_ONE_TO_ONE || (uint64_t)a.rows * a.cols < 256) return false;
     const uint64_t lefts = a.family == XC_ONE_TO_MANY ? 1 : a.n, mpl = a.family == XC_N_TO_MN ? a.m / a.n : a.m;
     const uint64_t mp = (mpl + 63) / 64 * 64, nr = (a.family == XC_N_TO_MN ? lefts : 1) * mp;
-    if (nr * a.rows * (a.cols + 22) * 4 > (16ull << 30) || nr * 80 + 4096 >= (1ull << 31)) return false;
+    const uint64_t copies = nr * a.rows * (a.cols + 22) * 4 + lefts * (a.rows + 6) * (a.cols + 89) * 8;
+    if (copies > (16ull << 30) || nr * 80 + 4096 >= (1ull << 31)) return false;
     const uint64_t group_rows = lefts * (mp / 64) * a.rows;
     if (a.cols > 64) return 4 * mpl >= 3 * mp && group_rows >= 48;
     return 20 * mpl >= 17 * mp || (2 * mpl >= mp && group_rows <= 128);

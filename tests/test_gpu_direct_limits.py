@@ -31,3 +31,21 @@ def test_more_tiles_than_one_launch_holds(cols, n, m):
     wide = torch.nn.functional.pad(l64, (cols - 1, cols - 1)).unfold(1, cols, 1)
     ref = torch.tensordot(wide, right[:, 0].double().cpu(), dims=([2], [1])).transpose(1, 2)
     np.testing.assert_allclose(got[::997].cpu().numpy(), ref.numpy(), rtol=1e-6)
+
+
+def test_copies_of_many_lefts_are_bounded():
+    """15 M lefts of 1x1, 60 MB: padded for the matrix kernel they would take 23 GB."""
+    x = xcorr()
+    n, m = 15_000_000, 8
+    left = torch.rand((n, 1, 1), device="cuda")
+    right = torch.rand((m, 1, 1), device="cuda")
+    out = torch.full((n * m, 1, 1), float("nan"), device="cuda")
+    with torch.cuda.stream(torch.cuda.Stream()):  # a workspace of its own
+        torch.cuda.synchronize()
+        before = torch.cuda.mem_get_info()[0]
+        print(f"{n} x {m} of 1x1", flush=True)
+        x.cross_corr("n_to_m", left, right, out=out, precision="fp32")
+        torch.cuda.synchronize()
+        assert before - torch.cuda.mem_get_info()[0] <= 16 << 30
+    ref = left.view(n, 1) * right.view(1, m)  # one product each, rounded once
+    assert torch.equal(out.view(n, m), ref)
