@@ -522,11 +522,11 @@ bool matrix_kernel_applies(const family_args& a) {
     return matrix < shifts;
 }
 
-// matrix: by direct_matrix_kernel, with direct_pairs_kernel behind it for data that is not finite;
-// false (nothing launched) if there is no memory for its copies.  False too where a grid does not
-// fit one launch.
+// matrix: by direct_matrix_kernel, with direct_pairs_kernel behind it for data that is not finite.
+// False (nothing launched) if there is no memory for the copies, unless the kernel is `asked` for by
+// the caller (then an error), or if a grid does not fit one launch.
 template <typename T>
-bool launch_direct_pairs(const family_args& a, const T* L, const T* R, T* O, hipStream_t s, bool matrix) {
+bool launch_direct_pairs(const family_args& a, const T* L, const T* R, T* O, hipStream_t s, bool matrix, bool asked) {
     constexpr int TY = kPairsTY;
     const int H = (int)a.rows, W = (int)a.cols;
     const uint32_t nl = a.family == XC_ONE_TO_MANY ? 1 : a.n;
@@ -570,7 +570,7 @@ bool launch_direct_pairs(const family_args& a, const T* L, const T* R, T* O, hip
     const uint64_t mblocks = blocks_for_order((uint32_t)units, k.tiles_y, mk.by_unit);
     if (!fits_one_launch(std::max(punits, nblocks), 256) || (matrix && !fits_one_launch(std::max(units, mblocks), 256)))
         return false;
-    T* Lc = static_cast<T*>(matrix ? workspace_if_free(WS_DIRECT, bytes, s) : workspace(WS_DIRECT, bytes, s));
+    T* Lc = static_cast<T*>(asked ? workspace(WS_DIRECT, bytes, s) : workspace_if_free(WS_DIRECT, bytes, s));
     if (!Lc) return false;
     T* Rq = Lc + lsize;
     uint32_t* flag = matrix ? reinterpret_cast<uint32_t*>(Rq + rsize) : nullptr;
@@ -849,10 +849,10 @@ void launch_direct(const family_args& a, const T* L, const T* R, T* O, const xc_
         fail(XC_ERR_UNSUPPORTED, "direct-method tile 2 (lanes over pairs) does not serve one_to_one");
     const bool free_choice = opt.tile == 0 && !keys;
     if (std::is_same<T, float>::value && free_choice && matrix_kernel_applies(a) &&
-        launch_direct_pairs<T>(a, L, R, O, s, true))
+        launch_direct_pairs<T>(a, L, R, O, s, true, false))
         return;
     if ((opt.tile == 2 || (free_choice && pairs_kernel_applies(a, sizeof(T) == 4))) &&
-        launch_direct_pairs<T>(a, L, R, O, s, false))
+        launch_direct_pairs<T>(a, L, R, O, s, false, opt.tile == 2))
         return;
     if (opt.tile == 2) fail(XC_ERR_INVALID_ARGUMENT, "problem too large for one launch");
     if constexpr (std::is_same<T, float>::value) {
