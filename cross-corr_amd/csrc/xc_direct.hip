@@ -614,24 +614,232 @@ bool launch_direct_pairs(const family_args& a, const T* L, const T* R, T* O, hip
 // No barriers until the groups' FP64 totals are added through LDS at the end, in a fixed order.
 //
 // Bound: FP32 FMAs (LDS a fifth of the FMAs' time): 22.8 T products/s at 40 pairs of 256^2, where
-// the register tiles run 17.8; n_to_m 2 x 6 of 100x120 349 -> 137 us, 1 pair of 512^2 9.5 -> 3.4 ms.  All lanes of a tile share one column range
-// and one row range, the unions over 16 shifts: (W/2 + 8)(H/2 + 8) products issued per W/2 * H/2,
-// where the register tiles' 64-dx waves issue W/2 + 32 columns and take 32 4-byte LDS reads per
-// 128 FMAs.  Panels that hold a NaN or an infinity are summed product by product, so that a
-// shift's sum never meets a value outside its overlap (0 * inf).
+// the register tiles run 17.8; n_to_m 2 x 6 of 100x120 349 -> 137 us, 1 pair of 512^2 9.5 -> 3.4 ms.
+// All lanes of a tile share one column range and one row range, the unions over 16 shifts: (W/2 +
+// 8)(H/2 + 8) products issued per W/2 * H/2, where the register tiles' 64-dx waves issue W/2 + 32
+// columns and take 32 4-byte LDS reads per 128 FMAs.  A value that is not finite reaches only the
+// shifts whose overlap holds it: its products are added after the panels (direct_shifts_nonfinite).
 struct ds_args {
     int family, H, W;
     uint32_t n, m, pairs, tiles_x, tiles_y;
 };
 
+struct ds_panel {
+    static constexpr int JP = 8, CP = 16;            // right rows x columns
+    static constexpr int NLR = JP + 15;              // left rows
+    static constexpr int RQ = 68, LQ = 129, LS = 5;  // quads: right part, left part of a group, left row stride (bank spread)
+    static constexpr int WQ = 4 * (RQ + LQ);         // quads of a wave
+};
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) f32x4 lds_quad;
+typedef __attribute__((address_space(3))) float lds_float;
+typedef __attribute__((address_space(3))) double lds_double;
+
+__device__ __forceinline__ void wave_lds_sync() {  // the wave's own LDS: ordering its accesses is enough
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+}
+
+// The products of the first JN right rows of a panel in LDS (rq, lq: a group's right and left part).
+template <int JN, typename Quad>
+__device__ __forceinline__ void sum_panel(const Quad* rq, const Quad* lq, int gx, int gy, float (&acc)[4][4],
+                                          double (&tot)[4][4]) {
+#pragma unroll 1
+    for (int q = 0; q < ds_panel::CP / 4; ++q) {
+        const Quad* rrow = rq + (q - gx + 3);
+        const Quad* lrow = lq + 4 * gy * ds_panel::LS + q;
+        float l[4][4];
+#pragma unroll
+        for (int y = 0; y < 3; ++y) {
+            const auto v = lrow[y * ds_panel::LS];
+            l[y + 1][0] = v.x, l[y + 1][1] = v.y, l[y + 1][2] = v.z, l[y + 1][3] = v.w;
+        }
+#pragma unroll
+        for (int j = 0; j < JN; ++j) {
+#pragma unroll
+            for (int y = 0; y < 3; ++y)
+#pragma unroll
+                for (int t = 0; t < 4; ++t) l[y][t] = l[y + 1][t];
+            const auto v = lrow[(j + 3) * ds_panel::LS];
+            l[3][0] = v.x, l[3][1] = v.y, l[3][2] = v.z, l[3][3] = v.w;
+            const auto w0 = rrow[j * 8], w1 = rrow[j * 8 + 1];
+            float w[8] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w};
+            asm volatile("" : "+v"(w[0]));  // not used: keeps the quad one 16-byte read
+#pragma unroll
+            for (int y = 0; y < 4; ++y)
+#pragma unroll
+                for (int t = 0; t < 4; ++t)
+#pragma unroll
+                    for (int x = 0; x < 4; ++x) acc[y][x] = fmaf(l[y][t], w[t - x + 4], acc[y][x]);
+        }
+        if (q & 1) {  // at most 64 products per FP32 sum
+#pragma unroll
+            for (int y = 0; y < 4; ++y)
+#pragma unroll
+                for (int x = 0; x < 4; ++x) tot[y][x] += (double)acc[y][x], acc[y][x] = 0.f;
+        }
+    }
+}
+
+// The sums of a wave that met a value that is not finite, again: the same sums with zeros in place of
+// these values, and then what they bring to the shifts whose overlap holds them.  A NaN makes NaN of
+// such a shift whatever its factor: bit masks of a row's NaNs against each shift's columns.  An infinity
+// meets its factors one by one.  Leaves the totals in the wave's LDS as the kernel does.  A call of its
+// own, so that the kernel keeps its registers.  Data with one NaN per right or left, with 1% of NaNs, and
+// finite data, us (the register tiles take as long either way): 2 x 6 of 100x120 215, 468, 140 (341); 4 x
+// 4 of 300^2 11730, 15240, 6100 (19900); 8 x 4 of 64^2 110, 192, 48 (90); 1 x 4 of 10^2 20, 21, 7 (13.6).
+__device__ __attribute__((noinline)) void direct_shifts_again(const float* Lp, const float* Rp, lds_quad* wave_lds, int H,
+                                                              int W, int dx0, int dy0, int js, int je, int clo,
+                                                              int cpanels, int panels) {
+    using P = ds_panel;
+    const int lane = threadIdx.x & 63, g = lane >> 4, l16 = lane & 15, gx = lane & 3, gy = (lane >> 2) & 3;
+    lds_quad* const rq = wave_lds + g * P::RQ;
+    lds_quad* const lq = wave_lds + 4 * P::RQ + g * P::LQ;
+    lds_float* const rp = reinterpret_cast<lds_float*>(rq);
+    lds_float* const lp = reinterpret_cast<lds_float*>(lq);
+    // This lane's values of panel p.
+    float pr[2 * P::JP], pl[P::NLR];
+    auto load = [&](int p) {
+        const int j0 = js + p / cpanels * P::JP, c = clo + p % cpanels * P::CP + l16, q0 = c - dx0 - 16;
+#pragma unroll
+        for (int k = 0; k < 2 * P::JP; ++k) {
+            const int j = j0 + (k >> 1), q = q0 + 16 * (k & 1);
+            pr[k] = j < je && q >= 0 && q < W ? Rp[(size_t)j * W + q] : 0.f;
+        }
+#pragma unroll
+        for (int k = 0; k < P::NLR; ++k) {
+            const int r = j0 + dy0 + k;
+            pl[k] = r >= 0 && r < H && c < W ? Lp[(size_t)r * W + c] : 0.f;
+        }
+    };
+    auto store = [&] {
+#pragma unroll
+        for (int k = 0; k < 2 * P::JP; ++k) rp[l16 + k * 16] = pr[k];
+#pragma unroll
+        for (int k = 0; k < P::NLR; ++k) lp[l16 + k * 4 * P::LS] = pl[k];
+        wave_lds_sync();
+    };
+    double tot[4][4];
+    int p0 = panels, p1 = -1;  // the panels with such values
+    {
+        float acc[4][4];
+#pragma unroll
+        for (int y = 0; y < 4; ++y)
+#pragma unroll
+            for (int x = 0; x < 4; ++x) acc[y][x] = 0.f, tot[y][x] = 0.0;
+        for (int p = 0; p < panels; ++p) {
+            load(p);
+            bool finite = true;
+#pragma unroll
+            for (int k = 0; k < 2 * P::JP; ++k) {
+                finite = finite & __builtin_isfinite(pr[k]);
+                pr[k] = __builtin_isfinite(pr[k]) ? pr[k] : 0.f;
+            }
+#pragma unroll
+            for (int k = 0; k < P::NLR; ++k) {
+                finite = finite & __builtin_isfinite(pl[k]);
+                pl[k] = __builtin_isfinite(pl[k]) ? pl[k] : 0.f;
+            }
+            if (!__all(finite)) p0 = min(p0, p), p1 = p;
+            store();
+            sum_panel<P::JP>(rq, lq, gx, gy, acc, tot);
+            wave_lds_sync();  // the next panel overwrites this one
+        }
+    }
+    uint32_t nan = 0;  // bit 4 y + x: shift (y, x) is NaN, or beyond the result's edges
+#pragma unroll
+    for (int y = 0; y < 4; ++y)
+#pragma unroll
+        for (int x = 0; x < 4; ++x)
+            nan |= dx0 + 4 * gx + x >= W || dy0 + 4 * gy + y >= H ? 1u << (4 * y + x) : 0u;
+    auto spread = [](uint32_t y) { return (y & 1) | (y & 2) << 3 | (y & 4) << 6 | (y & 8) << 9; };
+    for (int p = p0; p <= p1 && __any(nan != 0xffffu && js < je); ++p) {
+        const int j0 = js + p / cpanels * P::JP, c0 = clo + p % cpanels * P::CP, q0 = c0 - dx0 - 16;
+        const int jn = min(P::JP, je - j0), cn = min(P::CP, W - c0);
+        load(p);
+        store();
+        // per shift x: the panel's left columns whose right column lies in the matrix, and the right
+        // columns of all its left columns; left rows in the matrix
+        uint32_t cm[4], qm[4], rm = 0;
+#pragma unroll
+        for (int x = 0; x < 4; ++x) {
+            const int d = 16 - 4 * gx - x;  // right column of the window = left column of the panel + d
+            cm[x] = 0;
+#pragma unroll
+            for (int c = 0; c < P::CP; ++c) cm[x] |= c < cn && (uint32_t)(q0 + c + d) < (uint32_t)W ? 1u << c : 0u;
+            qm[x] = ((1u << cn) - 1) << d;
+        }
+#pragma unroll
+        for (int k = 0; k < P::NLR; ++k) rm |= (uint32_t)(j0 + dy0 + k) < (uint32_t)H ? 1u << k : 0u;
+#pragma unroll 1
+        for (int j = 0; j < P::JP; ++j) {
+            const float v0 = rp[l16 + j * 32], v1 = rp[l16 + j * 32 + 16];
+            if (__all(__builtin_isfinite(v0) && __builtin_isfinite(v1))) continue;
+            const uint32_t ym = j < jn ? rm >> (j + 4 * gy) & 15u : 0u;
+            const uint32_t nans = ((uint32_t)(__ballot(v0 != v0) >> (16 * g)) & 0xffffu) |
+                                  (uint32_t)(__ballot(v1 != v1) >> (16 * g)) << 16;
+#pragma unroll
+            for (int x = 0; x < 4; ++x) nan |= nans & qm[x] ? spread(ym) << x : 0u;
+            uint32_t infs = ((uint32_t)(__ballot(__builtin_isinf(v0)) >> (16 * g)) & 0xffffu) |
+                            (uint32_t)(__ballot(__builtin_isinf(v1)) >> (16 * g)) << 16;
+            for (; __any(infs != 0); infs &= infs - 1) {
+                const int q = infs ? __builtin_ctz(infs) : 16;
+                const float v = infs ? (float)rp[j * 32 + q] : 0.f;
+#pragma unroll
+                for (int x = 0; x < 4; ++x) {
+                    const int c = q - 16 + 4 * gx + x;
+#pragma unroll
+                    for (int y = 0; y < 4; ++y)
+                        if (infs && (uint32_t)c < (uint32_t)cn && (ym >> y & 1))
+                            tot[y][x] += (double)(v * lp[c + (j + 4 * gy + y) * 4 * P::LS]);
+                }
+            }
+        }
+#pragma unroll 1
+        for (int k = 0; k < P::NLR; ++k) {
+            const float v0 = lp[l16 + k * 4 * P::LS];
+            if (__all(__builtin_isfinite(v0))) continue;
+            uint32_t ym = 0;
+#pragma unroll
+            for (int y = 0; y < 4; ++y) ym |= (uint32_t)(k - 4 * gy - y) < (uint32_t)max(jn, 0) ? 1u << y : 0u;
+            const uint32_t nans = (uint32_t)(__ballot(v0 != v0) >> (16 * g)) & 0xffffu;
+#pragma unroll
+            for (int x = 0; x < 4; ++x) nan |= nans & cm[x] ? spread(ym) << x : 0u;
+            uint32_t infs = (uint32_t)(__ballot(__builtin_isinf(v0)) >> (16 * g)) & 0xffffu;
+            for (; __any(infs != 0); infs &= infs - 1) {
+                const int c = infs ? __builtin_ctz(infs) : 0;
+                const float v = infs ? (float)lp[c + k * 4 * P::LS] : 0.f;
+#pragma unroll
+                for (int x = 0; x < 4; ++x)
+#pragma unroll
+                    for (int y = 0; y < 4; ++y)
+                        if (infs && (cm[x] >> c & 1) && (ym >> y & 1)) {
+                            const float w = rp[(k - 4 * gy - y) * 32 + c + 16 - 4 * gx - x];
+                            if (!__builtin_isinf(w)) tot[y][x] += (double)(v * w);  // else it has met this one
+                        }
+            }
+        }
+#pragma unroll
+        for (int y = 0; y < 4; ++y)
+#pragma unroll
+            for (int x = 0; x < 4; ++x) nan |= tot[y][x] != tot[y][x] ? 1u << (4 * y + x) : 0u;
+        wave_lds_sync();  // the next panel, or the totals, overwrite this one
+    }
+    auto* const td = reinterpret_cast<lds_double*>(wave_lds) + g * 256;
+#pragma unroll
+    for (int y = 0; y < 4; ++y)
+#pragma unroll
+        for (int x = 0; x < 4; ++x)
+            td[(4 * gy + y) * 16 + 4 * gx + x] = nan >> (4 * y + x) & 1 ? __builtin_nan("") : tot[y][x];
+}
+
 template <int NW>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(3))) void direct_shifts_kernel(const float* __restrict__ L,
                                                                 const float* __restrict__ R, float* __restrict__ O,
                                                                 ds_args a) {
-    constexpr int JP = 8, CP = 16;           // panel: right rows x columns
-    constexpr int NLR = JP + 15;             // left rows of a panel
-    constexpr int RQ = 68, LQ = 129, LS = 5;  // quads: right part, left part of a group, left row stride (bank spread)
-    constexpr int WQ = 4 * (RQ + LQ);        // quads of a wave
+    constexpr int JP = ds_panel::JP, CP = ds_panel::CP, NLR = ds_panel::NLR;
+    constexpr int RQ = ds_panel::RQ, LQ = ds_panel::LQ, LS = ds_panel::LS, WQ = ds_panel::WQ;
     __shared__ float4 smem[NW * WQ];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int g = lane >> 4, l16 = lane & 15, gx = lane & 3, gy = (lane >> 2) & 3;
@@ -690,51 +898,6 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(3))) vo
     for (int y = 0; y < 4; ++y)
 #pragma unroll
         for (int x = 0; x < 4; ++x) acc[y][x] = 0.f, tot[y][x] = 0.0;
-    auto flush = [&] {
-#pragma unroll
-        for (int y = 0; y < 4; ++y)
-#pragma unroll
-            for (int x = 0; x < 4; ++x) {
-                tot[y][x] += (double)acc[y][x];
-                acc[y][x] = 0.f;
-            }
-    };
-    auto lds_sync = [] {  // the wave's own LDS: ordering its accesses is enough
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-    };
-
-    // The products of the first JN right rows of the panel in LDS.
-    auto sum_panel = [&](auto JN) {
-#pragma unroll 1
-        for (int q = 0; q < CP / 4; ++q) {
-            const float4* rrow = rq + (q - gx + 3);
-            const float4* lrow = lq + 4 * gy * LS + q;
-            float4 lv[4];
-#pragma unroll
-            for (int y = 0; y < 3; ++y) lv[y + 1] = lrow[y * LS];
-#pragma unroll
-            for (int j = 0; j < decltype(JN)::value; ++j) {
-#pragma unroll
-                for (int y = 0; y < 3; ++y) lv[y] = lv[y + 1];
-                lv[3] = lrow[(j + 3) * LS];
-                float4 w0 = rrow[j * 8];
-                const float4 w1 = rrow[j * 8 + 1];
-                asm volatile("" : "+v"(w0.x));  // not used: keeps the quad one 16-byte read
-                const float w[8] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w};
-#pragma unroll
-                for (int y = 0; y < 4; ++y) {
-                    const float l[4] = {lv[y].x, lv[y].y, lv[y].z, lv[y].w};
-#pragma unroll
-                    for (int t = 0; t < 4; ++t)
-#pragma unroll
-                        for (int x = 0; x < 4; ++x) acc[y][x] = fmaf(l[t], w[t - x + 4], acc[y][x]);
-                }
-            }
-            if (q & 1) flush();  // at most 64 products per FP32 sum
-        }
-    };
 
     const int panels = jpanels * cpanels, share = (cnt + 4 * NW - 1) / (4 * NW);
     fetch(js, clo);
@@ -747,42 +910,29 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(3))) vo
         const int rows_left = share - jp * JP;  // of the longest group
         if (++cp == cpanels) cp = 0, ++jp;
         if (p + 1 < panels) fetch(js + jp * JP, clo + cp * CP);
-        lds_sync();
+        wave_lds_sync();
         if (rows_left > JP / 2)
-            sum_panel(std::integral_constant<int, JP>{});
+            sum_panel<JP>(rq, lq, gx, gy, acc, tot);
         else
-            sum_panel(std::integral_constant<int, JP / 2>{});
-        lds_sync();  // the next panel overwrites this one
+            sum_panel<JP / 2>(rq, lq, gx, gy, acc, tot);
+        wave_lds_sync();  // the next panel overwrites this one
     }
-    // A value that is not finite makes a total of every lane that met it so, overlap or not (0 *
-    // inf): such a wave sums its shifts again, each over its own overlap only.
     bool finite = true;
 #pragma unroll
     for (int y = 0; y < 4; ++y)
 #pragma unroll
         for (int x = 0; x < 4; ++x) finite = finite & __builtin_isfinite(tot[y][x]);
-    if (!__all(finite)) {
-#pragma unroll 1
-        for (int o = 0; o < 16; ++o) {
-            const int dy = dy0 + 4 * gy + (o >> 2), dx = dx0 + 4 * gx + (o & 3);
-            double v = 0.0;
-            for (int j = max(js, -dy); j < min(je, H - dy); ++j) {
-                float part = 0.f;
-                for (int c = max(0, dx); c < min(W, W + dx); ++c)
-                    part = fmaf(Lp[(size_t)(j + dy) * W + c], Rp[(size_t)j * W + c - dx], part);
-                v += (double)part;
-            }
+    // The groups' totals, added in order.  A value that is not finite makes a total of every lane that
+    // met it so, overlap or not (0 * inf): such a wave sums again.
+    if (__all(finite)) {
+        double* const td = reinterpret_cast<double*>(smem + wave * WQ) + g * 256;
 #pragma unroll
-            for (int i = 0; i < 16; ++i)
-                if (i == o) tot[i >> 2][i & 3] = v;
-        }
+        for (int y = 0; y < 4; ++y)
+#pragma unroll
+            for (int x = 0; x < 4; ++x) td[(4 * gy + y) * 16 + 4 * gx + x] = tot[y][x];
+    } else {
+        direct_shifts_again(Lp, Rp, (lds_quad*)(float4*)(smem + wave * WQ), H, W, dx0, dy0, js, je, clo, cpanels, panels);
     }
-    // The groups' totals, added in order.
-    double* const td = reinterpret_cast<double*>(smem + wave * WQ) + g * 256;
-#pragma unroll
-    for (int y = 0; y < 4; ++y)
-#pragma unroll
-        for (int x = 0; x < 4; ++x) td[(4 * gy + y) * 16 + 4 * gx + x] = tot[y][x];
     __syncthreads();
     const int SX = 2 * W - 1, SY = 2 * H - 1;
     float* __restrict__ Op = O + (size_t)pair * SX * SY;
