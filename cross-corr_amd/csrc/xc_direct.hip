@@ -134,6 +134,27 @@ direct_plan plan_direct(const family_args& a, const xc_options& opt) {
     return d;
 }
 
+dk_args args_of(const family_args& a, const direct_plan& d) {
+    dk_args k{};
+    k.family = a.family;
+    k.H = (int)a.rows;
+    k.W = (int)a.cols;
+    k.n = a.family == XC_ONE_TO_ONE || a.family == XC_ONE_TO_MANY ? 1 : a.n;
+    k.m = a.family == XC_ONE_TO_ONE ? 1 : a.m;
+    k.mpl = a.family == XC_N_TO_MN ? a.m / a.n : 0;
+    k.tiles_x = d.tiles_x;
+    k.tiles_y = d.tiles_y;
+    k.chunks = d.chunks;
+    k.rows_per_chunk = d.rows_per_chunk;
+    k.groups_l = d.groups_l;
+    k.groups_r = d.groups_r;
+    k.nwx = d.nwx;
+    k.nwy = d.nwy;
+    k.len = d.len;
+    k.atomic = d.chunks > 1 ? 1 : 0;
+    return k;
+}
+
 // ---------------------------------------------------------------- lanes over pairs
 // Definition-based FP32 kernel for batches with many rights per left (one_to_many, n_to_m,
 // n_to_mn).  A wave takes one left and 64 of its rights (the pairs (left, right), one per
@@ -522,7 +543,35 @@ bool matrix_kernel_applies(const family_args& a) {
     return matrix < shifts;
 }
 
-// matrix: by direct_matrix_kernel, with direct_pairs_kernel behind it for data that is not finite.
+// The register tiles behind direct_matrix_kernel, in one chunk (no atomics, which would need a zeroed
+// output): the plan, and its kernel if it is one of the defaults for several rights per left.
+const void* tiles_behind(const family_args& a, direct_plan& d) {
+    xc_options o{};
+    o.split = 1;
+    d = plan_direct<float>(a, o);
+    const uint64_t nblocks = (uint64_t)d.tiles_x * d.tiles_y * d.groups_r * d.groups_l;
+    if (d.lds > 160 * 1024 || !fits_one_launch(nblocks, 64 * d.nwx * d.nwy)) return nullptr;
+    if (d.t.ty == 4 && d.t.rm == 2 && d.t.lm == 1 && d.t.jb == 2)
+        return reinterpret_cast<const void*>(&direct_kernel<float, 4, 2, 1, 2, true>);
+    if (d.t.ty == 2 && d.t.rm == 4 && d.t.lm == 2 && d.t.jb == 2)
+        return reinterpret_cast<const void*>(&direct_kernel<float, 2, 4, 2, 2, true>);
+    return nullptr;
+}
+
+void launch_tiles_behind(const family_args& a, const float* L, const float* R, float* O, const direct_plan& d,
+                         const void* fn, const uint32_t* flag, hipStream_t s) {
+    dk_args k = args_of(a, d);
+    k.only_if = flag;
+    if (d.lds > 65536) allow_dynamic_lds(fn, d.lds);
+    void* args[] = {(void*)&L, (void*)&R, (void*)&O, (void*)&k};
+    XC_HIP(hipLaunchKernel(fn, dim3(d.tiles_x * d.tiles_y * d.groups_r * d.groups_l), dim3(64 * d.nwx * d.nwy), args,
+                           d.lds, s));
+}
+
+// matrix: by direct_matrix_kernel, with another kernel behind it for data that is not finite: up to 39
+// rights per left the register tiles, from 40 on direct_pairs_kernel, whose lanes are then 5/8 busy.
+// us with a NaN, tiles / pairs behind (the tiles by themselves): 16 of 128^2 569 / 1167 (391), 32 of 200^2
+// 3170 / 3700 (3090), 16 x 12 of 64^2 484 / 640 (288).
 // False (nothing launched) if there is no memory for the copies, unless the kernel is `asked` for by
 // the caller (then an error), or if a grid does not fit one launch.
 template <typename T>
@@ -568,7 +617,10 @@ bool launch_direct_pairs(const family_args& a, const T* L, const T* R, T* O, hip
     // blocks are then the same units of several bands), unless that leaves XCDs idle
     mk.by_unit = (units + 7) / 8 * 8 * 10 <= units * 11;
     const uint64_t mblocks = blocks_for_order((uint32_t)units, k.tiles_y, mk.by_unit);
-    if (!fits_one_launch(std::max(punits, nblocks), 256) || (matrix && !fits_one_launch(std::max(units, mblocks), 256)))
+    direct_plan behind{};
+    const void* tiles = matrix && k.mpl < 40 ? tiles_behind(a, behind) : nullptr;
+    if ((!tiles && !fits_one_launch(std::max(punits, nblocks), 256)) ||
+        (matrix && !fits_one_launch(std::max(units, mblocks), 256)))
         return false;
     T* Lc = static_cast<T*>(asked ? workspace(WS_DIRECT, bytes, s) : workspace_if_free(WS_DIRECT, bytes, s));
     if (!Lc) return false;
@@ -588,6 +640,10 @@ bool launch_direct_pairs(const family_args& a, const T* L, const T* R, T* O, hip
             timed td("direct_kernel", s);
             hipLaunchKernelGGL(direct_matrix_kernel, grid, block, 0, s, Lc, Rq, O, mk, flag);
             XC_HIP(hipGetLastError());
+        }
+        if (tiles) {
+            launch_tiles_behind(a, L, R, O, behind, tiles, flag, s);
+            return true;
         }
     }
     dim3 grid((uint32_t)nblocks), block(256);
@@ -1028,23 +1084,7 @@ void launch_direct(const family_args& a, const T* L, const T* R, T* O, const xc_
     const uint64_t nblocks = (uint64_t)d.tiles_x * d.tiles_y * d.chunks * d.groups_r * d.groups_l;
     if (nblocks == 0 || !fits_one_launch(nblocks, 64 * d.nwx * d.nwy))
         fail(XC_ERR_INVALID_ARGUMENT, "problem too large for one launch");
-    dk_args k{};
-    k.family = a.family;
-    k.H = (int)a.rows;
-    k.W = (int)a.cols;
-    k.n = a.family == XC_ONE_TO_ONE || a.family == XC_ONE_TO_MANY ? 1 : a.n;
-    k.m = a.family == XC_ONE_TO_ONE ? 1 : a.m;
-    k.mpl = a.family == XC_N_TO_MN ? a.m / a.n : 0;
-    k.tiles_x = d.tiles_x;
-    k.tiles_y = d.tiles_y;
-    k.chunks = d.chunks;
-    k.rows_per_chunk = d.rows_per_chunk;
-    k.groups_l = d.groups_l;
-    k.groups_r = d.groups_r;
-    k.nwx = d.nwx;
-    k.nwy = d.nwy;
-    k.len = d.len;
-    k.atomic = d.chunks > 1 ? 1 : 0;
+    dk_args k = args_of(a, d);
     if (k.atomic) {
         const uint64_t count = (uint64_t)a.pairs * (2 * a.cols - 1) * (2 * a.rows - 1);
         uint32_t zb = (uint32_t)std::min<uint64_t>((count + 255) / 256, 8192);

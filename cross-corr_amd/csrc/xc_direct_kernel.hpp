@@ -64,6 +64,7 @@ struct dk_args {
     uint32_t nwx, nwy;           // waves of a block along dx and along dy
     int len;                     // LDS elements per staged row
     int atomic;                  // 1: add into a zeroed output
+    const uint32_t* only_if;     // BEHIND: flag of the kernel before, 0 where that one has done the batch
 };
 
 template <typename T>
@@ -80,8 +81,9 @@ constexpr int cols_per_step() {
 }
 
 // One block: dx in [dxb, dxb + 64*nwx), dy in [dyb, dyb + TY*nwy), the right rows of its
-// chunk, one group of LM left x RM right matrices.
-template <typename T, int TY, int RM, int LM, int JB>
+// chunk, one group of LM left x RM right matrices.  BEHIND: a launch that leaves at once unless
+// *only_if.
+template <typename T, int TY, int RM, int LM, int JB, bool BEHIND = false>
 __global__ __launch_bounds__(512) void direct_kernel(const T* __restrict__ L, const T* __restrict__ R,
                                                      T* __restrict__ O, dk_args a) {
     constexpr int CW = cols_per_step<T, TY, LM, JB>();
@@ -91,6 +93,9 @@ __global__ __launch_bounds__(512) void direct_kernel(const T* __restrict__ L, co
     using Tot = typename total_of<T>::type;
     extern __shared__ __attribute__((aligned(16))) char smem_raw[];
     T* buf = reinterpret_cast<T*>(smem_raw);  // [2][JB][RM][len]
+
+    if constexpr (BEHIND)
+        if (*a.only_if == 0) return;
 
     const int H = a.H, W = a.W;
     const int SX = 2 * W - 1, SY = 2 * H - 1;

@@ -61,3 +61,31 @@ def test_only_the_overlaps_show_it(family, rows, cols, n, m, side, kind):
     shown = ~fine & ~np.isnan(ref)
     np.testing.assert_array_equal(got[shown], ref[shown].astype(np.float32))
     np.testing.assert_array_equal(got[fine], clean[fine])
+
+
+@pytest.mark.parametrize("kind", ["nan", "mixed"])
+@pytest.mark.parametrize("family,rows,cols,n,m", [("one_to_many", 90, 80, 1, 16), ("n_to_m", 33, 47, 12, 20),
+                                                  ("n_to_mn", 64, 50, 3, 48), ("one_to_many", 128, 300, 1, 9)])
+def test_behind_the_matrix_kernel(family, rows, cols, n, m, kind):
+    """Up to 39 rights per left the matrix kernel leaves such a batch to the register tiles, and serves
+    finite data after it as before."""
+    x = xcorr()
+    rng = np.random.default_rng(6)
+    left, right = seeded((n, rows, cols), "u01", 93, np.float32), seeded((m, rows, cols), "u01", 94, np.float32)
+    shape = x.result_shape(family, rows, cols, n, m)
+
+    def call(l, r, kernel="direct_pairs_kernel<f32> matrix instructions", **kw):
+        out = torch.full(shape, 7.0, device="cuda")
+        print(f"matrix {family} {l.shape} {r.shape}", flush=True)
+        x.cross_corr(family, torch.from_numpy(l).cuda(), torch.from_numpy(r).cuda(), out=out, precision="fp32", **kw)
+        torch.cuda.synchronize()
+        assert x.last_launch()["kernel"].startswith(kernel)
+        return out.cpu().numpy()
+
+    clean = call(left, right)
+    r = right.copy()
+    spoil(r[m // 2:m // 2 + 1], kind, rng)
+    got = call(left, r)
+    assert not np.isfinite(got).all()
+    np.testing.assert_array_equal(got, call(left, r, "direct_kernel<f32> ty", tile=1, split=1))
+    np.testing.assert_array_equal(call(left, right), clean)
