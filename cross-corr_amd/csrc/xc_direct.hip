@@ -378,7 +378,7 @@ __global__ __launch_bounds__(256) void pairs_copy_right_kernel(const T* __restri
 // with 149 registers, and twice as long where the second was idle.  16 x 64 of 64^2 700 -> 465 us.
 // Columns are the union over 16 dx, rounded up to 16 (about 16 more than a single dx has), rows
 // the union over 4 dy.  A zero of the copies' padding must not meet an infinity or a NaN: a batch
-// that holds one (*nonfinite) is left to direct_pairs_kernel, which reads the same copies.
+// that holds one (*nonfinite) is left to the kernel behind this one (launch_direct_pairs).
 constexpr int kMatrixPadC = 20;  // zero columns of the left copy before column 0
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void direct_matrix_kernel(
     const float* __restrict__ Lc, const float* __restrict__ Rq, float* __restrict__ O, dp_args a,
@@ -1004,13 +1004,41 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(3))) vo
 
 // Waves per block, each with four of the tile's 4 NW shares of right rows: more waves while the
 // shares keep about 4 rows and the tiles are too few to balance the 256 CUs (the longer the sums,
-// the more of them it takes).  Measured us with 1 / 2 / 4 waves: 1 pair of 64^2 43 / 24 / 18, 8 of
-// 128^2 194 / 150 / 114, 64 of 64^2 72 / 70 / 90, 40 of 32^2 14 / 13 / 18, 40 of 256^2 7630 / 7880 /
-// 8110, 64 of 50x80 87 / 92 / 107.
+// the more of them it takes), and where even four waves a tile leave places on the chip, until a share has
+// the 4 rows of a half panel.  Measured us with 1 / 2 / 4 waves: 1 pair of 64^2 43 / 24 / 18, 8 of 128^2
+// 194 / 150 / 114, 64 of 64^2 72 / 70 / 90, 40 of 32^2 14 / 13 / 18, 40 of 256^2 7630 / 7880 / 8110, 64
+// of 50x80 87 / 92 / 107; 2 / 4 waves: 1 pair of 39x344 118 / 76, of 33x321 112 / 72.
 int direct_shifts_waves(uint64_t tiles, uint32_t rows) {
     int nw = 1;
     while (nw < 4 && rows >= 20u * nw && tiles * nw < 72ull * rows) nw *= 2;
+    if (tiles <= 768)
+        while (nw < 4 && rows > 16u * nw) nw *= 2;
     return nw;
+}
+
+// Whether the register tiles take less time than the 16 x 16 shifts for batches of one right per left,
+// where neither fills the chip and a wave's own chain of steps counts.  Both are estimated, in us: the
+// shifts from a tile's panels (a half one for a last share of up to 4 rows) and the products issued, the
+// tiles from a block's steps (rows of its chunk, in turns of 4) times columns, longer the more blocks
+// share the chip.  640 shapes of 6 to 400 rows and columns were measured with both, 1 to 12 pairs: the
+// estimates are off by 6% and 9%, and on the wrong side by more than 3% at 5 shapes in 268 (by 11% at
+// most).  us, shifts / tiles: 129x37 28.3 / 20.0, 126x37 19.1 / 15.3, 26x335 72 / 53, 65x124 45 / 34, 128^2
+// 44.5 / 43.9, 54x61 16.6 / 27.9, 130^2 79 / 121.  Up to 5 rows (7 to 18 us; the tiles up to
+// a fifth less) the shifts stay.
+bool register_tiles_faster(const family_args& a) {
+    if (rights_per_left(a) > 1 || (a.family == XC_N_TO_M && a.n > 1) || a.rows <= 5) return false;
+    const double W = a.cols, tx = (2 * a.cols - 1 + 15) / 16, ty = (2 * a.rows - 1 + 15) / 16;
+    const int nw = direct_shifts_waves((uint64_t)a.pairs * (uint64_t)(tx * ty), a.rows);
+    const uint32_t share = (a.rows + 4 * nw - 1) / (4 * nw), rest = share % 8;
+    const double panel = 5.04 * (share / 8 + (rest > 4)) + (rest > 0 && rest <= 4 ? 3.09 : 0.0);
+    const double chain = 3.4 + std::ceil(W / 16) * panel;
+    const double issue = a.pairs * tx * ty * 256 * (a.rows / 2.0 + 8) * (W / 2 + 8) / 20.7e6;
+    const double shifts = std::pow(std::pow(chain, 1.6) + std::pow(issue, 1.6), 1 / 1.6);
+    const direct_plan d = plan_direct<float>(a, xc_options{});
+    const uint32_t rows = d.rows_per_chunk ? d.rows_per_chunk : a.rows, steps = (rows + d.t.jb - 1) / d.t.jb;
+    const double waves = (double)d.tiles_x * d.tiles_y * d.chunks * d.groups_r * d.groups_l * d.nwx * d.nwy;
+    const double tiles = 3.9 + (d.chunks > 1 ? 1.95 : 0.0) + steps * (W + 23) * (0.056 + 2.05e-5 * waves);
+    return tiles < shifts;
 }
 
 // False (nothing launched) where the grid does not fit one launch.
@@ -1068,7 +1096,7 @@ void launch_direct(const family_args& a, const T* L, const T* R, T* O, const xc_
         // 1850, 64x1000 2950 / 4960, 1000x20 640 / 1150; its buffer offsets need matrices below
         // 2^31 bytes.
         if (free_choice && 16ull * a.rows >= a.cols && (uint64_t)a.rows * a.cols < (1u << 29) &&
-            launch_direct_shifts(a, L, R, O, s))
+            !register_tiles_faster(a) && launch_direct_shifts(a, L, R, O, s))
             return;
     }
     direct_plan d = plan_direct<T>(a, opt);
