@@ -697,10 +697,14 @@ __device__ __forceinline__ void wave_lds_sync() {  // the wave's own LDS: orderi
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
 }
 
-// The products of the first JN right rows of a panel in LDS (rq, lq: a group's right and left part).
+// The products of the first JN right rows of a panel in LDS (rq, lq: a group's right and left part).  An
+// FP32 sum takes 8 columns of the panel's rows, at most 64 products; `narrow` (matrices of one panel's
+// columns) 4, since the register tiles' sums of such matrices ended with each step's rows: 100x12, signed
+// data, relative error in the 2-norm 9.6e-8 with 8 columns, 7.8e-8 with 4, the
+// tiles 9.0e-8.
 template <int JN, typename Quad>
-__device__ __forceinline__ void sum_panel(const Quad* rq, const Quad* lq, int gx, int gy, float (&acc)[4][4],
-                                          double (&tot)[4][4]) {
+__device__ __forceinline__ void sum_panel(const Quad* rq, const Quad* lq, int gx, int gy, bool narrow,
+                                          float (&acc)[4][4], double (&tot)[4][4]) {
 #pragma unroll 1
     for (int q = 0; q < ds_panel::CP / 4; ++q) {
         const Quad* rrow = rq + (q - gx + 3);
@@ -729,7 +733,7 @@ __device__ __forceinline__ void sum_panel(const Quad* rq, const Quad* lq, int gx
 #pragma unroll
                     for (int x = 0; x < 4; ++x) acc[y][x] = fmaf(l[y][t], w[t - x + 4], acc[y][x]);
         }
-        if (q & 1) {  // at most 64 products per FP32 sum
+        if ((q & 1) || narrow) {
 #pragma unroll
             for (int y = 0; y < 4; ++y)
 #pragma unroll
@@ -799,7 +803,7 @@ __device__ __attribute__((noinline)) void direct_shifts_again(const float* Lp, c
             }
             if (!__all(finite)) p0 = min(p0, p), p1 = p;
             store();
-            sum_panel<P::JP>(rq, lq, gx, gy, acc, tot);
+            sum_panel<P::JP>(rq, lq, gx, gy, W <= P::CP, acc, tot);
             wave_lds_sync();  // the next panel overwrites this one
         }
     }
@@ -968,9 +972,9 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(3))) vo
         if (p + 1 < panels) fetch(js + jp * JP, clo + cp * CP);
         wave_lds_sync();
         if (rows_left > JP / 2)
-            sum_panel<JP>(rq, lq, gx, gy, acc, tot);
+            sum_panel<JP>(rq, lq, gx, gy, W <= CP, acc, tot);
         else
-            sum_panel<JP / 2>(rq, lq, gx, gy, acc, tot);
+            sum_panel<JP / 2>(rq, lq, gx, gy, W <= CP, acc, tot);
         wave_lds_sync();  // the next panel overwrites this one
     }
     bool finite = true;

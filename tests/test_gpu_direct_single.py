@@ -29,3 +29,22 @@ def test_kernel_and_parity(family, rows, cols, n, m, kernel):
     l64, r64 = left.astype(np.float64), right.astype(np.float64)
     err, _ = norm_error(out.cpu().numpy(), oracle_family(family, l64, r64), oracle_family(family, l64, r64, absval=True))
     assert err <= 1e-6, (family, rows, cols, err)
+
+
+@pytest.mark.parametrize("rows,cols,m", [(100, 12, 6), (16, 16, 4), (60, 16, 3), (130, 9, 5)])
+@pytest.mark.parametrize("dist", ["u01", "u11", "normal"])
+def test_narrow_matrices_are_as_exact_as_by_the_register_tiles(rows, cols, m, dist):
+    """Relative error in the 2-norm over several batches, against the kernel that served them before."""
+    x = xcorr()
+    wrong, total = {0: 0.0, 1: 0.0}, 0.0
+    for seed in range(8):
+        left, right = seeded((1, rows, cols), dist, 300 + seed, np.float32), seeded((m, rows, cols), dist, 400 + seed, np.float32)
+        ref = oracle_family("one_to_many", left.astype(np.float64), right.astype(np.float64))
+        total += (ref ** 2).sum()
+        for tile in wrong:
+            out = x.cross_corr("one_to_many", torch.from_numpy(left).cuda(), torch.from_numpy(right).cuda(),
+                               precision="fp32", tile=tile)
+            assert x.last_launch()["kernel"].startswith(TILES if tile else SHIFTS)
+            wrong[tile] += ((out.cpu().numpy().astype(np.float64).reshape(ref.shape) - ref) ** 2).sum()
+    print(rows, cols, dist, [(v / total) ** 0.5 for v in wrong.values()])
+    assert wrong[0] <= wrong[1]
