@@ -1023,26 +1023,30 @@ int direct_shifts_waves(uint64_t tiles, uint32_t rows) {
 // Whether the register tiles take less time than the 16 x 16 shifts for batches of one right per left,
 // where neither fills the chip and a wave's own chain of steps counts.  Both are estimated, in us: the
 // shifts from a tile's panels (a half one for a last share of up to 4 rows) and the products issued, the
-// tiles from a block's steps (rows of its chunk, in turns of 4) times columns, longer the more blocks
-// share the chip.  640 shapes of 6 to 400 rows and columns were measured with both, 1 to 12 pairs: the
-// estimates are off by 6% and 9%, and on the wrong side by more than 3% at 5 shapes in 268 (by 11% at
-// most).  us, shifts / tiles: 129x37 28.3 / 20.0, 126x37 19.1 / 15.3, 26x335 72 / 53, 65x124 45 / 34, 128^2
-// 44.5 / 43.9, 54x61 16.6 / 27.9, 130^2 79 / 121.  Up to 5 rows (7 to 18 us; the tiles up to
-// a fifth less) the shifts stay.
+// tiles from a block's steps (rows of its chunk, in turns of 4) times columns, longer the more waves
+// share the chip; more than it holds at once, 4096, take a second round, which the estimate does not
+// know.  1358 shapes of 6 to 512 rows and columns, 1 to 12 pairs, were measured with both: the estimates
+// are off by 7% and 9%.  The shifts by themselves are more than 3% slower than the tiles at 271 shapes, by
+// up to 1.9 times; the choice at 28, by up to 1.15 times, and it is 1.29 times as fast on average.  us,
+// shifts / tiles: 129x37 28.3 / 20.0, 26x335 72 / 53, 65x124 45 / 34, 64x128 30.1 / 25.5, 128^2 45.4 /
+// 44.1, 54x61 16.6 / 27.9, 130^2 79 / 121, 256x64 45 / 55.  Up to 5 rows (7 to 18 us; the tiles up to a
+// fifth less) the shifts stay.
 bool register_tiles_faster(const family_args& a) {
     if (rights_per_left(a) > 1 || (a.family == XC_N_TO_M && a.n > 1) || a.rows <= 5) return false;
+    const direct_plan d = plan_direct<float>(a, xc_options{});
+    const double waves = (double)d.tiles_x * d.tiles_y * d.chunks * d.groups_r * d.groups_l * d.nwx * d.nwy;
+    if (waves > 4096) return false;
     const double W = a.cols, tx = (2 * a.cols - 1 + 15) / 16, ty = (2 * a.rows - 1 + 15) / 16;
     const int nw = direct_shifts_waves((uint64_t)a.pairs * (uint64_t)(tx * ty), a.rows);
     const uint32_t share = (a.rows + 4 * nw - 1) / (4 * nw), rest = share % 8;
-    const double panel = 5.04 * (share / 8 + (rest > 4)) + (rest > 0 && rest <= 4 ? 3.09 : 0.0);
+    const double panel = 5.07 * (share / 8 + (rest > 4)) + (rest > 0 && rest <= 4 ? 3.18 : 0.0);
     const double chain = 3.4 + std::ceil(W / 16) * panel;
-    const double issue = a.pairs * tx * ty * 256 * (a.rows / 2.0 + 8) * (W / 2 + 8) / 20.7e6;
-    const double shifts = std::pow(std::pow(chain, 1.6) + std::pow(issue, 1.6), 1 / 1.6);
-    const direct_plan d = plan_direct<float>(a, xc_options{});
+    const double issue = a.pairs * tx * ty * 256 * (a.rows / 2.0 + 8) * (W / 2 + 8) / 19.8e6;
+    const double shifts = std::pow(std::pow(chain, 1.84) + std::pow(issue, 1.84), 1 / 1.84);
     const uint32_t rows = d.rows_per_chunk ? d.rows_per_chunk : a.rows, steps = (rows + d.t.jb - 1) / d.t.jb;
-    const double waves = (double)d.tiles_x * d.tiles_y * d.chunks * d.groups_r * d.groups_l * d.nwx * d.nwy;
-    const double tiles = 3.9 + (d.chunks > 1 ? 1.95 : 0.0) + steps * (W + 23) * (0.056 + 2.05e-5 * waves);
-    return tiles < shifts;
+    const double tiles = 3.6 + (d.chunks > 1 ? 2.0 : 0.0) +
+                         steps * (W + 24) * (0.0575 + 0.0775 * std::pow(waves / 4096, 1.13));
+    return tiles < 1.02 * shifts;
 }
 
 // False (nothing launched) where the grid does not fit one launch.

@@ -15,8 +15,10 @@ TILES, SHIFTS = "direct_kernel<f32> ty", "direct_kernel<f32> 16x16 shifts"
 
 @pytest.mark.parametrize("family,rows,cols,n,m,kernel", [
     ("one_to_one", 129, 37, 1, 1, TILES), ("one_to_one", 26, 335, 1, 1, TILES), ("one_to_one", 65, 124, 1, 1, TILES),
+    ("one_to_one", 64, 128, 1, 1, TILES),
     ("n_to_mn", 13, 146, 3, 3, TILES), ("one_to_many", 8, 76, 1, 1, TILES), ("one_to_one", 54, 61, 1, 1, SHIFTS),
-    ("one_to_one", 130, 130, 1, 1, SHIFTS), ("one_to_one", 17, 17, 1, 1, SHIFTS), ("n_to_mn", 34, 72, 2, 2, SHIFTS),
+    ("one_to_one", 130, 130, 1, 1, SHIFTS), ("one_to_one", 256, 64, 1, 1, SHIFTS),
+    ("one_to_one", 17, 17, 1, 1, SHIFTS), ("n_to_mn", 34, 72, 2, 2, SHIFTS),
     ("one_to_many", 129, 37, 1, 2, SHIFTS)])
 def test_kernel_and_parity(family, rows, cols, n, m, kernel):
     x = xcorr()
