@@ -210,7 +210,7 @@ __global__ __launch_bounds__(NT) void rows_fwd_regs_kernel(const Tin* __restrict
     extern __shared__ double2 buf[];
     const regs_pos<LOGPC> ps((int)threadIdx.x);
     const int t0 = ps.t0, t = ps.t, i = ps.i;
-    const regs_roots<LOGPC> rr = load_roots<LOGPC>(i, tw);
+    const auto rr = load_roots<LOGPC, exact_roots<Tin>>(i, tw);
     // this block's items: x * per + k + j * bpx, j = 0, 1, ... below min((x + 1) * per, items)
     const uint32_t nx = gridDim.x >= 8 ? 8 : 1;
     const uint32_t x = blockIdx.x % nx, kb = blockIdx.x / nx, bpx = gridDim.x / nx;
@@ -418,7 +418,8 @@ constexpr int cols_threads(int logP) { return logP <= 9 ? 64 : kFT; }
 // 128^2 15.9 -> 13.6 us, of 512^2 32.2 -> 28.6, 1 x 16 of 256^2 40.0 -> 37.4; 1 x 24 46.6 -> 46.0, 1 x
 // 32 55.2 -> 56.1).  G = 2 above 4608 waves (the batch 772 -> 740 in one run), G = 1 below (1 x 4 of
 // 256^2 20.7 against 22.1, 64 x 64 of 128^2 37.7 against 39.7).
-template <int LOGPR>
+// X: regs_roots (the batch's data are double).
+template <int LOGPR, bool X>
 __global__ __launch_bounds__(cols_threads(LOGPR)) void cols_group_kernel(
     const double2* __restrict__ SL, const double2* __restrict__ SR, double2* __restrict__ Z,
     const uint2* __restrict__ ptab, const uint2* __restrict__ mdims, uint32_t nl, int family, uint32_t n, uint32_t m,
@@ -433,7 +434,7 @@ __global__ __launch_bounds__(cols_threads(LOGPR)) void cols_group_kernel(
     const uint32_t k = cg * C + ps.t;
     const bool ok = k < Kc;
     double2* wb = buf + at<LOGPR>(ps.t0, 0);
-    const regs_roots<LOGPR> rr = load_roots<LOGPR>(ps.i, tw);
+    const auto rr = load_roots<LOGPR, X>(ps.i, tw);
     auto column = [&](const double2* S, uint32_t mat, uint32_t rows, int i, double2 (&u)[8]) {
         const __amdgpu_buffer_rsrc_t rs = buf_of(S + (size_t)mat * Kc * Hs, Kc * Hs * 16u);
         const uint32_t so = (k * Hs + (uint32_t)i) * 16u;
@@ -484,7 +485,7 @@ __global__ __launch_bounds__(cols_threads(LOGPR)) void cols_group_kernel(
     }
 }
 
-template <int LOGPR, int MODE>
+template <int LOGPR, int MODE, bool X>
 __global__ __launch_bounds__(cols_threads(LOGPR)) void cols_kernel(const double2* __restrict__ S, double2* __restrict__ Lhat,
                                                    double2* __restrict__ Z, const uint2* __restrict__ ptab,
                                                    const uint2* __restrict__ mdims, uint32_t nl, int family,
@@ -518,7 +519,7 @@ __global__ __launch_bounds__(cols_threads(LOGPR)) void cols_kernel(const double2
         const uint32_t k = k0 + ps.t;
         const bool ok = k < Kc;
         double2* wb = buf + at<LOGPR>(t0, 0);
-        const regs_roots<LOGPR> rr = load_roots<LOGPR>(i, tw);
+        const auto rr = load_roots<LOGPR, X>(i, tw);
         const __amdgpu_buffer_rsrc_t rs = buf_of(Sm, Kc * Hs * 16u), rl = buf_of(Ll, Kc * (uint32_t)P * 16u);
         const uint32_t so = (k * Hs + (uint32_t)i) * 16u, lo = ok ? (k * (uint32_t)P + (uint32_t)i) * 16u : kOut;
         const uint32_t rows = ok ? Hq : 0;
@@ -719,7 +720,7 @@ __global__ __launch_bounds__(NT) void rows_inv_regs_kernel(const double2* __rest
     const uint32_t z0 = g << (LOGT + 1);
     if (z_gap(z0, 2 * T, H, Ys)) return;  // between the two halves of the result
     const regs_pos<LOGPC> ps((int)threadIdx.x);
-    const regs_roots<LOGPC> rr = load_roots<LOGPC>(ps.i, tw);
+    const auto rr = load_roots<LOGPC, exact_roots<Tout>>(ps.i, tw);
     // Columns kk0 + Q q of row pair tq: A, B (conjugated) -> slots kk and Pc - kk of conj(Y), Y[k] =
     // A[k] + i B[k] extended by A[Pc-k] = conj(A[k]), B[Pc-k] = conj(B[k]).
     {
@@ -841,13 +842,16 @@ __global__ __launch_bounds__(rows3<LOGN>::NT) void rows_fwd3_kernel(
     extern __shared__ double2 buf[];
     const regs_pos<LOGN> ps((int)threadIdx.x);
     const int sub = ps.t, tt = sub / 3, m = sub - 3 * tt, i = ps.i;
-    const regs_roots<LOGN> rr = load_roots<LOGN>(i, tw);
+    const auto rr = load_roots<LOGN, exact_roots<Tin>>(i, tw);
     // the split: row rw of the group (an A or a B of row pair tq) at k = k0 + FS q
     const int rw = (int)threadIdx.x & (2 * T - 1), tq = rw >> 1, odd = rw & 1;
     const int k0 = (int)threadIdx.x >> (G::LOGT + 1);
-    double2 w1[G::FQ];
+    double2 w1[G::FQ], w2[G::FQ];
 #pragma unroll
-    for (int q = 0; q < G::FQ; ++q) w1[q] = tw3[(k0 + FS * q) * (kTw3 / P)];
+    for (int q = 0; q < G::FQ; ++q) {
+        w1[q] = tw3[(k0 + FS * q) * (kTw3 / P)];
+        if constexpr (exact_roots<Tin>) w2[q] = tw3[2 * (k0 + FS * q) * (kTw3 / P)];
+    }
     const uint32_t nx = gridDim.x >= 8 ? 8 : 1;
     const uint32_t x = blockIdx.x % nx, kb = blockIdx.x / nx, bpx = gridDim.x / nx;
     const uint32_t per = (items + nx - 1) / nx;
@@ -924,7 +928,7 @@ __global__ __launch_bounds__(rows3<LOGN>::NT) void rows_fwd3_kernel(
                     f[mm] = make_double2(0.5 * (zs[2 * a] + zs[2 * b]), hs * (zd[2 * a] - zd[2 * b]));
                 }
                 double2 x0, x1, x2;
-                dft3(f[0], cmul(w1[q], f[1]), cmul(csqr(w1[q]), f[2]), x0, x1, x2);
+                dft3(f[0], cmul(w1[q], f[1]), cmul(exact_roots<Tin> ? w2[q] : csqr(w1[q]), f[2]), x0, x1, x2);
                 const uint32_t off = row < cur.Hm ? ((uint32_t)k * Hs + row) * 16u : kOut;
                 buf_store(x0, rs, off, 0);
                 buf_store(x1, rs, off, N * Hs * 16u);
@@ -962,7 +966,7 @@ __global__ __launch_bounds__(rows3<LOGN>::NT) void rows_inv3_kernel(
     if (z_gap(z0, 2 * T, H, Ys)) return;
     const regs_pos<LOGN> ps((int)threadIdx.x);
     const int sub = ps.t, tt = sub / 3, m = sub - 3 * tt, i = ps.i;
-    const regs_roots<LOGN> rr = load_roots<LOGN>(i, tw);
+    const auto rr = load_roots<LOGN, exact_roots<Tout>>(i, tw);
     // The extension: row pair tq at k = k0 + IS q, the bins k, N + k and N - k of both rows (Z holds
     // them conjugated).
     {
@@ -970,13 +974,14 @@ __global__ __launch_bounds__(rows3<LOGN>::NT) void rows_inv3_kernel(
         const uint32_t za = z0 + 2 * tq;
         const bool oka = out_row_of_z(za, H, Ys) >= 0, okb = out_row_of_z(za + 1, H, Ys) >= 0;
         const __amdgpu_buffer_rsrc_t rz = buf_of(Z + (size_t)item * Kc * Ys, Kc * Ys * 16u);
-        double2 A[G::IQ][3], B[G::IQ][3], w1[G::IQ];
+        double2 A[G::IQ][3], B[G::IQ][3], w1[G::IQ], wx[G::IQ];
 #pragma unroll
         for (int q = 0; q < G::IQ; ++q) {
             const int k = k0 + IS * q;
             const uint32_t lo = ((uint32_t)k * Ys + za) * 16u, hi = ((uint32_t)(N - k) * Ys + za) * 16u;
             const bool ka = oka && k <= N / 2, kb = okb && k <= N / 2;
             w1[q] = tw3[(k <= N / 2 ? k : 0) * (kTw3 / P)];
+            if constexpr (exact_roots<Tout>) wx[q] = tw3[2 * (k <= N / 2 ? k : 0) * (kTw3 / P)];
             A[q][0] = buf_load(rz, ka ? lo : kOut, 0);
             B[q][0] = buf_load(rz, kb ? lo + 16u : kOut, 0);
             A[q][1] = buf_load(rz, ka ? lo : kOut, N * Ys * 16u);
@@ -988,7 +993,7 @@ __global__ __launch_bounds__(rows3<LOGN>::NT) void rows_inv3_kernel(
         for (int q = 0; q < G::IQ; ++q) {
             const int k = k0 + IS * q;
             if (k > N / 2) continue;
-            const double2 w2 = csqr(w1[q]);
+            const double2 w2 = exact_roots<Tout> ? wx[q] : csqr(w1[q]);
             double2 a[3], b[3];
             dft3(A[q][0], A[q][1], cconj(A[q][2]), a[0], a[1], a[2]);
             dft3(B[q][0], B[q][1], cconj(B[q][2]), b[0], b[1], b[2]);
@@ -1302,7 +1307,7 @@ void launch_job(const fftk_job& j, const Tio* L, const Tio* R, Tio* O, const fft
     auto cols = [&](const char* name, const double2* S, double2* Zout, auto MODE, uint32_t items,
                     uint32_t q0) {
         with_logp(g.logPr, [&](auto LP) {
-            auto k = cols_kernel<decltype(LP)::value, decltype(MODE)::value>;
+            auto k = cols_kernel<decltype(LP)::value, decltype(MODE)::value, exact_roots<Tio>>;
             allow_lds(k, g.vc.lds);
             launch_timed(name, timing, k, dim3(items * g.cg), dim3(cols_threads(g.logPr)), g.vc.lds, s, S, LH, Zout,
                          ptab, mdims, j.nl, j.family, j.n, j.m, q0, items, H, g.Hs, g.Kc, g.Ys, g.vc.logT, tw);
@@ -1316,7 +1321,7 @@ void launch_job(const fftk_job& j, const Tio* L, const Tio* R, Tio* O, const fft
         with_logp(g.logPr, [&](auto LP) {
             constexpr int LOGPR = decltype(LP)::value;
             if constexpr (regs_of<LOGPR>::ON) {
-                auto k = cols_group_kernel<LOGPR>;
+                auto k = cols_group_kernel<LOGPR, exact_roots<Tio>>;
                 allow_lds(k, g.vc.lds);
                 const uint32_t items = (nq + G - 1) / G;
                 launch_timed("fftk_cols", timing, k, dim3(items * g.cg), dim3(cols_threads(g.logPr)), g.vc.lds, s,

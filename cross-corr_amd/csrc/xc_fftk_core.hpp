@@ -98,9 +98,16 @@ __device__ __forceinline__ void dft8_last(double2 t0, double2 t1, double2 t2, do
     u[3] = make_double2(fma(c, p3, e3.x), fma(-c, q3, e3.y));
     u[7] = make_double2(fma(-c, p3, e3.x), fma(c, q3, e3.y));
 }
-// s = a + w b, d = a - w b = 2 a - s: 6 FMAs where product, sum and difference took 8
-// instructions.
+// s = a + w b, d = a - w b = 2 a - s: 6 FMAs where product, sum and difference (X) take 8
+// instructions; d has the rounding of s too.
+template <bool X>
 __device__ __forceinline__ void bfly(double2 a, double2 w, double2 b, double2& s, double2& d) {
+    if constexpr (X) {
+        const double2 p = cmul(w, b);
+        d = csub(a, p);
+        s = cadd(a, p);
+        return;
+    }
     s.x = fma(w.x, b.x, fma(-w.y, b.y, a.x));
     s.y = fma(w.x, b.y, fma(w.y, b.x, a.y));
     d.x = fma(2.0, a.x, -s.x);
@@ -149,27 +156,61 @@ __device__ __forceinline__ void regs_sync() {
 // a twiddled radix-2 or 4 pass multiplies 4 or 6 of a thread's 8 values where a radix-8 pass
 // multiplies 7 and forms 6 powers: per 8 points 92 FP64 instructions against 124 at 16 points,
 // 196 against 232 at 128, 312 against 340 at 1024 (234 against 248 at 256).
-template <int LOGP>
+//
+// X (double data): more roots of a pass are the table's own.  Powers and rotations of a single root
+// carry its rounding and their own: results of unsigned values of 64^2 were 4.0e-16 off in the 2-norm
+// with one root per pass and are 2.1e-16 off with these (2.3e-16 with a short radix first and powers one
+// by one); n_to_m 16 x 64 of 64^2 50 -> 59 us.  Float results round at 6e-8, where neither shows.
+template <int LOGP, bool X = false>
 struct regs_roots {
     static constexpr int REM = LOGP % 3;
     static constexpr int N8 = LOGP / 3 - 1;  // twiddled radix-8 passes
     static constexpr int N = N8 + (REM ? 1 : 0);
     double2 w[N];
+    const double2* tw;  // X: the table
 };
+// A pass's further roots with X.  Radix 8: powers 2 to 4 of the root w; radix 2: the root at i + P/8 (w2);
+// radix 4: that and w^2 (w3).  Read where the pass before ends, so that they are in flight during the
+// exchange, whose registers are free: kept from the start of the kernel they spill, and w read here too
+// is waited for (16 x 64 of 64^2 60 us, 64 of 128^2 36.5 -> 39.7).
+struct pass_roots {
+    double2 w2, w3, w4;
+};
+template <int LOGP, int LOGPP>
+__device__ __forceinline__ pass_roots load_pass_roots(int i, const double2* __restrict__ tw) {
+    asm volatile("" : "+v"(i));  // here, not hoisted
+    pass_roots x;
+    if constexpr (LOGP - LOGPP >= 3) {
+        const int e = (i & ((1 << LOGPP) - 1)) << (kLogMaxP - LOGPP - 3);
+        x.w2 = tw[2 * e];
+        x.w4 = tw[4 * e];
+        x.w3 = tw[3 * e];
+    } else {
+        const int e = i << (kLogMaxP - LOGP);
+        x.w2 = tw[e + kSlab / 8];
+        if constexpr (LOGP - LOGPP == 2) x.w3 = tw[2 * e];
+    }
+    return x;
+}
+// Whether kernels on data of type T take the roots X.
+template <typename T>
+constexpr bool exact_roots = sizeof(T) == 8;
+
 // Pass roots at lane position i: w[j] = exp(-2 pi i k / (8p)), k = i mod p, p = 8^(j+1) for the
 // twiddled radix-8 passes, exp(-2 pi i i / P) for a last radix-2 or 4 pass.  Kernels load them
 // once, before their first transform: a table read inside a pass would wait on memory after
 // every LDS exchange.
-template <int LOGP>
-__device__ __forceinline__ regs_roots<LOGP> load_roots(int i, const double2* __restrict__ tw) {
-    using RR = regs_roots<LOGP>;
-    regs_roots<LOGP> rr;
+template <int LOGP, bool X = false>
+__device__ __forceinline__ regs_roots<LOGP, X> load_roots(int i, const double2* __restrict__ tw) {
+    using RR = regs_roots<LOGP, X>;
+    RR rr;
 #pragma unroll
     for (int j = 0; j < RR::N8; ++j) {
         const int logpp = 3 + 3 * j;
         rr.w[j] = tw[(i & ((1 << logpp) - 1)) << (kLogMaxP - logpp - 3)];
     }
     if constexpr (RR::REM != 0) rr.w[RR::N8] = tw[i << (kLogMaxP - LOGP)];
+    if constexpr (X) rr.tw = tw;
     return rr;
 }
 
@@ -250,33 +291,34 @@ __device__ __forceinline__ void lane_exchange(double2 (&u)[8]) {
     for (int r = 0; r < 8; ++r) u[r] = v[r];
 }
 
-template <int LOGP, int LOGPP>
+template <int LOGP, int LOGPP, bool X>
 __device__ __forceinline__ void fft_regs_next(double2 (&u)[8], double2* wb, int tl, int i,
-                                              const regs_roots<LOGP>& rr);
+                                              const regs_roots<LOGP, X>& rr);
 
 // Twiddled passes of fft_regs from p = 2^LOGPP on (u[r] = element i + Q r); the last one leaves
 // its outputs i + (P/8) r in registers.
-template <int LOGP, int LOGPP>
+template <int LOGP, int LOGPP, bool X>
 __device__ __forceinline__ void fft_regs_passes(double2 (&u)[8], double2* wb, int tl, int i,
-                                                const regs_roots<LOGP>& rr) {
+                                                const regs_roots<LOGP, X>& rr, const pass_roots& x) {
     // The root passes through an empty asm so that its powers are formed here, in this pass:
     // otherwise the compiler hoists the power chains of every pass (and keeps them for a second
     // transform with the same roots), which costs tens of VGPRs.
     double2 w1 = rr.w[LOGPP / 3 - 1];
     asm volatile("" : "+v"(w1.x), "+v"(w1.y));
     if constexpr (LOGP - LOGPP == 1) {  // radix 2: butterfly i + Q m takes u[m], u[m + 4]
-        bfly(u[0], w1, u[4], u[0], u[4]);
-        bfly(u[1], rot8<1>(w1), u[5], u[1], u[5]);
-        bfly(u[2], mul_mi(w1), u[6], u[2], u[6]);
-        bfly(u[3], rot8<3>(w1), u[7], u[3], u[7]);
+        const double2 wr = X ? x.w2 : rot8<1>(w1);
+        bfly<X>(u[0], w1, u[4], u[0], u[4]);
+        bfly<X>(u[1], wr, u[5], u[1], u[5]);
+        bfly<X>(u[2], mul_mi(w1), u[6], u[2], u[6]);
+        bfly<X>(u[3], X ? mul_mi(x.w2) : rot8<3>(w1), u[7], u[3], u[7]);
     } else if constexpr (LOGP - LOGPP == 2) {  // radix 4: butterfly i + Q m takes u[m + 2 r]
 #pragma unroll
         for (int m = 0; m < 2; ++m) {
-            const double2 wm = m ? rot8<1>(w1) : w1;
-            const double2 w2 = csqr(wm);
+            const double2 wm = m ? (X ? x.w2 : rot8<1>(w1)) : w1;
+            const double2 w2 = X ? (m ? mul_mi(x.w3) : x.w3) : csqr(wm);
             double2 t0, t1, t2, t3;
-            bfly(u[m], w2, u[m + 4], t0, t1);
-            bfly(cmul(u[m + 2], wm), cmul(w2, wm), u[m + 6], t2, t3);
+            bfly<X>(u[m], w2, u[m + 4], t0, t1);
+            bfly<X>(cmul(u[m + 2], wm), cmul(w2, wm), u[m + 6], t2, t3);
             u[m] = cadd(t0, t2);
             u[m + 4] = csub(t0, t2);
             u[m + 2] = make_double2(t1.x + t3.y, t1.y - t3.x);
@@ -286,12 +328,12 @@ __device__ __forceinline__ void fft_regs_passes(double2 (&u)[8], double2* wb, in
         // The powers as a tree (squares take 3 instructions and the chain is 3 long, not 6); the
         // products of the upper four inputs go into the first level's sums (bfly): 93 FP64
         // instructions against 105.
-        const double2 w2 = csqr(w1), w3 = cmul(w2, w1), w4 = csqr(w2);
+        const double2 w2 = X ? x.w2 : csqr(w1), w3 = X ? x.w3 : cmul(w2, w1), w4 = X ? x.w4 : csqr(w2);
         double2 t0, t1, t2, t3, s0, s1, s2, s3;
-        bfly(u[0], w4, u[4], t0, t1);
-        bfly(cmul(u[1], w1), cmul(w4, w1), u[5], s0, s1);
-        bfly(cmul(u[2], w2), csqr(w3), u[6], t2, t3);
-        bfly(cmul(u[3], w3), cmul(w4, w3), u[7], s2, s3);
+        bfly<X>(u[0], w4, u[4], t0, t1);
+        bfly<X>(cmul(u[1], w1), cmul(w4, w1), u[5], s0, s1);
+        bfly<X>(cmul(u[2], w2), X ? cmul(w4, w2) : csqr(w3), u[6], t2, t3);
+        bfly<X>(cmul(u[3], w3), cmul(w4, w3), u[7], s2, s3);
         dft8_last(t0, t1, t2, t3, s0, s1, s2, s3, u);
         regs_sync<regs_of<LOGP>::BLOCK>();
         if constexpr (LOGPP + 3 < LOGP) fft_regs_next<LOGP, LOGPP + 3>(u, wb, tl, i, rr);
@@ -301,10 +343,12 @@ __device__ __forceinline__ void fft_regs_passes(double2 (&u)[8], double2* wb, in
 // From the outputs of the radix-8 pass before p = 2^LOGPP (element ((i - k) << 3) + k + r p/8 in
 // u[r], k = i mod p/8) to the pass at p: a short last pass takes them by lane swaps, a radix-8
 // one through LDS.
-template <int LOGP, int LOGPP>
+template <int LOGP, int LOGPP, bool X>
 __device__ __forceinline__ void fft_regs_next(double2 (&u)[8], double2* wb, int tl, int i,
-                                              const regs_roots<LOGP>& rr) {
+                                              const regs_roots<LOGP, X>& rr) {
     constexpr int Q = 1 << (LOGP - 3);
+    pass_roots x;
+    if constexpr (X) x = load_pass_roots<LOGP, LOGPP>(i, rr.tw);
     if constexpr (LOGP - LOGPP < 3) {
         lane_exchange<LOGP - LOGPP>(u);
     } else {
@@ -325,7 +369,7 @@ __device__ __forceinline__ void fft_regs_next(double2 (&u)[8], double2* wb, int 
             for (int r = 0; r < 8; ++r) u[r] = wb[at<LOGP>(tl, i + Q * r)];
         }
     }
-    fft_regs_passes<LOGP, LOGPP>(u, wb, tl, i, rr);
+    fft_regs_passes<LOGP, LOGPP>(u, wb, tl, i, rr, x);
 }
 
 // FFTs entered and left in registers, for P = 2^LOGP of 16..2048 points (regs_of).  Thread
@@ -341,8 +385,8 @@ __device__ __forceinline__ void fft_regs_next(double2 (&u)[8], double2* wb, int 
 // block: every thread of it must call.  (tl, i) are passed in (regs_pos) so that a kernel
 // calling twice can keep the compiler from holding the first call's LDS addresses in registers
 // for the second.
-template <int LOGP, bool HALF = false>
-__device__ __forceinline__ void fft_regs(double2 (&u)[8], double2* wb, const regs_roots<LOGP>& rr, int tl,
+template <int LOGP, bool HALF = false, bool X>
+__device__ __forceinline__ void fft_regs(double2 (&u)[8], double2* wb, const regs_roots<LOGP, X>& rr, int tl,
                                          int i) {
     static_assert(LOGP >= 4 && regs_of<LOGP>::ON, "register FFTs take 16..2048 points");
     if constexpr (HALF)

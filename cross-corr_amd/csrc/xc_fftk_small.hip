@@ -81,11 +81,11 @@ __global__ __launch_bounds__((small_geom<LR, LC>::NT)) void small_spec_kernel(
         W = d.y;
     }
     const regs_pos<LR> pc(tp);
-    const regs_roots<LR> rrc = load_roots<LR>(pc.i, tw);
+    const auto rrc = load_roots<LR, exact_roots<Tin>>(pc.i, tw);
     // Rows rho and rho + Pr/4 in one transform (H <= Pr/2): Pr/4 of them, on half the threads.
     if (G::NT < 128 || tp < G::NT / 2) {
         const regs_pos<LC> pr(tp);
-        const regs_roots<LC> rr = load_roots<LC>(pr.i, tw);
+        const auto rr = load_roots<LC, exact_roots<Tin>>(pr.i, tw);
         const uint32_t a = pr.t, b = a + G::Pr / 4;
         const bool oka = a < H && pr.t < G::Pr / 4, okb = b < H && pr.t < G::Pr / 4;
         const Tin* xa = X + (oka ? (size_t)a * W : 0);
@@ -170,7 +170,7 @@ __global__ __launch_bounds__((pairs_geom<LR, LC, PS>::NT), 4) void small_pairs_k
     const bool wave0 = tp < 64;  // holds column 0 (selects in every wave cost 60 instructions)
     double2 u[PS][8];
     {
-        const regs_roots<LR> rr = load_roots<LR>(i, tw);
+        const auto rr = load_roots<LR, exact_roots<Tout>>(i, tw);
         const size_t nyq = (size_t)G::NC * G::Pr;
 #pragma unroll
         for (int h = 0; h < PS; ++h) {
@@ -215,7 +215,7 @@ __global__ __launch_bounds__((pairs_geom<LR, LC, PS>::NT), 4) void small_pairs_k
         }
     }
     const regs_pos<LC> pr(tp);
-    const regs_roots<LC> rr = load_roots<LC>(pr.i, tw);
+    const auto rr = load_roots<LC, exact_roots<Tout>>(pr.i, tw);
     const int SX = 2 * (int)W - 1;
     Tout* Oq = O + (ooff ? ooff[q] : (size_t)q * (2 * H - 1) * SX);
     const int wlo = (int)W - 1, whi = -(G::Pc - (int)W + 1);
