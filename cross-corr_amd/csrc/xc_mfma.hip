@@ -487,14 +487,16 @@ __device__ __forceinline__ void mfma_tile(const float* __restrict__ Lp, const fl
     }
 }
 
-template <int KIND, int WX, int WY, int KC, int FLUSH, bool KAHAN, int OCC, int JR>
+// BEHIND: for the batches that mfma_rights_kernel leaves (*only_if != 0).  A template flag: the test at
+// the start of every launch costs fp16x3 1..4 % (one pair of 32^2 51.4 -> 53.7 us, of 256^2 351 -> 357).
+template <int KIND, int WX, int WY, int KC, int FLUSH, bool KAHAN, int OCC, int JR, bool BEHIND>
 __global__ __launch_bounds__(256, OCC) void mfma_kernel(const float* __restrict__ L, const float* __restrict__ R,
                                                       float* __restrict__ O, int family, uint32_t rows,
                                                       uint32_t cols, uint32_t n, uint32_t m, uint32_t tiles_x,
                                                       uint32_t tiles_y, uint32_t skip_area,
                                                       const uint32_t* __restrict__ only_if) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
-    if (only_if && *only_if == 0) return;  // mfma_rights_kernel has done the batch
+    if (BEHIND && *only_if == 0) return;
     const int H = (int)rows, W = (int)cols;
     uint32_t bid = xcd_remap(blockIdx.x, gridDim.x);
     const uint32_t tx = bid % tiles_x;
@@ -810,14 +812,14 @@ __device__ __forceinline__ void mfma_rows_tile(const float* __restrict__ Lp, con
     }
 }
 
-template <int KIND, int NS, int KC, int FLUSH, int OCC, bool PIPE_ROWS>
+template <int KIND, int NS, int KC, int FLUSH, int OCC, bool PIPE_ROWS, bool BEHIND>
 __global__ __launch_bounds__(256, OCC) void mfma_rows_kernel(const float* __restrict__ L, const float* __restrict__ R,
                                                            float* __restrict__ O, int family, uint32_t rows,
                                                            uint32_t cols, uint32_t n, uint32_t m, uint32_t tiles_x,
                                                            uint32_t tiles_y, uint32_t skip_area,
                                                            const uint32_t* __restrict__ only_if) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
-    if (only_if && *only_if == 0) return;  // mfma_rights_kernel has done the batch
+    if (BEHIND && *only_if == 0) return;
     const int H = (int)rows, W = (int)cols;
     uint32_t bid = xcd_remap(blockIdx.x, gridDim.x);
     const uint32_t tx = bid % tiles_x;
@@ -1089,48 +1091,48 @@ __global__ __launch_bounds__(256) void frame_kernel(const float* __restrict__ Ln
     }
 }
 
-template <int KIND, int WX, int WY, int KC, int FLUSH, bool KAHAN, int OCC, int JR = 1>
+template <int KIND, int WX, int WY, int KC, int FLUSH, bool KAHAN, int OCC, int JR = 1, bool BEHIND = false>
 void launch(const family_args& a, const float* L, const float* R, float* O, uint32_t skip_area, hipStream_t s,
-            const uint32_t* only_if) {
+            const uint32_t* only_if = nullptr) {
     using G = geom<WX, WY, split_traits<KIND>::planes, KC, JR>;
     const uint32_t SX = 2 * a.cols - 1, SY = 2 * a.rows - 1;
     const uint32_t tiles_x = (SX + G::BX - 1) / G::BX;
     const uint32_t tiles_y = (SY + G::BY - 1) / G::BY;
     const uint64_t nblocks = (uint64_t)tiles_x * tiles_y * a.pairs;
     if (nblocks > 0x7fffffffULL) fail(XC_ERR_INVALID_ARGUMENT, "problem too large for one launch");
-    allow_dynamic_lds(reinterpret_cast<const void*>(&mfma_kernel<KIND, WX, WY, KC, FLUSH, KAHAN, OCC, JR>), G::BYTES);
+    allow_dynamic_lds(reinterpret_cast<const void*>(&mfma_kernel<KIND, WX, WY, KC, FLUSH, KAHAN, OCC, JR, BEHIND>), G::BYTES);
     dim3 grid((uint32_t)nblocks), block(256);
-    if (!only_if)
+    if (!BEHIND)
         record_launch(KIND == XC_PREC_BF16X3   ? "mfma_kernel<bf16x3>"
                   : KIND == XC_PREC_FP16X3 ? "mfma_kernel<fp16x3>"
                   : KIND == XC_PREC_BF16   ? "mfma_kernel<bf16>"
                                            : "mfma_kernel<fp16>",
                   grid, block, G::BYTES, a.rows, a.cols, a.pairs, 1);
-    timed tm("mfma_kernel", s, !only_if);
-    hipLaunchKernelGGL((mfma_kernel<KIND, WX, WY, KC, FLUSH, KAHAN, OCC, JR>), grid, block, G::BYTES, s, L, R, O, a.family, a.rows, a.cols, a.n,
+    timed tm("mfma_kernel", s, !BEHIND);
+    hipLaunchKernelGGL((mfma_kernel<KIND, WX, WY, KC, FLUSH, KAHAN, OCC, JR, BEHIND>), grid, block, G::BYTES, s, L, R, O, a.family, a.rows, a.cols, a.n,
                        a.m, tiles_x, tiles_y, skip_area, only_if);
     XC_HIP(hipGetLastError());
 }
 
-template <int KIND, int NS, int KC, int FLUSH, int OCC, bool PIPE_ROWS = (OCC == 1)>
+template <int KIND, int NS, int KC, int FLUSH, int OCC, bool PIPE_ROWS = (OCC == 1), bool BEHIND = false>
 void launch_rows(const family_args& a, const float* L, const float* R, float* O, uint32_t skip_area, hipStream_t s,
-            const uint32_t* only_if) {
+            const uint32_t* only_if = nullptr) {
     using G = rgeom<NS, split_traits<KIND>::planes, KC>;
     const uint32_t SX = 2 * a.cols - 1, SY = 2 * a.rows - 1;
     const uint32_t tiles_x = (SX + G::BX - 1) / G::BX;
     const uint32_t tiles_y = (SY + G::BY - 1) / G::BY;
     const uint64_t nblocks = (uint64_t)tiles_x * tiles_y * a.pairs;
     if (nblocks > 0x7fffffffULL) fail(XC_ERR_INVALID_ARGUMENT, "problem too large for one launch");
-    allow_dynamic_lds(reinterpret_cast<const void*>(&mfma_rows_kernel<KIND, NS, KC, FLUSH, OCC, PIPE_ROWS>), G::BYTES);
+    allow_dynamic_lds(reinterpret_cast<const void*>(&mfma_rows_kernel<KIND, NS, KC, FLUSH, OCC, PIPE_ROWS, BEHIND>), G::BYTES);
     dim3 grid((uint32_t)nblocks), block(256);
-    if (!only_if)
+    if (!BEHIND)
         record_launch(KIND == XC_PREC_BF16X3   ? "mfma_rows_kernel<bf16x3>"
                   : KIND == XC_PREC_FP16X3 ? "mfma_rows_kernel<fp16x3>"
                   : KIND == XC_PREC_BF16   ? "mfma_rows_kernel<bf16>"
                                            : "mfma_rows_kernel<fp16>",
                   grid, block, G::BYTES, a.rows, a.cols, a.pairs, 1);
-    timed tm("mfma_kernel", s, !only_if);
-    hipLaunchKernelGGL((mfma_rows_kernel<KIND, NS, KC, FLUSH, OCC, PIPE_ROWS>), grid, block, G::BYTES, s, L, R, O, a.family, a.rows,
+    timed tm("mfma_kernel", s, !BEHIND);
+    hipLaunchKernelGGL((mfma_rows_kernel<KIND, NS, KC, FLUSH, OCC, PIPE_ROWS, BEHIND>), grid, block, G::BYTES, s, L, R, O, a.family, a.rows,
                        a.cols, a.n, a.m, tiles_x, tiles_y, skip_area, only_if);
     XC_HIP(hipGetLastError());
 }
@@ -1360,7 +1362,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
 
 template <int KIND>
 void launch_tile(const family_args& a, const float* L, const float* R, float* O, uint32_t tile, uint32_t skip_area,
-                 hipStream_t s, const uint32_t* only_if = nullptr);
+                 hipStream_t s);
+template <int KIND>
+void launch_tile_behind(const family_args& a, const float* L, const float* R, float* O, uint32_t skip_area,
+                        const uint32_t* only_if, hipStream_t s);
 
 // Whether mfma_rights_kernel serves this batch by default.  Its time does not shrink with a group's
 // missing rights: 3/4 of the slots busy, or 17/20 up to 64 columns (48 of 256^2 1341 us against
@@ -1431,7 +1436,7 @@ bool launch_rights(const family_args& a, const float* L, const float* R, float* 
         hipLaunchKernelGGL(mfma_rights_kernel<KIND>, grid, block, 0, s, Lc, Rq, O, k, flag);
         XC_HIP(hipGetLastError());
     }
-    launch_tile<KIND>(a, L, R, O, 0, skip_area, s, flag);
+    launch_tile_behind<KIND>(a, L, R, O, skip_area, flag, s);
     return true;
 }
 
@@ -1632,25 +1637,37 @@ uint32_t mfma_candidate_tile(int i) { return kMfmaCandidates[i]; }
 
 namespace {
 
+uint32_t default_tile(const family_args& a) { return a.cols <= 64 ? 6 : 9; }
+
 template <int KIND>
 void launch_tile(const family_args& a, const float* L, const float* R, float* O, uint32_t tile, uint32_t skip_area,
-                 hipStream_t s, const uint32_t* only_if) {
-    if (tile == 0) tile = a.cols <= 64 ? 6 : 9;
+                 hipStream_t s) {
+    if (tile == 0) tile = default_tile(a);
     switch (tile) {
-    case 1: launch<KIND, 4, 1, 128, 4, false, 2>(a, L, R, O, skip_area, s, only_if); break;
-    case 2: launch<KIND, 4, 1, 256, 2, true, 1>(a, L, R, O, skip_area, s, only_if); break;
-    case 3: launch<KIND, 4, 1, 128, 2, true, 1>(a, L, R, O, skip_area, s, only_if); break;
-    case 4: launch<KIND, 4, 1, 128, 8, false, 2>(a, L, R, O, skip_area, s, only_if); break;
-    case 5: launch<KIND, 4, 1, 64, 8, false, 2>(a, L, R, O, skip_area, s, only_if); break;
-    case 6: launch<KIND, 2, 2, 64, 4, false, 2>(a, L, R, O, skip_area, s, only_if); break;
-    case 7: launch<KIND, 4, 1, 128, 8, false, 2, 2>(a, L, R, O, skip_area, s, only_if); break;
-    case 8: launch<KIND, 4, 1, 128, 8, false, 1, 2>(a, L, R, O, skip_area, s, only_if); break;
-    case 9: launch_rows<KIND, 2, 128, 8, 2>(a, L, R, O, skip_area, s, only_if); break;
-    case 10: launch_rows<KIND, 2, 64, 8, 2>(a, L, R, O, skip_area, s, only_if); break;
-    case 11: launch_rows<KIND, 2, 128, 4, 2>(a, L, R, O, skip_area, s, only_if); break;
-    case 12: launch_rows<KIND, 1, 64, 8, 3>(a, L, R, O, skip_area, s, only_if); break;
+    case 1: launch<KIND, 4, 1, 128, 4, false, 2>(a, L, R, O, skip_area, s); break;
+    case 2: launch<KIND, 4, 1, 256, 2, true, 1>(a, L, R, O, skip_area, s); break;
+    case 3: launch<KIND, 4, 1, 128, 2, true, 1>(a, L, R, O, skip_area, s); break;
+    case 4: launch<KIND, 4, 1, 128, 8, false, 2>(a, L, R, O, skip_area, s); break;
+    case 5: launch<KIND, 4, 1, 64, 8, false, 2>(a, L, R, O, skip_area, s); break;
+    case 6: launch<KIND, 2, 2, 64, 4, false, 2>(a, L, R, O, skip_area, s); break;
+    case 7: launch<KIND, 4, 1, 128, 8, false, 2, 2>(a, L, R, O, skip_area, s); break;
+    case 8: launch<KIND, 4, 1, 128, 8, false, 1, 2>(a, L, R, O, skip_area, s); break;
+    case 9: launch_rows<KIND, 2, 128, 8, 2>(a, L, R, O, skip_area, s); break;
+    case 10: launch_rows<KIND, 2, 64, 8, 2>(a, L, R, O, skip_area, s); break;
+    case 11: launch_rows<KIND, 2, 128, 4, 2>(a, L, R, O, skip_area, s); break;
+    case 12: launch_rows<KIND, 1, 64, 8, 3>(a, L, R, O, skip_area, s); break;
     default: fail(XC_ERR_INVALID_ARGUMENT, "tile code " + std::to_string(tile) + " is not in the MFMA tile catalog");
     }
+}
+
+// The default tile, for the batches that mfma_rights_kernel leaves.
+template <int KIND>
+void launch_tile_behind(const family_args& a, const float* L, const float* R, float* O, uint32_t skip_area,
+                        const uint32_t* only_if, hipStream_t s) {
+    if (default_tile(a) == 6)
+        launch<KIND, 2, 2, 64, 4, false, 2, 1, true>(a, L, R, O, skip_area, s, only_if);
+    else
+        launch_rows<KIND, 2, 128, 8, 2, false, true>(a, L, R, O, skip_area, s, only_if);
 }
 
 }  // namespace

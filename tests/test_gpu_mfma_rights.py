@@ -57,3 +57,20 @@ def test_values_that_the_split_does_not_hold(prec, side, value):
     np.testing.assert_array_equal(got, tiles)
     again, _ = run("n_to_m", left, right, prec)
     np.testing.assert_array_equal(again, clean)
+
+
+@pytest.mark.parametrize("prec,value", [("bf16x3", np.nan), ("fp16x3", 1e5)])
+def test_values_that_the_split_does_not_hold_above_64_columns(prec, value):
+    """The same where the default tile is the one of rows kernels."""
+    left = seeded((1, 50, 81), "u11", 75, np.float32)
+    right = seeded((50, 50, 81), "u11", 76, np.float32)
+    clean, kernel = run("one_to_many", left, right, prec)
+    assert kernel == f"mfma_rights_kernel<{prec}>"
+    r = right.copy()
+    r[49, 7, 80] = value
+    got, _ = run("one_to_many", left, r, prec)
+    tiles, kernel = run("one_to_many", left, r, prec, tile=9)
+    assert kernel == f"mfma_rows_kernel<{prec}>"
+    np.testing.assert_array_equal(got, tiles)
+    again, _ = run("one_to_many", left, right, prec)
+    np.testing.assert_array_equal(again, clean)
