@@ -91,26 +91,32 @@ def fft_lengths(H, W, pow2_rows=False):
     return Pr, Pc
 
 
-def kernel_bytes(name, H, W, n, m, k, pow2_rows=False):
+def kernel_bytes(name, H, W, n, m, k, pow2_rows=False, elem=4):
     """Algorithmic HBM bytes of one launch of a kernel of the FFT methods (n left, m right
-    matrices of H x W, k results): every array the kernel must read is read once and every
-    array it must write is written once."""
+    matrices of H x W of `elem` bytes a value, k results): every array the kernel must read is
+    read once and every array it must write is written once."""
     Pr, Pc = fft_lengths(H, W, pow2_rows)
     Kc = Pc // 2 + 1
     SY, SX = 2 * H - 1, 2 * W - 1
-    out = k * SY * SX * 4
+    out = k * SY * SX * elem
     if name == "fftk_rows_fwd":
-        return (n + m) * (H * W * 4 + Kc * H * 16)
+        return (n + m) * (H * W * elem + Kc * H * 16)
     if name == "fftk_cols":
         return m * Kc * H * 16 + n * Kc * Pr * 16 + k * Kc * SY * 16
     if name == "fftk_cols_left":
         return n * (Kc * H * 16 + Kc * Pr * 16)
     if name == "fftk_rows_inv":
         return k * Kc * SY * 16 + out
+    # One-block kernels: half spectra of powers of two from 32 (fftk_small_fits).
+    half = max(32, pow2ceil(2 * H - 1)) * (max(32, pow2ceil(2 * W - 1)) // 2 + 1) * 16
+    if name == "fftk_small_spec":
+        return (n + m) * (H * W * elem + half)
+    if name == "fftk_small_pairs":
+        return (n + m) * half + out
     pr, pc = 2 * H, 2 * W
     spec = pr * (pc // 2 + 1) * 16
     if name == "fft_scatter":
-        return (n + m) * (H * W * 4 + pr * pc * 8)
+        return (n + m) * (H * W * elem + pr * pc * 8)
     if name == "rocfft_forward":
         return (n + m) * (pr * pc * 8 + spec)
     if name == "fft_hadamard":
@@ -341,7 +347,8 @@ def main():
         if "ms_per_step" in a:
             t = kernels_of(lambda: x.cross_corr(family, L, R, out=o, precision="auto"), steps)
             pow2 = line["auto_selected"] == "fft64/2"
-            line["roofline"] = roofline(t, lambda kk: kernel_bytes(kk, H, W, n if fam > 1 else 1, m, k, pow2),
+            line["roofline"] = roofline(t, lambda kk: kernel_bytes(kk, H, W, n if fam > 1 else 1, m, k, pow2,
+                                                                 lnp.itemsize),
                                         lambda kk: 2.0 * k * float(H * W) ** 2)
         if "ms_per_step" in res.get("fp32", {}) and "ms_per_step" in a:
             line["auto_vs_fp32_direct"] = res["fp32"]["ms_per_step"] / a["ms_per_step"]
