@@ -187,7 +187,7 @@ def _raw_stream_getter():
 def _stream(stream):
     global _raw_stream
     if stream is not None:
-        return stream
+        return ctypes.c_void_p(stream)  # a number: strings and bytes would pass as addresses
     if _raw_stream is None:
         _raw_stream = _raw_stream_getter()
     return _raw_stream()

@@ -128,3 +128,12 @@ def test_device_checks_refuse_bad_inputs():
     with pytest.raises(x.XcError, match="torch"):
         x.validate_result(a.numpy(), a)
 
+
+
+@pytest.mark.parametrize("bad", ["default", b"default", 1.0])
+def test_a_stream_is_a_number(bad):
+    """ctypes would pass a string's or bytes' own address as the stream."""
+    with pytest.raises(TypeError):
+        xcorr()._stream(bad)
+    assert xcorr()._stream(4096).value == 4096
+    assert xcorr()._stream(0).value is None
