@@ -630,7 +630,10 @@ bool launch_direct_pairs(const family_args& a, const T* L, const T* R, T* O, hip
     hipLaunchKernelGGL(pairs_copy_left_kernel<T>, dim3(blocks_for(lsize)), dim3(256), 0, s, L, Lc, nl, H, W, k.Hl,
                        k.Wl, TY - 1, padc, flag);
     XC_HIP(hipGetLastError());
-    hipLaunchKernelGGL(pairs_copy_right_kernel<T>, dim3(blocks_for(rsize / 4)), dim3(256), 0, s, R, Rq, nr, a.m,
+    // with a flag it reads the lefts too, of which there may be far more than rights (62544 pairs of 5212
+    // lefts of 1x2 1999 us with blocks for 12 rights only, the tiles 58)
+    const uint64_t copied = std::max(rsize / 4, flag ? lsize / 4 : 0);
+    hipLaunchKernelGGL(pairs_copy_right_kernel<T>, dim3(blocks_for(copied)), dim3(256), 0, s, R, Rq, nr, a.m,
                        a.family == XC_N_TO_MN ? nl : 0u, k.mp, k.mpl, H, W, k.Q4, k.PL, Lc, lsize, flag);
     XC_HIP(hipGetLastError());
     if constexpr (std::is_same<T, float>::value) {
