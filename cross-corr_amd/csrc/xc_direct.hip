@@ -496,14 +496,25 @@ uint64_t pairs_kernel_waves(const family_args& a) {
            ((2 * a.cols - 1 + 3) / 4);
 }
 
+bool one_row_by_pairs(const family_args& a) {
+    return a.rows == 1 && a.cols > 32 && a.cols <= 256 && a.family != XC_N_TO_M;
+}
+
 // Whether the lanes-over-pairs kernel serves this batch by default: at least 48 rights per left
 // (a wave's lanes at least 3/4 busy below 64), its copy of the rights (the other kernels need
-// none) at most 16 GiB, and enough waves.  Double data, and float data with every lane busy: 2048
-// waves (against the register tiles 0.45-0.9x at 128-1024 waves, 1.14x at 2048, 1.6-2.2x from
-// 4096).  Float data with idle lanes competes with the 16 x 16 shifts kernel: a wave's time does
-// not shrink with its pairs, so the line lies at waves * (busy lanes)^3 = 4500, at least 7 lanes
-// in 10 busy.  Measured us, pairs / shifts: 48 of 128^2 869 / 635, 100 of 128^2 1563 / 1287, 4 x 50
-// of 100^2 950 / 1283, 56 of 200^2 3805 / 4499, 80 of 256^2 16620 / 15070, 100 of 256^2 17350 / 18830.
+// none) at most 16 GiB, and enough waves.  Double data: 2048 waves (against the register tiles
+// 0.45-0.9x at 128-1024 waves, 1.14x at 2048, 1.6-2.2x from 4096).  Float data competes with the matrix
+// kernel, whose 16 dx and 16 columns are mostly padding in narrow matrices, and with the 16 x 16 shifts,
+// whose 16 dx are; a wave's time does not shrink with its pairs, so the lines lie at waves * (busy
+// lanes)^3, by columns.  Up to 4 all of 2048 waves (us, pairs / the faster of the two: 20 x 186 of 142x1
+// 80 / 365, 24 x 107 of 305x1 208 / 1064, 28 x 78 of 397x3 743 / 1500, 4 x 218 of 205x3 103 / 191); 5 columns
+// 2000 (51 x 73 of 365x5 1914 / 2260, 323 of 380x5 242 / 221); 6 to 12 4000 (17 x 49 of 283x7 304 / 413, 3 x 78 of
+// 247x8 171 / 98, 113 calls past 4500 0.87 of the time, 2 x 271 of 247x8 285 / 163); 13 to 15 columns none (54 calls
+// 1.4 times).  One row, whose few steps the matrix kernel's four waves share: 33 to 256 columns, rights of
+// one left only and 6000 waves (20253 of 1x37 25 / 31, 39512 of 1x63 68 / 95, 12316 of 1x87 34 / 42, 12400 of
+// 1x38 51 / 24, 3 x 5345 of 1x300 283 / 263, n_to_m 17 x 1056 of 1x98 208 / 59).  The last rule is for batches
+// whose copies are too large for the matrix kernel: against the 16 x 16 shifts 100 of 128^2 1563 / 1287, 4 x 50
+// of 100^2 950 / 1283, 56 of 200^2 3805 / 4499, 80 of 256^2 16620 / 15070.
 bool pairs_kernel_applies(const family_args& a, bool float_data) {
     const uint32_t mpl = rights_per_left(a);
     if (mpl < 48) return false;
@@ -512,8 +523,11 @@ bool pairs_kernel_applies(const family_args& a, bool float_data) {
     const uint64_t copy = slots * a.rows * (a.cols + 24) * sizeof(float);
     if (copy > (16ull << 30)) return false;
     const double busy = (double)mpl / (double)((mpl + 63) / 64 * 64), waves = (double)pairs_kernel_waves(a);
-    if (!float_data || busy == 1.0) return waves >= 2048;
-    return busy >= 0.7 && waves * busy * busy * busy >= 4500;
+    if (!float_data || a.cols <= 4) return waves >= 2048;
+    const double full = waves * busy * busy * busy;
+    if (a.cols <= 12) return full >= (a.cols == 5 ? 2000 : 4000);
+    if (one_row_by_pairs(a)) return waves >= 6000;
+    return busy == 1.0 ? waves >= 2048 : busy >= 0.7 && full >= 4500;
 }
 
 // Whether direct_matrix_kernel serves this float batch by default: its copies of both sides at most 16
@@ -522,9 +536,8 @@ bool pairs_kernel_applies(const family_args& a, bool float_data) {
 // the matrix kernel's also six steps per wave for its start and end, and 0.6 of its longest wave,
 // which small grids wait for.  Measured us, matrix / shifts: 8 of 128^2 127 / 115, 10 of 128^2 127 / 143,
 // 48 of 128^2 298 / 590, 64 of 128^2 380 / 800 (lanes over pairs 898), 16 of 64^2 34 / 27, 32 of 64^2 37 / 47,
-// 20 x 10 of 64^2 149 / 190, 64 of 32^2 18 / 14, 256 of 32^2 28 / 33, 8 of 256^2 1228 / 1552.  Below 16 columns most of
-// its 16 dx and 16 columns are padding: the lanes-over-pairs kernel keeps the batches it serves (200 x 64 of
-// 10^2 59 / 86 us).
+// 20 x 10 of 64^2 149 / 190, 64 of 32^2 18 / 14, 256 of 32^2 28 / 33, 8 of 256^2 1228 / 1552.  Up to
+// 12 columns, and for single rows, the lanes-over-pairs kernel is asked first (200 x 64 of 10^2 59 / 86 us).
 bool matrix_kernel_applies(const family_args& a) {
     const uint32_t mpl = rights_per_left(a);
     if (mpl == 0) return false;
@@ -533,7 +546,7 @@ bool matrix_kernel_applies(const family_args& a) {
     const double H = a.rows, W = a.cols;
     const double copies = slots * H * (W + 27) + lefts * (H + 6) * (W + 55);
     if (copies * sizeof(float) > (double)(16ull << 30) || slots * 64 >= (double)(1u << 31)) return false;
-    if (a.cols < 16 && pairs_kernel_applies(a, true)) return false;
+    if ((a.cols <= 12 || one_row_by_pairs(a)) && pairs_kernel_applies(a, true)) return false;
     const double SX = (2 * a.cols - 1 + 15) / 16 * 16, SY = (2 * a.rows - 1 + 3) / 4 * 4;
     const double SYs = (2 * a.rows - 1 + 15) / 16 * 16;
     const double step = 512 / 2.4e3, waves = groups * (SX / 16) * (SY / 4) * 4;  // us of a step; waves
