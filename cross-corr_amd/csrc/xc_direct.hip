@@ -530,6 +530,15 @@ bool pairs_kernel_applies(const family_args& a, bool float_data) {
     return busy == 1.0 ? waves >= 2048 : busy >= 0.7 && full >= 4500;
 }
 
+bool matrix_copies_fit(const family_args& a) {
+    const uint32_t mpl = rights_per_left(a);
+    if (mpl == 0) return false;
+    const double lefts = a.family == XC_ONE_TO_MANY ? 1 : a.n, H = a.rows, W = a.cols;
+    const double slots = (a.family == XC_N_TO_MN ? lefts : 1) * ((mpl + 15) / 16 * 16);
+    const double copies = slots * H * (W + 27) + lefts * (H + 6) * (W + 55);
+    return copies * sizeof(float) <= (double)(16ull << 30) && slots * 64 < (double)(1u << 31);
+}
+
 // Whether direct_matrix_kernel serves this float batch by default: its copies of both sides at most 16
 // GiB, and a shorter estimated time than the 16 x 16 shifts kernel's.  Both estimates are products
 // issued (the padding of tiles and of groups of 16 rights among them) over a rate, plus the launches;
@@ -540,12 +549,9 @@ bool pairs_kernel_applies(const family_args& a, bool float_data) {
 // 12 columns, and for single rows, the lanes-over-pairs kernel is asked first (200 x 64 of 10^2 59 / 86 us).
 bool matrix_kernel_applies(const family_args& a) {
     const uint32_t mpl = rights_per_left(a);
-    if (mpl == 0) return false;
+    if (!matrix_copies_fit(a)) return false;
     const double lefts = a.family == XC_ONE_TO_MANY ? 1 : a.n, groups = lefts * ((mpl + 15) / 16);
-    const double slots = (a.family == XC_N_TO_MN ? lefts : 1) * ((mpl + 15) / 16 * 16);
     const double H = a.rows, W = a.cols;
-    const double copies = slots * H * (W + 27) + lefts * (H + 6) * (W + 55);
-    if (copies * sizeof(float) > (double)(16ull << 30) || slots * 64 >= (double)(1u << 31)) return false;
     if ((a.cols <= 12 || one_row_by_pairs(a)) && pairs_kernel_applies(a, true)) return false;
     const double SX = (2 * a.cols - 1 + 15) / 16 * 16, SY = (2 * a.rows - 1 + 3) / 4 * 4;
     const double SYs = (2 * a.rows - 1 + 15) / 16 * 16;
@@ -1065,6 +1071,41 @@ bool register_tiles_faster(const family_args& a) {
     return tiles < 1.02 * shifts;
 }
 
+// The kernel for float batches of up to 12 rows with several results per left or right, where the 16 dy of
+// the shifts and the 4 waves of the matrix kernel are partly padding and a call takes little more than its
+// launches: all three times are estimated, in us (the tiles and shifts as above, with the tiles' products
+// per step and the shifts' cost per tile; the matrix kernel from its products and waves), over 1250 shapes of
+// 1 to 32 rows, 1 to 400 columns and up to 300000 results with an error of 16, 8 and 11%.  The choice takes
+// 1.025 times the fastest kernel's time there; without it 1.09, up to 3 times as long as the tiles (us, tiles):
+// 1792 x 3 of 4x53 257 us (tiles 73), 848 x 5 of 5x75 371 (174), 21 x 10 of 1x44 15.4 (7.4), 1098 x 6
+// of 4x19 80 (39), 6 x 793 of 3x7 17.6 (13.7), 14 x 499 of 4x74 61 by the matrix kernel (153).
+enum class few_rows { none, tiles, shifts, matrix };
+few_rows few_rows_choice(const family_args& a) {
+    if (a.rows > 12 || (rights_per_left(a) < 2 && (a.family != XC_N_TO_M || a.n < 2))) return few_rows::none;
+    if ((a.cols <= 12 || one_row_by_pairs(a)) && pairs_kernel_applies(a, true)) return few_rows::none;
+    const direct_plan d = plan_direct<float>(a, xc_options{});
+    const double H = a.rows, W = a.cols, tx = (2 * a.cols - 1 + 15) / 16, ty = (2 * a.rows - 1 + 15) / 16;
+    const double turns = std::ceil(W / 16);
+    const double tile_waves = (double)d.tiles_x * d.tiles_y * d.chunks * d.groups_r * d.groups_l * d.nwx * d.nwy;
+    const uint32_t rows = d.rows_per_chunk ? d.rows_per_chunk : a.rows, steps = (rows + d.t.jb - 1) / d.t.jb;
+    const double tiles = 5.4 + (d.chunks > 1 ? 1.8 : 0.0) + steps * (W + 24) * (d.t.ty * d.t.rm * d.t.lm / 8.0) *
+                                                                (0.041 + 0.077 * std::pow(tile_waves / 4096, 1.1));
+    const double shift_tiles = a.pairs * tx * ty;
+    const int nw = direct_shifts_waves((uint64_t)shift_tiles, a.rows);
+    const uint32_t share = (a.rows + 4 * nw - 1) / (4 * nw), rest = share % 8;
+    const double panel = 3.2 * (share / 8 + (rest > 4)) + (rest > 0 && rest <= 4 ? 2.5 : 0.0);
+    const double shifts = 4.1 + turns * panel + shift_tiles * (0.37e-3 + 1.3e-6 * (H + 60) * (W + 16.5));
+    double matrix = HUGE_VAL;
+    if (matrix_copies_fit(a)) {
+        const double groups = (a.family == XC_ONE_TO_MANY ? 1.0 : a.n) * ((rights_per_left(a) + 15) / 16);
+        const double bands = (2 * a.rows - 1 + 3) / 4, waves = groups * tx * bands * 4;
+        matrix = 13.8 + waves * (256 * (H / 2 + 0.21) * (W / 2 + 8.2) * 2.36e-8 + 0.66e-3) +
+                 0.098 * (H / 4) * std::ceil((W + 15) / 16);
+    }
+    if (tiles < 0.9 * shifts && tiles < matrix) return few_rows::tiles;
+    return shifts < matrix ? few_rows::shifts : few_rows::matrix;
+}
+
 // False (nothing launched) where the grid does not fit one launch.
 bool launch_direct_shifts(const family_args& a, const float* L, const float* R, float* O, hipStream_t s) {
     ds_args k{};
@@ -1106,10 +1147,12 @@ void launch_direct(const family_args& a, const T* L, const T* R, T* O, const xc_
     if (opt.tile == 2 && rights_per_left(a) == 0)
         fail(XC_ERR_UNSUPPORTED, "direct-method tile 2 (lanes over pairs) does not serve one_to_one");
     const bool free_choice = opt.tile == 0 && !keys;
-    if (std::is_same<T, float>::value && free_choice && matrix_kernel_applies(a) &&
+    const few_rows few = std::is_same<T, float>::value && free_choice ? few_rows_choice(a) : few_rows::none;
+    if (std::is_same<T, float>::value && free_choice &&
+        (few == few_rows::none ? matrix_kernel_applies(a) : few == few_rows::matrix) &&
         launch_direct_pairs<T>(a, L, R, O, s, true, false))
         return;
-    if ((opt.tile == 2 || (free_choice && pairs_kernel_applies(a, sizeof(T) == 4))) &&
+    if ((opt.tile == 2 || (free_choice && few == few_rows::none && pairs_kernel_applies(a, sizeof(T) == 4))) &&
         launch_direct_pairs<T>(a, L, R, O, s, false, opt.tile == 2))
         return;
     if (opt.tile == 2) fail(XC_ERR_INVALID_ARGUMENT, "problem too large for one launch");
@@ -1119,8 +1162,9 @@ void launch_direct(const family_args& a, const T* L, const T* R, T* O, const xc_
         // the register tiles: 20x100 29 / 41, 20x300 110 / 109, 20x1000 833 / 676, 40x1000 1970 /
         // 1850, 64x1000 2950 / 4960, 1000x20 640 / 1150; its buffer offsets need matrices below
         // 2^31 bytes.
-        if (free_choice && 16ull * a.rows >= a.cols && (uint64_t)a.rows * a.cols < (1u << 29) &&
-            !register_tiles_faster(a) && launch_direct_shifts(a, L, R, O, s))
+        const bool apt = few == few_rows::shifts ||
+                         (few != few_rows::tiles && 16ull * a.rows >= a.cols && !register_tiles_faster(a));
+        if (free_choice && apt && (uint64_t)a.rows * a.cols < (1u << 29) && launch_direct_shifts(a, L, R, O, s))
             return;
     }
     direct_plan d = plan_direct<T>(a, opt);
