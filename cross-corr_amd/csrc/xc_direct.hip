@@ -1071,24 +1071,25 @@ bool register_tiles_faster(const family_args& a) {
     return tiles < 1.02 * shifts;
 }
 
-// The kernel for float batches of up to 12 rows with several results per left or right, where the 16 dy of
-// the shifts and the 4 waves of the matrix kernel are partly padding and a call takes little more than its
-// launches: all three times are estimated, in us (the tiles and shifts as above, with the tiles' products
-// per step and the shifts' cost per tile; the matrix kernel from its products and waves), over 1250 shapes of
-// 1 to 32 rows, 1 to 400 columns and up to 300000 results with an error of 16, 8 and 11%.  The choice takes
-// 1.025 times the fastest kernel's time there; without it 1.09, up to 3 times as long as the tiles (us, tiles):
-// 1792 x 3 of 4x53 257 us (tiles 73), 848 x 5 of 5x75 371 (174), 21 x 10 of 1x44 15.4 (7.4), 1098 x 6
-// of 4x19 80 (39), 6 x 793 of 3x7 17.6 (13.7), 14 x 499 of 4x74 61 by the matrix kernel (153).
+// The kernel for float batches of several results of up to 12 rows, where the 16 dy of the shifts and the 4
+// waves of the matrix kernel are partly padding and a call may take little more than its launches: all
+// three times are estimated, in us (the tiles and shifts as above, with the tiles' products per step and the
+// shifts' cost per tile; the matrix kernel from its products and waves), over 1650 shapes of 1 to 32 rows,
+// 1 to 400 columns and up to 300000 results with an error of 16, 8 and 11%.  The choice takes 1.025 times the
+// fastest kernel's time there; without it 1.08, up to 3 times as long as the tiles (us, tiles): 1792 x 3 of
+// 4x53 257 (73), 848 x 5 of 5x75 371 (174), 1549 pairs of 10x97 433 (216), 4092 of 2x22 51 (30), 1098 x 6 of 4x19
+// 80 (39), 21 x 10 of 1x44 15.4 (7.4), 6 x 793 of 3x7 17.6 (13.7), 14 x 499 of 4x74 61 by the matrix kernel
+// (153).  With several rights per left the shifts, the more exact ones, keep what they are 10% slower at.
 enum class few_rows { none, tiles, shifts, matrix };
 few_rows few_rows_choice(const family_args& a) {
-    if (a.rows > 12 || (rights_per_left(a) < 2 && (a.family != XC_N_TO_M || a.n < 2))) return few_rows::none;
+    if (a.rows > 12 || a.pairs < 2) return few_rows::none;
     if ((a.cols <= 12 || one_row_by_pairs(a)) && pairs_kernel_applies(a, true)) return few_rows::none;
     const direct_plan d = plan_direct<float>(a, xc_options{});
     const double H = a.rows, W = a.cols, tx = (2 * a.cols - 1 + 15) / 16, ty = (2 * a.rows - 1 + 15) / 16;
     const double turns = std::ceil(W / 16);
     const double tile_waves = (double)d.tiles_x * d.tiles_y * d.chunks * d.groups_r * d.groups_l * d.nwx * d.nwy;
     const uint32_t rows = d.rows_per_chunk ? d.rows_per_chunk : a.rows, steps = (rows + d.t.jb - 1) / d.t.jb;
-    const double tiles = 5.4 + (d.chunks > 1 ? 1.8 : 0.0) + steps * (W + 24) * (d.t.ty * d.t.rm * d.t.lm / 8.0) *
+    const double tiles = 5.4 + (d.chunks > 1 ? 1.8 : 0.0) + steps * (W + 24) * (d.t.ty * d.t.rm * d.t.lm * d.t.jb / 16.0) *
                                                                 (0.041 + 0.077 * std::pow(tile_waves / 4096, 1.1));
     const double shift_tiles = a.pairs * tx * ty;
     const int nw = direct_shifts_waves((uint64_t)shift_tiles, a.rows);
@@ -1102,7 +1103,7 @@ few_rows few_rows_choice(const family_args& a) {
         matrix = 13.8 + waves * (256 * (H / 2 + 0.21) * (W / 2 + 8.2) * 2.36e-8 + 0.66e-3) +
                  0.098 * (H / 4) * std::ceil((W + 15) / 16);
     }
-    if (tiles < 0.9 * shifts && tiles < matrix) return few_rows::tiles;
+    if (tiles < (rights_per_left(a) > 1 ? 0.9 : 1.0) * shifts && tiles < matrix) return few_rows::tiles;
     return shifts < matrix ? few_rows::shifts : few_rows::matrix;
 }
 

@@ -1,6 +1,6 @@
-"""GPU checks of the FP32 direct method's default kernel for batches of up to 12 rows with several rights
-per left, where register tiles, 16 x 16 shifts and the matrix kernel take turns: the kernel taken at shapes
-measured well to either side of the lines, and parity with the CPU oracle (normalised error <= 1e-6)."""
+"""GPU checks of the FP32 direct method's default kernel for batches of up to 12 rows, where the register
+tiles, the 16 x 16 shifts and the matrix kernel take turns: the kernel taken at shapes measured well to
+either side of the lines, and parity with the CPU oracle (normalised error <= 1e-6)."""
 import numpy as np
 import pytest
 
@@ -19,6 +19,8 @@ MATRIX = "direct_pairs_kernel<f32> matrix instructions"
     ("one_to_many", 2, 21, 1, 655, TILES), ("n_to_m", 3, 19, 389, 2, TILES), ("n_to_m", 6, 33, 300, 4, TILES),
     ("n_to_m", 1, 2, 436, 20, TILES), ("one_to_many", 1, 1, 1, 80, SHIFTS), ("n_to_mn", 3, 14, 9, 63, SHIFTS),
     ("n_to_m", 12, 12, 3, 4, SHIFTS), ("one_to_many", 11, 40, 1, 6, SHIFTS), ("n_to_m", 4, 74, 14, 200, MATRIX),
+    ("n_to_mn", 10, 97, 1549, 1549, TILES), ("n_to_mn", 2, 22, 4092, 4092, TILES), ("n_to_mn", 3, 47, 62, 62, TILES),
+    ("n_to_mn", 12, 12, 5, 5, SHIFTS),
     ("one_to_many", 2, 298, 1, 223, MATRIX), ("n_to_m", 12, 100, 4, 100, MATRIX)])
 def test_kernel_and_parity(family, rows, cols, n, m, kernel):
     x = xcorr()
