@@ -1046,14 +1046,15 @@ int ilog2_ceil(uint32_t x) {
 }
 
 // Twiddle tables in device memory of the code object (no allocation): tw[j] =
-// exp(-2 pi i j / 4096) and tw3[j] = exp(-2 pi i j / 12288).  The host computes them and
-// copies them in once per device.
-__device__ double2 g_tw[kSlab];
+// exp(-2 pi i j / 4096), tw[4096 + N + j] = exp(-2 pi i j / N) for N = 2, 4 .. 2048 and j < N (the same
+// values side by side: packed_roots), and tw3[j] = exp(-2 pi i j / 12288).  The host computes them, in long
+// double (the angle rounded to double is up to 4e-16 off), and copies them in once per device.
+__device__ double2 g_tw[2 * kSlab];
 __device__ double2 g_tw3[kTw3];
 
 std::vector<double2> twiddle_values() {
-    std::vector<double2> h(kSlab);
-    const double two_pi = 6.283185307179586476925286766559;
+    std::vector<double2> h(2 * kSlab);
+    const long double two_pi = 6.283185307179586476925286766559005768L;
     for (int j = 0; j < kSlab; ++j) {
         // exact at the eighths of the circle, where cos/sin of the rounded argument are not
         const int oct = j % (kSlab / 8);
@@ -1068,19 +1069,21 @@ std::vector<double2> twiddle_values() {
                                             {0.70710678118654752440, 0.70710678118654752440}};
             h[j] = make_double2(c8[j / (kSlab / 8)][0], c8[j / (kSlab / 8)][1]);
         } else {
-            const double a = two_pi * (double)j / (double)kSlab;
-            h[j] = make_double2(std::cos(a), -std::sin(a));
+            const long double a = two_pi * j / kSlab;
+            h[j] = make_double2((double)std::cos(a), (double)-std::sin(a));
         }
     }
+    for (int n = 2; n < kSlab; n *= 2)
+        for (int j = 0; j < n; ++j) h[packed_roots(n) + j] = h[j * (kSlab / n)];
     return h;
 }
 
 std::vector<double2> twiddle3_values() {
     std::vector<double2> h(kTw3);
-    const double two_pi = 6.283185307179586476925286766559;
+    const long double two_pi = 6.283185307179586476925286766559005768L;
     for (int j = 0; j < kTw3; ++j) {
-        const double a = two_pi * (double)j / (double)kTw3;
-        h[j] = make_double2(std::cos(a), -std::sin(a));
+        const long double a = two_pi * j / kTw3;
+        h[j] = make_double2((double)std::cos(a), (double)-std::sin(a));
     }
     // exact at the twelfths of the circle (the radix-3 and radix-4 points)
     const double s3 = 0.86602540378443864676;
@@ -1110,7 +1113,7 @@ const device_tables& tables_of_device() {
         XC_HIP(hipGetSymbolAddress(reinterpret_cast<void**>(&t.tw), HIP_SYMBOL(g_tw)));
         XC_HIP(hipGetSymbolAddress(reinterpret_cast<void**>(&t.tw3), HIP_SYMBOL(g_tw3)));
         const std::vector<double2> h = twiddle_values(), h3 = twiddle3_values();
-        XC_HIP(hipMemcpy(t.tw, h.data(), sizeof(double2) * kSlab, hipMemcpyHostToDevice));
+        XC_HIP(hipMemcpy(t.tw, h.data(), sizeof(double2) * h.size(), hipMemcpyHostToDevice));
         XC_HIP(hipMemcpy(t.tw3, h3.data(), sizeof(double2) * kTw3, hipMemcpyHostToDevice));
         t.ready = true;
     }

@@ -9,13 +9,15 @@
 
 namespace xc {
 
-// The current device's table of exp(-2 pi i j / 4096), j = 0..4095 (xc_fftk.hip).
+// The current device's table of exp(-2 pi i j / 4096), j = 0..4095, and packed_roots (xc_fftk.hip).
 const double2* fftk_twiddles();
 
 namespace {
 
 constexpr int kLogMaxP = 12;          // longest transform: 4096 (the twiddle table's length)
 constexpr int kSlab = 1 << kLogMaxP;  // twiddle table entries
+// Where the roots of length n = 2, 4 .. 2048 lie side by side behind the table.
+constexpr int packed_roots(int n) { return kSlab + n; }
 
 // LDS slot of element j of transform t (length P = 2^LOGP): one pad slot per 8 values, and a
 // transform stride of 9P/8 + 1 slots, so that lanes touching the same j of consecutive
@@ -159,8 +161,8 @@ __device__ __forceinline__ void regs_sync() {
 //
 // X (double data): more roots of a pass are the table's own.  Powers and rotations of a single root
 // carry its rounding and their own: results of unsigned values of 64^2 were 4.0e-16 off in the 2-norm
-// with one root per pass and are 2.1e-16 off with these (2.3e-16 with a short radix first and powers one
-// by one); n_to_m 16 x 64 of 64^2 50 -> 59 us.  Float results round at 6e-8, where neither shows.
+// with one root per pass and are 2.0e-16 off with these (2.3e-16 with a short radix first and powers one
+// by one); n_to_m 16 x 64 of 64^2 50 -> 60 us.  Float results round at 6e-8, where neither shows.
 template <int LOGP, bool X = false>
 struct regs_roots {
     static constexpr int REM = LOGP % 3;
@@ -172,7 +174,8 @@ struct regs_roots {
 // A pass's further roots with X.  Radix 8: powers 2 to 4 of the root w; radix 2: the root at i + P/8 (w2);
 // radix 4: that and w^2 (w3).  Read where the pass before ends, so that they are in flight during the
 // exchange, whose registers are free: kept from the start of the kernel they spill, and w read here too
-// is waited for (16 x 64 of 64^2 60 us, 64 of 128^2 36.5 -> 39.7).
+// is waited for (64 of 128^2 36.5 -> 39.7 us).  From the tables where a length's roots lie side by side: at the
+// strides of the 4096-point table every lane's root is in a line of its own (50 x 27 of 191x61 609 us, 546 so).
 struct pass_roots {
     double2 w2, w3, w4;
 };
@@ -180,15 +183,15 @@ template <int LOGP, int LOGPP>
 __device__ __forceinline__ pass_roots load_pass_roots(int i, const double2* __restrict__ tw) {
     asm volatile("" : "+v"(i));  // here, not hoisted
     pass_roots x;
+    constexpr int PP = 1 << LOGPP, P = 1 << LOGP;
     if constexpr (LOGP - LOGPP >= 3) {
-        const int e = (i & ((1 << LOGPP) - 1)) << (kLogMaxP - LOGPP - 3);
-        x.w2 = tw[2 * e];
-        x.w4 = tw[4 * e];
-        x.w3 = tw[3 * e];
+        const int e = i & (PP - 1);
+        x.w2 = tw[packed_roots(4 * PP) + e];
+        x.w4 = tw[packed_roots(2 * PP) + e];
+        x.w3 = tw[packed_roots(8 * PP) + 3 * e];
     } else {
-        const int e = i << (kLogMaxP - LOGP);
-        x.w2 = tw[e + kSlab / 8];
-        if constexpr (LOGP - LOGPP == 2) x.w3 = tw[2 * e];
+        x.w2 = tw[packed_roots(P) + P / 8 + i];
+        if constexpr (LOGP - LOGPP == 2) x.w3 = tw[packed_roots(P / 2) + i];
     }
     return x;
 }
