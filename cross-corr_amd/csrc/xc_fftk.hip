@@ -808,6 +808,7 @@ struct rows3 {
     static constexpr int FQ = 3, IQ = 2;                    // and their number: k = 0..N/2
     static_assert(NT % 64 == 0 && NT <= 1024 && (1 << LOGT) == T && 8 * NT == T * P, "rows3 geometry");
     static_assert(FS * FQ > N / 2 && IS * IQ > N / 2, "rows3 steps");
+    static_assert(NT < P || (NT % P == 0 && 2 * T % (NT / P) == 0), "rows3 output rows");
 };
 
 // tw3[j] = exp(-2 pi i j / 12288): the P-th roots for P = 3 * 2^n <= 12288, one table per
@@ -1028,11 +1029,15 @@ __global__ __launch_bounds__(rows3<LOGN>::NT) void rows_inv3_kernel(
     __syncthreads();
     const int SX = 2 * (int)W - 1;
     Tout* Oq = O + (ooff ? ooff[q0 + item] : (size_t)(q0 + item) * (2 * H - 1) * SX);
+    // The block's threads take as many rows at once as they hold P columns: at 48 and 96 points one row
+    // each time leaves most of them idle (527 pairs of 230x18 48 us; 25 before rows went through LDS).
+    constexpr int RP = G::NT >= P ? G::NT / P : 1, TR = G::NT >= P ? P : G::NT;  // rows; threads of each
+    const int zr = (int)threadIdx.x / TR, x0 = (int)threadIdx.x - zr * TR;
 #pragma unroll
-    for (int z = 0; z < 2 * T; ++z) {
-        const int oy = out_row_of_z(z0 + z, H, Ys);
+    for (int z1 = 0; z1 < 2 * T; z1 += RP) {
+        const int z = z1 + zr, oy = out_row_of_z(z0 + z, H, Ys);
         if (oy < 0) continue;
-        for (int ox = (int)threadIdx.x; ox < SX; ox += G::NT) {
+        for (int ox = x0; ox < SX; ox += TR) {
             const int c = ox - ((int)W - 1);
             Oq[(size_t)oy * SX + ox] = rows[z * P + (c < 0 ? c + P : c)];
         }
