@@ -1187,6 +1187,14 @@ struct fftk_geom {
     size_t s_bytes, sl_bytes, col_bytes, z_bytes;  // S per right and per left, Lhat per left, Z per pair
 };
 
+// Whether the one-block kernels serve H x W.  Not 129 to 192 columns, up to 16 rows: rows of 384 points, which
+// they don't have, let the three passes take half the time (one pair of 2x180 24 / 11.5 us, 72 x 13 of 2x150
+// 84 / 38; of 32x512 points at 16x150 25 / 14).
+bool small_serves(uint32_t H, uint32_t W) {
+    const int lr = std::max(5, ilog2_ceil(2 * H - 1)), lc = std::max(5, ilog2_ceil(2 * W - 1));
+    return fftk_small_fits(lr, lc) && (lc < 9 || 2 * W - 1 > 384);
+}
+
 // plain: the layout that takes the least memory per matrix (no one-block kernels, no rounding of
 // the column strides).
 fftk_geom geom_of(uint32_t H, uint32_t W, bool pow2_rows = false, bool plain = false) {
@@ -1222,7 +1230,7 @@ fftk_geom geom_of(uint32_t H, uint32_t W, bool pow2_rows = false, bool plain = f
     g.sl_bytes = g.s_bytes;
     g.logPrs = std::max(5, g.logPr);
     g.logPcs = std::max(5, ilog2_ceil(2 * W - 1));
-    g.small = !plain && fftk_small_fits(g.logPrs, g.logPcs);
+    g.small = !plain && small_serves(H, W);
     if (g.small) {
         g.col_bytes = sizeof(double2) * (size_t)((1u << g.logPcs) / 2 + 1) << g.logPrs;
         g.s_bytes = g.col_bytes;
@@ -1598,8 +1606,8 @@ uint32_t fftk_row_len(uint32_t cols) {
 }
 
 std::pair<uint32_t, uint32_t> fftk_class(uint32_t rows, uint32_t cols) {
-    const int lr = std::max(5, ilog2_ceil(2 * rows - 1)), lc = std::max(5, ilog2_ceil(2 * cols - 1));
-    if (fftk_small_fits(lr, lc)) return {1u << lr, 1u << lc};
+    if (small_serves(rows, cols))
+        return {1u << std::max(5, ilog2_ceil(2 * rows - 1)), 1u << std::max(5, ilog2_ceil(2 * cols - 1))};
     return {fftk_col_len(rows), fftk_row_len(cols)};
 }
 

@@ -110,7 +110,7 @@ constexpr size_t kFftkExtra = size_t(4) << 30;
 uint32_t fftk_col_len(uint32_t rows);
 uint32_t fftk_row_len(uint32_t cols);
 // Matrices of equal fftk_class may share a job: the lengths above, or those of the one-block
-// kernels where they take the size (fftk_small_fits).
+// kernels where they serve the size (small_serves).
 std::pair<uint32_t, uint32_t> fftk_class(uint32_t rows, uint32_t cols);
 void fftk_prepare();  // device tables the kernels read (call before stream capture)
 void fftk_launch_f32(const fftk_job& j, const float* L, const float* R, float* O, const fftk_ws& ws, hipStream_t s);
