@@ -256,7 +256,7 @@ xc_status xc_fft_cross_corr_f32(xc_family family, const float* left, const float
         // Normalised float results come from the own FP64 FFT where it takes the size: the same
         // values with the error of one FP32 rounding (2.5e-8 of the result in the 2-norm; the FP32
         // transforms left 1.5e-7), 4 kernels instead of 8 with rocFFT's.  n_to_m 4 x 16 of 200^2:
-        // 163 us through rocFFT and 74 so; the unnormalised layout needs the 2H x 2W transforms.
+        // 163 us through rocFFT and 68 so; the unnormalised layout needs the 2H x 2W transforms.
         if (normalize && rows <= 2048 && cols <= 2048)
             xc::run_fftk_f32(a, left, right, out, 0, false, (hipStream_t)stream);
         else

@@ -1137,10 +1137,10 @@ bool launch_direct_shifts(const family_args& a, const float* L, const float* R, 
 template <typename T>
 void launch_direct(const family_args& a, const T* L, const T* R, T* O, const xc_options& opt, hipStream_t s) {
     if (a.cols > (uint32_t)kMaxCols) fail(XC_ERR_UNSUPPORTED, "direct kernel: cols above 32768");
-    // tile 0, with no register tile or work distribution requested: float data by the matrix kernel
-    // where it applies, then the lanes-over-pairs kernel where it applies, else (float data) the 16 x
-    // 16 shifts kernel; 1: the register-tile kernel;
-    // 2: the lanes-over-pairs kernel (float and double data alike)
+    // tile 0, with no register tile or work distribution requested: float data of few rows by
+    // few_rows_choice, other by the matrix kernel where it applies, then the lanes-over-pairs kernel where it
+    // applies, else (float data) the 16 x 16 shifts kernel where the tiles are not faster; 1: the
+    // register-tile kernel; 2: the lanes-over-pairs kernel (float and double data alike)
     if (opt.tile > 2)
         fail(XC_ERR_INVALID_ARGUMENT, "direct-method tile must be 0 (default), 1 (register tiles) or 2 (lanes over pairs)");
     const bool keys = opt.shifts_per_thread || opt.right_mats_per_thread || opt.left_mats_per_thread ||

@@ -387,7 +387,10 @@ xc_status xc_kernel_timing(int enable);
 xc_status xc_kernel_times(char* buf, size_t len, size_t* needed);
 
 const char* xc_last_error(void);             /* thread-local; "" if none */
-const xc_launch_desc* xc_last_launch(void);  /* thread-local; last launch this thread enqueued */
+/* Thread-local: the launch that the last call of this thread enqueued.  `kernel` labels the path that was
+ * chosen: data with infinities or NaNs may have been computed by a kernel enqueued behind it, and a launch
+ * of many small pairs may have been one of several. */
+const xc_launch_desc* xc_last_launch(void);
 const char* xc_version(void);
 /* Describe the device the library runs on (name, CUs, clock); returns XC_ERR_HIP without a GPU. */
 xc_status xc_device_info(char* buf, size_t len);
