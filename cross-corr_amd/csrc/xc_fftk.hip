@@ -393,6 +393,12 @@ __device__ __forceinline__ bool z_gap(uint32_t z0, uint32_t rows, uint32_t H, ui
 // Threads per block of the column kernel: one wave for wave-owned register transforms (up to
 // 512 points; C = 512 / Pr columns per block, so that a pair's last column group wastes at
 // most a wave), 256 for the block-owned and slab transforms.
+// Rows of each half of a column of Z that are stored: whole 128-byte lines, with outputs of the transform that
+// nothing reads past the result's.  Partly written lines are read back first where Z does not stay in the
+// Infinity Cache (8 x 67 of 100x200: cols 143 -> 131 us, rows_inv 157 -> 142; of 100x420 322 -> 283, 280 -> 267; whole
+// 64-byte sectors only 316 and 278).
+__device__ __forceinline__ uint32_t z_lines(uint32_t rows, uint32_t Ys) { return min((rows + 7) & ~7u, Ys / 2); }
+
 constexpr int cols_threads(int logP) { return logP <= 9 ? 64 : kFT; }
 
 // cols: block (item, group of C columns k).  mode 0: item = left matrix l, writes its full
@@ -403,7 +409,7 @@ constexpr int cols_threads(int logP) { return logP <= 9 ? 64 : kFT; }
 // table of an uneven batch): X = the same FFT of SR[r][k], then a second FFT of
 // conj(Lhat) * X: the conjugate of Pr * IFFT_rho(Lhat * conj(X)), whose circular row rho goes to
 // Z[item][k][z_row(rho)] (column stride Ys; the rows between the result's two halves are
-// dropped).
+// dropped, but for those of a line that has result rows: z_lines).
 // Blocks are ordered column-group major through the XCD remap, so the pairs that read the
 // same Lhat columns run on one XCD and find them in its L2.
 // cols_group: block (group of C columns k, G consecutive pairs from q0 + item G): the columns of
@@ -474,12 +480,13 @@ __global__ __launch_bounds__(cols_threads(LOGPR)) void cols_group_kernel(
         fft_regs<LOGPR>(u, wb, rr, tl, i);
         // z_row: rows below Hq (s < 4: Hq <= Pr / 2) in place, rows above Pr - Hq (s >= 4) down by
         // Pr - Ys
+        const uint32_t whole = z_lines(rows, Ys);
         const __amdgpu_buffer_rsrc_t rz = buf_of(Z + (size_t)p * Kc * Ys, Kc * Ys * 16u);
         const uint32_t zlo = (k * Ys + (uint32_t)i) * 16u, zhi = zlo - ((uint32_t)P - Ys) * 16u;
 #pragma unroll
         for (int s = 0; s < 8; ++s) {
             const uint32_t rho = (uint32_t)(i + Q * s);
-            const bool in = s < 4 ? rho < rows : rho + rows > (uint32_t)P;
+            const bool in = s < 4 ? rho < whole : rho + whole >= (uint32_t)P;
             buf_store(u[s], rz, in ? (s < 4 ? zlo : zhi) + 16u * Q * s : kOut, 0);
         }
     }
@@ -548,12 +555,13 @@ __global__ __launch_bounds__(cols_threads(LOGPR)) void cols_kernel(const double2
         fft_regs<LOGPR>(u, wb, rr, tl2, i2);
         // z_row: rows below Hq (r < 4: Hq <= Pr / 2) in place, rows above Pr - Hq (r >= 4) down by
         // Pr - Ys; indices from the opaque i2, so that those of the loads are not kept live.
+        const uint32_t whole = z_lines(rows, Ys);
         const __amdgpu_buffer_rsrc_t rz = buf_of(Z + (size_t)item * Kc * Ys, Kc * Ys * 16u);
         const uint32_t zlo = (k * Ys + (uint32_t)i2) * 16u, zhi = zlo - ((uint32_t)P - Ys) * 16u;
 #pragma unroll
         for (int r = 0; r < 8; ++r) {
             const uint32_t rho = (uint32_t)(i2 + Q * r);
-            const bool in = r < 4 ? rho < rows : rho + rows > (uint32_t)P;
+            const bool in = r < 4 ? rho < whole : rho + whole >= (uint32_t)P;
             buf_store(u[r], rz, in ? (r < 4 ? zlo : zhi) + 16u * Q * r : kOut, 0);
         }
         return;
