@@ -396,8 +396,15 @@ __device__ __forceinline__ bool z_gap(uint32_t z0, uint32_t rows, uint32_t H, ui
 // Rows of each half of a column of Z that are stored: whole 128-byte lines, with outputs of the transform that
 // nothing reads past the result's.  Partly written lines are read back first where Z does not stay in the
 // Infinity Cache (8 x 67 of 100x200: cols 143 -> 131 us, rows_inv 157 -> 142; of 100x420 322 -> 283, 280 -> 267; whole
-// 64-byte sectors only 316 and 278).
-__device__ __forceinline__ uint32_t z_lines(uint32_t rows, uint32_t Ys) { return min((rows + 7) & ~7u, Ys / 2); }
+// 64-byte sectors only 316 and 278).  From 64 rows; of few rows the lines' rest is most of them (72 x 13 of 2x150
+// 37.5 -> 42.8).
+__device__ __forceinline__ uint32_t z_lines(uint32_t rows, uint32_t Ys) {
+    return rows < 64 ? rows : min((rows + 7) & ~7u, Ys / 2);
+}
+// The first row rho of the second half that is stored.
+__device__ __forceinline__ uint32_t z_second(uint32_t rows, uint32_t whole, uint32_t P) {
+    return rows < 64 ? P - rows + 1 : P - whole;
+}
 
 constexpr int cols_threads(int logP) { return logP <= 9 ? 64 : kFT; }
 
@@ -480,13 +487,13 @@ __global__ __launch_bounds__(cols_threads(LOGPR)) void cols_group_kernel(
         fft_regs<LOGPR>(u, wb, rr, tl, i);
         // z_row: rows below Hq (s < 4: Hq <= Pr / 2) in place, rows above Pr - Hq (s >= 4) down by
         // Pr - Ys
-        const uint32_t whole = z_lines(rows, Ys);
+        const uint32_t whole = z_lines(rows, Ys), second = z_second(rows, whole, P);
         const __amdgpu_buffer_rsrc_t rz = buf_of(Z + (size_t)p * Kc * Ys, Kc * Ys * 16u);
         const uint32_t zlo = (k * Ys + (uint32_t)i) * 16u, zhi = zlo - ((uint32_t)P - Ys) * 16u;
 #pragma unroll
         for (int s = 0; s < 8; ++s) {
             const uint32_t rho = (uint32_t)(i + Q * s);
-            const bool in = s < 4 ? rho < whole : rho + whole >= (uint32_t)P;
+            const bool in = s < 4 ? rho < whole : rho >= second;
             buf_store(u[s], rz, in ? (s < 4 ? zlo : zhi) + 16u * Q * s : kOut, 0);
         }
     }
@@ -555,13 +562,13 @@ __global__ __launch_bounds__(cols_threads(LOGPR)) void cols_kernel(const double2
         fft_regs<LOGPR>(u, wb, rr, tl2, i2);
         // z_row: rows below Hq (r < 4: Hq <= Pr / 2) in place, rows above Pr - Hq (r >= 4) down by
         // Pr - Ys; indices from the opaque i2, so that those of the loads are not kept live.
-        const uint32_t whole = z_lines(rows, Ys);
+        const uint32_t whole = z_lines(rows, Ys), second = z_second(rows, whole, P);
         const __amdgpu_buffer_rsrc_t rz = buf_of(Z + (size_t)item * Kc * Ys, Kc * Ys * 16u);
         const uint32_t zlo = (k * Ys + (uint32_t)i2) * 16u, zhi = zlo - ((uint32_t)P - Ys) * 16u;
 #pragma unroll
         for (int r = 0; r < 8; ++r) {
             const uint32_t rho = (uint32_t)(i2 + Q * r);
-            const bool in = r < 4 ? rho < whole : rho + whole >= (uint32_t)P;
+            const bool in = r < 4 ? rho < whole : rho >= second;
             buf_store(u[r], rz, in ? (r < 4 ? zlo : zhi) + 16u * Q * r : kOut, 0);
         }
         return;
