@@ -1204,10 +1204,14 @@ struct fftk_geom {
 
 // Whether the one-block kernels serve H x W.  Not 129 to 192 columns, up to 16 rows: rows of 384 points, which
 // they don't have, let the three passes take half the time (one pair of 2x180 24 / 11.5 us, 72 x 13 of 2x150
-// 84 / 38; of 32x512 points at 16x150 25 / 14).
+// 84 / 38; of 32x512 points at 16x150 25 / 14).  Nor 65 to 96 columns, up to 8 rows, padded to 32x256 instead of
+// 16x192 points (926 of 1x73 45 / 26, 446 of 3x71 35 / 22, one of 5x90 14.5 / 13.2, 20 x 50 of 8x96 33 / 33; with
+// more rows pairs that share their matrices lose: 16 x 64 of 20x80 42.5 / 47.5, 30 x 60 of 32x96 78 / 90).
 bool small_serves(uint32_t H, uint32_t W) {
     const int lr = std::max(5, ilog2_ceil(2 * H - 1)), lc = std::max(5, ilog2_ceil(2 * W - 1));
-    return fftk_small_fits(lr, lc) && (lc < 9 || 2 * W - 1 > 384);
+    if (lc == 9 && 2 * W - 1 <= 384) return false;
+    if (lc == 8 && 2 * W - 1 <= 192 && H <= 8) return false;
+    return fftk_small_fits(lr, lc);
 }
 
 // plain: the layout that takes the least memory per matrix (no one-block kernels, no rounding of

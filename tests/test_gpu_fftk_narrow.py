@@ -30,7 +30,8 @@ def test_parity(rows, cols, dtype, tol):
 
 @pytest.mark.parametrize("dtype,tol", [(np.float32, 1e-6), (np.float64, 1e-9)])
 @pytest.mark.parametrize("rows,cols,small", [(1, 128, True), (1, 129, False), (16, 129, False), (9, 192, False),
-                                             (2, 193, True), (16, 193, True), (17, 150, False)])
+                                             (2, 193, True), (16, 193, True), (17, 150, False)]
+                         + [(8, 64, True), (8, 65, False), (1, 96, False), (9, 65, True), (8, 97, True)])
 def test_flat(rows, cols, small, dtype, tol):
     left, right = seeded((2, rows, cols), "u11", 63, dtype), seeded((3, rows, cols), "u01", 64, dtype)
     x = xcorr()
